@@ -184,11 +184,21 @@ __device__ __forceinline__ void density_column(const KArgs& a, const NoiseLds& T
     }
 }
 
-// Wave-level work queue: lane 0 takes the next 64-element item, all lanes get it.
-__device__ __forceinline__ int next_item(int* queue) {
-    int item = 0;
-    if ((threadIdx.x & 63) == 0) item = atomicAdd(queue, 1);
-    return __shfl(item, 0);
+// Items of the crossing kernels: wave w of the grid starts with grab w (`per_grab`
+// consecutive items), without the queue, and takes later grabs from the atomic counter.
+// One counter serves about 77 grabs per us, so when every wave of a full grid (3,072 for
+// one chunk) took its first, mostly failing, grab there, that alone was 40 us.  Waves are
+// numbered across the workgroups, so the few items of a small chunk spread over the CUs.
+__device__ __forceinline__ int grid_waves() { return (int)(gridDim.x * (blockDim.x >> 6)); }
+__device__ __forceinline__ int first_grab(int per_grab) {
+    return ((int)(threadIdx.x >> 6) * (int)gridDim.x + (int)blockIdx.x) * per_grab;
+}
+__device__ __forceinline__ int next_grab(int* queue, int per_grab, int total) {
+    const int given = grid_waves() * per_grab;  // the waves' first grabs
+    if (given >= total) return total;
+    int at = 0;
+    if ((threadIdx.x & 63) == 0) at = atomicAdd(queue, per_grab);
+    return given + __shfl(at, 0);
 }
 
 // Items of a persistent kernel shared within the workgroup: workgroup b owns items b,
@@ -895,21 +905,17 @@ template <bool kCount>
 __global__ __attribute__((amdgpu_waves_per_eu(6, 8))) __launch_bounds__(kCrossThreads) void k_edge_cross(KArgs a,
                                                                                                           int chunks) {
     __shared__ NoiseLds T;
-    load_noise_tables(T, a.perm, a.grads);
     const int total = a.item_prefix[chunks];
-    const int lane = threadIdx.x & 63;
     // One global queue (sharing items within workgroups instead measured slower: clipmap
     // 93.2 -> 94.5 ms).  A grab takes up to 4 consecutive items, as many as still leave
     // every wave 8 grabs: one counter serves ~77,000 grabs per ms, which items of a few
     // microseconds (a heightfield's y-edges) would otherwise wait on, and the chunk of
     // an item is found by one search per grab, the grab's later items walking forward.
-    const int waves = (int)(gridDim.x * (blockDim.x >> 6));
-    const int per_grab = max(1, min(4, total / (8 * waves)));
-    for (;;) {
-        int first = 0;
-        if (lane == 0) first = atomicAdd(&a.queue[1], per_grab);
-        first = __shfl(first, 0);
-        if (first >= total) break;
+    const int per_grab = max(1, min(4, total / (8 * grid_waves())));
+    if ((int)blockIdx.x * per_grab >= total) return;  // no wave of this workgroup has an item
+    load_noise_tables(T, a.perm, a.grads);
+    const int lane = threadIdx.x & 63;
+    for (int first = first_grab(per_grab); first < total; first = next_grab(&a.queue[1], per_grab, total)) {
         const int end = min(first + per_grab, total);
         int lo = 0, hi = chunks;  // last chunk with item_prefix[c] <= first
         while (hi - lo > 1) {
@@ -1056,13 +1062,12 @@ template <bool kCount, int kG>
 __global__ __attribute__((amdgpu_waves_per_eu(6, 8))) __launch_bounds__(kCrossThreads) void k_edge_cross_group(
     KArgs a, int chunks) {
     __shared__ NoiseLds T;
-    load_noise_tables(T, a.perm, a.grads);
     constexpr int kPerItem = 64 / kG;
     const int total = a.item_prefix[chunks];
+    if ((int)blockIdx.x >= total) return;  // no wave of this workgroup has an item
+    load_noise_tables(T, a.perm, a.grads);
     const int lane = threadIdx.x & 63;
-    for (;;) {
-        const int item = next_item(&a.queue[1]);
-        if (item >= total) break;
+    for (int item = first_grab(1); item < total; item = next_grab(&a.queue[1], 1, total)) {
         int lo = 0, hi = chunks;  // last chunk with item_prefix[c] <= item
         while (hi - lo > 1) {
             const int mid = (lo + hi) >> 1;
@@ -1111,8 +1116,9 @@ __global__ __attribute__((amdgpu_waves_per_eu(6, 8))) __launch_bounds__(kCrossTh
     __shared__ NoiseLds T;
     __shared__ int sp_k[kSpWaves][64];    // per wave: kbest of each edge of the item
     __shared__ float sp_h[kSpWaves][64];  // and the height term there
-    load_noise_tables(T, a.perm, a.grads);
     const int total = a.item_prefix[chunks];
+    if ((int)blockIdx.x >= total) return;  // no wave of this workgroup has an item
+    load_noise_tables(T, a.perm, a.grads);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int row = lane >> 4, sub = lane & 15;
     const FieldParams& Fp = a.F;
@@ -1120,9 +1126,7 @@ __global__ __attribute__((amdgpu_waves_per_eu(6, 8))) __launch_bounds__(kCrossTh
     const bool ends = !a.fp16;
     const Geometry& G = a.G;
     unsigned nh = 0, nc = 0, ne = 0;
-    for (;;) {
-        const int item = next_item(&a.queue[1]);
-        if (item >= total) break;
+    for (int item = first_grab(1); item < total; item = next_grab(&a.queue[1], 1, total)) {
         int lo = 0, hi = chunks;  // last chunk with item_prefix[c] <= item
         while (hi - lo > 1) {
             const int mid = (lo + hi) >> 1;
