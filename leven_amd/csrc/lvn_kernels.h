@@ -26,7 +26,7 @@ struct KArgs {
     int precise;             // QEF: compensated FP32 sums + FP64 re-solve
     unsigned long long* work;  // optional work counters (see lvn_batch_work), else null
     int* queue;              // kNumQueues work-queue heads, zeroed by launch_clear_counters
-    int* item_prefix;        // chunks + 1 edge-item offsets (k_edge_items)
+    int* item_prefix;        // chunks + 1 edge-item offsets (k_edge_data)
     int cus;                 // compute units of the device
     int persist_per_cu;      // persistent workgroups per CU (edge crossing)
     int density_per_cu;      // persistent workgroups per CU (density)
