@@ -29,7 +29,7 @@ struct KArgs {
     int* item_prefix;        // chunks + 1 edge-item offsets (k_edge_data)
     int cus;                 // compute units of the device
     int persist_per_cu;      // persistent workgroups per CU (edge crossing)
-    int density_per_cu;      // persistent workgroups per CU (density)
+    int density_per_cu;      // persistent workgroups per CU (density), 0 = by the number of items
     int height_lines;        // 1: x/z-edge sample heights evaluated once per line (k_height_lines)
     const int* slot_map;     // batch entry -> arena slot, or null for the identity
     int row_blocks;          // workgroups over the batch for the bookkeeping kernels
@@ -67,6 +67,10 @@ void launch_voxel_compact(const KArgs& a, int chunks, hipStream_t s);
 void launch_qef(const KArgs& a, int chunks, hipStream_t s);
 void launch_emit(const KArgs& a, int chunks, hipStream_t s);
 
+// y-segments per density column when the launch shapes leave it open.
+int default_ysplit(const Geometry& G, int field_kind, int chunks);
+// Density workgroups per CU when the launch shapes leave it open.
+int default_density_per_cu(const Geometry& G, int ysplit, int chunks, int cus);
 // Lanes per edge in the crossing stage when the launch shapes leave it open.
 int default_cross_lanes(int chunks);
 // cross_lanes value of the sample-parallel crossing kernel (16 lanes per edge in the

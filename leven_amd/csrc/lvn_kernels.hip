@@ -2165,11 +2165,32 @@ static unsigned persistent_blocks(const KArgs& a, int per_cu, long items) {
     return (unsigned)std::max(1L, std::min((long)per_cu * a.cus, (items + 15) / 16));
 }
 
+// A column item evaluates the height term once and then its y-segment.  With the cave term
+// the segment is the cost (a 66-sample column is 0.18 ms of dependent octaves), so few
+// chunks are cut finely, down to two samples, until about 20,000 items fill the chip, and
+// never below three segments, which balance caves against sky; without it each segment
+// repeats the whole height term, so a cut pays only until about 3,400 items are in flight.
+// Measured (density stage, us; caves / reference terrain): one chunk 39 / 14 with 6
+// segments, 16 / 12 with these; 8 chunks 51 / 17 -> 40 / 17; 24 chunks 83 / 29 -> 74 / 24;
+// 96 chunks 347 / 54 -> 216 / 46; 500 chunks 1,087 / 202 -> 914 / 156 (with the workgroups
+// below).
+int default_ysplit(const Geometry& G, int field_kind, int chunks) {
+    const long items = (long)G.col_groups * std::max(1, chunks);
+    if (field_kind == LVN_FIELD_TERRAIN_CAVES) return (int)std::clamp(20000L / items, 3L, (long)G.F / 2);
+    return (int)std::clamp(3400L / items, 1L, std::min(11L, (long)G.F / 2));
+}
+// Two workgroups per CU once one per CU has every wave busy (500 chunks: 1,040 -> 914 us
+// with caves, 202 -> 156 without); below that a second one only loads tables.
+int default_density_per_cu(const Geometry& G, int ysplit, int chunks, int cus) {
+    return (long)G.col_groups * ysplit * chunks > 16L * cus ? 2 : 1;
+}
+
 void launch_density(const KArgs& a, int chunks, hipStream_t s) {
     const long items = (long)a.G.col_groups * a.ysplit * chunks;
-    // One workgroup per CU by default (density_per_cu); the tuner tries two, which the
-    // kernel's register caps let a CU hold at once.
-    const unsigned blocks = persistent_blocks(a, a.density_per_cu, items);
+    // density_per_cu workgroups per CU (two fit, by the kernel's register caps), or one per
+    // item where there are fewer items than that.
+    const int per_cu = a.density_per_cu ? a.density_per_cu : default_density_per_cu(a.G, a.ysplit, chunks, a.cus);
+    const unsigned blocks = (unsigned)std::max(1L, std::min((long)per_cu * a.cus, items));
     if (a.work)
         hipLaunchKernelGGL(k_density<true>, dim3(blocks), dim3(1024), 0, s, a, chunks);
     else
@@ -2211,7 +2232,7 @@ static int cross_lanes(const KArgs& a, int chunks) {
     return a.cross_lanes > 0 ? a.cross_lanes : default_cross_lanes(chunks);
 }
 
-constexpr int kEdgeDataBlocks = 256;
+constexpr int kEdgeDataBlocks = 1024;
 
 template <int kG>
 static void launch_cross_group(const KArgs& a, int chunks, hipStream_t s) {

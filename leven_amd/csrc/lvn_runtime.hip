@@ -353,7 +353,6 @@ KArgs make_kargs(char* arena, const SlotLayout& L, const Geometry& G, const Caps
     a.item_prefix = item_prefix;
     a.cus = cus;
     a.persist_per_cu = kDefaultPersistPerCu;
-    a.density_per_cu = kDefaultDensityPerCu;
     a.height_lines = 0;
     a.row_blocks = kDefaultRowBlocks;
     a.voxel_blocks = kDefaultVoxelBlocks;
@@ -458,10 +457,10 @@ static void set_cached(ChunkDesc& cd, const FieldEntry* cached) {
     cd.old_mat = (uint64_t)(uintptr_t)cached->d_mat;
 }
 
-// Launch shapes of the one-chunk forms: split density columns 6 ways.
+// Launch shapes of the one-chunk forms.
 static KArgs single_args(const Ctx* c) {
     KArgs a = c->kargs();
-    a.ysplit = 6;
+    a.ysplit = default_ysplit(a.G, a.F.kind, 1);
     return a;
 }
 
@@ -647,13 +646,13 @@ static int stage_batch(Batch* b, int n, const lvn_chunk_req* reqs) {
     return LVN_OK;
 }
 
-// The batch's launch shapes with the automatic column split resolved: small batches
-// split the density columns to fill the GPU.
+// The batch's launch shapes with the automatic ones resolved.
 static lvn_tuning effective_tuning(const Batch* b) {
     lvn_tuning t = b->tuning;
-    if (t.density_ysplit == 0) t.density_ysplit = b->n >= 64 ? 1 : 6;
+    if (t.density_ysplit == 0) t.density_ysplit = default_ysplit(b->ctx.G, g_state.fp.kind, b->n);
     if (t.cross_lanes == 0) t.cross_lanes = default_cross_lanes(b->n);
-    if (t.density_per_cu == 0) t.density_per_cu = kDefaultDensityPerCu;
+    if (t.density_per_cu == 0)
+        t.density_per_cu = default_density_per_cu(b->ctx.G, t.density_ysplit, b->n, b->ctx.cus);
     if (t.height_lines == 0) t.height_lines = b->n >= kHeightLinesMinChunks ? 2 : 1;
     return t;
 }
@@ -1069,7 +1068,7 @@ int lvn_generate_chunk_mesh_noalloc(int32_t n, uint32_t flags, const int32_t min
                          reinterpret_cast<Counters*>(base + t.counters), reinterpret_cast<const DevOp*>(base + t.ops),
                          reinterpret_cast<const int*>(base + t.index), flags, reinterpret_cast<int*>(base + t.queue),
                          reinterpret_cast<int*>(base + t.prefix), d.cus);
-    a.ysplit = 6;  // the one-chunk forms' density column split (single_args)
+    a.ysplit = default_ysplit(a.G, a.F.kind, 1);  // as the other one-chunk form (single_args)
     launch_pipeline(a, 1, st);
     LVN_HIP(hipGetLastError());
     LVN_HIP(hipMemcpyAsync(&k, base + t.counters, sizeof(Counters), hipMemcpyDeviceToHost, st));

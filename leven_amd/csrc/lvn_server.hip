@@ -94,7 +94,7 @@ struct Server {
     int error = LVN_OK;
 
     std::mutex tuning_mu;          // launch shapes (lvn_server_set_tuning), read at each launch
-    lvn_tuning tuning = {0, kDefaultPersistPerCu, kDefaultRowBlocks, kDefaultVoxelBlocks, 0, kDefaultDensityPerCu, 0, {0}};
+    lvn_tuning tuning = {0, kDefaultPersistPerCu, kDefaultRowBlocks, kDefaultVoxelBlocks, 0, 0, 0, {0}};
 
     std::mutex cache_mu;           // cache, ticket_key and stats (read by lvn_server_get_mesh / _stats)
     std::map<Key, Entry> cache;
@@ -371,10 +371,10 @@ int Server::launch(Lane& L, const std::vector<Job>& batch, const std::vector<int
     a.dens_cols = a.F.kind != LVN_FIELD_TERRAIN_CAVES && !a.fp16 ? 1 : 0;
     a.mat_free = 1;  // and chunks without brushes their materials
     // zero fields: the automatic choice by batch size
-    a.ysplit = t.density_ysplit ? t.density_ysplit : n >= 32 ? 1 : 6;
+    a.ysplit = t.density_ysplit ? t.density_ysplit : default_ysplit(a.G, a.F.kind, n);
     a.height_lines = t.height_lines ? (t.height_lines == 2 ? 1 : 0) : (n >= kHeightLinesMinChunks ? 1 : 0);
     a.persist_per_cu = t.persistent_per_cu;
-    a.density_per_cu = t.density_per_cu ? t.density_per_cu : kDefaultDensityPerCu;
+    a.density_per_cu = t.density_per_cu;
     a.row_blocks = t.row_blocks;
     a.voxel_blocks = t.voxel_blocks;
     a.cross_lanes = t.cross_lanes;
