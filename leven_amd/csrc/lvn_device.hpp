@@ -78,6 +78,8 @@ __device__ __forceinline__ float recip_1_2(float d) {
     return fmaf(fmaf(-d, q1, 1.f), r1, q1);
 }
 
+__device__ __forceinline__ float clamp01(float v) { return fminf(fmaxf(v, 0.f), 1.f); }
+
 // One snoise2 corner (cl/simplex.cl:123-153).  The squared distance and the
 // gradient dot product are fused multiply-adds, as the restatement defines them
 // (the reference's -cl-fast-relaxed-math build, src/compute.cpp:213, allows it).
@@ -87,7 +89,7 @@ __device__ __forceinline__ float recip_1_2(float d) {
 // every noise value feeds either fBm's fma chain, which starts at +0 (a zero noise
 // value then adds +0 to a sum that is never -0), or the ridged form's fabsf.
 __device__ __forceinline__ float corner2(const NoiseLds& T, int texel, float fx, float fy) {
-    const float r = fmaxf(0.5f - fmaf(fy, fy, fx * fx), 0.f);
+    const float r = clamp01(0.5f - fmaf(fy, fy, fx * fx));
     const float2 g = T.gxy[T.perm[texel] & 15];
     const float t = r * r;
     return (t * t) * fmaf(g.y, fy, g.x * fx);
@@ -120,7 +122,7 @@ __device__ __forceinline__ float snoise2(const NoiseLds& T, float px, float py) 
 // r is clamped at +0 as in corner2.
 __device__ __forceinline__ float corner3(const NoiseLds& T, int texel, int zrow, float fx, float fy, float fz) {
     const int w = T.perm[texel];
-    const float r = fmaxf(0.6f - fmaf(fz, fz, fmaf(fy, fy, fx * fx)), 0.f);
+    const float r = clamp01(0.6f - fmaf(fz, fz, fmaf(fy, fy, fx * fx)));
     const int j = T.perm[zrow + w] & 15;
     const float2 g = T.gxy[j];
     const float t = r * r;
@@ -189,7 +191,6 @@ __device__ __forceinline__ float fbm3(const NoiseLds& T, int octaves, float freq
     return n;
 }
 
-__device__ __forceinline__ float clamp01(float v) { return fminf(fmaxf(v, 0.f), 1.f); }
 
 // RidgedMultiFractal, cl/noise.cl:42-81 (pow(f, -1) as 1 / f).
 __device__ __forceinline__ float ridged(const NoiseLds& T, int octaves, float lac, float gain, float offset, float x,
@@ -224,9 +225,19 @@ __device__ __forceinline__ float leven_terrain(const NoiseLds& T, float x, float
     return n + b2;
 }
 
+// A kernel's field kind: its template argument, or the descriptor's in the kernels that
+// are not timed (kAnyField).  A kernel built for one kind holds no other kind's code, whose
+// live values cost it scalar registers.
+constexpr int kAnyField = -1;
+template <int kKind>
+__device__ __forceinline__ int field_kind(const FieldParams& F) {
+    return kKind == kAnyField ? F.kind : kKind;
+}
+
 // Height term H(x, z) of every field kind: density = y - H (cl/noise.cl:265-266).
+template <int kKind>
 __device__ __forceinline__ float height_term(const FieldParams& F, const NoiseLds& T, float x, float z) {
-    if (F.kind == LVN_FIELD_LEVEN_TERRAIN) return 900.f * leven_terrain(T, x, z);
+    if (field_kind<kKind>(F) == LVN_FIELD_LEVEN_TERRAIN) return 900.f * leven_terrain(T, x, z);
     return F.hamp * fbm2(T, F.hoct, F.hfreq, F.hlac, F.hgain, x, z);
 }
 
@@ -238,14 +249,199 @@ __device__ __forceinline__ float cave_term(const FieldParams& F, const NoiseLds&
 // density = max(a, cave) with a = y - H.  The cave term is bounded by F.cave_cut
 // (|snoise3| <= 1.19 times the sum of octave amplitudes, minus the threshold);
 // when a exceeds it, max(a, cave) == a exactly and the cave term is skipped.
+template <int kKind>
 __device__ __forceinline__ float combine(const FieldParams& F, const NoiseLds& T, float a, float x, float y, float z) {
-    if (F.kind != LVN_FIELD_TERRAIN_CAVES || a > F.cave_cut) return a;
+    if (field_kind<kKind>(F) != LVN_FIELD_TERRAIN_CAVES || a > F.cave_cut) return a;
     return fmaxf(a, cave_term(F, T, x, y, z));
 }
 
-__device__ __forceinline__ float density(const FieldParams& F, const NoiseLds& T, float x, float y, float z) {
-    const float a = y - height_term(F, T, x, z);
-    return combine(F, T, a, x, y, z);
+// ---------------------------------------------------------------------------
+// leven's height term at the four points of a central difference, (x + h, z), (x - h, z),
+// (x, z + h), (x, z - h).  They lie 0.002 apart, so at almost every octave all four of a
+// lane's points fall into one simplex cell, and the cell's gradients (all of snoise2's LDS
+// reads and their addresses) are found once for them.  Each point's value is formed by
+// snoise2's own expressions, so nothing changes in it; a wave with a lane whose points
+// straddle a cell takes the plain form for that octave.  A coordinate's three values
+// c[0..2] = (c, c + h, c - h) are scaled octave by octave as fbm2 and ridged scale a point's.
+// Only for this field: the others' frequencies and lacunarities are powers of two and edges
+// sample them at multiples of 1/16 voxel, so the points around which they are differenced
+// lie on cell borders so often that no wave has 64 lanes without one (measured there: no
+// LDS read saved, 10% more VALU).
+// ---------------------------------------------------------------------------
+
+__device__ constexpr int kNear2X[4] = {1, 2, 0, 0}, kNear2Z[4] = {0, 0, 1, 2};
+
+__device__ __forceinline__ void snoise2_near(const NoiseLds& T, const float x[3], const float z[3], float out[4]) {
+    const float F2 = 0.366025403784f;
+    const float G2 = 0.211324865405f;
+    const float C2 = 1.f - 2.f * G2;
+    float fx[4], fy[4], cx = 0.f, cy = 0.f;
+    bool upper = false, same = true;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float px = x[kNear2X[i]], py = z[kNear2Z[i]];
+        const float s = (px + py) * F2;
+        const float pix = floorf(px + s);
+        const float piy = floorf(py + s);
+        const float t = (pix + piy) * G2;
+        fx[i] = px - (pix - t);
+        fy[i] = py - (piy - t);
+        const bool u = fx[i] > fy[i];
+        if (i == 0) {
+            cx = pix;
+            cy = piy;
+            upper = u;
+        } else {
+            same = same && pix == cx && piy == cy && u == upper;
+        }
+    }
+    if (__ballot(!same) == 0) {
+        const int base = ((int)cy & 255) * kPermPitch + ((int)cx & 255) + 1;
+        const int o1x = upper ? 1 : 0, o1y = 1 - o1x;
+        const float ox = (float)o1x, oy = (float)o1y;
+        const float2 g0 = T.gxy[T.perm[base] & 15];
+        const float2 g1 = T.gxy[T.perm[base + o1y * kPermPitch + o1x] & 15];
+        const float2 g2 = T.gxy[T.perm[base + kPermPitch + 1] & 15];
+        auto corner = [](float2 g, float ax, float ay) {  // corner2 with its gradient at hand
+            const float r = fmaxf(0.5f - fmaf(ay, ay, ax * ax), 0.f);
+            const float t = r * r;
+            return (t * t) * fmaf(g.y, ay, g.x * ax);
+        };
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float n0 = corner(g0, fx[i], fy[i]);
+            const float n1 = corner(g1, (fx[i] - ox) + G2, (fy[i] - oy) + G2);
+            const float n2 = corner(g2, fx[i] - C2, fy[i] - C2);
+            out[i] = 70.f * ((n0 + n1) + n2);
+        }
+        return;
+    }
+    float px[4], py[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        px[i] = x[kNear2X[i]];
+        py[i] = z[kNear2Z[i]];
+    }
+#pragma unroll 1
+    for (int k = 0; k < 4; ++k) {  // one copy of snoise2's code: the points rotate through it
+        const float n = snoise2(T, px[0], py[0]), ax = px[0], ay = py[0];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            px[i] = px[i + 1];
+            py[i] = py[i + 1];
+            out[i] = out[i + 1];
+        }
+        px[3] = ax;
+        py[3] = ay;
+        out[3] = n;
+    }
+}
+
+// leven's 900 * Terrain as one loop over its 14 octaves (8 ridged, 4 of the billow, 2 of
+// the base), for the point (x[0], z[0]) when N is 1 or the four near points when N is 4:
+// leven_terrain's steps in its order, with one copy of the noise's code: written out, the four
+// points' octaves made the crossing kernel 39 KB of code.  (leven_terrain stays written out:
+// its three parts are independent chains, which overlap there.)
+struct LevenExpo {  // 1 / lacunarity^o as RidgedMultiFractal's loop forms it
+    float v[7];
+    constexpr LevenExpo() : v() {
+        float freq = 1.f;
+        for (int o = 0; o < 7; ++o) {
+            v[o] = 1.f / freq;
+            freq = freq * 2.114352f;
+        }
+    }
+};
+__constant__ constexpr LevenExpo kLevenExpo{};
+
+template <int N>
+__device__ __forceinline__ void leven_heights(const NoiseLds& T, const float x[], const float z[], float out[]) {
+    constexpr int M = N == 1 ? 1 : 3;
+    float qx[M], qy[M], px[M], py[M], signal[N], sum[N], v[N], amp = 1.f, lac = 2.114352f, gain = 0.f;
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+        px[j] = qx[j] = x[j] * (1.f / 2000.f);
+        py[j] = qy[j] = z[j] * (1.f / 2000.f);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) signal[i] = sum[i] = v[i] = 0.f;
+#pragma unroll 1
+    for (int step = 0; step < 14; ++step) {
+        if (step == 8 || step == 12) {  // the next part starts
+            const bool billow = step == 8;
+            const float freq = billow ? 0.24f : 0.63f;
+#pragma unroll
+            for (int j = 0; j < M; ++j) {
+                px[j] = (billow ? -4.33f * qx[j] : qx[j]) * freq;
+                py[j] = (billow ? 7.98f * qy[j] : qy[j]) * freq;
+            }
+            lac = billow ? 1.8754f : 2.2f;
+            gain = billow ? 0.433f : 0.15f;
+            amp = 1.f;
+#pragma unroll
+            for (int i = 0; i < N; ++i) sum[i] = 0.f;
+        }
+        if constexpr (N == 1)
+            v[0] = snoise2(T, px[0], py[0]);
+        else
+            snoise2_near(T, px, py, v);
+        if (step < 8) {
+            const float expo = step == 0 ? 1.f : kLevenExpo.v[step - 1];
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const float weight = clamp01(signal[i] * 1.5241f);
+                float s = 1.f - fabsf(v[i]);
+                s = s * (step == 0 ? s : weight);
+                signal[i] = s;
+                sum[i] = step == 0 ? s : sum[i] + s * expo;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < N; ++i) sum[i] = fmaf(v[i], amp, sum[i]);
+            amp = amp * gain;
+        }
+#pragma unroll
+        for (int j = 0; j < M; ++j) {
+            px[j] = px[j] * lac;
+            py[j] = py[j] * lac;
+        }
+        if (step == 7) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) out[i] = clamp01(0.8f * (sum[i] * (1.f / (float)7)));
+        } else if (step == 11) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const float billow = 0.6f * sum[i];
+                out[i] = ((0.5f * billow) + 0.5f) * out[i];
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const float b2 = 0.6f * sum[i];
+        out[i] = 900.f * (out[i] + ((b2 * 0.5f) + 0.5f));
+    }
+}
+
+// height_term in the small form, for calls that are rare.
+template <int kKind>
+__device__ __forceinline__ float height_small(const FieldParams& F, const NoiseLds& T, float x, float z) {
+    if (field_kind<kKind>(F) != LVN_FIELD_LEVEN_TERRAIN) return height_term<kKind>(F, T, x, z);
+    float out;
+    leven_heights<1>(T, &x, &z, &out);
+    return out;
+}
+
+// height_term at (x + h, z), (x - h, z), (x, z + h), (x, z - h).
+template <int kKind>
+__device__ __forceinline__ void height_near(const FieldParams& F, const NoiseLds& T, const float x[3], const float z[3],
+                                            float out[4]) {
+    if (field_kind<kKind>(F) == LVN_FIELD_LEVEN_TERRAIN) {
+        leven_heights<4>(T, x, z, out);
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) out[i] = height_term<kKind>(F, T, x[kNear2X[i]], z[kNear2Z[i]]);
 }
 
 // ---------------------------------------------------------------------------

@@ -30,6 +30,7 @@ struct KArgs {
     int cus;                 // compute units of the device
     int persist_per_cu;      // persistent workgroups per CU (edge crossing)
     int density_per_cu;      // persistent workgroups per CU (density), 0 = by the number of items
+    int load;                // chunk_load of the launch's chunks, 0 = their number
     int height_lines;        // 1: x/z-edge sample heights evaluated once per line (k_height_lines)
     const int* slot_map;     // batch entry -> arena slot, or null for the identity
     int row_blocks;          // workgroups over the batch for the bookkeeping kernels
@@ -71,8 +72,16 @@ void launch_emit(const KArgs& a, int chunks, hipStream_t s);
 int default_ysplit(const Geometry& G, int field_kind, int chunks);
 // Density workgroups per CU when the launch shapes leave it open.
 int default_density_per_cu(const Geometry& G, int ysplit, int chunks, int cus);
+// What `chunks` chunks count for in the crossing stage's choices, `coarse` being the sum of
+// their sample scales / 4.
+inline int chunk_load(int field_kind, long chunks, long coarse) {
+    const long load = field_kind == LVN_FIELD_TERRAIN_CAVES ? chunks + coarse : chunks;
+    return (int)(load < (1L << 24) ? load : 1L << 24);
+}
 // Lanes per edge in the crossing stage when the launch shapes leave it open.
-int default_cross_lanes(int chunks);
+int default_cross_lanes(const Geometry& G, int field_kind, int load);
+// 1: line heights (k_height_lines) when the launch shapes leave it open.
+int default_height_lines(const Geometry& G, int field_kind, int load);
 // cross_lanes value of the sample-parallel crossing kernel (16 lanes per edge in the
 // search, 6 in the normal).
 constexpr int kCrossSampleParallel = 16;

@@ -109,7 +109,7 @@ __device__ __forceinline__ bool chunk_mat_free(const KArgs& a, const ChunkDesc& 
     return a.mat_free && cd.op_count == 0 && cd.mode != kModeCached;
 }
 
-template <bool kCount>
+template <bool kCount, int kKind>
 __device__ __forceinline__ void density_column(const KArgs& a, const NoiseLds& T, int chunk, int seg, int g) {
     const Geometry& G = a.G;
     const int F = G.F;
@@ -144,7 +144,7 @@ __device__ __forceinline__ void density_column(const KArgs& a, const NoiseLds& T
     uint64_t* P = slot_ptr<uint64_t>(a, chunk, a.L.planes) + (long)g * F;
     const float wx = (float)(x * cd.scale + cd.off[0]);
     const float wz = (float)(z * cd.scale + cd.off[2]);
-    const float H = height_term(a.F, T, wx, wz);
+    const float H = height_term<kKind>(a.F, T, wx, wz);
     if (seg == 0 && valid) slot_ptr<float>(a, chunk, a.L.h_cols)[col] = H;  // read by the crossing kernels
     float* dens = slot_ptr<float>(a, chunk, a.L.density);
     __half* dens16 = slot_ptr<__half>(a, chunk, a.L.density);
@@ -152,7 +152,7 @@ __device__ __forceinline__ void density_column(const KArgs& a, const NoiseLds& T
     uint64_t word = 0;
     for (int y = y0; y < y1; ++y) {
         const float wy = (float)(y * cd.scale + cd.off[1]);
-        const float d = combine(a.F, T, wy - H, wx, wy, wz);
+        const float d = combine<kKind>(a.F, T, wy - H, wx, wy, wz);
         if constexpr (kCount) caves += (a.F.kind == LVN_FIELD_TERRAIN_CAVES && !((wy - H) > a.F.cave_cut)) ? 1u : 0u;
         const int idx = field_index(G, x, y, z);
         const uint8_t m = d < 0.f ? (uint8_t)a.defmat : (uint8_t)kAir;
@@ -184,21 +184,14 @@ __device__ __forceinline__ void density_column(const KArgs& a, const NoiseLds& T
     }
 }
 
-// Items of the crossing kernels: wave w of the grid starts with grab w (`per_grab`
+// Items of the queued crossing kernel: wave w of the grid starts with grab w (`per_grab`
 // consecutive items), without the queue, and takes later grabs from the atomic counter.
 // One counter serves about 77 grabs per us, so when every wave of a full grid (3,072 for
 // one chunk) took its first, mostly failing, grab there, that alone was 40 us.  Waves are
-// numbered across the workgroups, so the few items of a small chunk spread over the CUs.
+// numbered across the workgroups, so few items spread over the CUs.
 __device__ __forceinline__ int grid_waves() { return (int)(gridDim.x * (blockDim.x >> 6)); }
 __device__ __forceinline__ int first_grab(int per_grab) {
-    return ((int)(threadIdx.x >> 6) * (int)gridDim.x + (int)blockIdx.x) * per_grab;
-}
-__device__ __forceinline__ int next_grab(int* queue, int per_grab, int total) {
-    const int given = grid_waves() * per_grab;  // the waves' first grabs
-    if (given >= total) return total;
-    int at = 0;
-    if ((threadIdx.x & 63) == 0) at = atomicAdd(queue, per_grab);
-    return given + __shfl(at, 0);
+    return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) * (int)gridDim.x + (int)blockIdx.x) * per_grab;
 }
 
 // Items of a persistent kernel shared within the workgroup: workgroup b owns items b,
@@ -211,7 +204,7 @@ __device__ __forceinline__ int wg_next_item(int* next, int total) {
     const int mine = (total - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
     int j = 0;
     if ((threadIdx.x & 63) == 0) j = atomicAdd(next, 1);
-    j = __shfl(j, 0);
+    j = __builtin_amdgcn_readfirstlane(j);
     return j < mine ? (int)blockIdx.x + (int)gridDim.x * j : -1;
 }
 
@@ -225,7 +218,7 @@ __device__ __forceinline__ int wg_next_item(int* next, int total) {
 // SIMD; some SGPRs spill into VGPR lanes), which the tuner takes where the pass is a
 // chain of height-term lookups per column (the reference's terrain field: 0.69 -> 0.57 ms
 // on its clipmap batch); the cave field's pass takes the same time either way.
-template <bool kCount>
+template <bool kCount, int kKind>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_num_sgpr(80), amdgpu_waves_per_eu(8, 8))) void k_density(
     KArgs a, int chunks) {
     __shared__ NoiseLds T;
@@ -241,7 +234,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_num_sgpr(80), amdgpu_wa
         const int chunk = item / items_per_chunk;
         const int r = item - chunk * items_per_chunk;
         const int seg = r / groups;
-        density_column<kCount>(a, T, chunk, seg, r - seg * groups);
+        density_column<kCount, kKind>(a, T, chunk, seg, r - seg * groups);
     }
 }
 
@@ -481,7 +474,7 @@ __global__ __launch_bounds__(256) void k_edge_compact(KArgs a) {
     const int* base = slot_ptr<const int>(a, chunk, a.L.e_base);
     const int* base_y = slot_ptr<const int>(a, chunk, a.L.e_base_y);
     int* ids = slot_ptr<int>(a, chunk, a.L.e_ids);
-    int* order = slot_ptr<int>(a, chunk, a.L.e_order);
+    int2* order = slot_ptr<int2>(a, chunk, a.L.e_order);
     const int S = G.shift, cap = a.caps.edges, ey_total = a.counters[chunk].edges_y;
     const int lane = threadIdx.x & 63;
     const uint64_t lt = lanemask_lt(lane);
@@ -490,7 +483,7 @@ __global__ __launch_bounds__(256) void k_edge_compact(KArgs a) {
         if (k < cap) {
             ids[k] = id;
             const int pos = is_y ? ky : ey_total + (k - ky);
-            if (pos < cap) order[pos] = k;
+            if (pos < cap) order[pos] = make_int2(k, id);
         }
     };
     const int groups = (G.edge_rows + 63) >> 6;
@@ -574,7 +567,7 @@ __global__ __launch_bounds__(256) void k_edge_compact(KArgs a) {
 // every line holding a crossing x- or z-edge are evaluated once, before the crossing
 // kernels, by the expressions those kernels use (bit-identical values), and read back
 // there.  Line (sel, x, z), sel 0 for x-edges and 1 for z-edges, starts at:
-__device__ __forceinline__ int hline_index(int H, int sel, int x, int z) { return ((sel * H + z) * H + x) * kLineSamples; }
+__device__ __forceinline__ int hline_index(int H, int sel, int x, int z) { return ((sel * H + z) * H + x) * kLineStride; }
 
 // Position of the j-th set bit (from 0) of m; m has more than j set bits.
 __device__ __forceinline__ int nth_bit(uint64_t m, int j) {
@@ -603,7 +596,7 @@ __device__ __forceinline__ int nth_bit(uint64_t m, int j) {
 // needed are the OR over y of the chunk's edge rows (x-edge or z-edge words); the lanes
 // run over their samples only.  Chunks whose edges take no density crossings (the
 // cached-field form) are skipped.
-template <bool kCount>
+template <bool kCount, int kKind>
 __global__ __launch_bounds__(1024) void k_height_lines(KArgs a, int chunks) {
     __shared__ NoiseLds T;
     __shared__ int next_local;
@@ -646,7 +639,7 @@ __global__ __launch_bounds__(1024) void k_height_lines(KArgs a, int chunks) {
             const float p1x = (float)(w0x + (sel == 0 ? cd.scale : 0));
             const float p1z = (float)(w0z + (sel == 1 ? cd.scale : 0));
             const float cur = (float)k * 0.0625f;  // = the sequential scan's running sum (exact)
-            out[x * kLineSamples + (k - 1)] = height_term(a.F, T, p0x + (p1x - p0x) * cur, p0z + (p1z - p0z) * cur);
+            out[x * kLineStride + (k - 1)] = height_term<kKind>(a.F, T, p0x + (p1x - p0x) * cur, p0z + (p1z - p0z) * cur);
             ++nh;
         }
         if constexpr (kCount) atomicAdd(&a.work[2], (unsigned long long)nh);
@@ -656,52 +649,82 @@ __global__ __launch_bounds__(1024) void k_height_lines(KArgs a, int chunks) {
 // The normal of FindEdgeIntersectionInfo (cl/density_field.cl:131-150): central
 // differences with h = 0.001 at the arg-min sample t of the edge p0 -> p1, whose height
 // term `Hbest` is reused when it was evaluated there.
+template <int kKind>
 __device__ __forceinline__ float4 crossing_normal(const FieldParams& Fp, const NoiseLds& T, int axis, bool ends_known,
                                                   float tbest, float Hbest, float p0x, float p0y, float p0z, float p1x,
                                                   float p1y, float p1z, unsigned& nh, unsigned& nc) {
-    const bool caves = Fp.kind == LVN_FIELD_TERRAIN_CAVES;
     const float px = p0x + (p1x - p0x) * tbest;
     const float py = p0y + (p1y - p0y) * tbest;
     const float pz = p0z + (p1z - p0z) * tbest;
     const float h = 0.001f;
     // The height at the arg-min sample is only known when it was evaluated there.
     const bool hb_known = axis == 1 || !(ends_known && (tbest == 0.f || tbest == 1.f));
-    const float H0 = hb_known ? Hbest : height_term(Fp, T, px, pz);
-    const float Hxp = height_term(Fp, T, px + h, pz);
-    const float Hxm = height_term(Fp, T, px - h, pz);
-    const float Hzp = height_term(Fp, T, px, pz + h);
-    const float Hzm = height_term(Fp, T, px, pz - h);
-    const float dx = combine(Fp, T, py - Hxp, px + h, py, pz) - combine(Fp, T, py - Hxm, px - h, py, pz);
-    const float dy = combine(Fp, T, (py + h) - H0, px, py + h, pz) - combine(Fp, T, (py - h) - H0, px, py - h, pz);
-    const float dz = combine(Fp, T, py - Hzp, px, py, pz + h) - combine(Fp, T, py - Hzm, px, py, pz - h);
+    const float H0 = hb_known ? Hbest : height_small<kKind>(Fp, T, px, pz);
+    const float x[3] = {px, px + h, px - h}, y[3] = {py, py + h, py - h}, z[3] = {pz, pz + h, pz - h};
+    float H[4];
+    height_near<kKind>(Fp, T, x, z, H);
     nh += hb_known ? 4u : 5u;
-    if (caves) {
-        nc += !((py - Hxp) > Fp.cave_cut) + !((py - Hxm) > Fp.cave_cut) + !(((py + h) - H0) > Fp.cave_cut) +
-              !(((py - h) - H0) > Fp.cave_cut) + !((py - Hzp) > Fp.cave_cut) + !((py - Hzm) > Fp.cave_cut);
+    // the six samples, combine() each
+    float d[6] = {py - H[0], py - H[1], y[1] - H0, y[2] - H0, py - H[2], py - H[3]};
+    if (field_kind<kKind>(Fp) == LVN_FIELD_TERRAIN_CAVES) {
+        constexpr int ix[6] = {1, 2, 0, 0, 0, 0}, iy[6] = {0, 0, 1, 2, 0, 0}, iz[6] = {0, 0, 0, 0, 1, 2};
+#pragma unroll
+        for (int i = 0; i < 6; ++i) {
+            nc += !(d[i] > Fp.cave_cut) ? 1u : 0u;
+            d[i] = combine<kKind>(Fp, T, d[i], x[ix[i]], y[iy[i]], z[iz[i]]);
+        }
     }
-    const float3 n = normalize_or_zero(dx, dy, dz);
+    const float3 n = normalize_or_zero(d[0] - d[1], d[2] - d[3], d[4] - d[5]);
     return make_float4(n.x, n.y, n.z, tbest);
 }
 
 // FindEdgeIntersectionInfo, cl/density_field.cl:96-151: first arg-min of |d|
 // over t = k/16, then a central-difference normal with h = 0.001.  The height
-// term of samples that share (x, z) is evaluated once: per y-edge, and per x- or
-// z-edge line (`hl`, k_height_lines); the two end samples are the stored field
+// term of samples that share (x, z) is evaluated once: per column (`colH`, a y-edge's, from
+// the density pass), and per x- or z-edge line (`hl`, k_height_lines); the two end samples are the stored field
 // samples when the field is FP32.
+template <int kKind>
 __device__ __forceinline__ float4 density_crossing(const KArgs& a, const NoiseLds& T, const ChunkDesc& cd, int x, int y, int z,
-                                   int axis, bool ends_known, float d_start, float d_end, const float* hl, unsigned& nh,
-                                   unsigned& nc) {
+                                   int axis, bool ends_known, float d_start, float d_end, const float* hl,
+                                   float colH, unsigned& nh, unsigned& nc) {
     const FieldParams& Fp = a.F;
-    const bool caves = Fp.kind == LVN_FIELD_TERRAIN_CAVES;
+    const bool caves = field_kind<kKind>(Fp) == LVN_FIELD_TERRAIN_CAVES;
     const int w0x = x * cd.scale + cd.off[0], w0y = y * cd.scale + cd.off[1], w0z = z * cd.scale + cd.off[2];
     const float p0x = (float)w0x, p0y = (float)w0y, p0z = (float)w0z;
     const float p1x = (float)(w0x + (axis == 0 ? cd.scale : 0));
     const float p1y = (float)(w0y + (axis == 1 ? cd.scale : 0));
     const float p1z = (float)(w0z + (axis == 2 ? cd.scale : 0));
-    const float colH = axis == 1 ? height_term(Fp, T, p0x, p0z) : 0.f;
-    nh += axis == 1 ? 1u : 0u;
     float minV = 3.402823466e+38f, tbest = 0.f, Hbest = colH, cur = 0.f;
     const bool lines = a.height_lines != 0 && axis != 1;
+    // Without the cave term a sample is y - H, and every H is at hand for a y-edge (its
+    // column's) and with line heights, which lie in one 64-byte line and are loaded together
+    // (one after another, the 15 loads' latency was the larger part of an x- or z-edge item).
+    if (!caves && ends_known && (lines || axis == 1)) {
+        float Hl[kLineStride];
+        if (lines) {
+#pragma unroll
+            for (int q = 0; q < kLineStride / 4; ++q) {
+                const float4 v = reinterpret_cast<const float4*>(hl)[q];  // 16-byte aligned: lines are 64 bytes
+                Hl[4 * q] = v.x;
+                Hl[4 * q + 1] = v.y;
+                Hl[4 * q + 2] = v.z;
+                Hl[4 * q + 3] = v.w;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k <= 16; ++k) {
+            const float t = (float)k * 0.0625f;  // = the running sum below (exact)
+            const float H = lines && k >= 1 && k <= kLineSamples ? Hl[k >= 1 && k <= kLineSamples ? k - 1 : 0] : colH;
+            const float py = p0y + (p1y - p0y) * t;
+            const float d = k == 0 ? fabsf(d_start) : k == 16 ? fabsf(d_end) : fabsf(py - H);
+            if (d < minV) {
+                tbest = t;
+                minV = d;
+                Hbest = H;
+            }
+        }
+        return crossing_normal<kKind>(Fp, T, axis, ends_known, tbest, Hbest, p0x, p0y, p0z, p1x, p1y, p1z, nh, nc);
+    }
     float Hn = lines ? hl[0] : 0.f;  // the next interior sample's line height, loaded a sample ahead
     for (int k = 0; k <= 16; ++k) {
         const float px = p0x + (p1x - p0x) * cur;
@@ -718,12 +741,12 @@ __device__ __forceinline__ float4 density_crossing(const KArgs& a, const NoiseLd
                     H = Hn;
                     if (k < kLineSamples) Hn = hl[k];
                 } else {
-                    H = height_term(Fp, T, px, pz);
+                    H = height_term<kKind>(Fp, T, px, pz);
                     ++nh;
                 }
             }
             nc += (caves && !((py - H) > Fp.cave_cut)) ? 1u : 0u;
-            d = fabsf(combine(Fp, T, py - H, px, py, pz));
+            d = fabsf(combine<kKind>(Fp, T, py - H, px, py, pz));
         }
         if (d < minV) {
             tbest = cur;
@@ -732,7 +755,7 @@ __device__ __forceinline__ float4 density_crossing(const KArgs& a, const NoiseLd
         }
         cur = cur + 0.0625f;
     }
-    return crossing_normal(Fp, T, axis, ends_known, tbest, Hbest, p0x, p0y, p0z, p1x, p1y, p1z, nh, nc);
+    return crossing_normal<kKind>(Fp, T, axis, ends_known, tbest, Hbest, p0x, p0y, p0z, p1x, p1y, p1z, nh, nc);
 }
 
 // A brush through scalar loads: its address is the same in every lane, the ops and their
@@ -866,12 +889,12 @@ __device__ __forceinline__ bool edge_touched(const KArgs& a, int chunk, const Ch
 }
 
 // One compacted edge's density crossing; edges with brush data are k_edge_data's.
-template <bool kCount>
-__device__ __forceinline__ void cross_edge(const KArgs& a, const NoiseLds& T, int chunk, int i) {
+template <bool kCount, int kKind>
+__device__ __forceinline__ void cross_edge(const KArgs& a, const NoiseLds& T, int chunk, int i, int id) {
     const Geometry& G = a.G;
     const ChunkDesc& cd = a.chunks[chunk];
     EdgeAt e;
-    if (!decode_edge(G, slot_ptr<int>(a, chunk, a.L.e_ids)[i], e)) {
+    if (!decode_edge(G, id, e)) {
         atomicOr(&a.counters[chunk].status, kStatusLookupMiss);
         return;
     }
@@ -879,8 +902,9 @@ __device__ __forceinline__ void cross_edge(const KArgs& a, const NoiseLds& T, in
     const bool ends = !a.fp16;
     const float2 de = ends ? edge_ends(a, chunk, cd, e.x, e.y, e.z, e.axis, e.i0, e.i1) : make_float2(0.f, 0.f);
     const float* hl = slot_ptr<const float>(a, chunk, a.L.h_lines) + hline_index(G.H, e.axis == 2 ? 1 : 0, e.x, e.z);
+    const float colH = e.axis == 1 ? slot_ptr<const float>(a, chunk, a.L.h_cols)[e.x + G.F * e.z] : 0.f;
     unsigned nh = 0, nc = 0;
-    const float4 out = density_crossing(a, T, cd, e.x, e.y, e.z, e.axis, ends, de.x, de.y, hl, nh, nc);
+    const float4 out = density_crossing<kKind>(a, T, cd, e.x, e.y, e.z, e.axis, ends, de.x, de.y, hl, colH, nh, nc);
     if constexpr (kCount) {
         atomicAdd(&a.work[2], (unsigned long long)nh);
         atomicAdd(&a.work[3], (unsigned long long)nc);
@@ -899,14 +923,30 @@ __device__ __forceinline__ int edge_items_y(const Counters& c, int per_item) {
 __device__ __forceinline__ int edge_items_xz(const Counters& c, int per_item) {
     return (c.edges - min(c.edges_y, c.edges) + per_item - 1) / per_item;
 }
-// Edge rank (index into e_ids / e_data) of item j's slot `e`, or -1 past the end.
-__device__ __forceinline__ int edge_of_item(const KArgs& a, int chunk, int j, int e, int per_item) {
+// Slot `e` of the chunk's item j: the edge's rank (index into e_ids / e_data) and id, rank -1
+// past the end.
+__device__ __forceinline__ int2 edge_of_item(const KArgs& a, int chunk, int j, int e, int per_item) {
     const Counters& c = a.counters[chunk];
     const int ey = min(c.edges_y, c.edges), ny = (ey + per_item - 1) / per_item;
     const int pos = j < ny ? j * per_item + e : ey + (j - ny) * per_item + e;
-    if (j < ny ? pos >= ey : pos >= c.edges) return -1;
-    const int i = slot_ptr<const int>(a, chunk, a.L.e_order)[pos];
-    return (unsigned)i < (unsigned)c.edges ? i : -1;  // entries past a capped list are not written
+    if (j < ny ? pos >= ey : pos >= c.edges) return make_int2(-1, 0);
+    const int2 o = slot_ptr<const int2>(a, chunk, a.L.e_order)[pos];
+    return (unsigned)o.x < (unsigned)c.edges ? o : make_int2(-1, 0);  // entries past a capped list are not written
+}
+
+// The last chunk c with prefix[c] <= item (prefix ascends from 0, item < prefix[chunks]): the
+// wave looks at 64 chunks spread over the range at once, so 4,096 chunks take two loads,
+// where a binary search waits for 11 one after another.
+__device__ __forceinline__ int chunk_of_item(const int* prefix, int chunks, int item) {
+    const int lane = threadIdx.x & 63;
+    int lo = 0, n = chunks;
+    while (n > 1) {
+        const int step = (n + 63) >> 6, at = lane * step;
+        const int found = __popcll(__ballot(at < n && prefix[lo + at] <= item));  // >= 1: lane 0's holds
+        lo += (found - 1) * step;
+        n = min(step, n - (found - 1) * step);
+    }
+    return lo;
 }
 
 // Items of `per_item` edges (64 / lanes per edge) over all chunks: item_prefix[c] =
@@ -1018,32 +1058,72 @@ __global__ __launch_bounds__(kEdgeDataThreads) void k_edge_data(KArgs a, int chu
 // a third of the wave slots empty.
 constexpr int kCrossThreads = 768;
 
-template <bool kCount>
+template <bool kCount, int kKind>
 __global__ __attribute__((amdgpu_waves_per_eu(6, 8))) __launch_bounds__(kCrossThreads) void k_edge_cross(KArgs a,
                                                                                                           int chunks) {
     __shared__ NoiseLds T;
+    __shared__ int next_local;
     const int total = a.item_prefix[chunks];
-    // One global queue (sharing items within workgroups instead measured slower: clipmap
-    // 93.2 -> 94.5 ms).  A grab takes up to 4 consecutive items, as many as still leave
-    // every wave 8 grabs: one counter serves ~77,000 grabs per ms, which items of a few
-    // microseconds (a heightfield's y-edges) would otherwise wait on, and the chunk of
-    // an item is found by one search per grab, the grab's later items walking forward.
-    const int per_grab = max(1, min(4, total / (8 * grid_waves())));
-    if ((int)blockIdx.x * per_grab >= total) return;  // no wave of this workgroup has an item
-    load_noise_tables(T, a.perm, a.grads);
+    if ((int)blockIdx.x >= total) return;  // no wave of this workgroup has an item
+    if (threadIdx.x == 0) next_local = 0;
+    load_noise_tables(T, a.perm, a.grads);  // ends with a barrier
     const int lane = threadIdx.x & 63;
-    for (int first = first_grab(per_grab); first < total; first = next_grab(&a.queue[1], per_grab, total)) {
-        const int end = min(first + per_grab, total);
-        int lo = 0, hi = chunks;  // last chunk with item_prefix[c] <= first
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (a.item_prefix[mid] <= first) lo = mid; else hi = mid;
+    // Cave items cost several times more underground than above, so they come from the one
+    // global queue (sharing within workgroups measured slower: clipmap 93.2 -> 94.5 ms), in
+    // grabs that shrink as the work runs out: half a wave's share of what is left when the
+    // wave last looked, from 16 items down to 1.  Without the cave term items are short
+    // and alike, and 82,000 of them through a counter that serves 77 grabs per us were the
+    // whole of the kernel's time (0.92 ms on the reference's clipmap, its waves waiting 78%
+    // of it): there each workgroup owns every gridDim-th block of items (of 8 once its
+    // waves have 8 each, so that neighbours share a chunk's lines) and its waves share them
+    // through an LDS counter.
+    constexpr bool kQueue = kKind == LVN_FIELD_TERRAIN_CAVES || kKind == kAnyField;
+    const int block_log = total >= 96 * (int)gridDim.x ? 3 : 0;
+    const int waves = grid_waves();
+    auto share = [&](int from) { return min(16, max(1, (total - from) / (2 * waves))); };
+    const int given = share(0) * waves;  // the waves' first grabs
+    int item, end = 0;
+    auto local_item = [&]() {
+        int j = 0;
+        if (lane == 0) j = atomicAdd(&next_local, 1);
+        j = __builtin_amdgcn_readfirstlane(j);
+        const long at = ((((long)(j >> block_log) * gridDim.x) + blockIdx.x) << block_log) + (j & ((1 << block_log) - 1));
+        return at < total ? (int)at : total;
+    };
+    auto next_of = [&](int cur) {  // the wave's item after `cur`, or total
+        if constexpr (!kQueue) return local_item();
+        if (cur + 1 < end) return cur + 1;
+        if (given >= total) return total;
+        const int n = share(cur);
+        int at = 0;
+        if (lane == 0) at = atomicAdd(&a.queue[1], n);
+        at = given + __builtin_amdgcn_readfirstlane(at);
+        end = min(at + n, total);
+        return min(at, total);
+    };
+    if constexpr (kQueue) {
+        item = first_grab(share(0));
+        end = min(item + share(0), total);
+    } else {
+        item = local_item();
+    }
+    if (item >= total) return;
+    int chunk = chunk_of_item(a.item_prefix, chunks, item);
+    int2 o = edge_of_item(a, chunk, item - a.item_prefix[chunk], lane, 64);
+    for (;;) {
+        // the next item's edges are on their way while this one's are crossed
+        const int next = next_of(item);
+        int next_chunk = chunk;
+        int2 o_next = make_int2(-1, 0);
+        if (next < total) {
+            if (next < item || a.item_prefix[chunk + 1] <= next) next_chunk = chunk_of_item(a.item_prefix, chunks, next);
+            o_next = edge_of_item(a, next_chunk, next - a.item_prefix[next_chunk], lane, 64);
         }
-        for (int item = first; item < end; ++item) {
-            while (a.item_prefix[lo + 1] <= item) ++lo;  // item < item_prefix[chunks] stops it
-            const int i = edge_of_item(a, lo, item - a.item_prefix[lo], lane, 64);
-            if (i >= 0) cross_edge<kCount>(a, T, lo, i);
-        }
+        if (o.x >= 0) cross_edge<kCount, kKind>(a, T, chunk, o.x, o.y);
+        if (next >= total) break;
+        item = next;
+        chunk = next_chunk;
+        o = o_next;
     }
 }
 
@@ -1053,19 +1133,20 @@ __global__ __attribute__((amdgpu_waves_per_eu(6, 8))) __launch_bounds__(kCrossTh
 // arg-min (smallest |d|, then smallest k, as the sequential scan decides), then the
 // six normal samples are spread over the group.  Every value is computed by the
 // same expression as in density_crossing, so results are identical.
-template <bool kCount, int kG>
-__device__ __forceinline__ void cross_edge_group(const KArgs& a, const NoiseLds& T, int chunk, int i, int sub) {
+template <bool kCount, int kKind, int kG>
+__device__ __forceinline__ void cross_edge_group(const KArgs& a, const NoiseLds& T, int chunk, int i, int id,
+                                                 int sub) {
     const Geometry& G = a.G;
     const ChunkDesc& cd = a.chunks[chunk];
     EdgeAt e;
-    if (!decode_edge(G, slot_ptr<int>(a, chunk, a.L.e_ids)[i], e)) {
+    if (!decode_edge(G, id, e)) {
         if (sub == 0) atomicOr(&a.counters[chunk].status, kStatusLookupMiss);
         return;
     }
     const int x = e.x, y = e.y, z = e.z, axis = e.axis, i0 = e.i0, i1 = e.i1;
     if (edge_touched(a, chunk, cd, i0, i1)) return;  // k_edge_data's
     const FieldParams& Fp = a.F;
-    const bool caves = Fp.kind == LVN_FIELD_TERRAIN_CAVES;
+    const bool caves = field_kind<kKind>(Fp) == LVN_FIELD_TERRAIN_CAVES;
     const bool ends = !a.fp16;
     const float2 de = ends ? edge_ends(a, chunk, cd, x, y, z, axis, i0, i1) : make_float2(0.f, 0.f);
     const float d_start = de.x, d_end = de.y;
@@ -1075,8 +1156,7 @@ __device__ __forceinline__ void cross_edge_group(const KArgs& a, const NoiseLds&
     const float p1y = (float)(w0y + (axis == 1 ? cd.scale : 0));
     const float p1z = (float)(w0z + (axis == 2 ? cd.scale : 0));
     unsigned nh = 0, nc = 0;
-    const float colH = axis == 1 ? height_term(Fp, T, p0x, p0z) : 0.f;
-    nh += (axis == 1 && sub == 0) ? 1u : 0u;
+    const float colH = axis == 1 ? slot_ptr<const float>(a, chunk, a.L.h_cols)[x + G.F * z] : 0.f;
     const float* hl = slot_ptr<const float>(a, chunk, a.L.h_lines) + hline_index(G.H, axis == 2 ? 1 : 0, x, z);
     float minV = 3.402823466e+38f, Hbest = colH;
     int kbest = 17;
@@ -1099,12 +1179,12 @@ __device__ __forceinline__ void cross_edge_group(const KArgs& a, const NoiseLds&
                     H = Hn;
                     if (k + kG <= kLineSamples) Hn = hl[k + kG - 1];
                 } else {
-                    H = height_term(Fp, T, px, pz);
+                    H = height_term<kKind>(Fp, T, px, pz);
                     ++nh;
                 }
             }
             nc += (caves && !((py - H) > Fp.cave_cut)) ? 1u : 0u;
-            d = fabsf(combine(Fp, T, py - H, px, py, pz));
+            d = fabsf(combine<kKind>(Fp, T, py - H, px, py, pz));
         }
         if (d < minV) {
             minV = d;
@@ -1132,18 +1212,19 @@ __device__ __forceinline__ void cross_edge_group(const KArgs& a, const NoiseLds&
     constexpr int kR = (6 + kG - 1) / kG;
     float vals[kR];
 #pragma unroll
-    for (int r = 0; r < kR; ++r) {
-        vals[r] = 0.f;
+    for (int r = 0; r < kR; ++r) vals[r] = 0.f;
+#pragma unroll 1
+    for (int r = 0; r < kR; ++r) {  // one copy of the field's code
         const int j = r * kG + sub;  // normal sample j: +x, -x, +y, -y, +z, -z
         if (j >= 6) continue;
         const float sx = j == 0 ? h : j == 1 ? -h : 0.f;
         const float sz = j == 4 ? h : j == 5 ? -h : 0.f;
         float H;
         if (j == 2 || j == 3) {
-            H = hb_known ? Hbest : height_term(Fp, T, px, pz);
+            H = hb_known ? Hbest : height_term<kKind>(Fp, T, px, pz);
             nh += (!hb_known && j == 2) ? 1u : 0u;
         } else {
-            H = height_term(Fp, T, j < 2 ? px + sx : px, j < 2 ? pz : pz + sz);
+            H = height_term<kKind>(Fp, T, j < 2 ? px + sx : px, j < 2 ? pz : pz + sz);
             ++nh;
         }
         const float qx = j < 2 ? px + sx : px;
@@ -1151,7 +1232,9 @@ __device__ __forceinline__ void cross_edge_group(const KArgs& a, const NoiseLds&
         const float qz = j >= 4 ? pz + sz : pz;
         const float aa = qy - H;
         nc += (caves && !(aa > Fp.cave_cut)) ? 1u : 0u;
-        vals[r] = combine(Fp, T, aa, qx, qy, qz);
+        const float val = combine<kKind>(Fp, T, aa, qx, qy, qz);
+#pragma unroll
+        for (int q = 0; q < kR; ++q) vals[q] = q == r ? val : vals[q];
     }
     float v[6];
 #pragma unroll
@@ -1165,23 +1248,21 @@ __device__ __forceinline__ void cross_edge_group(const KArgs& a, const NoiseLds&
     if (sub == 0) slot_ptr<float4>(a, chunk, a.L.e_data)[i] = make_float4(n.x, n.y, n.z, tbest);
 }
 
-template <bool kCount, int kG>
+template <bool kCount, int kKind, int kG>
 __global__ __attribute__((amdgpu_waves_per_eu(6, 8))) __launch_bounds__(kCrossThreads) void k_edge_cross_group(
     KArgs a, int chunks) {
     __shared__ NoiseLds T;
+    __shared__ int next_local;
     constexpr int kPerItem = 64 / kG;
     const int total = a.item_prefix[chunks];
     if ((int)blockIdx.x >= total) return;  // no wave of this workgroup has an item
-    load_noise_tables(T, a.perm, a.grads);
+    if (threadIdx.x == 0) next_local = 0;
+    load_noise_tables(T, a.perm, a.grads);  // ends with a barrier
     const int lane = threadIdx.x & 63;
-    for (int item = first_grab(1); item < total; item = next_grab(&a.queue[1], 1, total)) {
-        int lo = 0, hi = chunks;  // last chunk with item_prefix[c] <= item
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (a.item_prefix[mid] <= item) lo = mid; else hi = mid;
-        }
-        const int i = edge_of_item(a, lo, item - a.item_prefix[lo], lane / kG, kPerItem);
-        if (i >= 0) cross_edge_group<kCount, kG>(a, T, lo, i, lane & (kG - 1));
+    for (int item = wg_next_item(&next_local, total); item >= 0; item = wg_next_item(&next_local, total)) {
+        const int lo = chunk_of_item(a.item_prefix, chunks, item);
+        const int2 o = edge_of_item(a, lo, item - a.item_prefix[lo], lane / kG, kPerItem);
+        if (o.x >= 0) cross_edge_group<kCount, kKind, kG>(a, T, lo, o.x, o.y, lane & (kG - 1));
     }
 }
 
@@ -1216,37 +1297,36 @@ __device__ __forceinline__ void argmin_step(uint32_t& d, int& k, float& H) {
     H = take ? oh : H;
 }
 
-template <bool kCount>
+template <bool kCount, int kKind>
 __global__ __attribute__((amdgpu_waves_per_eu(6, 8))) __launch_bounds__(kCrossThreads) void k_edge_cross_sp(KArgs a,
                                                                                                              int chunks) {
     __shared__ NoiseLds T;
+    __shared__ int next_local;
     __shared__ int sp_k[kSpWaves][64];    // per wave: kbest of each edge of the item
     __shared__ float sp_h[kSpWaves][64];  // and the height term there
     const int total = a.item_prefix[chunks];
     if ((int)blockIdx.x >= total) return;  // no wave of this workgroup has an item
-    load_noise_tables(T, a.perm, a.grads);
+    if (threadIdx.x == 0) next_local = 0;
+    load_noise_tables(T, a.perm, a.grads);  // ends with a barrier
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int row = lane >> 4, sub = lane & 15;
     const FieldParams& Fp = a.F;
-    const bool caves = Fp.kind == LVN_FIELD_TERRAIN_CAVES;
+    const bool caves = field_kind<kKind>(Fp) == LVN_FIELD_TERRAIN_CAVES;
     const bool ends = !a.fp16;
     const Geometry& G = a.G;
     unsigned nh = 0, nc = 0, ne = 0;
-    for (int item = first_grab(1); item < total; item = next_grab(&a.queue[1], 1, total)) {
-        int lo = 0, hi = chunks;  // last chunk with item_prefix[c] <= item
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (a.item_prefix[mid] <= item) lo = mid; else hi = mid;
-        }
+    for (int item = wg_next_item(&next_local, total); item >= 0; item = wg_next_item(&next_local, total)) {
+        const int lo = chunk_of_item(a.item_prefix, chunks, item);
         const int chunk = lo;
         const ChunkDesc& cd = a.chunks[chunk];
         // ---- each lane loads its own edge
-        int ei = edge_of_item(a, chunk, item - a.item_prefix[chunk], lane, 64);
+        const int2 o = edge_of_item(a, chunk, item - a.item_prefix[chunk], lane, 64);
+        int ei = o.x;
         int exyz = 0;
         float eH = 0.f, eS = 0.f, eE = 0.f;
         if (ei >= 0) {
             EdgeAt e;
-            if (!decode_edge(G, slot_ptr<int>(a, chunk, a.L.e_ids)[ei], e)) {
+            if (!decode_edge(G, o.y, e)) {
                 atomicOr(&a.counters[chunk].status, kStatusLookupMiss);
                 ei = -1;
             } else if (edge_touched(a, chunk, cd, e.i0, e.i1)) {  // k_edge_data's
@@ -1300,12 +1380,12 @@ __global__ __attribute__((amdgpu_waves_per_eu(6, 8))) __launch_bounds__(kCrossTh
                             H = slot_ptr<const float>(a, chunk, a.L.h_lines)[hline_index(G.H, axis == 2 ? 1 : 0, x, z) +
                                                                              (k - 1)];
                         } else {
-                            H = height_term(Fp, T, px, pz);
+                            H = height_term<kKind>(Fp, T, px, pz);
                             ++nh;
                         }
                     }
                     nc += (caves && !((py - H) > Fp.cave_cut)) ? 1u : 0u;
-                    d = fabsf(combine(Fp, T, py - H, px, py, pz));
+                    d = fabsf(combine<kKind>(Fp, T, py - H, px, py, pz));
                 }
                 // the scan takes a sample only when |d| < its running minimum (from FLT_MAX):
                 // lane 15 tries sample 0 before sample 16
@@ -1338,7 +1418,7 @@ __global__ __attribute__((amdgpu_waves_per_eu(6, 8))) __launch_bounds__(kCrossTh
             const float p1y = (float)(w0y + (axis == 1 ? cd.scale : 0));
             const float p1z = (float)(w0z + (axis == 2 ? cd.scale : 0));
             slot_ptr<float4>(a, chunk, a.L.e_data)[ei] =
-                crossing_normal(Fp, T, axis, ends, (float)kb * 0.0625f, hb, (float)w0x, (float)w0y, (float)w0z, p1x, p1y,
+                crossing_normal<kKind>(Fp, T, axis, ends, (float)kb * 0.0625f, hb, (float)w0x, (float)w0y, (float)w0z, p1x, p1y,
                                 p1z, nh, nc);
             ++ne;
         }
@@ -2159,6 +2239,23 @@ void launch_clear_counters(const KArgs& a, int n, hipStream_t s) {
                        a.counters, n, a.queue);
 }
 
+// A kernel over the field, built for the launch's field kind; the work-counting form takes
+// any kind.  Further template arguments follow the kind.
+#define LVN_LAUNCH_KIND(kernel, grid, block, ...)                                                                 \
+    do {                                                                                                          \
+        if (a.work)                                                                                               \
+            hipLaunchKernelGGL((kernel<true, kAnyField __VA_OPT__(, ) __VA_ARGS__>), grid, block, 0, s, a, chunks);  \
+        else if (a.F.kind == LVN_FIELD_LEVEN_TERRAIN)                                                             \
+            hipLaunchKernelGGL((kernel<false, LVN_FIELD_LEVEN_TERRAIN __VA_OPT__(, ) __VA_ARGS__>), grid, block, 0,  \
+                               s, a, chunks);                                                                     \
+        else if (a.F.kind == LVN_FIELD_TERRAIN_CAVES)                                                             \
+            hipLaunchKernelGGL((kernel<false, LVN_FIELD_TERRAIN_CAVES __VA_OPT__(, ) __VA_ARGS__>), grid, block, 0,  \
+                               s, a, chunks);                                                                     \
+        else                                                                                                      \
+            hipLaunchKernelGGL((kernel<false, LVN_FIELD_HEIGHTFIELD __VA_OPT__(, ) __VA_ARGS__>), grid, block, 0, s, \
+                               a, chunks);                                                                        \
+    } while (0)
+
 // per_cu workgroups per CU (at most two: the LDS table limit), fewer when the work is
 // small.
 static unsigned persistent_blocks(const KArgs& a, int per_cu, long items) {
@@ -2191,10 +2288,7 @@ void launch_density(const KArgs& a, int chunks, hipStream_t s) {
     // item where there are fewer items than that.
     const int per_cu = a.density_per_cu ? a.density_per_cu : default_density_per_cu(a.G, a.ysplit, chunks, a.cus);
     const unsigned blocks = (unsigned)std::max(1L, std::min((long)per_cu * a.cus, items));
-    if (a.work)
-        hipLaunchKernelGGL(k_density<true>, dim3(blocks), dim3(1024), 0, s, a, chunks);
-    else
-        hipLaunchKernelGGL(k_density<false>, dim3(blocks), dim3(1024), 0, s, a, chunks);
+    LVN_LAUNCH_KIND(k_density, dim3(blocks), dim3(1024));
 }
 void launch_csg(const KArgs& a, int chunks, hipStream_t s) {
     hipLaunchKernelGGL(k_csg, dim3(kCsgSlabs, chunks), dim3(256), 0, s, a);
@@ -2224,12 +2318,35 @@ void launch_edge_compact(const KArgs& a, int chunks, hipStream_t s) {
     const long groups = (a.G.edge_rows + 63) / 64;
     hipLaunchKernelGGL(k_edge_compact, dim3(chunk_blocks(chunks, 64L * groups, a.row_blocks), chunks), dim3(256), 0, s, a);
 }
-// Lanes per edge of the crossing stage: the tuned value, else by batch size (a
-// typical chunk has a few hundred 64-edge items; kG multiplies the waves).
-int default_cross_lanes(int chunks) { return chunks <= 1 ? 8 : chunks <= 3 ? 4 : chunks <= 9 ? 2 : 1; }
+// Lanes per edge of the crossing stage: the tuned value, else by field and batch size (a
+// typical 64^3 chunk has a few hundred 64-edge items, a chunk of N^3 about (N / 64)^2 of
+// that; kG lanes multiply the waves and divide each wave's chain of dependent octaves).
+// Crossing stage measured at 1 / 2 / 4 / 8 lanes (us): heightfield, 8 chunks 36/33/28/25,
+// 32 chunks 52/42/35/35, 200 chunks 88/84/98/108, 500 chunks 196/198/253/302; caves, 1 chunk
+// 131/67/46/32, 8 chunks 86/87/75/74, 64 chunks 415/339/382/406, 96 chunks 501/519/594/638;
+// the reference's terrain, whose 14 octaves a term make the longest chains, 1 chunk
+// 61/51/38/22, 64 chunks 87/84/79/54, 300 chunks 151/155/181/134, 500 chunks 242/261/360/268.
+// Sampled coarsely, caves cross more of the edges (17,000 a chunk at voxel size 1, 170,000
+// and more at 32: 50 such chunks 2,485 us with 1 lane, 2,700 with 2), hence chunk_load.
+static long full_chunks(const Geometry& G, int load) { return std::max(1L, (long)load * G.N * G.N / 4096); }
+
+int default_cross_lanes(const Geometry& G, int field_kind, int load) {
+    const long n = full_chunks(G, load);
+    if (field_kind == LVN_FIELD_LEVEN_TERRAIN) return n <= 350 ? 8 : 1;
+    if (field_kind == LVN_FIELD_TERRAIN_CAVES) return n <= 10 ? 8 : n <= 80 ? 2 : 1;
+    return n <= 12 ? 8 : n <= 48 ? 4 : n <= 400 ? 2 : 1;
+}
+
+// Line heights pay where several crossings share a line, as caves make them, and the pass
+// before the crossings is short beside these: 200 chunks of caves 1,406 -> 1,219 us, 32
+// chunks 263 -> 254, one chunk 131 -> 136.  A surface crosses a line about once: 1,800
+// chunks of the reference's terrain 903 without, 944 with.
+int default_height_lines(const Geometry& G, int field_kind, int load) {
+    return field_kind == LVN_FIELD_TERRAIN_CAVES && full_chunks(G, load) >= 64 ? 1 : 0;
+}
 
 static int cross_lanes(const KArgs& a, int chunks) {
-    return a.cross_lanes > 0 ? a.cross_lanes : default_cross_lanes(chunks);
+    return a.cross_lanes > 0 ? a.cross_lanes : default_cross_lanes(a.G, a.F.kind, a.load ? a.load : chunks);
 }
 
 constexpr int kEdgeDataBlocks = 1024;
@@ -2237,20 +2354,14 @@ constexpr int kEdgeDataBlocks = 1024;
 template <int kG>
 static void launch_cross_group(const KArgs& a, int chunks, hipStream_t s) {
     const dim3 grid(persistent_blocks(a, a.persist_per_cu, 512L * kG * chunks));
-    if (a.work)
-        hipLaunchKernelGGL((k_edge_cross_group<true, kG>), grid, dim3(kCrossThreads), 0, s, a, chunks);
-    else
-        hipLaunchKernelGGL((k_edge_cross_group<false, kG>), grid, dim3(kCrossThreads), 0, s, a, chunks);
+    LVN_LAUNCH_KIND(k_edge_cross_group, grid, dim3(kCrossThreads), kG);
 }
 
 void launch_edge_cross(const KArgs& a, int chunks, hipStream_t s) {
     if (a.height_lines) {
         const long line_items = 2L * a.G.H * chunks;
         const dim3 line_grid(persistent_blocks(a, 2, line_items));  // 63 SGPRs: two workgroups per CU stay resident
-        if (a.work)
-            hipLaunchKernelGGL(k_height_lines<true>, line_grid, dim3(1024), 0, s, a, chunks);
-        else
-            hipLaunchKernelGGL(k_height_lines<false>, line_grid, dim3(1024), 0, s, a, chunks);
+        LVN_LAUNCH_KIND(k_height_lines, line_grid, dim3(1024));
     }
     const int g = cross_lanes(a, chunks);
     // 1,024 waves of brush and cached edges (of a few chunks: 96 KB of hermite data), and
@@ -2268,19 +2379,13 @@ void launch_edge_cross(const KArgs& a, int chunks, hipStream_t s) {
     case 8: launch_cross_group<8>(a, chunks, s); return;
     case kCrossSampleParallel: {
         const dim3 grid(persistent_blocks(a, a.persist_per_cu, 512L * chunks));
-        if (a.work)
-            hipLaunchKernelGGL(k_edge_cross_sp<true>, grid, dim3(kCrossThreads), 0, s, a, chunks);
-        else
-            hipLaunchKernelGGL(k_edge_cross_sp<false>, grid, dim3(kCrossThreads), 0, s, a, chunks);
+        LVN_LAUNCH_KIND(k_edge_cross_sp, grid, dim3(kCrossThreads));
         return;
     }
     default: break;
     }
     const dim3 grid(persistent_blocks(a, a.persist_per_cu, 512L * chunks));
-    if (a.work)
-        hipLaunchKernelGGL(k_edge_cross<true>, grid, dim3(kCrossThreads), 0, s, a, chunks);
-    else
-        hipLaunchKernelGGL(k_edge_cross<false>, grid, dim3(kCrossThreads), 0, s, a, chunks);
+    LVN_LAUNCH_KIND(k_edge_cross, grid, dim3(kCrossThreads));
 }
 void launch_voxel_rows(const KArgs& a, int chunks, hipStream_t s) {
     hipLaunchKernelGGL(k_voxel_rows, dim3(chunk_blocks(chunks, a.G.voxel_segs, a.row_blocks), chunks), dim3(256), 0, s, a);

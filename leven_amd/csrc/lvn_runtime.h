@@ -154,6 +154,8 @@ struct Batch {
     hipGraphExec_t exec = nullptr;   // captured pipeline for `graph_n` chunks
     hipGraph_t graph = nullptr;
     int graph_n = -1;
+    long coarse = 0;                 // sum of the staged chunks' sample scales / 4 (chunk_load)
+    int graph_lanes = 0, graph_lines = 0;  // crossing shapes the graph was captured with
     const void* graph_ops = nullptr;   // op arrays the graph was captured with
     const void* graph_index = nullptr;
     uint64_t graph_gen = 0;
@@ -168,8 +170,6 @@ struct Batch {
 
 // Launch-shape defaults shared by every form (the batched form overrides them per batch).
 constexpr int kDefaultPersistPerCu = 2;
-// Batches from this many chunks evaluate x/z-edge line heights once per line by default.
-constexpr int kHeightLinesMinChunks = 64;
 constexpr int kDefaultRowBlocks = 8192;
 constexpr int kDefaultVoxelBlocks = 8192;
 
@@ -181,7 +181,8 @@ KArgs make_kargs(char* arena, const SlotLayout& L, const Geometry& G, const Caps
                  int* item_prefix, int cus);
 Geometry make_geometry(int n);
 Caps make_caps(const Geometry& G, int edge_cap, int voxel_cap);
-SlotLayout make_layout(const Geometry& G, const Caps& c);
+// lines: room for the line heights of k_height_lines (KArgs::height_lines stays 0 without it).
+SlotLayout make_layout(const Geometry& G, const Caps& c, bool lines = true);
 void fill_chunk_desc(ChunkDesc& cd, const int32_t* min, int32_t size, int N);
 // A chunk size the pipeline accepts for N voxels per chunk: a positive multiple of
 // N * LEAF_SIZE_SCALE (sampleScale = size / (N * 4) >= 1, src/compute_density_field.cpp:149).

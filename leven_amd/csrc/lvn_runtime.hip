@@ -205,7 +205,7 @@ Caps make_caps(const Geometry& G, int edge_cap, int voxel_cap) {
     return c;
 }
 
-SlotLayout make_layout(const Geometry& G, const Caps& c) {
+SlotLayout make_layout(const Geometry& G, const Caps& c, bool lines) {
     SlotLayout L;
     uint64_t o = 0;
     auto take = [&](uint64_t bytes) {
@@ -226,8 +226,8 @@ SlotLayout make_layout(const Geometry& G, const Caps& c) {
     L.e_base_y = take((uint64_t)G.edge_rows * 4);
     L.e_ids = take((uint64_t)c.edges * 4);
     L.e_data = take((uint64_t)c.edges * 16);
-    L.e_order = take((uint64_t)c.edges * 4);
-    L.h_lines = take((uint64_t)2 * G.H * G.H * kLineSamples * 4);
+    L.e_order = take((uint64_t)c.edges * 8);
+    L.h_lines = take(lines ? (uint64_t)2 * G.H * G.H * kLineStride * 4 : 0);
     L.h_cols = take((uint64_t)G.F * G.F * 4);
     L.v_mask = take((uint64_t)G.voxel_segs * 8);
     L.v_count = take((uint64_t)G.voxel_segs * 4);
@@ -640,20 +640,24 @@ static int stage_batch(Batch* b, int n, const lvn_chunk_req* reqs) {
     LVN_HIP(hipMemcpyAsync(c->d_chunks, c->h_chunks, sizeof(ChunkDesc) * n, hipMemcpyHostToDevice, c->stream));
     LVN_HIP(hipStreamSynchronize(c->stream));
     b->n = n;
+    b->coarse = 0;
+    for (int i = 0; i < n; ++i) b->coarse += c->h_chunks[i].scale / 4;
     b->simplified = false;
     b->slot_of.clear();
     for (int i = 0; i < n; ++i) b->slot_of[make_key(reqs[i].min, reqs[i].size)] = i;
     return LVN_OK;
 }
 
+static int batch_load(const Batch* b) { return chunk_load(g_state.fp.kind, b->n, b->coarse); }
+
 // The batch's launch shapes with the automatic ones resolved.
 static lvn_tuning effective_tuning(const Batch* b) {
     lvn_tuning t = b->tuning;
     if (t.density_ysplit == 0) t.density_ysplit = default_ysplit(b->ctx.G, g_state.fp.kind, b->n);
-    if (t.cross_lanes == 0) t.cross_lanes = default_cross_lanes(b->n);
+    if (t.cross_lanes == 0) t.cross_lanes = default_cross_lanes(b->ctx.G, g_state.fp.kind, batch_load(b));
     if (t.density_per_cu == 0)
         t.density_per_cu = default_density_per_cu(b->ctx.G, t.density_ysplit, b->n, b->ctx.cus);
-    if (t.height_lines == 0) t.height_lines = b->n >= kHeightLinesMinChunks ? 2 : 1;
+    if (t.height_lines == 0) t.height_lines = default_height_lines(b->ctx.G, g_state.fp.kind, batch_load(b)) ? 2 : 1;
     return t;
 }
 
@@ -787,7 +791,7 @@ static NoAllocLayout noalloc_layout(int n) {
     NoAllocLayout t;
     t.G = make_geometry(n);
     t.caps = make_caps(t.G, LVN_NOALLOC_MAX_EDGES, LVN_NOALLOC_MAX_VOXELS);
-    t.L = make_layout(t.G, t.caps);
+    t.L = make_layout(t.G, t.caps, false);
     uint64_t o = t.L.slot_bytes;
     auto take = [&](uint64_t bytes) {
         const uint64_t at = o;
@@ -1122,13 +1126,14 @@ int lvn_batch_run(lvn_batch* bh) {
     if (!g_state.init) return LVN_ERR_STATE;  // the library was shut down
     if (b->n == 0) return LVN_OK;
     Ctx* c = &b->ctx;
-    if (b->graph_n != b->n || b->graph_ops != c->d_ops || b->graph_index != c->d_op_index ||
+    const lvn_tuning t = effective_tuning(b);  // may change with the staged chunks' scales
+    if (b->graph_n != b->n || b->graph_lanes != t.cross_lanes || b->graph_lines != t.height_lines || b->graph_ops != c->d_ops || b->graph_index != c->d_op_index ||
         b->graph_gen != g_state.generation) {
         if (b->exec) LVN_HIP(hipGraphExecDestroy(b->exec));
         if (b->graph) LVN_HIP(hipGraphDestroy(b->graph));
         b->exec = nullptr;
         b->graph = nullptr;
-        const KArgs a = batch_args(b);
+        const KArgs a = batch_args(b, t);
         LVN_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
         launch_pipeline(a, b->n, c->stream);
         LVN_HIP(hipStreamEndCapture(c->stream, &b->graph));
@@ -1137,6 +1142,8 @@ int lvn_batch_run(lvn_batch* bh) {
         b->graph_ops = c->d_ops;
         b->graph_index = c->d_op_index;
         b->graph_gen = g_state.generation;
+        b->graph_lanes = t.cross_lanes;
+        b->graph_lines = t.height_lines;
     }
     b->simplified = false;
     LVN_HIP(hipGraphLaunch(b->exec, c->stream));

@@ -371,8 +371,11 @@ int Server::launch(Lane& L, const std::vector<Job>& batch, const std::vector<int
     a.dens_cols = a.F.kind != LVN_FIELD_TERRAIN_CAVES && !a.fp16 ? 1 : 0;
     a.mat_free = 1;  // and chunks without brushes their materials
     // zero fields: the automatic choice by batch size
+    long coarse = 0;
+    for (int i = 0; i < n; ++i) coarse += L.h_chunks[i].scale / 4;
+    a.load = chunk_load(a.F.kind, n, coarse);
     a.ysplit = t.density_ysplit ? t.density_ysplit : default_ysplit(a.G, a.F.kind, n);
-    a.height_lines = t.height_lines ? (t.height_lines == 2 ? 1 : 0) : (n >= kHeightLinesMinChunks ? 1 : 0);
+    a.height_lines = t.height_lines ? (t.height_lines == 2 ? 1 : 0) : default_height_lines(a.G, a.F.kind, a.load);
     a.persist_per_cu = t.persistent_per_cu;
     a.density_per_cu = t.density_per_cu;
     a.row_blocks = t.row_blocks;

@@ -22,6 +22,7 @@ constexpr int kGradEntries = 16;
 // Interior samples (k = 1..15 of the 17) of an x- or z-edge line whose heights are
 // evaluated once per line (k_height_lines).
 constexpr int kLineSamples = 15;
+constexpr int kLineStride = 16;  // floats per line: one 64-byte stretch
 
 constexpr int kAir = LVN_MATERIAL_AIR;    // src/volume_materials.h:9
 constexpr int kNone = LVN_MATERIAL_NONE;  // src/volume_materials.h:8
