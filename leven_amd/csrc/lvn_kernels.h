@@ -86,7 +86,27 @@ int default_height_lines(const Geometry& G, int field_kind, int load);
 // search, 6 in the normal).
 constexpr int kCrossSampleParallel = 16;
 
-// Whole pipeline for chunk slots [0, chunks), counters cleared first.
+// A mesh's three arrays (vertices, triangles, seam nodes) copied by one launch; pinned host
+// memory or device memory on either side, addresses and sizes multiples of 4.
+struct MeshCopy {
+    const char* src[3];
+    char* dst[3];
+    uint64_t bytes[3];
+};
+void launch_copy_mesh(const MeshCopy& c, hipStream_t s);
+
+// Chunk slot 0's counters and, back to back from kExportHeader bytes on, the mesh that
+// generateChunkMesh exports of it into `out` (pinned host memory).
+constexpr int kExportHeader = 64;
+void launch_export(const KArgs& a, char* out, hipStream_t s);
+
+// Chunk slot 0's descriptor and its op batch from pinned host memory into a.chunks, a.ops
+// and a.op_index, counters cleared.
+void launch_stage_chunk(const KArgs& a, const ChunkDesc* chunk, const DevOp* ops, const int* index, hipStream_t s);
+
+// The pipeline's stages for chunk slots [0, chunks).
+void launch_stages(const KArgs& a, int chunks, hipStream_t s);
+// The same, counters cleared first.
 void launch_pipeline(const KArgs& a, int chunks, hipStream_t s);
 
 }  // namespace lvn

@@ -2220,6 +2220,46 @@ __global__ __launch_bounds__(64 * kEmitWaves) void k_emit(KArgs a) {
     }
 }
 
+// One mesh read back into the caller's pinned buffers by one launch and one wait.  Bound by
+// the host link (57 GB/s).  Three hipMemcpy calls and a read of the chunk's counters, each
+// waited for, took 64 chunks of 1.2 MB 3.3 ms; this and counters read once per run take 1.9.
+// Copies in the widest units that addresses and sizes allow.
+template <typename Word>
+__device__ __forceinline__ void copy_words(const char* src, char* dst, uint64_t bytes) {
+    const Word* s = reinterpret_cast<const Word*>(src);
+    Word* d = reinterpret_cast<Word*>(dst);
+    const uint64_t n = bytes / sizeof(Word), step = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += step) d[i] = s[i];
+}
+__global__ __launch_bounds__(256) void k_copy_mesh(MeshCopy c) {
+    const uint64_t odd = (uint64_t)c.src[blockIdx.y] | (uint64_t)c.dst[blockIdx.y] | c.bytes[blockIdx.y];
+    if ((odd & 15) == 0)
+        copy_words<uint4>(c.src[blockIdx.y], c.dst[blockIdx.y], c.bytes[blockIdx.y]);
+    else if ((odd & 7) == 0)
+        copy_words<uint2>(c.src[blockIdx.y], c.dst[blockIdx.y], c.bytes[blockIdx.y]);
+    else
+        copy_words<uint32_t>(c.src[blockIdx.y], c.dst[blockIdx.y], c.bytes[blockIdx.y]);
+}
+
+// The one-chunk forms' export as the pipeline's last kernel: the counters and the mesh in one
+// pass to the host, so the caller waits once instead of for the counters, then three device
+// copies into the mesh cache and one read-back; the cache's copy now runs beside the host's.
+// Bound by the host link: 2 MB of a 64^3 cave chunk in 45 us.  With k_stage_chunk that call
+// went 297 -> 286 us, a two-step edit 779 -> 720, a 16^3 chunk 145 -> 125.
+__global__ __launch_bounds__(256) void k_export(KArgs a, char* out) {
+    const Counters k = a.counters[0];
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *reinterpret_cast<Counters*>(out) = k;
+    if (k.status || k.edges == 0) return;
+    const uint64_t bv = k.quads > 0 ? 48ull * k.voxels : 0, bt = 24ull * k.quads, bs = 48ull * k.seams;
+    char* at = out + kExportHeader;
+    if (blockIdx.y == 0)
+        copy_words<uint4>(slot_ptr<const char>(a, 0, a.L.verts), at, bv);
+    else if (blockIdx.y == 1)
+        copy_words<uint2>(slot_ptr<const char>(a, 0, a.L.tris), at + bv, bt);
+    else
+        copy_words<uint2>(slot_ptr<const char>(a, 0, a.L.seams), at + bv + bt, bs);
+}
+
 static inline unsigned ceil_div(long a, long b) { return (unsigned)((a + b - 1) / b); }
 
 // Zero the per-chunk counters (a kernel rather than a memset node, so that a
@@ -2230,9 +2270,29 @@ __global__ __launch_bounds__(256) void k_clear_counters(Counters* c, int n, int*
     if (i < kNumQueues) queue[i] = 0;
 }
 
+// The one-chunk forms' inputs, read from pinned host memory by the pipeline's first kernel
+// (a descriptor and 68 bytes an op) instead of up to three copies and a clear launched ahead
+// of it: about 20 us of a one-chunk call were spent before its first stage.
+__global__ __launch_bounds__(256) void k_stage_chunk(const ChunkDesc* chunk, const DevOp* ops, const int* index,
+                                                     ChunkDesc* d_chunk, DevOp* d_ops, int* d_index, Counters* c,
+                                                     int* queue) {
+    static_assert(sizeof(ChunkDesc) % 4 == 0 && sizeof(DevOp) == 64, "copied in words");
+    const int t = threadIdx.x, n = chunk->op_count;
+    if (t < (int)(sizeof(ChunkDesc) / 4)) reinterpret_cast<uint32_t*>(d_chunk)[t] = reinterpret_cast<const uint32_t*>(chunk)[t];
+    if (t == 0) *c = Counters{0, 0, 0, 0, 0, 0, 0, 0};
+    if (t < kNumQueues) queue[t] = 0;
+    for (int i = t; i < 4 * n; i += 256) reinterpret_cast<uint4*>(d_ops)[i] = reinterpret_cast<const uint4*>(ops)[i];
+    for (int i = t; i < n; i += 256) d_index[i] = index[i];
+}
+
 // ---------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------
+
+void launch_stage_chunk(const KArgs& a, const ChunkDesc* chunk, const DevOp* ops, const int* index, hipStream_t s) {
+    hipLaunchKernelGGL(k_stage_chunk, dim3(1), dim3(256), 0, s, chunk, ops, index, const_cast<ChunkDesc*>(a.chunks),
+                       const_cast<DevOp*>(a.ops), const_cast<int*>(a.op_index), a.counters, a.queue);
+}
 
 void launch_clear_counters(const KArgs& a, int n, hipStream_t s) {
     hipLaunchKernelGGL(k_clear_counters, dim3(ceil_div(std::max(n, kNumQueues), 256)), dim3(256), 0, s,
@@ -2289,6 +2349,14 @@ void launch_density(const KArgs& a, int chunks, hipStream_t s) {
     const int per_cu = a.density_per_cu ? a.density_per_cu : default_density_per_cu(a.G, a.ysplit, chunks, a.cus);
     const unsigned blocks = (unsigned)std::max(1L, std::min((long)per_cu * a.cus, items));
     LVN_LAUNCH_KIND(k_density, dim3(blocks), dim3(1024));
+}
+void launch_copy_mesh(const MeshCopy& c, hipStream_t s) {
+    const uint64_t most = std::max(c.bytes[0], std::max(c.bytes[1], c.bytes[2]));
+    const unsigned blocks = std::clamp(ceil_div((long)(most / 16), 256), 1u, 256u);
+    hipLaunchKernelGGL(k_copy_mesh, dim3(blocks, 3), dim3(256), 0, s, c);
+}
+void launch_export(const KArgs& a, char* out, hipStream_t s) {
+    hipLaunchKernelGGL(k_export, dim3(128, 3), dim3(256), 0, s, a, out);
 }
 void launch_csg(const KArgs& a, int chunks, hipStream_t s) {
     hipLaunchKernelGGL(k_csg, dim3(kCsgSlabs, chunks), dim3(256), 0, s, a);
@@ -2427,9 +2495,13 @@ void launch_stage(const KArgs& a, int chunks, int i, hipStream_t s) {
     }
 }
 
+void launch_stages(const KArgs& a, int chunks, hipStream_t s) {
+    for (int i = 0; i < kNumStages; ++i) launch_stage(a, chunks, i, s);
+}
+
 void launch_pipeline(const KArgs& a, int chunks, hipStream_t s) {
     launch_clear_counters(a, chunks, s);
-    for (int i = 0; i < kNumStages; ++i) launch_stage(a, chunks, i, s);
+    launch_stages(a, chunks, s);
 }
 
 }  // namespace lvn

@@ -125,6 +125,7 @@ struct Ctx {
     int* d_op_index = nullptr;
     int* h_op_index = nullptr;
     int ops_cap = 0, idx_cap = 0;
+    uint64_t ops_gen = 0;  // bumped when an op array moves (a freed one's address may come back)
     int* d_queue = nullptr;
     int* d_item_prefix = nullptr;
     int cus = 0;
@@ -134,10 +135,9 @@ struct Ctx {
     ClassPool mesh_pool;
     hipGraphExec_t exec = nullptr;       // the one-chunk pipeline, captured on first use
     hipGraph_t graph = nullptr;
-    const void* graph_ops = nullptr;     // op arrays the graph was captured with
-    const void* graph_index = nullptr;
+    uint64_t graph_ops = 0;              // ops_gen of the op arrays the graph was captured with
     uint64_t graph_gen = 0;              // global generation the graph was captured with
-    float* h_verts = nullptr;   // pinned read-back staging for one chunk's mesh (caps sized)
+    char* h_stage = nullptr;    // pinned staging: one chunk's counters, then its mesh (caps sized)
     SeamState* seams = nullptr; // seam stitching buffers, made on first use
     SimpState* simp = nullptr;  // simplifier buffers, made on first use
 
@@ -151,13 +151,13 @@ struct Ctx {
 struct Batch {
     Ctx ctx;
     int n = 0;                       // staged chunks
+    bool counted = false;            // ctx.h_counters holds the last run's counters of every staged chunk
     hipGraphExec_t exec = nullptr;   // captured pipeline for `graph_n` chunks
     hipGraph_t graph = nullptr;
     int graph_n = -1;
     long coarse = 0;                 // sum of the staged chunks' sample scales / 4 (chunk_load)
     int graph_lanes = 0, graph_lines = 0;  // crossing shapes the graph was captured with
-    const void* graph_ops = nullptr;   // op arrays the graph was captured with
-    const void* graph_index = nullptr;
+    uint64_t graph_ops = 0;            // ops_gen of the op arrays the graph was captured with
     uint64_t graph_gen = 0;
     unsigned long long* d_work = nullptr;
     lvn_tuning tuning = {0, 2, 8192, 8192, 0, 0, 0, {0}};  // 0 = by batch size
@@ -172,6 +172,13 @@ struct Batch {
 constexpr int kDefaultPersistPerCu = 2;
 constexpr int kDefaultRowBlocks = 8192;
 constexpr int kDefaultVoxelBlocks = 8192;
+
+// Device address of pinned host memory, or null for any other memory.
+char* pinned_view(void* p);
+// A mesh in device memory into the caller's host buffers (null ones are skipped), waited
+// for: one launch on `s` when they are pinned, else copies through the runtime.
+int read_mesh(const char* verts, size_t bv, const char* tris, size_t bt, const char* seams, size_t bs, lvn_vertex* v,
+              int32_t* tri, lvn_seam_node* sn, hipStream_t s);
 
 DevOp make_dev_op(const lvn_csg_op& op);
 // Kernel arguments of one arena with the default launch shapes of the one-chunk forms

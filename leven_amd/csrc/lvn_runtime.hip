@@ -312,6 +312,7 @@ int Ctx::allocate(int n, uint32_t fl, int nslots, int edge_cap, int voxel_cap) {
 }
 
 int Ctx::ensure_ops(int nops, int nidx) {
+    if (nops > ops_cap || nidx > idx_cap) ++ops_gen;
     if (nops > ops_cap) {
         if (d_ops) LVN_HIP(hipFree(d_ops));
         if (h_ops) LVN_HIP(hipHostFree(h_ops));
@@ -368,7 +369,7 @@ Ctx::~Ctx() {
     if (stream) (void)hipStreamSynchronize(stream);
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
-    if (h_verts) (void)hipHostFree(h_verts);
+    if (h_stage) (void)hipHostFree(h_stage);
     if (seams) destroy_seam_state(seams);
     if (simp) destroy_simp_state(simp);
     if (d_arena) (void)hipFree(d_arena);
@@ -426,8 +427,9 @@ char* ClassPool::take(size_t bytes, size_t* cap) {
     return static_cast<char*>(base.take(c));
 }
 
-// Upload one chunk descriptor + its op batch to slot 0.
-static int upload_single(Ctx* c, const ChunkDesc& cd_in, const std::vector<lvn_csg_op>& ops) {
+// One chunk descriptor + its op batch into the pinned staging, which the pipeline's first
+// kernel reads (launch_stage_chunk).  No call returns while work that reads it is pending.
+static int stage_single(Ctx* c, const ChunkDesc& cd_in, const std::vector<lvn_csg_op>& ops) {
     const int n = (int)ops.size();
     int r = c->ensure_ops(std::max(n, 1), std::max(n, 1));
     if (r) return r;
@@ -438,12 +440,6 @@ static int upload_single(Ctx* c, const ChunkDesc& cd_in, const std::vector<lvn_c
     c->h_chunks[0] = cd_in;
     c->h_chunks[0].op_start = 0;
     c->h_chunks[0].op_count = n;
-    if (n) {
-        LVN_HIP(hipMemcpyAsync(c->d_ops, c->h_ops, sizeof(DevOp) * n, hipMemcpyHostToDevice, c->stream));
-        LVN_HIP(hipMemcpyAsync(c->d_op_index, c->h_op_index, sizeof(int) * n, hipMemcpyHostToDevice, c->stream));
-    }
-    LVN_HIP(hipMemcpyAsync(c->d_chunks, c->h_chunks, sizeof(ChunkDesc), hipMemcpyHostToDevice, c->stream));
-    launch_clear_counters(c->kargs(), 1, c->stream);
     return LVN_OK;
 }
 
@@ -464,21 +460,32 @@ static KArgs single_args(const Ctx* c) {
     return a;
 }
 
-// The whole pipeline for slot 0 as one graph launch (captured once, again when the op
-// arrays move).
+// Pinned staging for the largest mesh a slot can hold, behind its counters.
+static int ensure_stage(Ctx* c) {
+    if (c->h_stage) return LVN_OK;
+    const size_t bytes = kExportHeader + 48 * (size_t)c->caps.voxels + 24 * (size_t)c->caps.quads +
+                         48 * (size_t)c->caps.seams;
+    LVN_HIP(hipHostMalloc(&c->h_stage, bytes, hipHostMallocDefault));
+    return LVN_OK;
+}
+
+// The whole pipeline for slot 0 and the export of its mesh into the staging as one graph
+// launch (captured once, again when the op arrays move).
 static int run_pipeline_graph(Ctx* c) {
-    if (!c->exec || c->graph_ops != c->d_ops || c->graph_index != c->d_op_index ||
-        c->graph_gen != g_state.generation) {
+    if (!c->exec || c->graph_ops != c->ops_gen || c->graph_gen != g_state.generation) {
         if (c->exec) LVN_HIP(hipGraphExecDestroy(c->exec));
         if (c->graph) LVN_HIP(hipGraphDestroy(c->graph));
         c->exec = nullptr;
         c->graph = nullptr;
+        const int r = ensure_stage(c);
+        if (r) return r;
         LVN_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        launch_pipeline(single_args(c), 1, c->stream);
+        launch_stage_chunk(single_args(c), c->h_chunks, c->h_ops, c->h_op_index, c->stream);
+        launch_stages(single_args(c), 1, c->stream);
+        launch_export(single_args(c), c->h_stage, c->stream);
         LVN_HIP(hipStreamEndCapture(c->stream, &c->graph));
         LVN_HIP(hipGraphInstantiate(&c->exec, c->graph, nullptr, nullptr, 0));
-        c->graph_ops = c->d_ops;
-        c->graph_index = c->d_op_index;
+        c->graph_ops = c->ops_gen;
         c->graph_gen = g_state.generation;
     }
     LVN_HIP(hipGraphLaunch(c->exec, c->stream));
@@ -491,9 +498,10 @@ static int run_field(Ctx* c, const int32_t* min, int32_t size, const std::vector
     ChunkDesc cd;
     fill_chunk_desc(cd, min, size, c->N);
     set_cached(cd, cached);
-    int r = upload_single(c, cd, ops);
+    int r = stage_single(c, cd, ops);
     if (r) return r;
     const KArgs a = single_args(c);
+    launch_stage_chunk(a, c->h_chunks, c->h_ops, c->h_op_index, c->stream);
     launch_density(a, 1, c->stream);  // or the cached field's materials
     if (!ops.empty()) launch_csg(a, 1, c->stream);
     launch_edge_rows(a, 1, c->stream);
@@ -582,27 +590,71 @@ static int cache_mesh(Ctx* c, const Counters& k, MeshEntry* m) {
     m->d = c->mesh_pool.take(std::max<size_t>(bv + bt + bs, 1), &m->cap);
     if (!m->d) return LVN_ERR_NOMEM;
     const char* slot = c->d_arena;
-    if (bv) LVN_HIP(hipMemcpyAsync(m->d, slot + c->L.verts, bv, hipMemcpyDeviceToDevice, c->stream));
-    if (bt) LVN_HIP(hipMemcpyAsync(m->d + bv, slot + c->L.tris, bt, hipMemcpyDeviceToDevice, c->stream));
-    if (bs) LVN_HIP(hipMemcpyAsync(m->d + bv + bt, slot + c->L.seams, bs, hipMemcpyDeviceToDevice, c->stream));
+    if (bv + bt + bs == 0) return LVN_OK;
+    launch_copy_mesh({{slot + c->L.verts, slot + c->L.tris, slot + c->L.seams},
+                      {m->d, m->d + bv, m->d + bv + bt},
+                      {bv, bt, bs}}, c->stream);
+    LVN_HIP(hipGetLastError());
     return LVN_OK;
 }
 
 // ExportMeshBuffer (src/compute_octree.cpp:326-347): a cached mesh into the caller's
-// buffers through pinned staging (one read-back, one host copy per array).
-static int export_mesh(Ctx* c, const MeshEntry& m, lvn_vertex* v, int32_t* tri, lvn_seam_node* s) {
+// buffers through pinned staging (one read-back, one host copy per array); `staged` when the
+// pipeline's export has put it there.
+static int export_mesh(Ctx* c, const MeshEntry& m, bool staged, lvn_vertex* v, int32_t* tri, lvn_seam_node* s) {
     const size_t bv = 48 * (size_t)m.V, bt = 12 * (size_t)m.T, bs = 48 * (size_t)m.S;
     if (bv + bt + bs == 0) return LVN_OK;
-    if (!c->h_verts) {  // staging sized for the largest mesh a slot can hold
-        LVN_HIP(hipHostMalloc(&c->h_verts, 48 * (size_t)c->caps.voxels + 24 * (size_t)c->caps.quads +
-                                               48 * (size_t)c->caps.seams, hipHostMallocDefault));
+    if (!staged) {
+        const int r = ensure_stage(c);
+        if (r) return r;
+        LVN_HIP(hipMemcpyAsync(c->h_stage + kExportHeader, m.d, bv + bt + bs, hipMemcpyDeviceToHost, c->stream));
+        LVN_HIP(hipStreamSynchronize(c->stream));
     }
-    char* h = reinterpret_cast<char*>(c->h_verts);
-    LVN_HIP(hipMemcpyAsync(h, m.d, bv + bt + bs, hipMemcpyDeviceToHost, c->stream));
-    LVN_HIP(hipStreamSynchronize(c->stream));
+    const char* h = c->h_stage + kExportHeader;
     if (bv && v) std::memcpy(v, h, bv);
     if (bt && tri) std::memcpy(tri, h + bv, bt);
     if (bs && s) std::memcpy(s, h + bv + bt, bs);
+    return LVN_OK;
+}
+
+char* pinned_view(void* p) {
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();  // memory the runtime does not know
+        return nullptr;
+    }
+    return at.type == hipMemoryTypeHost ? static_cast<char*>(at.devicePointer) : nullptr;
+}
+
+int read_mesh(const char* verts, size_t bv, const char* tris, size_t bt, const char* seams, size_t bs, lvn_vertex* v,
+              int32_t* tri, lvn_seam_node* sn, hipStream_t s) {
+    MeshCopy c = {{verts, tris, seams}, {nullptr, nullptr, nullptr}, {v ? bv : 0, tri ? bt : 0, sn ? bs : 0}};
+    void* out[3] = {v, tri, sn};
+    bool pinned = true;
+    for (int i = 0; i < 3; ++i) {
+        if (!c.bytes[i]) continue;
+        c.dst[i] = pinned_view(out[i]);
+        pinned = pinned && c.dst[i] && ((uintptr_t)c.dst[i] & 3) == 0;
+    }
+    if (c.bytes[0] + c.bytes[1] + c.bytes[2] == 0) return LVN_OK;
+    if (pinned) {
+        launch_copy_mesh(c, s);
+        LVN_HIP(hipGetLastError());
+        LVN_HIP(hipStreamSynchronize(s));
+        return LVN_OK;
+    }
+    for (int i = 0; i < 3; ++i)
+        if (c.bytes[i]) LVN_HIP(hipMemcpy(out[i], c.src[i], c.bytes[i], hipMemcpyDeviceToHost));
+    return LVN_OK;
+}
+
+// The last run's counters of every staged chunk in ctx.h_counters, read once per run.
+static int count_batch(Batch* b) {
+    if (b->counted) return LVN_OK;
+    Ctx* c = &b->ctx;
+    LVN_HIP(hipMemcpyAsync(c->h_counters, c->d_counters, sizeof(Counters) * b->n, hipMemcpyDeviceToHost, c->stream));
+    LVN_HIP(hipStreamSynchronize(c->stream));
+    b->counted = true;
     return LVN_OK;
 }
 
@@ -640,6 +692,7 @@ static int stage_batch(Batch* b, int n, const lvn_chunk_req* reqs) {
     LVN_HIP(hipMemcpyAsync(c->d_chunks, c->h_chunks, sizeof(ChunkDesc) * n, hipMemcpyHostToDevice, c->stream));
     LVN_HIP(hipStreamSynchronize(c->stream));
     b->n = n;
+    b->counted = false;
     b->coarse = 0;
     for (int i = 0; i < n; ++i) b->coarse += c->h_chunks[i].scale / 4;
     b->simplified = false;
@@ -687,7 +740,7 @@ static KArgs batch_args(const Batch* b) { return batch_args(b, effective_tuning(
 // One pass of the pipeline without the graph, each stage bracketed by HIP events.
 static int time_stages(Batch* b, const KArgs& a, float* stage_ms) {
     Ctx* c = &b->ctx;
-    b->simplified = false;
+    b->simplified = b->counted = false;
     hipEvent_t ev[kNumStages + 1];
     for (auto& e : ev) LVN_HIP(hipEventCreate(&e));
     launch_clear_counters(a, std::max(b->n, 1), c->stream);
@@ -991,6 +1044,7 @@ int lvn_generate_chunk_mesh(lvn_ctx* ctx, const int32_t min[3], int32_t size, lv
     const Key key = make_key(min, size);
     auto it = c->meshes.find(key);
     const MeshEntry* m = nullptr;
+    bool staged = false;
     if (it != c->meshes.end()) {
         m = &it->second;  // LoadOctree cache hit (src/compute_octree.cpp:157-163)
     } else {
@@ -1003,13 +1057,12 @@ int lvn_generate_chunk_mesh(lvn_ctx* ctx, const int32_t min[3], int32_t size, lv
         ChunkDesc cd;
         fill_chunk_desc(cd, min, size, c->N);
         set_cached(cd, cached);
-        int r = upload_single(c, cd, ops);
+        int r = stage_single(c, cd, ops);
         if (r) return r;
         r = run_pipeline_graph(c);
         if (r) return r;
-        Counters k;
-        r = read_counters(c, &k);
-        if (r) return r;
+        LVN_HIP(hipStreamSynchronize(c->stream));
+        const Counters k = *reinterpret_cast<const Counters*>(c->h_stage);
         if (k.status) return LVN_ERR_OVERFLOW;
         if (!ops.empty()) {
             r = store_field(c, key, k.edges, (int)g_state.ops.size());
@@ -1020,12 +1073,13 @@ int lvn_generate_chunk_mesh(lvn_ctx* ctx, const int32_t min[3], int32_t size, lv
         r = cache_mesh(c, k, &fresh);
         if (r) return r;
         m = &(c->meshes[key] = fresh);
+        staged = true;
     }
     *nv = m->V;
     *nt = m->T;
     *ns = m->S;
     if (m->V > v_cap || m->T > tri_cap || m->S > s_cap) return LVN_ERR_CAPACITY;
-    return export_mesh(c, *m, v, tri, s);
+    return export_mesh(c, *m, staged, v, tri, s);
 }
 
 int lvn_generate_chunk_mesh_noalloc(int32_t n, uint32_t flags, const int32_t min[3], int32_t size, lvn_vertex* v,
@@ -1127,7 +1181,7 @@ int lvn_batch_run(lvn_batch* bh) {
     if (b->n == 0) return LVN_OK;
     Ctx* c = &b->ctx;
     const lvn_tuning t = effective_tuning(b);  // may change with the staged chunks' scales
-    if (b->graph_n != b->n || b->graph_lanes != t.cross_lanes || b->graph_lines != t.height_lines || b->graph_ops != c->d_ops || b->graph_index != c->d_op_index ||
+    if (b->graph_n != b->n || b->graph_lanes != t.cross_lanes || b->graph_lines != t.height_lines || b->graph_ops != c->ops_gen ||
         b->graph_gen != g_state.generation) {
         if (b->exec) LVN_HIP(hipGraphExecDestroy(b->exec));
         if (b->graph) LVN_HIP(hipGraphDestroy(b->graph));
@@ -1139,13 +1193,12 @@ int lvn_batch_run(lvn_batch* bh) {
         LVN_HIP(hipStreamEndCapture(c->stream, &b->graph));
         LVN_HIP(hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
         b->graph_n = b->n;
-        b->graph_ops = c->d_ops;
-        b->graph_index = c->d_op_index;
+        b->graph_ops = c->ops_gen;
         b->graph_gen = g_state.generation;
         b->graph_lanes = t.cross_lanes;
         b->graph_lines = t.height_lines;
     }
-    b->simplified = false;
+    b->simplified = b->counted = false;
     LVN_HIP(hipGraphLaunch(b->exec, c->stream));
     return LVN_OK;
 }
@@ -1244,7 +1297,7 @@ int lvn_batch_work(lvn_batch* bh, uint64_t* work) {
     KArgs a = batch_args(b);
     a.work = b->d_work;
     LVN_HIP(hipMemsetAsync(b->d_work, 0, sizeof(unsigned long long) * 8, c->stream));
-    b->simplified = false;
+    b->simplified = b->counted = false;
     if (b->n) launch_pipeline(a, b->n, c->stream);
     unsigned long long h[8];
     LVN_HIP(hipMemcpyAsync(h, b->d_work, sizeof(h), hipMemcpyDeviceToHost, c->stream));
@@ -1258,8 +1311,8 @@ int lvn_batch_counts(lvn_batch* bh, int32_t* counts) {
     if (!b || !counts) return LVN_ERR_INVALID;
     Ctx* c = &b->ctx;
     if (b->n == 0) return LVN_OK;
-    LVN_HIP(hipMemcpyAsync(c->h_counters, c->d_counters, sizeof(Counters) * b->n, hipMemcpyDeviceToHost, c->stream));
-    LVN_HIP(hipStreamSynchronize(c->stream));
+    const int r = count_batch(b);
+    if (r) return r;
     for (int i = 0; i < b->n; ++i) {
         const Counters& k = c->h_counters[i];
         counts[6 * i + 0] = k.edges;
@@ -1277,10 +1330,9 @@ int lvn_batch_get_mesh(lvn_batch* bh, int32_t i, lvn_vertex* v, int32_t v_cap, i
     Batch* b = reinterpret_cast<Batch*>(bh);
     if (!b || i < 0 || i >= b->n || !nv || !nt || !ns) return LVN_ERR_INVALID;
     Ctx* c = &b->ctx;
-    Counters k;
-    LVN_HIP(hipMemcpyAsync(&c->h_counters[i], c->d_counters + i, sizeof(Counters), hipMemcpyDeviceToHost, c->stream));
-    LVN_HIP(hipStreamSynchronize(c->stream));
-    k = c->h_counters[i];
+    const int r = count_batch(b);
+    if (r) return r;
+    const Counters k = c->h_counters[i];
     if (k.status) return LVN_ERR_OVERFLOW;
     const bool simp = b->simplified && (size_t)(2 * i + 1) < b->simp_counts.size();
     const int V = simp ? b->simp_counts[2 * i] : k.edges > 0 && k.quads > 0 ? k.voxels : 0;
@@ -1291,10 +1343,8 @@ int lvn_batch_get_mesh(lvn_batch* bh, int32_t i, lvn_vertex* v, int32_t v_cap, i
     *ns = S;
     if (V > v_cap || T > tri_cap || S > s_cap) return LVN_ERR_CAPACITY;
     const char* slot = c->d_arena + (uint64_t)i * c->L.slot_bytes;
-    if (V && v) LVN_HIP(hipMemcpy(v, slot + c->L.verts, sizeof(lvn_vertex) * (size_t)V, hipMemcpyDeviceToHost));
-    if (T && tri) LVN_HIP(hipMemcpy(tri, slot + c->L.tris, 12 * (size_t)T, hipMemcpyDeviceToHost));
-    if (S && s) LVN_HIP(hipMemcpy(s, slot + c->L.seams, sizeof(lvn_seam_node) * (size_t)S, hipMemcpyDeviceToHost));
-    return LVN_OK;
+    return read_mesh(slot + c->L.verts, sizeof(lvn_vertex) * (size_t)V, slot + c->L.tris, 12 * (size_t)T,
+                     slot + c->L.seams, sizeof(lvn_seam_node) * (size_t)S, v, tri, s, c->stream);
 }
 
 int lvn_debug_chunk_stages(lvn_ctx* ctx, const int32_t min[3], int32_t size, const lvn_csg_op* ops, int32_t nops,

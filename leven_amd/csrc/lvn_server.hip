@@ -634,12 +634,8 @@ int lvn_server_get_mesh(lvn_server* sh, int64_t ticket, lvn_vertex* v, int32_t v
     if (e.nv > v_cap || e.nt > tri_cap || e.ns > s_cap) return LVN_ERR_CAPACITY;
     const Ctx& c = s->arena;
     const char* slot = c.d_arena + (uint64_t)e.slot * c.L.slot_bytes;
-    if (e.nv && v && hipMemcpy(v, slot + c.L.verts, sizeof(lvn_vertex) * (size_t)e.nv, hipMemcpyDeviceToHost))
-        return LVN_ERR_DEVICE;
-    if (e.nt && tri && hipMemcpy(tri, slot + c.L.tris, 12 * (size_t)e.nt, hipMemcpyDeviceToHost)) return LVN_ERR_DEVICE;
-    if (e.ns && sn && hipMemcpy(sn, slot + c.L.seams, sizeof(lvn_seam_node) * (size_t)e.ns, hipMemcpyDeviceToHost))
-        return LVN_ERR_DEVICE;
-    return LVN_OK;
+    return read_mesh(slot + c.L.verts, sizeof(lvn_vertex) * (size_t)e.nv, slot + c.L.tris, 12 * (size_t)e.nt,
+                     slot + c.L.seams, sizeof(lvn_seam_node) * (size_t)e.ns, v, tri, sn, c.stream);
 }
 
 int lvn_server_set_tuning(lvn_server* sh, const lvn_tuning* t) {
