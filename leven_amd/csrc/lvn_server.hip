@@ -451,6 +451,7 @@ void Server::admit_and_launch() {
         if (r != LVN_OK) {
             std::lock_guard<std::mutex> lock(mu);
             error = r;
+            cv.notify_all();  // a drain may be waiting already
         }
     }
 }
