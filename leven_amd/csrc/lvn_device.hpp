@@ -478,24 +478,27 @@ __device__ __forceinline__ float3 normalize_or_zero(float x, float y, float z) {
 // Octree codes (cl/octree.cl:34-72)
 // ---------------------------------------------------------------------------
 
-__device__ __forceinline__ uint32_t code_for_position(int x, int y, int z, int depth) {
-    uint32_t code = 1;
-    for (int d = depth - 1; d >= 0; --d)
-        code = (code << 3) | (uint32_t)((((x >> d) & 1) << 2) | (((y >> d) & 1) << 1) | ((z >> d) & 1));
-    return code;
+// The codes interleave x, y and z (bits 3 d + 2, 3 d + 1, 3 d) below a leading one at bit
+// 3 depth; depth is at most 6, so a coordinate's six bits are spread and gathered by masks.
+__device__ __forceinline__ uint32_t spread3(uint32_t v) {
+    v = (v | (v << 8)) & 0x300fu;
+    v = (v | (v << 4)) & 0x30c3u;
+    return (v | (v << 2)) & 0x9249u;
+}
+__device__ __forceinline__ int gather3(uint32_t v) {
+    v &= 0x9249u;
+    v = (v | (v >> 2)) & 0x30c3u;
+    v = (v | (v >> 4)) & 0x300fu;
+    return (int)((v | (v >> 8)) & 0x3fu);
 }
 
-__device__ __forceinline__ int3 position_for_code(uint32_t code, int max_depth) {
-    const int node_depth = (32 - __clz(code)) / 3;
-    int3 p = make_int3(0, 0, 0);
-    for (int i = max_depth - node_depth; i < max_depth; ++i) {
-        const uint32_t c = code & 7u;
-        code >>= 3;
-        p.x |= (int)((c >> 2) & 1u) << i;
-        p.y |= (int)((c >> 1) & 1u) << i;
-        p.z |= (int)(c & 1u) << i;
-    }
-    return p;
+__device__ __forceinline__ uint32_t code_for_position(int x, int y, int z, int depth) {
+    return (1u << (3 * depth)) | (spread3((uint32_t)x) << 2) | (spread3((uint32_t)y) << 1) | spread3((uint32_t)z);
+}
+
+// The position of a leaf's code (leading one at bit 3 depth).
+__device__ __forceinline__ int3 position_for_code(uint32_t code, int depth) {
+    return make_int3(gather3(code >> 2), gather3(code >> 1), gather3(code & ~(1u << (3 * depth))));
 }
 
 }  // namespace lvn

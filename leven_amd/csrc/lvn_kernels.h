@@ -47,8 +47,6 @@ struct KArgs {
 // line-height passes share their items within workgroups instead; the rest are spare).
 constexpr int kNumQueues = 8;
 
-enum ScanKind { kScanEdges = 0, kScanVoxels = 1, kScanQuadsSeams = 2 };
-
 void launch_clear_counters(const KArgs& a, int n, hipStream_t s);
 
 constexpr int kNumStages = LVN_NUM_STAGES;
@@ -59,13 +57,12 @@ void launch_stage(const KArgs& a, int chunks, int i, hipStream_t s);
 // Stage launchers: `chunks` chunk slots [0, chunks) processed by one launch each.
 void launch_density(const KArgs& a, int chunks, hipStream_t s);
 void launch_csg(const KArgs& a, int chunks, hipStream_t s);
-void launch_edge_rows(const KArgs& a, int chunks, hipStream_t s);
-void launch_scan(const KArgs& a, int chunks, ScanKind kind, hipStream_t s);
-void launch_edge_compact(const KArgs& a, int chunks, hipStream_t s);
+void launch_rows(const KArgs& a, int chunks, hipStream_t s);             // solid, edge and voxel rows
+void launch_scan_rows(const KArgs& a, int chunks, hipStream_t s);        // edge rows and voxel segments
+void launch_compact(const KArgs& a, int chunks, hipStream_t s);          // edge lists and voxel codes
 void launch_edge_cross(const KArgs& a, int chunks, hipStream_t s);
-void launch_voxel_rows(const KArgs& a, int chunks, hipStream_t s);
-void launch_voxel_compact(const KArgs& a, int chunks, hipStream_t s);
 void launch_qef(const KArgs& a, int chunks, hipStream_t s);
+void launch_scan_quads_seams(const KArgs& a, int chunks, hipStream_t s);
 void launch_emit(const KArgs& a, int chunks, hipStream_t s);
 
 // y-segments per density column when the launch shapes leave it open.

@@ -109,6 +109,13 @@ __device__ __forceinline__ bool chunk_mat_free(const KArgs& a, const ChunkDesc& 
     return a.mat_free && cd.op_count == 0 && cd.mode != kModeCached;
 }
 
+// A chunk whose samples the density pass found all solid or all air (and no brush or cached
+// field changes): it has no edges and no voxels, and the bookkeeping kernels pass it by.  Half
+// of a clipmap's chunks are such.
+__device__ __forceinline__ bool chunk_uniform(const KArgs& a, int chunk) {
+    return chunk_mat_free(a, a.chunks[chunk]) && a.counters[chunk].sides != (kSomeSolid | kSomeAir);
+}
+
 template <bool kCount, int kKind>
 __device__ __forceinline__ void density_column(const KArgs& a, const NoiseLds& T, int chunk, int seg, int g) {
     const Geometry& G = a.G;
@@ -149,7 +156,8 @@ __device__ __forceinline__ void density_column(const KArgs& a, const NoiseLds& T
     float* dens = slot_ptr<float>(a, chunk, a.L.density);
     __half* dens16 = slot_ptr<__half>(a, chunk, a.L.density);
     unsigned caves = 0;
-    uint64_t word = 0;
+    uint64_t word = 0, solid = 0, air = 0;
+    const uint64_t all = __ballot(valid);
     for (int y = y0; y < y1; ++y) {
         const float wy = (float)(y * cd.scale + cd.off[1]);
         const float d = combine<kKind>(a.F, T, wy - H, wx, wy, wz);
@@ -168,6 +176,8 @@ __device__ __forceinline__ void density_column(const KArgs& a, const NoiseLds& T
         }
         if (planes) {
             const uint64_t bits = __ballot(valid && m != (uint8_t)kAir);
+            solid |= bits;
+            air |= all & ~bits;
             const int j = (y - y0) & 63;
             if (lane == j) word = bits;
             if (j == 63 || y == y1 - 1) {
@@ -175,6 +185,9 @@ __device__ __forceinline__ void density_column(const KArgs& a, const NoiseLds& T
             }
         }
     }
+    if (planes && lane == 0)
+        slot_ptr<uint8_t>(a, chunk, a.L.sides)[seg * G.col_groups + g] =
+            (uint8_t)((solid ? kSomeSolid : 0) | (air ? kSomeAir : 0));
     if constexpr (kCount) {
         if (valid) {
             atomicAdd(&a.work[0], 1ull);
@@ -290,7 +303,7 @@ __global__ __launch_bounds__(256) void k_csg(KArgs a) {
 // ---------------------------------------------------------------------------
 // Edge classification (FindFieldEdges, cl/density_field.cl:41-76) as bit rows.
 // k_solid_rows packs the post-CSG "not air" test of every sample into rows of
-// F bits (y, z fixed); k_edge_rows turns three neighbouring rows into the x, y
+// F bits (y, z fixed); k_rows turns three neighbouring rows into the x, y
 // and z edge masks of a hermite row with a few 64-bit operations, so a chunk's
 // 3 H^3 edge slots are classified by H^2 threads.
 // ---------------------------------------------------------------------------
@@ -305,6 +318,14 @@ __global__ __launch_bounds__(256) void k_solid_rows(KArgs a) {
     const uint32_t* mat = slot_ptr<const uint32_t>(a, chunk, a.L.mat);
     uint64_t* S = slot_ptr<uint64_t>(a, chunk, a.L.solid);
     if (chunk_mat_free(a, a.chunks[chunk])) {  // uniform over the workgroup
+        // the sides its items met, for the kernels from here on (an atomic per item instead
+        // cost the density pass 50 us on 1,800 chunks)
+        const uint8_t* met = slot_ptr<const uint8_t>(a, chunk, a.L.sides);
+        int mine = 0;
+        for (int i = lane; i < G.col_groups * a.ysplit; i += 64) mine |= met[i];
+        const int sides = (__ballot(mine & kSomeSolid) ? kSomeSolid : 0) | (__ballot(mine & kSomeAir) ? kSomeAir : 0);
+        if (blockIdx.x == 0 && threadIdx.x == 0) a.counters[chunk].sides = sides;
+        if (sides != (kSomeSolid | kSomeAir)) return;
         // Row (y, z) is bits [F z, F z + F) of plane y: a 64-bit window of two or three
         // consecutive group words, then F - 64 bits above it (none when F <= 64).
         const uint64_t* P = slot_ptr<const uint64_t>(a, chunk, a.L.planes);
@@ -351,17 +372,21 @@ __global__ __launch_bounds__(256) void k_solid_rows(KArgs a) {
     }
 }
 
-__global__ __launch_bounds__(256) void k_edge_rows(KArgs a) {
-    const int chunk = blockIdx.y;
+// Edge rows by the first `edge_blocks` workgroups of a chunk, voxel rows by the others: both
+// read only the solid rows, so one launch serves both (and the kernels after it: one scan,
+// one compaction), three launches of about 5 us less for one chunk.  A row without edges
+// stores its count alone: its words are never read (the QEF and the line heights look only
+// at rows with edges), which were 70% of the 243 MB of words of a clipmap batch.
+// Row counts are packed: edges in the low half, y-edges in the high half.
+__device__ __forceinline__ void edge_rows(const KArgs& a, int chunk, int thread, int threads) {
     const Geometry& G = a.G;
     const int H = G.H, F = G.F;
     const uint64_t* S = slot_ptr<const uint64_t>(a, chunk, a.L.solid);
     uint64_t* E = slot_ptr<uint64_t>(a, chunk, a.L.e_rows);
-    int* count = slot_ptr<int>(a, chunk, a.L.e_count);
-    int* count_y = slot_ptr<int>(a, chunk, a.L.e_count_y);
+    uint32_t* count = slot_ptr<uint32_t>(a, chunk, a.L.e_count);
     const uint64_t mlo = H >= 64 ? ~0ull : ((1ull << H) - 1ull);  // x in [0, H)
     const uint64_t mhi = H > 64 ? 1ull : 0ull;                     // x = 64
-    for (int r = thread_in_chunk(); r < G.edge_rows; r += threads_per_chunk()) {
+    for (int r = thread; r < G.edge_rows; r += threads) {
         const int z = div_magic(r, G.magic_h), y = r - z * H;
         const int s0 = y + F * z;
         const uint64_t alo = S[2 * s0], ahi = S[2 * s0 + 1];                   // (y, z)
@@ -372,68 +397,125 @@ __global__ __launch_bounds__(256) void k_edge_rows(KArgs a) {
         const uint64_t ylo = (alo ^ blo) & mlo, yhi = (ahi ^ bhi) & mhi;
         const uint64_t zlo = (alo ^ clo) & mlo, zhi = (ahi ^ chi) & mhi;
         const uint64_t hi = xhi | (yhi << 1) | (zhi << 2);
-        E[4 * r] = xlo;
-        E[4 * r + 1] = ylo;
-        E[4 * r + 2] = zlo;
-        E[4 * r + 3] = hi;
-        count[r] = __popcll(xlo) + __popcll(ylo) + __popcll(zlo) + __popcll(hi);
-        count_y[r] = __popcll(ylo) + (int)((hi >> 1) & 1ull);
+        const int ny = __popcll(ylo) + (int)((hi >> 1) & 1ull);
+        const int n = __popcll(xlo) + __popcll(ylo) + __popcll(zlo) + __popcll(hi);
+        if (n) {
+            E[4 * r] = xlo;
+            E[4 * r + 1] = ylo;
+            E[4 * r + 2] = zlo;
+            E[4 * r + 3] = hi;
+        }
+        count[r] = (uint32_t)n | ((uint32_t)ny << 16);
     }
 }
 
-// ---------------------------------------------------------------------------
-// Exclusive scan of segment counts, one workgroup per chunk (replaces the
-// recursive Scan / ExclusiveScan with its blocking readback, src/compute.cpp:344-396).
-// ---------------------------------------------------------------------------
-// Exclusive scan of count[0, n) into base[0, n) by one 1024-thread workgroup;
-// returns the total to every thread.
-__device__ __forceinline__ int block_scan(const int* count, int* base, int n, int* buf) {
-    const int tid = threadIdx.x;
-    const int per = (n + 1023) / 1024;
-    const int b0 = min(n, tid * per), b1 = min(n, b0 + per);
-    int sum = 0;
-    for (int i = b0; i < b1; ++i) sum += count[i];
-    __syncthreads();
-    buf[tid] = sum;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-        const int v = tid >= off ? buf[tid - off] : 0;
-        __syncthreads();
-        buf[tid] += v;
-        __syncthreads();
+// A voxel is active when its 8 corners are not all solid or all air (FindActiveVoxels,
+// cl/octree.cl:142-223): over a voxel row, the AND and OR of the four sample rows around it
+// and their x + 1 shifts.  Segment `seg` of 64 voxels holds 64 / N voxel rows.
+__device__ __forceinline__ void voxel_rows(const KArgs& a, int chunk, int thread, int threads) {
+    const Geometry& G = a.G;
+    const int N = G.N, F = G.F;
+    const uint64_t* S = slot_ptr<const uint64_t>(a, chunk, a.L.solid);
+    uint64_t* vmask = slot_ptr<uint64_t>(a, chunk, a.L.v_mask);
+    const int per_seg = N >= 64 ? 1 : 64 / N;
+    const uint64_t nmask = N >= 64 ? ~0ull : ((1ull << N) - 1ull);
+    for (int seg = thread; seg < G.voxel_segs; seg += threads) {
+        uint64_t m = 0;
+        for (int k = 0; k < per_seg; ++k) {
+            const int vr = seg * per_seg + k;  // voxel row y + N z
+            const int y = vr & (N - 1), z = vr >> G.depth;
+            const int s0 = y + F * z;
+            const int rows[4] = {s0, s0 + 1, s0 + F, s0 + F + 1};
+            uint64_t all = ~0ull, any = 0ull;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const uint64_t lo = S[2 * rows[c]], hi = S[2 * rows[c] + 1];
+                const uint64_t nx = shift_next(lo, hi);
+                all &= lo & nx;
+                any |= lo | nx;
+            }
+            m |= ((any & ~all) & nmask) << (k * N);
+        }
+        vmask[seg] = m;
     }
-    int run = buf[tid] - sum;
-    for (int i = b0; i < b1; ++i) {
-        base[i] = run;
-        run += count[i];
-    }
-    return buf[1023];
 }
 
-// Edge (kScanEdges) or voxel (kScanVoxels) scan: the stage is a template parameter
-// (with a runtime selector hipcc, ROCm 7.2, gfx950, kept one stage's counter
-// address for the other's total).
-template <int KIND>
-__global__ __launch_bounds__(1024) void k_scan(KArgs a) {
-    __shared__ int buf[1024];
+__global__ __launch_bounds__(256) void k_rows(KArgs a, int edge_blocks) {
     const int chunk = blockIdx.y;
+    if (chunk_uniform(a, chunk)) return;
+    if ((int)blockIdx.x < edge_blocks)
+        edge_rows(a, chunk, thread_in_chunk(), edge_blocks * 256);
+    else
+        voxel_rows(a, chunk, thread_in_chunk() - edge_blocks * 256, ((int)gridDim.x - edge_blocks) * 256);
+}
+
+// ---------------------------------------------------------------------------
+// Exclusive scans, one workgroup per chunk and list (replaces the recursive Scan /
+// ExclusiveScan with its blocking readback, src/compute.cpp:344-396).
+// ---------------------------------------------------------------------------
+// Two counts scanned at once, in the halves of a 64-bit sum: get(i) for i in [0, n), put(i,
+// sum before i); the total is returned to every thread.  Each of the 1,024 threads sums a
+// run of elements, its wave scans the sums by shuffles, and one barrier joins the waves (the
+// 10-step scan through LDS with two barriers a step, once per count, took 8.5 us for a
+// 64^3 chunk's rows; this takes 4).
+constexpr int kScanThreads = 1024;
+template <typename Get, typename Put>
+__device__ __forceinline__ uint64_t block_scan(int n, uint64_t* wsum, Get get, Put put) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int per = (n + kScanThreads - 1) / kScanThreads;
+    const int b0 = min(n, tid * per), b1 = min(n, b0 + per);
+    uint64_t sum = 0;
+    for (int i = b0; i < b1; ++i) sum += get(i);
+    uint64_t run = sum;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint64_t u = __shfl_up(run, off);
+        if (lane >= off) run += u;
+    }
+    __syncthreads();  // wsum may still be read from an earlier scan
+    if (lane == 63) wsum[wave] = run;
+    __syncthreads();
+    uint64_t before = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < kScanThreads / 64; ++w) {
+        const uint64_t v = wsum[w];
+        if (w < wave) before += v;
+        total += v;
+    }
+    uint64_t at = before + run - sum;
+    for (int i = b0; i < b1; ++i) {
+        put(i, at);
+        at += get(i);
+    }
+    return total;
+}
+__device__ __forceinline__ uint64_t halves(uint32_t packed) { return (packed & 0xffffu) | ((uint64_t)(packed >> 16) << 32); }
+
+// Edge rows (blockIdx.x 0) and voxel segments (1).
+__global__ __launch_bounds__(kScanThreads) void k_scan_rows(KArgs a) {
+    __shared__ uint64_t wsum[kScanThreads / 64];
+    const int chunk = blockIdx.y;
+    if (chunk_uniform(a, chunk)) return;  // its counters stay cleared
     Counters* cnt = a.counters + chunk;
-    if constexpr (KIND == kScanEdges) {
-        const int t = block_scan(slot_ptr<const int>(a, chunk, a.L.e_count), slot_ptr<int>(a, chunk, a.L.e_base),
-                                 a.G.edge_rows, buf);
-        const int ty = block_scan(slot_ptr<const int>(a, chunk, a.L.e_count_y), slot_ptr<int>(a, chunk, a.L.e_base_y),
-                                  a.G.edge_rows, buf);
+    if (blockIdx.x == 0) {
+        const uint32_t* count = slot_ptr<const uint32_t>(a, chunk, a.L.e_count);
+        int2* base = slot_ptr<int2>(a, chunk, a.L.e_base);
+        const uint64_t t = block_scan(a.G.edge_rows, wsum, [&](int i) { return halves(count[i]); },
+                                      [&](int i, uint64_t at) { base[i] = make_int2((int)(uint32_t)at, (int)(at >> 32)); });
         if (threadIdx.x == 0) {
-            cnt->edges = min(t, a.caps.edges);
-            cnt->edges_y = min(ty, a.caps.edges);
-            if (t > a.caps.edges) atomicOr(&cnt->status, kStatusEdgeOverflow);
+            const int n = (int)(uint32_t)t;
+            cnt->edges = min(n, a.caps.edges);
+            cnt->edges_y = min((int)(t >> 32), a.caps.edges);
+            if (n > a.caps.edges) atomicOr(&cnt->status, kStatusEdgeOverflow);
         }
     } else {
-        const int t = block_scan(slot_ptr<const int>(a, chunk, a.L.v_count), slot_ptr<int>(a, chunk, a.L.v_base),
-                                 a.G.voxel_segs, buf);
+        const uint64_t* mask = slot_ptr<const uint64_t>(a, chunk, a.L.v_mask);
+        int* base = slot_ptr<int>(a, chunk, a.L.v_base);
+        const int n = (int)block_scan(a.G.voxel_segs, wsum, [&](int i) { return (uint64_t)__popcll(mask[i]); },
+                                      [&](int i, uint64_t at) { base[i] = (int)at; });
         if (threadIdx.x == 0) {
-            cnt->voxels = min(t, a.caps.voxels);
-            if (t > a.caps.voxels) atomicOr(&cnt->status, kStatusVoxelOverflow);
+            cnt->voxels = min(n, a.caps.voxels);
+            if (n > a.caps.voxels) atomicOr(&cnt->status, kStatusVoxelOverflow);
         }
     }
 }
@@ -466,13 +548,11 @@ __device__ __forceinline__ uint64_t readlane64(uint64_t v, int j) {
     return ((uint64_t)hi << 32) | lo;
 }
 
-__global__ __launch_bounds__(256) void k_edge_compact(KArgs a) {
-    const int chunk = blockIdx.y;
+__device__ __forceinline__ void edge_compact(const KArgs& a, int chunk, int wave, int waves) {
     const Geometry& G = a.G;
     const uint64_t* E = slot_ptr<const uint64_t>(a, chunk, a.L.e_rows);
-    const int* count = slot_ptr<const int>(a, chunk, a.L.e_count);
-    const int* base = slot_ptr<const int>(a, chunk, a.L.e_base);
-    const int* base_y = slot_ptr<const int>(a, chunk, a.L.e_base_y);
+    const uint32_t* count = slot_ptr<const uint32_t>(a, chunk, a.L.e_count);
+    const int2* base = slot_ptr<const int2>(a, chunk, a.L.e_base);
     int* ids = slot_ptr<int>(a, chunk, a.L.e_ids);
     int2* order = slot_ptr<int2>(a, chunk, a.L.e_order);
     const int S = G.shift, cap = a.caps.edges, ey_total = a.counters[chunk].edges_y;
@@ -487,21 +567,22 @@ __global__ __launch_bounds__(256) void k_edge_compact(KArgs a) {
         }
     };
     const int groups = (G.edge_rows + 63) >> 6;
-    for (int g = wave_in_chunk(); g < groups; g += waves_per_chunk()) {
+    for (int g = wave; g < groups; g += waves) {
         const int rl = (g << 6) + lane;
-        int cnt = 0, kb = 0, kyb = 0;
+        const int cnt = rl < G.edge_rows ? (int)(count[rl] & 0xffffu) : 0;
+        uint64_t live = __ballot(cnt != 0);
+        if (!live) continue;
+        int kb = 0, kyb = 0;
         uint64_t w0 = 0, w1 = 0, w2 = 0, w3 = 0;
-        if (rl < G.edge_rows) {
-            cnt = count[rl];
-            kb = base[rl];
-            kyb = base_y[rl];
+        if (cnt) {  // a row without edges has no words
+            const int2 b = base[rl];
+            kb = b.x;
+            kyb = b.y;
             w0 = E[4 * rl];
             w1 = E[4 * rl + 1];
             w2 = E[4 * rl + 2];
             w3 = E[4 * rl + 3];
         }
-        uint64_t live = __ballot(cnt != 0);
-        if (!live) continue;
         if (wave_sum(cnt) < kDenseRow * __popcll(live)) {  // sparse rows: one lane per row
             if (cnt == 0) continue;
             const int z = div_magic(rl, G.magic_h), y = rl - z * G.H;
@@ -614,12 +695,14 @@ __global__ __launch_bounds__(1024) void k_height_lines(KArgs a, int chunks) {
         const int r = item - chunk * per_chunk;
         const int sel = r / H, z = r - sel * H;
         const ChunkDesc cd = a.chunks[chunk];  // a copy: the sample loop's stores could alias it
-        if (cd.mode == kModeCached) continue;  // uniform over the wave
+        if (cd.mode == kModeCached || a.counters[chunk].edges == 0) continue;  // uniform over the wave
+        const uint32_t* count = slot_ptr<const uint32_t>(a, chunk, a.L.e_count);
         const uint64_t* E = slot_ptr<const uint64_t>(a, chunk, a.L.e_rows);
         const int word = sel == 0 ? 0 : 2;  // x-edge or z-edge bits of x < 64
         uint64_t lo = 0, hi = 0;
         for (int y = lane; y < H; y += 64) {
             const int row = y + H * z;
+            if ((count[row] & 0xffffu) == 0) continue;  // its words are not stored
             lo |= E[4 * row + word];
             hi |= (E[4 * row + 3] >> word) & 1ull;  // bit 0: x-edge, bit 2: z-edge at x = 64
         }
@@ -1503,40 +1586,6 @@ __device__ __forceinline__ int dominant_material(const int* m) {
     return maxMaterial;
 }
 
-// A voxel is active when its 8 corners are not all solid or all air: over a
-// voxel row, the AND and OR of the four sample rows around it and their x + 1
-// shifts.  Segment `seg` of 64 voxels holds 64 / N voxel rows.
-__global__ __launch_bounds__(256) void k_voxel_rows(KArgs a) {
-    const int chunk = blockIdx.y;
-    const Geometry& G = a.G;
-    const int N = G.N, F = G.F;
-    const uint64_t* S = slot_ptr<const uint64_t>(a, chunk, a.L.solid);
-    uint64_t* vmask = slot_ptr<uint64_t>(a, chunk, a.L.v_mask);
-    int* vcount = slot_ptr<int>(a, chunk, a.L.v_count);
-    const int per_seg = N >= 64 ? 1 : 64 / N;
-    const uint64_t nmask = N >= 64 ? ~0ull : ((1ull << N) - 1ull);
-    for (int seg = thread_in_chunk(); seg < G.voxel_segs; seg += threads_per_chunk()) {
-        uint64_t m = 0;
-        for (int k = 0; k < per_seg; ++k) {
-            const int vr = seg * per_seg + k;  // voxel row y + N z
-            const int y = vr & (N - 1), z = vr >> G.depth;
-            const int s0 = y + F * z;
-            const int rows[4] = {s0, s0 + 1, s0 + F, s0 + F + 1};
-            uint64_t all = ~0ull, any = 0ull;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const uint64_t lo = S[2 * rows[c]], hi = S[2 * rows[c] + 1];
-                const uint64_t nx = shift_next(lo, hi);
-                all &= lo & nx;
-                any |= lo | nx;
-            }
-            m |= ((any & ~all) & nmask) << (k * N);
-        }
-        vmask[seg] = m;
-        vcount[seg] = __popcll(m);
-    }
-}
-
 // The octree codes of every segment's active voxels in linear order; the corner
 // materials, edge mask and dominant material are found by the QEF kernel, which reads
 // the corners anyway.  A wave takes 64 consecutive segments and loads their masks and
@@ -1546,8 +1595,7 @@ __global__ __launch_bounds__(256) void k_voxel_rows(KArgs a) {
 // contiguous store.  Where they are sparse, each lane walks its own segment (one lane
 // per segment alone scattered the dense segments' stores: 4.4 bytes reached HBM per
 // byte of codes on the clipmap batch).  Both walks write the same codes.
-__global__ __launch_bounds__(256) void k_voxel_compact(KArgs a) {
-    const int chunk = blockIdx.y;
+__device__ __forceinline__ void voxel_compact(const KArgs& a, int chunk, int wave, int waves) {
     const Geometry& G = a.G;
     const uint64_t* vmask = slot_ptr<const uint64_t>(a, chunk, a.L.v_mask);
     const int* vbase = slot_ptr<const int>(a, chunk, a.L.v_base);
@@ -1556,16 +1604,12 @@ __global__ __launch_bounds__(256) void k_voxel_compact(KArgs a) {
     const int lane = threadIdx.x & 63;
     const uint64_t lt = lanemask_lt(lane);
     const int groups = (G.voxel_segs + 63) >> 6;
-    for (int g = wave_in_chunk(); g < groups; g += waves_per_chunk()) {
+    for (int g = wave; g < groups; g += waves) {
         const int sl = (g << 6) + lane;
-        uint64_t ml = 0;
-        int bl = 0;
-        if (sl < G.voxel_segs) {
-            ml = vmask[sl];
-            bl = vbase[sl];
-        }
-        uint64_t live = __ballot(ml != 0);
+        const uint64_t own = sl < G.voxel_segs ? vmask[sl] : 0;
+        uint64_t ml = own, live = __ballot(ml != 0);
         if (!live) continue;
+        const int bl = ml ? vbase[sl] : 0;
         if (wave_sum(__popcll(ml)) < kDenseRow * __popcll(live)) {  // sparse: one lane per segment
             int i = bl;
             while (ml && i < cap) {
@@ -1589,6 +1633,17 @@ __global__ __launch_bounds__(256) void k_voxel_compact(KArgs a) {
                 vcode[i] = (int)code_for_position(x, y, z, G.depth);
             }
         }
+    }
+}
+
+// Edge lists by the first `edge_blocks` workgroups of a chunk, voxel codes by the others.
+__global__ __launch_bounds__(256) void k_compact(KArgs a, int edge_blocks) {
+    const int chunk = blockIdx.y;
+    const Counters& c = a.counters[chunk];
+    if ((int)blockIdx.x < edge_blocks) {
+        if (c.edges) edge_compact(a, chunk, wave_in_chunk(), edge_blocks * 4);
+    } else {
+        if (c.voxels) voxel_compact(a, chunk, wave_in_chunk() - edge_blocks * 4, ((int)gridDim.x - edge_blocks) * 4);
     }
 }
 
@@ -1651,7 +1706,7 @@ __device__ __forceinline__ void qef_fast(const KArgs& a, int chunk, const ChunkD
                                          float4& nrm) {
     const Geometry& G = a.G;
     const uint64_t* erows = slot_ptr<const uint64_t>(a, chunk, a.L.e_rows);
-    const int* eb = slot_ptr<const int>(a, chunk, a.L.e_base);
+    const int2* eb = slot_ptr<const int2>(a, chunk, a.L.e_base);
     const float4* ed = slot_ptr<float4>(a, chunk, a.L.e_data);
     const float fscale = (float)cd.scale;
 
@@ -1666,7 +1721,7 @@ __device__ __forceinline__ void qef_fast(const KArgs& a, int chunk, const ChunkD
         const int r = (p.y + (j & 1)) + G.H * (p.z + (j >> 1));
 #pragma unroll
         for (int q = 0; q < 4; ++q) rw[j][q] = erows[4 * r + q];
-        rb[j] = eb[r];
+        rb[j] = eb[r].x;
     }
     int ke[12];
 #pragma unroll
@@ -1866,7 +1921,7 @@ __device__ __forceinline__ void qef_precise(const KArgs& a, int chunk, const Chu
                                             float4& nrm) {
     const Geometry& G = a.G;
     const uint64_t* erows = slot_ptr<const uint64_t>(a, chunk, a.L.e_rows);
-    const int* eb = slot_ptr<const int>(a, chunk, a.L.e_base);
+    const int2* eb = slot_ptr<const int2>(a, chunk, a.L.e_base);
     const float4* ed = slot_ptr<float4>(a, chunk, a.L.e_data);
     const float fscale = (float)cd.scale;
 
@@ -1878,7 +1933,7 @@ __device__ __forceinline__ void qef_precise(const KArgs& a, int chunk, const Chu
         const int r = (p.y + (j & 1)) + G.H * (p.z + (j >> 1));
 #pragma unroll
         for (int q = 0; q < 4; ++q) rw[j][q] = erows[4 * r + q];
-        rb[j] = eb[r];
+        rb[j] = eb[r].x;
     }
     int ke[12];
 #pragma unroll
@@ -2018,9 +2073,8 @@ __global__ __launch_bounds__(256) void k_qef(KArgs a) {
     int* vemask = slot_ptr<int>(a, chunk, a.L.v_emask);
     int* vmat = slot_ptr<int>(a, chunk, a.L.v_mat);
     float4* verts = slot_ptr<float4>(a, chunk, a.L.verts);
-    int* qcount = slot_ptr<int>(a, chunk, a.L.q_count);
+    uint32_t* qcount = slot_ptr<uint32_t>(a, chunk, a.L.q_count);
     uint64_t* smask = slot_ptr<uint64_t>(a, chunk, a.L.s_mask);
-    int* scount = slot_ptr<int>(a, chunk, a.L.s_count);
     const int lane = threadIdx.x & 63;
     const int N = G.N;
     for (int base = wave_in_chunk() << 6; base < V; base += waves_per_chunk() << 6) {
@@ -2054,27 +2108,28 @@ __global__ __launch_bounds__(256) void k_qef(KArgs a) {
         const uint64_t b0 = __ballot(nq & 1), b1 = __ballot(nq & 2), sm = __ballot(seam);
         if (lane == 0) {
             const int seg = base >> 6;
-            qcount[seg] = __popcll(b0) + 2 * __popcll(b1);
+            qcount[seg] = (uint32_t)(__popcll(b0) + 2 * __popcll(b1)) | ((uint32_t)__popcll(sm) << 16);
             smask[seg] = sm;
-            scount[seg] = __popcll(sm);
         }
     }
 }
 
 // Quad and seam scans of one chunk in one workgroup (the segment count is the
 // chunk's voxel count, known only on the device).
-__global__ __launch_bounds__(1024) void k_scan_quads_seams(KArgs a) {
-    __shared__ int buf[1024];
+__global__ __launch_bounds__(kScanThreads) void k_scan_quads_seams(KArgs a) {
+    __shared__ uint64_t wsum[kScanThreads / 64];
     const int chunk = blockIdx.y;
     Counters* cnt = a.counters + chunk;
     const int n = (cnt->voxels + 63) >> 6;
-    const int q = block_scan(slot_ptr<const int>(a, chunk, a.L.q_count), slot_ptr<int>(a, chunk, a.L.q_base), n, buf);
+    if (n == 0) return;  // the counters stay cleared
+    const uint32_t* count = slot_ptr<const uint32_t>(a, chunk, a.L.q_count);
+    int2* base = slot_ptr<int2>(a, chunk, a.L.q_base);
+    const uint64_t t = block_scan(n, wsum, [&](int i) { return halves(count[i]); },
+                                  [&](int i, uint64_t at) { base[i] = make_int2((int)(uint32_t)at, (int)(at >> 32)); });
     if (threadIdx.x == 0) {
+        const int q = (int)(uint32_t)t, sn = (int)(t >> 32);
         cnt->quads = min(q, a.caps.quads);
         if (q > a.caps.quads) atomicOr(&cnt->status, kStatusQuadOverflow);
-    }
-    const int sn = block_scan(slot_ptr<const int>(a, chunk, a.L.s_count), slot_ptr<int>(a, chunk, a.L.s_base), n, buf);
-    if (threadIdx.x == 0) {
         cnt->seams = min(sn, a.caps.seams);
         if (sn > a.caps.seams) atomicOr(&cnt->status, kStatusSeamOverflow);
     }
@@ -2104,9 +2159,8 @@ __global__ __launch_bounds__(64 * kEmitWaves) void k_emit(KArgs a) {
     const int* vmat = slot_ptr<const int>(a, chunk, a.L.v_mat);
     const uint64_t* vm = slot_ptr<const uint64_t>(a, chunk, a.L.v_mask);
     const int* vb = slot_ptr<const int>(a, chunk, a.L.v_base);
-    const int* qbase = slot_ptr<const int>(a, chunk, a.L.q_base);
+    const int2* qbase = slot_ptr<const int2>(a, chunk, a.L.q_base);  // quads, seam nodes
     const uint64_t* smask = slot_ptr<const uint64_t>(a, chunk, a.L.s_mask);
-    const int* sbase = slot_ptr<const int>(a, chunk, a.L.s_base);
     const float4* verts = slot_ptr<const float4>(a, chunk, a.L.verts);
     int* tris = slot_ptr<int>(a, chunk, a.L.tris);
     float4* seams = slot_ptr<float4>(a, chunk, a.L.seams);
@@ -2116,7 +2170,9 @@ __global__ __launch_bounds__(64 * kEmitWaves) void k_emit(KArgs a) {
         const int vi = base + lane, seg = base >> 6;
         // the voxel's own words, loaded together (a lane past the end reads the last voxel)
         const int vc = min(vi, V - 1);
-        const int em = vemask[vc], code = vcode[vc], m = vmat[vc], qb = qbase[seg];
+        const int em = vemask[vc], code = vcode[vc], m = vmat[vc];
+        const int2 qs = qbase[seg];
+        const int qb = qs.x;
         const uint64_t sm = smask[seg];
         const int qbits = vi < V ? (em >> 12) & 7 : 0;
         const int nq = __popc(qbits);
@@ -2194,7 +2250,7 @@ __global__ __launch_bounds__(64 * kEmitWaves) void k_emit(KArgs a) {
                 ++qi;
             }
             if (seam) {
-                const int si = sbase[seg] + __popcll(sm & lt);
+                const int si = qs.y + __popcll(sm & lt);
                 if (si < a.caps.seams) {
                     const float4 pos = verts[3 * vi], nrm = verts[3 * vi + 1];
                     reinterpret_cast<int4*>(seams)[3 * si] = make_int4(p.x, p.y, p.z, m);
@@ -2266,7 +2322,7 @@ static inline unsigned ceil_div(long a, long b) { return (unsigned)((a + b - 1) 
 // captured graph clears them correctly on every replay).
 __global__ __launch_bounds__(256) void k_clear_counters(Counters* c, int n, int* queue) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) c[i] = Counters{0, 0, 0, 0, 0, 0, 0, 0};
+    if (i < n) c[i] = Counters{};
     if (i < kNumQueues) queue[i] = 0;
 }
 
@@ -2279,7 +2335,7 @@ __global__ __launch_bounds__(256) void k_stage_chunk(const ChunkDesc* chunk, con
     static_assert(sizeof(ChunkDesc) % 4 == 0 && sizeof(DevOp) == 64, "copied in words");
     const int t = threadIdx.x, n = chunk->op_count;
     if (t < (int)(sizeof(ChunkDesc) / 4)) reinterpret_cast<uint32_t*>(d_chunk)[t] = reinterpret_cast<const uint32_t*>(chunk)[t];
-    if (t == 0) *c = Counters{0, 0, 0, 0, 0, 0, 0, 0};
+    if (t == 0) *c = Counters{};
     if (t < kNumQueues) queue[t] = 0;
     for (int i = t; i < 4 * n; i += 256) reinterpret_cast<uint4*>(d_ops)[i] = reinterpret_cast<const uint4*>(ops)[i];
     for (int i = t; i < n; i += 256) d_index[i] = index[i];
@@ -2369,22 +2425,23 @@ static unsigned chunk_blocks(int chunks, long threads, int target) {
     return (unsigned)std::min(full, share);
 }
 
-void launch_edge_rows(const KArgs& a, int chunks, hipStream_t s) {
+void launch_rows(const KArgs& a, int chunks, hipStream_t s) {
     const long solid_waves = (a.G.field_rows + kRowsPerBlock - 1) / kRowsPerBlock;
     hipLaunchKernelGGL(k_solid_rows, dim3(chunk_blocks(chunks, 64L * solid_waves, a.row_blocks), chunks), dim3(256), 0, s, a);
-    hipLaunchKernelGGL(k_edge_rows, dim3(chunk_blocks(chunks, a.G.edge_rows, a.row_blocks), chunks), dim3(256), 0, s, a);
+    const unsigned eb = chunk_blocks(chunks, a.G.edge_rows, a.row_blocks);
+    const unsigned vb = chunk_blocks(chunks, a.G.voxel_segs, a.row_blocks);
+    hipLaunchKernelGGL(k_rows, dim3(eb + vb, chunks), dim3(256), 0, s, a, (int)eb);
 }
-void launch_scan(const KArgs& a, int chunks, ScanKind kind, hipStream_t s) {
-    const dim3 grid(1, chunks), block(1024);
-    switch (kind) {
-    case kScanEdges: hipLaunchKernelGGL(k_scan<kScanEdges>, grid, block, 0, s, a); break;
-    case kScanVoxels: hipLaunchKernelGGL(k_scan<kScanVoxels>, grid, block, 0, s, a); break;
-    default: hipLaunchKernelGGL(k_scan_quads_seams, grid, block, 0, s, a); break;
-    }
+void launch_scan_rows(const KArgs& a, int chunks, hipStream_t s) {
+    hipLaunchKernelGGL(k_scan_rows, dim3(2, chunks), dim3(kScanThreads), 0, s, a);
 }
-void launch_edge_compact(const KArgs& a, int chunks, hipStream_t s) {
-    const long groups = (a.G.edge_rows + 63) / 64;
-    hipLaunchKernelGGL(k_edge_compact, dim3(chunk_blocks(chunks, 64L * groups, a.row_blocks), chunks), dim3(256), 0, s, a);
+void launch_scan_quads_seams(const KArgs& a, int chunks, hipStream_t s) {
+    hipLaunchKernelGGL(k_scan_quads_seams, dim3(1, chunks), dim3(kScanThreads), 0, s, a);
+}
+void launch_compact(const KArgs& a, int chunks, hipStream_t s) {
+    const unsigned eb = chunk_blocks(chunks, 64L * ((a.G.edge_rows + 63) / 64), a.row_blocks);
+    const unsigned vb = chunk_blocks(chunks, 64L * ((a.G.voxel_segs + 63) / 64), a.row_blocks);
+    hipLaunchKernelGGL(k_compact, dim3(eb + vb, chunks), dim3(256), 0, s, a, (int)eb);
 }
 // Lanes per edge of the crossing stage: the tuned value, else by field and batch size (a
 // typical 64^3 chunk has a few hundred 64-edge items, a chunk of N^3 about (N / 64)^2 of
@@ -2455,12 +2512,6 @@ void launch_edge_cross(const KArgs& a, int chunks, hipStream_t s) {
     const dim3 grid(persistent_blocks(a, a.persist_per_cu, 512L * chunks));
     LVN_LAUNCH_KIND(k_edge_cross, grid, dim3(kCrossThreads));
 }
-void launch_voxel_rows(const KArgs& a, int chunks, hipStream_t s) {
-    hipLaunchKernelGGL(k_voxel_rows, dim3(chunk_blocks(chunks, a.G.voxel_segs, a.row_blocks), chunks), dim3(256), 0, s, a);
-}
-void launch_voxel_compact(const KArgs& a, int chunks, hipStream_t s) {
-    hipLaunchKernelGGL(k_voxel_compact, dim3(chunk_blocks(chunks, a.G.voxel_segs, a.row_blocks), chunks), dim3(256), 0, s, a);
-}
 // The kernels below loop up to the chunk's voxel count, known only on the device.
 void launch_qef(const KArgs& a, int chunks, hipStream_t s) {
     const dim3 grid(chunk_blocks(chunks, a.caps.voxels, a.voxel_blocks), chunks);
@@ -2482,15 +2533,15 @@ void launch_stage(const KArgs& a, int chunks, int i, hipStream_t s) {
     switch (i) {
     case 0: launch_density(a, chunks, s); break;
     case 1: launch_csg(a, chunks, s); break;
-    case 2: launch_edge_rows(a, chunks, s); break;
-    case 3: launch_scan(a, chunks, kScanEdges, s); break;
-    case 4: launch_edge_compact(a, chunks, s); break;
+    case 2: launch_rows(a, chunks, s); break;  // edge and voxel rows
+    case 3: launch_scan_rows(a, chunks, s); break;
+    case 4: launch_compact(a, chunks, s); break;
     case 5: launch_edge_cross(a, chunks, s); break;
-    case 6: launch_voxel_rows(a, chunks, s); break;
-    case 7: launch_scan(a, chunks, kScanVoxels, s); break;
-    case 8: launch_voxel_compact(a, chunks, s); break;
+    case 6:
+    case 7:
+    case 8: break;  // the voxel stages run with the edges' (2, 3 and 4)
     case 9: launch_qef(a, chunks, s); break;
-    case 10: launch_scan(a, chunks, kScanQuadsSeams, s); break;
+    case 10: launch_scan_quads_seams(a, chunks, s); break;
     default: launch_emit(a, chunks, s); break;
     }
 }

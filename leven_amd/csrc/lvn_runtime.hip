@@ -219,28 +219,24 @@ SlotLayout make_layout(const Geometry& G, const Caps& c, bool lines) {
     L.orig = take(fs);
     L.solid = take((uint64_t)G.field_rows * 16);
     L.planes = take((uint64_t)G.col_groups * G.F * 8);
+    L.sides = take((uint64_t)G.col_groups * G.F);
     L.e_rows = take((uint64_t)G.edge_rows * 32);
     L.e_count = take((uint64_t)G.edge_rows * 4);
-    L.e_base = take((uint64_t)G.edge_rows * 4);
-    L.e_count_y = take((uint64_t)G.edge_rows * 4);
-    L.e_base_y = take((uint64_t)G.edge_rows * 4);
+    L.e_base = take((uint64_t)G.edge_rows * 8);
     L.e_ids = take((uint64_t)c.edges * 4);
     L.e_data = take((uint64_t)c.edges * 16);
     L.e_order = take((uint64_t)c.edges * 8);
     L.h_lines = take(lines ? (uint64_t)2 * G.H * G.H * kLineStride * 4 : 0);
     L.h_cols = take((uint64_t)G.F * G.F * 4);
     L.v_mask = take((uint64_t)G.voxel_segs * 8);
-    L.v_count = take((uint64_t)G.voxel_segs * 4);
     L.v_base = take((uint64_t)G.voxel_segs * 4);
     L.v_code = take((uint64_t)c.voxels * 4);
     L.v_emask = take((uint64_t)c.voxels * 4);
     L.v_mat = take((uint64_t)c.voxels * 4);
     L.q_count = take((uint64_t)c.seam_segs * 4);
-    L.q_base = take((uint64_t)c.seam_segs * 4);
+    L.q_base = take((uint64_t)c.seam_segs * 8);
     L.tris = take((uint64_t)c.quads * 24);
     L.s_mask = take((uint64_t)c.seam_segs * 8);
-    L.s_count = take((uint64_t)c.seam_segs * 4);
-    L.s_base = take((uint64_t)c.seam_segs * 4);
     L.seams = take((uint64_t)c.seams * 48);
     L.verts = take((uint64_t)c.voxels * 48);
     L.slot_bytes = o;
@@ -504,9 +500,9 @@ static int run_field(Ctx* c, const int32_t* min, int32_t size, const std::vector
     launch_stage_chunk(a, c->h_chunks, c->h_ops, c->h_op_index, c->stream);
     launch_density(a, 1, c->stream);  // or the cached field's materials
     if (!ops.empty()) launch_csg(a, 1, c->stream);
-    launch_edge_rows(a, 1, c->stream);
-    launch_scan(a, 1, kScanEdges, c->stream);
-    launch_edge_compact(a, 1, c->stream);
+    launch_rows(a, 1, c->stream);
+    launch_scan_rows(a, 1, c->stream);
+    launch_compact(a, 1, c->stream);
     launch_edge_cross(a, 1, c->stream);
     LVN_HIP(hipGetLastError());
     return LVN_OK;
@@ -514,11 +510,8 @@ static int run_field(Ctx* c, const int32_t* min, int32_t size, const std::vector
 
 static int run_mesh(Ctx* c) {
     KArgs a = c->kargs();
-    launch_voxel_rows(a, 1, c->stream);
-    launch_scan(a, 1, kScanVoxels, c->stream);
-    launch_voxel_compact(a, 1, c->stream);
     launch_qef(a, 1, c->stream);
-    launch_scan(a, 1, kScanQuadsSeams, c->stream);
+    launch_scan_quads_seams(a, 1, c->stream);
     launch_emit(a, 1, c->stream);
     LVN_HIP(hipGetLastError());
     return LVN_OK;

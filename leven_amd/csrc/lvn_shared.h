@@ -79,13 +79,16 @@ struct SlotLayout {
     uint64_t solid;                       // field_rows x 2 words: bit x = sample (x, y, z) is not air
     uint64_t planes;                      // col_groups x F words, [g][y] bit c: column 64 g + c of plane y
                                           // is not air (chunks whose materials are not stored)
-    uint64_t e_rows, e_count, e_base, e_ids, e_data;  // e_rows: edge_rows x {x, y, z, x = 64} words
-    uint64_t e_count_y, e_base_y, e_order;  // y-edges per row and their scan; crossing order (y-edges first)
+    uint64_t sides;                       // per density item: kSomeSolid, kSomeAir (such chunks)
+    uint64_t e_rows;                      // edge_rows x {x, y, z, x = 64} words (rows with edges only)
+    uint64_t e_count, e_base;             // per edge row: edges | y-edges << 16; {edges, y-edges} before it
+    uint64_t e_ids, e_data;
+    uint64_t e_order;                     // {rank, id} in crossing order (y-edges first)
     uint64_t h_lines;                     // heights at k/16 (k = 1..15) along x- and z-edge lines, 2 x H x H x 15 f32
     uint64_t h_cols;                      // the height term of each field column (x, z), F x F f32 (fresh fields)
-    uint64_t v_mask, v_count, v_base, v_code, v_emask, v_mat;
-    uint64_t q_count, q_base, tris;
-    uint64_t s_mask, s_count, s_base, seams, verts;
+    uint64_t v_mask, v_base, v_code, v_emask, v_mat;
+    uint64_t q_count, q_base, tris;       // per 64 voxels: quads | seam nodes << 16; {quads, seam nodes} before
+    uint64_t s_mask, seams, verts;
 };
 
 // Per-chunk request descriptor.
@@ -113,8 +116,11 @@ struct Counters {
     int status;      // 0 ok, else LVN_ERR_OVERFLOW bits
     int resolved;    // precise QEF: vertices re-solved in FP64
     int edges_y;     // y-edges among `edges` (capped like edges)
-    int pad;
+    int sides;       // kSomeSolid, kSomeAir: what the density pass met (chunks without stored materials)
 };
+
+constexpr int kSomeSolid = 1;
+constexpr int kSomeAir = 2;
 
 constexpr int kStatusEdgeOverflow = 1;
 constexpr int kStatusVoxelOverflow = 2;
