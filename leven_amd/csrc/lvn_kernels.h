@@ -27,6 +27,7 @@ struct KArgs {
     unsigned long long* work;  // optional work counters (see lvn_batch_work), else null
     int* queue;              // kNumQueues work-queue heads, zeroed by launch_clear_counters
     int* item_prefix;        // chunks + 1 edge-item offsets (k_edge_data)
+    int* special;            // the chunks with brushes or a cached field: their number, then them
     int cus;                 // compute units of the device
     int persist_per_cu;      // persistent workgroups per CU (edge crossing)
     int density_per_cu;      // persistent workgroups per CU (density), 0 = by the number of items

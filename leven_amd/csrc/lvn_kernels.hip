@@ -84,6 +84,16 @@ __device__ __forceinline__ int edge_index_in_row(const uint64_t w[4], int base, 
     return base + k;
 }
 
+// Items of the queued crossing kernel: wave w of the grid starts with grab w (`per_grab`
+// consecutive items), without the queue, and takes later grabs from the atomic counter.
+// One counter serves about 77 grabs per us, so when every wave of a full grid (3,072 for
+// one chunk) took its first, mostly failing, grab there, that alone was 40 us.  Waves are
+// numbered across the workgroups, so few items spread over the CUs.
+__device__ __forceinline__ int grid_waves() { return (int)(gridDim.x * (blockDim.x >> 6)); }
+__device__ __forceinline__ int first_grab(int per_grab) {
+    return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) * (int)gridDim.x + (int)blockIdx.x) * per_grab;
+}
+
 // FP16 store that keeps the sign of every negative sample (an underflow to -0
 // would turn a solid sample into air under the reference's `density < 0` test,
 // cl/density_field.cl:34).
@@ -197,16 +207,6 @@ __device__ __forceinline__ void density_column(const KArgs& a, const NoiseLds& T
     }
 }
 
-// Items of the queued crossing kernel: wave w of the grid starts with grab w (`per_grab`
-// consecutive items), without the queue, and takes later grabs from the atomic counter.
-// One counter serves about 77 grabs per us, so when every wave of a full grid (3,072 for
-// one chunk) took its first, mostly failing, grab there, that alone was 40 us.  Waves are
-// numbered across the workgroups, so few items spread over the CUs.
-__device__ __forceinline__ int grid_waves() { return (int)(gridDim.x * (blockDim.x >> 6)); }
-__device__ __forceinline__ int first_grab(int per_grab) {
-    return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) * (int)gridDim.x + (int)blockIdx.x) * per_grab;
-}
-
 // Items of a persistent kernel shared within the workgroup: workgroup b owns items b,
 // b + gridDim.x, ... (`total` items in all; interleaved, so every workgroup gets items
 // of every chunk and their totals even out) and its waves take them through the LDS
@@ -252,51 +252,141 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_num_sgpr(80), amdgpu_wa
 }
 
 // ---------------------------------------------------------------------------
-// CSG material override (CSG_HermiteIndices + BrushMaterial,
-// cl/apply_csg_operation.cl:114-140,179-210): ops in order, the last op whose
-// brush contains a sample sets its material.  A chunk's samples are split into
-// kCsgSlabs z-slabs, one workgroup each, so the chunk with the most brushes is spread
-// over several CUs; each workgroup walks the ops in order over the (x, y) columns of
-// each op's bounding box within its slab.  Every sample belongs to one workgroup and
-// sees the ops in order (a barrier after each op), as in a single pass.
+// Brushes.  A chunk's op list is walked by whole waves: 64 ops are loaded at once, one per
+// lane, and each is then read lane by lane into scalar registers, so an op costs a dozen
+// v_readlane instead of two dependent memory round trips.
 // ---------------------------------------------------------------------------
-constexpr int kCsgSlabs = 8;
+struct WaveOps {
+    const DevOp* ops;
+    const int* index;
+    int n, group;       // ops in the list; the group of 64 held, or -1
+    uint32_t w[16];     // the lane's op
+
+    __device__ __forceinline__ WaveOps(const KArgs& a, const ChunkDesc& cd)
+        : ops(a.ops), index(a.op_index + cd.op_start), n(cd.op_count), group(-1) {}
+    // Holds ops 64 g .. 64 g + 63 of the list (a lane past its end holds the last op).
+    __device__ __forceinline__ void hold(int g) {
+        if (g == group) return;
+        group = g;
+        const int k = min(64 * g + (int)(threadIdx.x & 63), n - 1);
+        const uint4* p = reinterpret_cast<const uint4*>(ops + index[k]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint4 v = p[q];
+            w[4 * q] = v.x;
+            w[4 * q + 1] = v.y;
+            w[4 * q + 2] = v.z;
+            w[4 * q + 3] = v.w;
+        }
+    }
+    __device__ __forceinline__ DevOp mine() const {
+        DevOp op;
+        __builtin_memcpy(&op, w, sizeof(op));
+        return op;
+    }
+    // Op k of the list, the same in every lane.
+    __device__ __forceinline__ DevOp at(int k) {
+        static_assert(sizeof(DevOp) == 64, "16 words");
+        hold(k >> 6);
+        uint32_t u[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) u[i] = (uint32_t)__builtin_amdgcn_readlane((int)w[i], k & 63);
+        DevOp op;
+        __builtin_memcpy(&op, u, sizeof(op));
+        return op;
+    }
+};
+
+// The chunks with brushes or a cached field (k_clear_counters): special[0] of them, in
+// special[1 ..].
+__device__ __forceinline__ int special_chunks(const KArgs& a) { return a.special[0]; }
+__device__ __forceinline__ int special_chunk(const KArgs& a, int i) {
+    return __builtin_amdgcn_readfirstlane(a.special[1 + i]);
+}
+
+// Deals items 0, 1, ... of one list after another round `waves` waves: the first item of the
+// current list for this wave, given how many earlier lists' items were dealt.
+__device__ __forceinline__ int first_dealt(int wave, int dealt, int waves) {
+    return wave >= dealt ? wave - dealt : wave - dealt + waves;
+}
+
+// ---------------------------------------------------------------------------
+// CSG material override (CSG_HermiteIndices + BrushMaterial,
+// cl/apply_csg_operation.cl:114-140,179-210): the last op whose brush contains a sample sets
+// its material.  A wave takes a tile of 16 x 4 x 8 samples, finds the ops whose bounding
+// sphere reaches it (64 tests at a time) and walks those from the last to the first, a
+// sample being settled by the first that holds it.  Tiles of all brushed chunks are dealt
+// round the grid's waves.  (The ops one after another over each chunk, a barrier after
+// each, took 82 us for one chunk under 60 brushes and 103 us for 24 or 1,800 chunks.)
+// ---------------------------------------------------------------------------
+constexpr int kCsgX = 16, kCsgY = 4, kCsgZ = 8;  // 64 lanes over x and y, 8 layers each
+constexpr int kCsgBlocks = 1024;
 
 __global__ __launch_bounds__(256) void k_csg(KArgs a) {
-    const int chunk = blockIdx.y;
-    const ChunkDesc cd = a.chunks[chunk];  // a copy: the loops below store through pointers that could alias it
     const int F = a.G.F;
-    const int zs = (F + kCsgSlabs - 1) / kCsgSlabs;
-    const int z0 = (int)blockIdx.x * zs, z1 = min(F, z0 + zs);  // this workgroup's slab
-    if (cd.op_count == 0 || z0 >= z1) return;                    // uniform, before any barrier
-    uint8_t* mat = slot_ptr<uint8_t>(a, chunk, a.L.mat);
-    const float inv = 1.f / (float)cd.scale;
-    for (int k = 0; k < cd.op_count; ++k) {
-        const DevOp op = a.ops[a.op_index[cd.op_start + k]];
-        const float r = op.radius + 1.f;
-        int lo[3], hi[3];
-        const float o[3] = {op.ox, op.oy, op.oz};
-        for (int c = 0; c < 3; ++c) {
-            lo[c] = max(0, (int)floorf((o[c] - r - (float)cd.off[c]) * inv));
-            hi[c] = min(F - 1, (int)ceilf((o[c] + r - (float)cd.off[c]) * inv));
-        }
-        lo[2] = max(lo[2], z0);
-        hi[2] = min(hi[2], z1 - 1);
-        const int nx = hi[0] - lo[0] + 1, ny = hi[1] - lo[1] + 1;
-        if (nx > 0 && ny > 0 && hi[2] >= lo[2]) {
-            const uint8_t newm = op.type == 0 ? (uint8_t)op.material : (uint8_t)kAir;
-            for (int i = threadIdx.x; i < nx * ny; i += blockDim.x) {
-                const int y = lo[1] + i / nx;
-                const int x = lo[0] + (i - (y - lo[1]) * nx);
-                const float px = (float)(x * cd.scale + cd.off[0]);
-                const float py = (float)(y * cd.scale + cd.off[1]);
-                for (int z = lo[2]; z <= hi[2]; ++z) {
-                    const float pz = (float)(z * cd.scale + cd.off[2]);
-                    if (brush_density(op, px, py, pz) <= 0.f) mat[field_index(a.G, x, y, z)] = newm;
+    const int lane = threadIdx.x & 63;
+    const int waves = grid_waves();
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) * (int)gridDim.x + (int)blockIdx.x);
+    const int tx = (F + kCsgX - 1) / kCsgX, ty = (F + kCsgY - 1) / kCsgY, tz = (F + kCsgZ - 1) / kCsgZ;
+    const int items = tx * ty * tz, lists = special_chunks(a);
+    int dealt = 0;  // items of earlier chunks, modulo the number of waves
+    for (int q = 0; q < lists; ++q) {
+        const int chunk = special_chunk(a, q);
+        const ChunkDesc cd = a.chunks[chunk];  // a copy: the stores below could alias it
+        if (cd.op_count == 0) continue;
+        uint8_t* mat = slot_ptr<uint8_t>(a, chunk, a.L.mat);
+        WaveOps list(a, cd);
+        for (int j = first_dealt(wave, dealt, waves); j < items; j += waves) {
+            const int jz = j / (tx * ty), jy = (j - jz * tx * ty) / tx, jx = j - (jz * ty + jy) * tx;
+            const int x0 = jx * kCsgX, y0 = jy * kCsgY, z0 = jz * kCsgZ;
+            const int x = x0 + (lane & (kCsgX - 1)), y = y0 + lane / kCsgX;
+            const bool in = x < F && y < F;
+            // the tile's samples in voxels: its box and this lane's column
+            const float lo[3] = {(float)(x0 * cd.scale + cd.off[0]), (float)(y0 * cd.scale + cd.off[1]),
+                                 (float)(z0 * cd.scale + cd.off[2])};
+            const float hi[3] = {lo[0] + (float)((kCsgX - 1) * cd.scale), lo[1] + (float)((kCsgY - 1) * cd.scale),
+                                 lo[2] + (float)((kCsgZ - 1) * cd.scale)};
+            const float px = (float)(x * cd.scale + cd.off[0]), py = (float)(y * cd.scale + cd.off[1]);
+            unsigned settled = in ? 0u : 0xffu;  // a bit per layer
+            int to[kCsgZ];
+#pragma unroll
+            for (int l = 0; l < kCsgZ; ++l) {
+                to[l] = 0;
+                if (z0 + l >= F) settled |= 1u << l;
+            }
+            const unsigned outside = settled;
+            for (int g = (cd.op_count - 1) >> 6; g >= 0; --g) {
+                list.hold(g);
+                const DevOp op = list.mine();
+                const float r = op.radius + 1.f;
+                const float o[3] = {op.ox, op.oy, op.oz};
+                float d2 = 0.f;
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    const float d = fmaxf(fmaxf(lo[c] - o[c], o[c] - hi[c]), 0.f);
+                    d2 = d2 + d * d;
+                }
+                uint64_t near = __ballot(64 * g + lane < cd.op_count && !(d2 > r * r));
+                while (near && __ballot(settled != 0xffu)) {
+                    const int b = 63 - (int)__builtin_clzll(near);
+                    near &= ~(1ull << b);
+                    const DevOp u = list.at(64 * g + b);
+                    const int newm = u.type == 0 ? (int)(uint8_t)u.material : kAir;
+#pragma unroll
+                    for (int l = 0; l < kCsgZ; ++l) {
+                        const float pz = (float)((z0 + l) * cd.scale + cd.off[2]);
+                        const bool take = !((settled >> l) & 1u) && brush_density(u, px, py, pz) <= 0.f;
+                        to[l] = take ? newm : to[l];
+                        settled |= take ? 1u << l : 0u;
+                    }
                 }
             }
+            const unsigned write = settled & ~outside;
+#pragma unroll
+            for (int l = 0; l < kCsgZ; ++l)
+                if ((write >> l) & 1u) mat[field_index(a.G, x, y, z0 + l)] = (uint8_t)to[l];
         }
-        __syncthreads();
+        dealt = (dealt + items) % waves;
     }
 }
 
@@ -841,42 +931,24 @@ __device__ __forceinline__ float4 density_crossing(const KArgs& a, const NoiseLd
     return crossing_normal<kKind>(Fp, T, axis, ends_known, tbest, Hbest, p0x, p0y, p0z, p1x, p1y, p1z, nh, nc);
 }
 
-// A brush through scalar loads: its address is the same in every lane, the ops and their
-// index list are written before the launch and never by a kernel that reads them here.
-using ScalarWord = const uint32_t __attribute__((address_space(4)));
-__device__ __forceinline__ uint32_t scalar_word(const void* p, int word) {
-    return reinterpret_cast<ScalarWord*>(reinterpret_cast<uint64_t>(p))[word];
-}
-__device__ __forceinline__ DevOp scalar_op(const DevOp* ops, const int* index, int k) {
-    static_assert(sizeof(DevOp) == 64, "16 words");
-    const DevOp* p = ops + __builtin_amdgcn_readfirstlane((int)scalar_word(index, k));
-    DevOp op;
-    uint32_t w[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) w[i] = scalar_word(p, i);
-    __builtin_memcpy(&op, w, sizeof(op));
-    return op;
-}
-
 // FindEdgeIntersectionInfo of the CSG program, cl/apply_csg_operation.cl:443-477,
 // with BrushZeroCrossing (:86-110) and BrushNormal (:144-175): the first (t, op) in
 // the reference's t-outer, op-inner scan whose |d| is smallest, t = k/16; then the
 // normal of the last op holding that point.  Only t matters of the pair, so the scan's
 // answer is the smallest k among the samples of the smallest |d|, whatever order they are
-// visited in: the ops are the outer loop here (one uniform load each instead of 17), and
-// an op is sampled along the edge only when it can still win.  A brush's distance is
+// visited in: the ops are the outer loop here (each read once instead of 17 times), and an
+// op is sampled along the edge only when it can still win.  A brush's distance is
 // 1-Lipschitz (a rounded rotation and the FP32 steps stay within 1e-5 of the magnitudes
 // that enter it), so with |d| = m at the edge's middle no sample of the edge, at most half
 // an edge away, is below m - half: an op for which that exceeds the running minimum is
-// passed by.  All edges of the wave are the chunk's, `op_start` and `op_count` its list.
-__device__ __forceinline__ float4 brush_crossing(const KArgs& a, const ChunkDesc& cd, bool live, int x, int y, int z,
+// passed by.  All edges of the wave are one chunk's, `list` its ops.
+__device__ __forceinline__ float4 brush_crossing(WaveOps& list, const ChunkDesc& cd, bool live, int x, int y, int z,
                                                  int axis) {
     const int w0x = x * cd.scale + cd.off[0], w0y = y * cd.scale + cd.off[1], w0z = z * cd.scale + cd.off[2];
     const float p0x = (float)w0x, p0y = (float)w0y, p0z = (float)w0z;
     const float ex = (float)(w0x + (axis == 0 ? cd.scale : 0)) - p0x;
     const float ey = (float)(w0y + (axis == 1 ? cd.scale : 0)) - p0y;
     const float ez = (float)(w0z + (axis == 2 ? cd.scale : 0)) - p0z;
-    const int* index = a.op_index + cd.op_start;
     const int n = cd.op_count;
     constexpr int kMid = 8;
     const float half = (float)cd.scale * 0.5f;
@@ -884,7 +956,7 @@ __device__ __forceinline__ float4 brush_crossing(const KArgs& a, const ChunkDesc
     int kbest = 0;
     const float mx = p0x + ex * 0.5f, my = p0y + ey * 0.5f, mz = p0z + ez * 0.5f;
     for (int k = 0; k < n; ++k) {
-        const DevOp op = scalar_op(a.ops, index, k);
+        const DevOp op = list.at(k);
         const float d = fabsf(brush_density(op, mx, my, mz));
         if (d < minD) {
             minD = d;
@@ -892,7 +964,7 @@ __device__ __forceinline__ float4 brush_crossing(const KArgs& a, const ChunkDesc
         }
     }
     for (int k = 0; k < n; ++k) {
-        const DevOp op = scalar_op(a.ops, index, k);
+        const DevOp op = list.at(k);
         const float slack = 1e-5f * (((fabsf(mx - op.ox) + fabsf(my - op.oy)) + (fabsf(mz - op.oz) + half)) +
                                      ((fabsf(op.dx) + fabsf(op.dy)) + fabsf(op.dz)));
         const float reach = half + slack;
@@ -915,7 +987,7 @@ __device__ __forceinline__ float4 brush_crossing(const KArgs& a, const ChunkDesc
     float3 nrm = make_float3(0.f, 0.f, 0.f);
     bool open = live;  // the last op holding the point decides: the first one found from the end
     for (int k = n - 1; k >= 0 && __ballot(open) != 0; --k) {
-        const DevOp op = scalar_op(a.ops, index, k);
+        const DevOp op = list.at(k);
         if (!open || brush_density(op, px, py, pz) > 0.f) continue;
         const float dx = brush_density(op, px + h, py, pz) - brush_density(op, px - h, py, pz);
         const float dy = brush_density(op, px, py + h, pz) - brush_density(op, px, py - h, pz);
@@ -1067,9 +1139,8 @@ __device__ __forceinline__ void edge_items(const KArgs& a, int chunks, int per_i
 
 // The edges whose hermite data needs no field evaluation: those a brush touched, and in
 // the cached form every other one, which keeps its data from the old edge list.  The last
-// workgroup counts the crossing kernels' items meanwhile.  The others walk the chunks,
-// 64 descriptors at a time, and deal the 64-edge items of the chunks that have such edges
-// round the grid's waves.  Beside the crossing kernels' density path this one is short of
+// workgroup counts the crossing kernels' items meanwhile.  The others deal the 64-edge items
+// of the chunks that have such edges round the grid's waves.  Beside the crossing kernels' density path this one is short of
 // neither registers nor LDS, and a few brushed chunks of a batch (whose edges each scan the
 // chunk's op list) no longer hold a wave of the density queue: those were its tail.  One
 // brushed 64^3 chunk of the reference's terrain meshed in 598 -> 325 us, a two-step edit of
@@ -1087,51 +1158,48 @@ __global__ __launch_bounds__(kEdgeDataThreads) void k_edge_data(KArgs a, int chu
     const int waves = (int)((gridDim.x - 1) * (blockDim.x >> 6));
     // waves are numbered across the workgroups, so a few items spread over the CUs
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) * (int)(gridDim.x - 1) + (int)blockIdx.x);
+    const int lists = special_chunks(a);
     int dealt = 0;  // items of earlier chunks, modulo the number of waves
-    for (int base = 0; base < chunks; base += 64) {
-        const int c = base + lane;
-        uint64_t some = __ballot(c < chunks && (a.chunks[c].op_count > 0 || a.chunks[c].mode == kModeCached));
-        while (some) {
-            const int chunk = __builtin_amdgcn_readfirstlane(base + (int)__builtin_ctzll(some));
-            some &= some - 1ull;
-            const ChunkDesc cd = a.chunks[chunk];
-            const bool cached = cd.mode == kModeCached;
-            const int edges = a.counters[chunk].edges, items = (edges + 63) >> 6;
-            const int* ids = slot_ptr<const int>(a, chunk, a.L.e_ids);
-            float4* data = slot_ptr<float4>(a, chunk, a.L.e_data);
-            const int* oid = reinterpret_cast<const int*>(cd.old_ids);
-            const float4* odata = reinterpret_cast<const float4*>(cd.old_data);
-            for (int j = wave >= dealt ? wave - dealt : wave - dealt + waves; j < items; j += waves) {
-                const int i = 64 * j + lane;
-                const int id = i < edges ? ids[i] : 0;
-                EdgeAt e;
-                bool live = decode_edge(G, id, e) && i < edges;
-                if (i < edges && !live) atomicOr(&a.counters[chunk].status, kStatusLookupMiss);
-                const bool touched = live && edge_touched(a, chunk, cd, e.i0, e.i1);
-                if (__ballot(touched)) {
-                    const float4 out = brush_crossing(a, cd, touched, e.x, e.y, e.z, e.axis);
-                    if (touched) data[i] = out;
+    for (int q = 0; q < lists; ++q) {
+        const int chunk = special_chunk(a, q);
+        const ChunkDesc cd = a.chunks[chunk];
+        const bool cached = cd.mode == kModeCached;
+        const int edges = a.counters[chunk].edges, items = (edges + 63) >> 6;
+        const int* ids = slot_ptr<const int>(a, chunk, a.L.e_ids);
+        float4* data = slot_ptr<float4>(a, chunk, a.L.e_data);
+        const int* oid = reinterpret_cast<const int*>(cd.old_ids);
+        const float4* odata = reinterpret_cast<const float4*>(cd.old_data);
+        WaveOps list(a, cd);
+        for (int j = first_dealt(wave, dealt, waves); j < items; j += waves) {
+            const int i = 64 * j + lane;
+            const int id = i < edges ? ids[i] : 0;
+            EdgeAt e;
+            bool live = decode_edge(G, id, e) && i < edges;
+            if (i < edges && !live) atomicOr(&a.counters[chunk].status, kStatusLookupMiss);
+            const bool touched = live && edge_touched(a, chunk, cd, e.i0, e.i1);
+            if (__ballot(touched)) {
+                const float4 out = brush_crossing(list, cd, touched, e.x, e.y, e.z, e.axis);
+                if (touched) data[i] = out;
+            }
+            if (cached && live && !touched) {
+                int lo = 0, hi = cd.old_edges;
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    if (oid[mid] < id) lo = mid + 1; else hi = mid;
                 }
-                if (cached && live && !touched) {
-                    int lo = 0, hi = cd.old_edges;
-                    while (lo < hi) {
-                        const int mid = (lo + hi) >> 1;
-                        if (oid[mid] < id) lo = mid + 1; else hi = mid;
-                    }
-                    if (lo < cd.old_edges && oid[lo] == id) {
-                        data[i] = odata[lo];
-                    } else {
-                        data[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-                        atomicOr(&a.counters[chunk].status, kStatusLookupMiss);
-                    }
-                }
-                if constexpr (kCount) {
-                    if (touched) atomicAdd(&a.work[4], (unsigned long long)(17 * cd.op_count));
-                    if (touched || (cached && live)) atomicAdd(&a.work[6], 1ull);
+                if (lo < cd.old_edges && oid[lo] == id) {
+                    data[i] = odata[lo];
+                } else {
+                    data[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+                    atomicOr(&a.counters[chunk].status, kStatusLookupMiss);
                 }
             }
-            dealt = (dealt + items) % waves;
+            if constexpr (kCount) {
+                if (touched) atomicAdd(&a.work[4], (unsigned long long)(17 * cd.op_count));
+                if (touched || (cached && live)) atomicAdd(&a.work[6], 1ull);
+            }
         }
+        dealt = (dealt + items) % waves;
     }
 }
 
@@ -2320,10 +2388,34 @@ static inline unsigned ceil_div(long a, long b) { return (unsigned)((a + b - 1) 
 
 // Zero the per-chunk counters (a kernel rather than a memset node, so that a
 // captured graph clears them correctly on every replay).
-__global__ __launch_bounds__(256) void k_clear_counters(Counters* c, int n, int* queue) {
+// The first workgroup also lists the chunks with brushes or a cached field, which are few in
+// a batch: k_csg and k_edge_data walk that list instead of every descriptor (28 us of 1,800).
+constexpr int kClearThreads = 1024;
+__global__ __launch_bounds__(kClearThreads) void k_clear_counters(Counters* c, int n, int* queue, const ChunkDesc* chunks,
+                                                                  int* special) {
+    __shared__ int wcount[kClearThreads / 64];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) c[i] = Counters{};
+    if (blockIdx.x) return;
     if (i < kNumQueues) queue[i] = 0;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int count = 0;
+    for (int base = 0; base < n; base += kClearThreads) {
+        const int k = base + (int)threadIdx.x;
+        const bool listed = k < n && (chunks[k].op_count > 0 || chunks[k].mode == kModeCached);
+        const uint64_t hits = __ballot(listed);
+        if (lane == 0) wcount[wave] = __popcll(hits);
+        __syncthreads();
+        int before = count, all = count;
+        for (int w = 0; w < kClearThreads / 64; ++w) {
+            before += w < wave ? wcount[w] : 0;
+            all += wcount[w];
+        }
+        if (listed) special[1 + before + __popcll(hits & lanemask_lt(lane))] = k;
+        count = all;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) special[0] = count;
 }
 
 // The one-chunk forms' inputs, read from pinned host memory by the pipeline's first kernel
@@ -2331,11 +2423,15 @@ __global__ __launch_bounds__(256) void k_clear_counters(Counters* c, int n, int*
 // of it: about 20 us of a one-chunk call were spent before its first stage.
 __global__ __launch_bounds__(256) void k_stage_chunk(const ChunkDesc* chunk, const DevOp* ops, const int* index,
                                                      ChunkDesc* d_chunk, DevOp* d_ops, int* d_index, Counters* c,
-                                                     int* queue) {
+                                                     int* queue, int* special) {
     static_assert(sizeof(ChunkDesc) % 4 == 0 && sizeof(DevOp) == 64, "copied in words");
     const int t = threadIdx.x, n = chunk->op_count;
     if (t < (int)(sizeof(ChunkDesc) / 4)) reinterpret_cast<uint32_t*>(d_chunk)[t] = reinterpret_cast<const uint32_t*>(chunk)[t];
-    if (t == 0) *c = Counters{};
+    if (t == 0) {
+        *c = Counters{};
+        special[0] = n > 0 || chunk->mode == kModeCached ? 1 : 0;
+        special[1] = 0;
+    }
     if (t < kNumQueues) queue[t] = 0;
     for (int i = t; i < 4 * n; i += 256) reinterpret_cast<uint4*>(d_ops)[i] = reinterpret_cast<const uint4*>(ops)[i];
     for (int i = t; i < n; i += 256) d_index[i] = index[i];
@@ -2347,12 +2443,12 @@ __global__ __launch_bounds__(256) void k_stage_chunk(const ChunkDesc* chunk, con
 
 void launch_stage_chunk(const KArgs& a, const ChunkDesc* chunk, const DevOp* ops, const int* index, hipStream_t s) {
     hipLaunchKernelGGL(k_stage_chunk, dim3(1), dim3(256), 0, s, chunk, ops, index, const_cast<ChunkDesc*>(a.chunks),
-                       const_cast<DevOp*>(a.ops), const_cast<int*>(a.op_index), a.counters, a.queue);
+                       const_cast<DevOp*>(a.ops), const_cast<int*>(a.op_index), a.counters, a.queue, a.special);
 }
 
 void launch_clear_counters(const KArgs& a, int n, hipStream_t s) {
-    hipLaunchKernelGGL(k_clear_counters, dim3(ceil_div(std::max(n, kNumQueues), 256)), dim3(256), 0, s,
-                       a.counters, n, a.queue);
+    hipLaunchKernelGGL(k_clear_counters, dim3(ceil_div(std::max(n, 1), kClearThreads)), dim3(kClearThreads), 0, s,
+                       a.counters, n, a.queue, a.chunks, a.special);
 }
 
 // A kernel over the field, built for the launch's field kind; the work-counting form takes
@@ -2415,7 +2511,9 @@ void launch_export(const KArgs& a, char* out, hipStream_t s) {
     hipLaunchKernelGGL(k_export, dim3(128, 3), dim3(256), 0, s, a, out);
 }
 void launch_csg(const KArgs& a, int chunks, hipStream_t s) {
-    hipLaunchKernelGGL(k_csg, dim3(kCsgSlabs, chunks), dim3(256), 0, s, a);
+    // a few chunks have no more tiles than that many waves
+    const long tiles = (long)((a.G.F + kCsgX - 1) / kCsgX) * ((a.G.F + kCsgY - 1) / kCsgY) * ((a.G.F + kCsgZ - 1) / kCsgZ);
+    hipLaunchKernelGGL(k_csg, dim3((unsigned)std::min((long)kCsgBlocks, ceil_div(tiles * chunks, 4) + 0L)), dim3(256), 0, s, a);
 }
 // Workgroups per chunk for a kernel that loops over `threads` work items of 256-thread
 // workgroups: all of them for a few chunks, about `target` workgroups over a large batch.

@@ -127,7 +127,7 @@ struct Ctx {
     int ops_cap = 0, idx_cap = 0;
     uint64_t ops_gen = 0;  // bumped when an op array moves (a freed one's address may come back)
     int* d_queue = nullptr;
-    int* d_item_prefix = nullptr;
+    int* d_item_prefix = nullptr;  // KArgs::item_prefix (slots + 1), then KArgs::special (slots + 1)
     int cus = 0;
     std::map<Key, FieldEntry> fields;
     std::map<Key, MeshEntry> meshes;
@@ -185,7 +185,7 @@ DevOp make_dev_op(const lvn_csg_op& op);
 // (the tables and field of the global state).
 KArgs make_kargs(char* arena, const SlotLayout& L, const Geometry& G, const Caps& caps, const ChunkDesc* chunks,
                  Counters* counters, const DevOp* ops, const int* op_index, uint32_t flags, int* queue,
-                 int* item_prefix, int cus);
+                 int* item_prefix, int* special, int cus);
 Geometry make_geometry(int n);
 Caps make_caps(const Geometry& G, int edge_cap, int voxel_cap);
 // lines: room for the line heights of k_height_lines (KArgs::height_lines stays 0 without it).

@@ -300,7 +300,7 @@ int Ctx::allocate(int n, uint32_t fl, int nslots, int edge_cap, int voxel_cap) {
     LVN_HIP(hipHostMalloc(&h_chunks, sizeof(ChunkDesc) * slots, hipHostMallocDefault));
     LVN_HIP(hipHostMalloc(&h_counters, sizeof(Counters) * slots, hipHostMallocDefault));
     LVN_HIP(hipMalloc(&d_queue, sizeof(int) * kNumQueues));
-    LVN_HIP(hipMalloc(&d_item_prefix, sizeof(int) * (slots + 1)));
+    LVN_HIP(hipMalloc(&d_item_prefix, sizeof(int) * 2 * (slots + 1)));
     int dev = 0;
     LVN_HIP(hipGetDevice(&dev));
     LVN_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
@@ -328,7 +328,7 @@ int Ctx::ensure_ops(int nops, int nidx) {
 
 KArgs make_kargs(char* arena, const SlotLayout& L, const Geometry& G, const Caps& caps, const ChunkDesc* chunks,
                  Counters* counters, const DevOp* ops, const int* op_index, uint32_t flags, int* queue,
-                 int* item_prefix, int cus) {
+                 int* item_prefix, int* special, int cus) {
     KArgs a;
     std::memset(&a, 0, sizeof(a));
     a.arena = arena;
@@ -348,6 +348,7 @@ KArgs make_kargs(char* arena, const SlotLayout& L, const Geometry& G, const Caps
     a.precise = (flags & LVN_CTX_PRECISE_QEF) ? 1 : 0;
     a.queue = queue;
     a.item_prefix = item_prefix;
+    a.special = special;
     a.cus = cus;
     a.persist_per_cu = kDefaultPersistPerCu;
     a.height_lines = 0;
@@ -358,7 +359,7 @@ KArgs make_kargs(char* arena, const SlotLayout& L, const Geometry& G, const Caps
 
 KArgs Ctx::kargs() const {
     return make_kargs(d_arena, L, G, caps, d_chunks, d_counters, d_ops, d_op_index, flags, d_queue, d_item_prefix,
-                      cus);
+                      d_item_prefix + slots + 1, cus);
 }
 
 Ctx::~Ctx() {
@@ -830,7 +831,7 @@ struct NoAllocLayout {
     Geometry G;
     Caps caps;
     SlotLayout L;
-    uint64_t chunk, counters, ops, index, queue, prefix, bytes;
+    uint64_t chunk, counters, ops, index, queue, prefix, special, bytes;
 };
 
 static NoAllocLayout noalloc_layout(int n) {
@@ -850,6 +851,7 @@ static NoAllocLayout noalloc_layout(int n) {
     t.index = take(sizeof(int) * LVN_NOALLOC_MAX_OPS);
     t.queue = take(sizeof(int) * kNumQueues);
     t.prefix = take(sizeof(int) * 2);
+    t.special = take(sizeof(int) * 2);
     t.bytes = o;
     return t;
 }
@@ -1118,7 +1120,7 @@ int lvn_generate_chunk_mesh_noalloc(int32_t n, uint32_t flags, const int32_t min
     KArgs a = make_kargs(base, t.L, t.G, t.caps, reinterpret_cast<const ChunkDesc*>(base + t.chunk),
                          reinterpret_cast<Counters*>(base + t.counters), reinterpret_cast<const DevOp*>(base + t.ops),
                          reinterpret_cast<const int*>(base + t.index), flags, reinterpret_cast<int*>(base + t.queue),
-                         reinterpret_cast<int*>(base + t.prefix), d.cus);
+                         reinterpret_cast<int*>(base + t.prefix), reinterpret_cast<int*>(base + t.special), d.cus);
     a.ysplit = default_ysplit(a.G, a.F.kind, 1);  // as the other one-chunk form (single_args)
     launch_pipeline(a, 1, st);
     LVN_HIP(hipGetLastError());

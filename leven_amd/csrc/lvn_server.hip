@@ -183,7 +183,7 @@ int Server::init_lane(Lane& L) {
     LVN_TRY(hipMalloc(&L.d_slot_map, sizeof(int) * B));
     LVN_TRY(hipHostMalloc(&L.h_slot_map, sizeof(int) * B, hipHostMallocDefault));
     LVN_TRY(hipMalloc(&L.d_queue, sizeof(int) * kNumQueues));
-    LVN_TRY(hipMalloc(&L.d_item_prefix, sizeof(int) * (B + 1)));
+    LVN_TRY(hipMalloc(&L.d_item_prefix, sizeof(int) * 2 * (B + 1)));
     // op lists sized up front (1,024 stored ops, op lists of a full batch with up to 256
     // stored ops) so that a lane's first batches allocate nothing; more ops grow them
     L.ops_cap = 1024;
@@ -359,6 +359,7 @@ int Server::launch(Lane& L, const std::vector<Job>& batch, const std::vector<int
     a.slot_map = L.d_slot_map;
     a.queue = L.d_queue;
     a.item_prefix = L.d_item_prefix;
+    a.special = L.d_item_prefix + max_batch + 1;
     a.ops = L.d_ops;
     a.op_index = L.d_op_index;
     lvn_tuning t;
