@@ -537,6 +537,7 @@ __global__ __launch_bounds__(kSeamThreads) __attribute__((amdgpu_waves_per_eu(8,
     }
     __syncthreads();
     const int nleaves = min(s_nodes, J.node_cap);
+    __syncthreads();  // every wave has the leaf count before the first ancestor adds to s_nodes
 
     // 2. ancestors (ConstructParents, src/octree.cpp:29-88): a leaf inserts its parent
     //    chain up to the first parent already present.  A parent key held by a leaf
