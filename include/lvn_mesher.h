@@ -170,7 +170,7 @@ int lvn_generate_seam_mesh(lvn_ctx* ctx, const int32_t host_min[3], int32_t host
                            lvn_vertex* v, int32_t v_cap, int32_t* nv,
                            int32_t* tri, int32_t tri_cap, int32_t* nt);
 
-/* Many seams in one launch sequence, one workgroup per seam.  reqs[i] takes sources
+/* Many seams in one launch sequence.  reqs[i] takes sources
  * [first_source, first_source + n_sources) of `sources`; a source list shared by
  * several seams (the same nodes pointer) is uploaded once.  Per-seam results go to
  * outs[i] (status LVN_OK, LVN_ERR_INVALID or LVN_ERR_CAPACITY as above); the call

@@ -841,23 +841,30 @@ inline int per_seam_blocks(int m) { return std::max(1, std::min(256, 4096 / std:
 // ---------------------------------------------------------------------------
 //
 // The steps of one seam above, each run as one launch over the elements of every seam.
-// Work is cut into tiles of 1024 elements that belong to one seam (offered nodes of one
-// list, hash slots, leaves, nodes, the internal nodes of one level, pending calls); a tile list
+// Work is cut into tiles of elements that belong to one seam (offered nodes of one list,
+// hash slots, leaves, nodes, the internal nodes of one level, pending calls); a tile list
 // is made on the device from each seam's counts, so lists whose length only the device
-// knows (a level's nodes, a round's calls) need no read-back.  A seam's counts, level
+// knows (a level's nodes, a round's calls) need no read-back.  Tiles hold kSgTile elements,
+// or kSgSmallTile where the request is too small to give every CU a large one: a step is a
+// chain of dependent reads per element, and a thread walks its elements one after another.  A seam's counts, level
 // starts, call-list state and status live in its SeamRun record.  Counters shared by a
 // tile's threads are reserved once per tile (LDS histograms, workgroup scans) or once per
 // wave, so the per-seam atomics stay few.
 
 constexpr int kSgTile = 1024;
+constexpr int kSgSmallTile = 256;
 constexpr int kSgThreads = 256;
-constexpr int kSgPer = kSgTile / kSgThreads;
+constexpr int kSgPer = kSgTile / kSgThreads;  // elements of a thread in a large tile
 constexpr int kSgGrid = 2048;  // workgroups of the tile launches
-constexpr int kSgStage = 3072;  // calls a round tile stages in LDS (48 KB)
+constexpr int kSgRoundThreads = 1024;
+constexpr int kSgRoundGrid = 512;  // two workgroups per CU
+constexpr int kSgRoundWaves = kSgRoundThreads / 64;
+constexpr int kSgStage = 192;  // calls a wave of a round tile stages in LDS (48 KB; two workgroups per CU)
 constexpr int kSgLevels = 33;
+constexpr int kSgTop = 5;      // levels 0 .. kSgTop - 1 are walked by one workgroup per seam
 
 struct SeamRun {
-    int nodes, nleaves, nnodes, status;
+    int leaves, inner, status;  // leaves and internal nodes reserved (may pass the node cap: an overflow)
     int root, linked, rounds, stage;  // stage: calls reserved in the staging list this round
     int n, more;              // pending calls; 1 = calls still expand (2 = one was written this round)
     int tbase[8], ntiles;     // this seam's tiles in the current round's list (first position per sub-list)
@@ -888,7 +895,17 @@ struct SeamGrid {
     int* out_t;
     int m;
     int spread;  // tiles of each seam dealt over every XCD (requests of few seams)
+    int tile;    // elements of a tile
+    int lanes;   // lanes that make one seam's tile lists (a power of two, at most a wave)
+    __device__ int tiles_of(int n) const { return (n + tile - 1) / tile; }
+    __device__ int per() const { return tile / kSgThreads; }
 };
+
+// A seam's leaves, and all its nodes (an internal node follows the leaves).
+__device__ __forceinline__ int sg_leaves(const SeamRun& R, const SeamJobDev& J) { return min(R.leaves, J.node_cap); }
+__device__ __forceinline__ int sg_all_nodes(const SeamRun& R, const SeamJobDev& J) {
+    return R.leaves ? min(sg_leaves(R, J) + R.inner, J.node_cap) : 0;
+}
 
 __device__ __forceinline__ SeamScratch sg_scratch(const SeamGrid& g, int s) {
     return seam_scratch(g.scratch + g.jobs[s].scratch, g.jobs[s]);
@@ -964,6 +981,7 @@ __device__ __forceinline__ int lane_rank(uint64_t mask) {
 // sub-list (s + t) mod 8.  Shorter sub-lists are padded with empty tiles (seam -1).  A
 // seam's tiles keep their order: its tiles in one sub-list are consecutive, from base[x].
 constexpr int kXcds = 8;
+constexpr int64_t kSgSmallBelow = 1 << 20;  // requests of fewer leaves (a large tile per CU and more) take small tiles
 constexpr int kSpreadBelow = 64;  // requests of fewer seams spread each seam over every XCD
 
 // Reserves seam s's cnt tiles in the sub-lists (fill = their lengths so far, in LDS):
@@ -997,56 +1015,98 @@ __device__ int sg_pad(int4* out, const int* fill) {
     return kXcds * longest;
 }
 
-// Tile lists (one workgroup of 1024 threads, a thread per seam; workgroup b of a level
-// list makes level b's list at tiles + b * stride).  what: 0 a level's nodes, 1 a round's
-// pending calls of the seams still expanding, 2 the final quads, 3 hash slots, 4 leaves,
-// 5 nodes, 6 offered nodes (one list per source).
-__global__ __launch_bounds__(1024) void k_sg_tiles(SeamGrid g, int what, int4* tiles, int stride, int* total) {
+// A seam's place in the tile lists, made by the group's first lane and handed to all of it.
+__device__ __forceinline__ void sg_place_group(const SeamGrid& g, int s, int cnt, int* fill, int* base) {
+    if ((threadIdx.x & (g.lanes - 1)) == 0) sg_place(g.spread, s, cnt, fill, base);
+#pragma unroll
+    for (int x = 0; x < kXcds; ++x) base[x] = __shfl(base[x], 0, g.lanes);
+}
+// Inclusive scan over a seam's group of lanes.
+__device__ __forceinline__ int sg_group_scan(const SeamGrid& g, int v) {
+    const int lane = threadIdx.x & (g.lanes - 1);
+    for (int off = 1; off < g.lanes; off <<= 1) {
+        const int u = __shfl_up(v, off, g.lanes);
+        if (lane >= off) v += u;
+    }
+    return v;
+}
+
+// Tile lists, one workgroup of 1024 threads per list, g.lanes lanes per seam.  With one
+// thread per seam a request of one seam wrote its tiles one after another (four lists of
+// one seam of 6,000 leaves: 28 us in four launches, of 16 such seams 90 us); the group
+// takes them side by side and the four lists the host's sizes give are one launch.
+enum : int {
+    kSgListHash, kSgListOffered, kSgListLeaf, kSgListNode,  // made together, one workgroup each
+    kSgListLevel,  // the nodes of level blockIdx.x, at tiles + blockIdx.x * off.w
+    kSgListRound,  // pending calls of the seams that still expand
+    kSgListFinal,  // the final quads
+};
+__global__ __launch_bounds__(1024) void k_sg_tiles(SeamGrid g, int first, int4* tiles, int4 off) {
     __shared__ int fill[kXcds];
+    const int what = first + (first == kSgListHash ? (int)blockIdx.x : 0);
     const int l = blockIdx.x;
-    int4* out = tiles + (size_t)l * stride;
+    int4* out = tiles;
+    int* total;
+    switch (what) {
+    case kSgListHash: total = g.cnt + kSgCntHash; break;
+    case kSgListOffered: out += off.x; total = g.cnt + kSgCntOffered; break;
+    case kSgListLeaf: out += off.y; total = g.cnt + kSgCntLeaf; break;
+    case kSgListNode: out += off.z; total = g.cnt + kSgCntNode; break;
+    case kSgListLevel: out += (size_t)l * off.w; total = g.cnt + kSgCntLevel + l; break;
+    case kSgListRound: total = g.cnt + kSgCntRound; break;
+    default: total = g.cnt + kSgCntFinal;
+    }
     if (threadIdx.x < kXcds) fill[threadIdx.x] = 0;
     __syncthreads();
-    for (int s = threadIdx.x; s < g.m; s += blockDim.x) {
-        const SeamRun& R = g.run[s];
+    const int lane = threadIdx.x & (g.lanes - 1);
+    for (int s = threadIdx.x / g.lanes; s < g.m; s += blockDim.x / g.lanes) {
+        SeamRun& R = g.run[s];
         const SeamJobDev& J = g.jobs[s];
-        auto nt = [](int n) { return (n + kSgTile - 1) / kSgTile; };
         int cnt = 0;
         switch (what) {
-        case 0: cnt = R.status == 0 ? nt(R.lev[l + 1] - R.lev[l]) : 0; break;
-        case 1: cnt = R.status == 0 && R.linked && R.more ? nt(R.n) : 0; break;
-        case 2: cnt = R.status == 0 && R.linked ? nt(R.n) : 0; break;
-        case 3: cnt = nt(J.hash_cap); break;
-        case 4: cnt = nt(J.leaf_cap); break;
-        case 5: cnt = nt(J.node_cap); break;
-        default:
-            for (int si = 0; si < J.src_count; ++si) cnt += nt(g.srcs[J.src_begin + si].count);
+        case kSgListHash: cnt = g.tiles_of(J.hash_cap); break;
+        case kSgListLeaf: cnt = g.tiles_of(J.leaf_cap); break;
+        case kSgListNode: cnt = g.tiles_of(J.node_cap); break;
+        case kSgListLevel: cnt = R.status == 0 ? g.tiles_of(R.lev[l + 1] - R.lev[l]) : 0; break;
+        case kSgListRound: cnt = R.status == 0 && R.linked && R.more ? g.tiles_of(R.n) : 0; break;
+        case kSgListFinal: cnt = R.status == 0 && R.linked ? g.tiles_of(R.n) : 0; break;
+        default:  // a list of tiles per source, its lanes a source each
+            for (int s0 = 0; s0 < J.src_count; s0 += g.lanes) {
+                const int v = s0 + lane < J.src_count ? g.tiles_of(g.srcs[J.src_begin + s0 + lane].count) : 0;
+                cnt += __shfl(sg_group_scan(g, v), g.lanes - 1, g.lanes);
+            }
         }
         int base[kXcds];
-        sg_place(g.spread, s, cnt, fill, base);
-        if (what == 6) {
-            int t = 0;
-            for (int si = 0; si < J.src_count; ++si)
-                for (int j = 0; j < g.srcs[J.src_begin + si].count; j += kSgTile)
-                    out[sg_tile_index(g.spread, s, t++, base)] = make_int4(s, j, si, 0);
-        } else {
-            for (int t = 0; t < cnt; ++t) out[sg_tile_index(g.spread, s, t, base)] = make_int4(s, t * kSgTile, 0, 0);
-            if (what == 1) {
-                for (int x = 0; x < kXcds; ++x) g.run[s].tbase[x] = base[x];
-                g.run[s].ntiles = cnt;
+        sg_place_group(g, s, cnt, fill, base);
+        if (what == kSgListOffered) {
+            int t0 = 0;
+            for (int s0 = 0; s0 < J.src_count; s0 += g.lanes) {
+                const int si = s0 + lane;
+                const int v = si < J.src_count ? g.tiles_of(g.srcs[J.src_begin + si].count) : 0;
+                const int incl = sg_group_scan(g, v);
+                for (int j = 0; j < v; ++j)
+                    out[sg_tile_index(g.spread, s, t0 + incl - v + j, base)] = make_int4(s, j * g.tile, si, 0);
+                t0 += __shfl(incl, g.lanes - 1, g.lanes);
             }
+            continue;
+        }
+        for (int t = lane; t < cnt; t += g.lanes)
+            out[sg_tile_index(g.spread, s, t, base)] = make_int4(s, t * g.tile, 0, 0);
+        if (what == kSgListRound && lane == 0) {
+            for (int x = 0; x < kXcds; ++x) R.tbase[x] = base[x];
+            R.ntiles = cnt;
         }
     }
     __syncthreads();
     const int n = sg_pad(out, fill);
-    if (threadIdx.x == 0) total[l] = n;
+    if (threadIdx.x == 0) *total = n;
 }
 
 // Seam records and round counters cleared; every hash slot emptied.
 __global__ __launch_bounds__(kSgThreads) void k_sg_init(SeamGrid g, const int4* tiles) {
     for (int s = blockIdx.x * kSgThreads + threadIdx.x; s < g.m; s += gridDim.x * kSgThreads) {
         SeamRun& R = g.run[s];
-        R.nodes = R.nleaves = R.nnodes = R.status = 0;
+        R.leaves = R.inner = R.status = 0;
         R.root = -1;
         R.linked = R.rounds = R.stage = 0;
         R.n = R.more = 0;
@@ -1059,7 +1119,7 @@ __global__ __launch_bounds__(kSgThreads) void k_sg_init(SeamGrid g, const int4* 
     LVN_SG_TILES(tiles, g.cnt[kSgCntHash]) {
         const SeamJobDev& J = g.jobs[tl.x];
         SeamScratch S = sg_scratch(g, tl.x);
-        for (int r = 0; r < kSgPer; ++r) {
+        for (int r = 0; r < g.per(); ++r) {
             const int i = tl.y + threadIdx.x + r * kSgThreads;
             if (i >= J.hash_cap) continue;
             S.keys[i] = kEmptyKey;
@@ -1082,7 +1142,7 @@ __global__ __launch_bounds__(kSgThreads) void k_sg_select(SeamGrid g, const int4
         const int root_size = 2 * J.host_size;
         const int root_levels = __builtin_ctz((unsigned)root_size);
         const int mask = J.hash_cap - 1;
-        for (int r = 0; r < kSgPer; ++r) {
+        for (int r = 0; r < g.per(); ++r) {
             const int j = tl.y + threadIdx.x + r * kSgThreads;
             if (j >= src.count) continue;
             int mn[3];
@@ -1116,15 +1176,16 @@ __global__ __launch_bounds__(kSgThreads) void k_sg_leaves(SeamGrid g, const int4
         SeamRun& R = g.run[tl.x];
         SeamScratch S = sg_scratch(g, tl.x);
         const SgNodes Q = sg_nodes(S, J.node_cap);
-        const int i0 = tl.y + threadIdx.x * kSgPer;
+        const int per = g.per();
+        const int i0 = tl.y + threadIdx.x * per;
         uint64_t key[kSgPer];
         int cnt = 0;
 #pragma unroll
         for (int r = 0; r < kSgPer; ++r) {
-            key[r] = i0 + r < J.hash_cap ? S.keys[i0 + r] : kEmptyKey;
+            key[r] = r < per && i0 + r < J.hash_cap ? S.keys[i0 + r] : kEmptyKey;
             cnt += key[r] != kEmptyKey;
         }
-        int idx = sg_reserve(cnt, &R.nodes);
+        int idx = sg_reserve(cnt, &R.leaves);
 #pragma unroll
         for (int r = 0; r < kSgPer; ++r) {
             if (key[r] == kEmptyKey) continue;
@@ -1151,37 +1212,18 @@ __global__ __launch_bounds__(kSgThreads) void k_sg_leaves(SeamGrid g, const int4
     }
 }
 
-// Per seam between steps.  0: the leaves are counted; 1: the ancestors too; 2: level
-// counts become level starts and the root is found; 3: the contouring list starts with
-// the root's cell call.
-__global__ void k_sg_seam(SeamGrid g, int step) {
+// Per seam: level counts become level starts and the root is found.
+__global__ void k_sg_seam(SeamGrid g) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= g.m) return;
     const SeamJobDev& J = g.jobs[s];
     SeamRun& R = g.run[s];
-    if (step == 0) {
-        R.nleaves = min(R.nodes, J.node_cap);
-    } else if (step == 1) {
-        R.nnodes = R.nleaves ? min(R.nodes, J.node_cap) : 0;
-    } else if (step == 2) {
-        for (int l = 1; l <= kSgLevels; ++l) R.lev[l] += R.lev[l - 1];
-        for (int l = 0; l < kSgLevels; ++l) R.fill[l] = R.lev[l];
-        if (R.status == 0 && R.nleaves > 0) {
-            SeamScratch S = sg_scratch(g, s);
-            const int slot = hash_find(S.keys, J.hash_cap - 1, 0ull);
-            R.root = slot < 0 ? -1 : S.vals[slot];
-        }
-    } else {
-        R.linked = R.status == 0 && R.nleaves > 0 && R.root >= 0;
-        R.n = 0;
-        if (R.linked) {
-            SeamScratch S = sg_scratch(g, s);
-            if (R.root >= R.nleaves && ((S.shape[R.root] >> 56) & 1) == 0) {  // an internal root
-                S.list0[0] = make_call(R.root, -1, -1, -1, kCallCell);
-                R.n = 1;
-            }
-        }
-        R.more = R.n > 0;
+    for (int l = 1; l <= kSgLevels; ++l) R.lev[l] += R.lev[l - 1];
+    for (int l = 0; l < kSgLevels; ++l) R.fill[l] = R.lev[l];
+    if (R.status == 0 && R.leaves > 0) {
+        SeamScratch S = sg_scratch(g, s);
+        const int slot = hash_find(S.keys, J.hash_cap - 1, 0ull);
+        R.root = slot < 0 ? -1 : S.vals[slot];
     }
 }
 
@@ -1198,8 +1240,8 @@ __global__ __launch_bounds__(kSgThreads) void k_sg_ancestors(SeamGrid g, const i
         const SgNodes Q = sg_nodes(S, J.node_cap);
         const int mask = J.hash_cap - 1;
         const int root_size = 2 * J.host_size;
-        const int nleaves = R.nleaves;
-        for (int r = 0; r < kSgPer; ++r) {
+        const int nleaves = sg_leaves(R, J);
+        for (int r = 0; r < g.per(); ++r) {
             const int i = tl.y + threadIdx.x + r * kSgThreads;
             const bool leaf = i < nleaves;
             const uint64_t lk = leaf ? Q.key[i] : 0;
@@ -1226,7 +1268,7 @@ __global__ __launch_bounds__(kSgThreads) void k_sg_ancestors(SeamGrid g, const i
                 if (!fm) continue;
                 const int leader = __ffsll((unsigned long long)fm) - 1;
                 int base = 0;
-                if ((int)(threadIdx.x & 63) == leader) base = atomicAdd(&R.nodes, __popcll(fm));
+                if ((int)(threadIdx.x & 63) == leader) base = nleaves + atomicAdd(&R.inner, __popcll(fm));
                 base = __shfl(base, leader, 64);
                 if (!fresh) continue;
                 const int idx = base + lane_rank(fm);
@@ -1260,7 +1302,7 @@ __global__ __launch_bounds__(kSgThreads) void k_sg_links(SeamGrid g, const int4*
         SeamRun& R = g.run[tl.x];
         // the status can change while the tile runs (set by other tiles): one thread
         // decides for the workgroup, whose barriers follow
-        if (threadIdx.x == 0) skip = load_l2(&R.status) != 0 || tl.y >= R.nnodes;
+        if (threadIdx.x == 0) skip = load_l2(&R.status) != 0 || tl.y >= sg_all_nodes(R, J);
         if (threadIdx.x < kSgLevels) hist[threadIdx.x] = 0;
         __syncthreads();
         if (skip) {
@@ -1269,13 +1311,13 @@ __global__ __launch_bounds__(kSgThreads) void k_sg_links(SeamGrid g, const int4*
         }
         SeamScratch S = sg_scratch(g, tl.x);
         const SgNodes Q = sg_nodes(S, J.node_cap);
-        const int nnodes = R.nnodes;
-        for (int r = 0; r < kSgPer; ++r) {
+        const int nleaves = sg_leaves(R, J), nnodes = sg_all_nodes(R, J);
+        for (int r = 0; r < g.per(); ++r) {
             const int i = tl.y + threadIdx.x + r * kSgThreads;
             if (i >= nnodes) continue;
             const uint64_t k = Q.key[i];
             const int level = (int)(k >> 48);
-            if (i >= R.nleaves) atomicAdd(&hist[level], 1);  // internal nodes (created after the leaves)
+            if (i >= nleaves) atomicAdd(&hist[level], 1);  // internal nodes (created after the leaves)
             if (level == 0) continue;
             const uint64_t c = k & kCodeMask;
             const int slot = hash_find(S.keys, J.hash_cap - 1, (uint64_t)(level - 1) << 48 | (c >> 3));
@@ -1297,18 +1339,19 @@ __global__ __launch_bounds__(kSgThreads) void k_sg_links(SeamGrid g, const int4*
 __global__ __launch_bounds__(kSgThreads) void k_sg_order(SeamGrid g, const int4* tiles) {
     __shared__ int hist[kSgLevels], base[kSgLevels];
     LVN_SG_TILES(tiles, g.cnt[kSgCntNode]) {
+        const SeamJobDev& J = g.jobs[tl.x];
         SeamRun& R = g.run[tl.x];
-        if (R.status != 0 || tl.y >= R.nnodes || tl.y + kSgTile <= R.nleaves) continue;
+        const int nleaves = sg_leaves(R, J), nnodes = sg_all_nodes(R, J), per = g.per();
+        if (R.status != 0 || tl.y >= nnodes || tl.y + g.tile <= nleaves) continue;
         SeamScratch S = sg_scratch(g, tl.x);
-        const SgNodes Q = sg_nodes(S, g.jobs[tl.x].node_cap);
+        const SgNodes Q = sg_nodes(S, J.node_cap);
         if (threadIdx.x < kSgLevels) hist[threadIdx.x] = 0;
         __syncthreads();
-        const int nnodes = R.nnodes, nleaves = R.nleaves;
         int lv[kSgPer];
 #pragma unroll
         for (int r = 0; r < kSgPer; ++r) {
             const int i = tl.y + threadIdx.x + r * kSgThreads;
-            lv[r] = i >= nleaves && i < nnodes ? (int)(Q.key[i] >> 48) : -1;
+            lv[r] = r < per && i >= nleaves && i < nnodes ? (int)(Q.key[i] >> 48) : -1;
             if (lv[r] >= 0) atomicAdd(&hist[lv[r]], 1);
         }
         __syncthreads();
@@ -1324,9 +1367,33 @@ __global__ __launch_bounds__(kSgThreads) void k_sg_order(SeamGrid g, const int4*
     }
 }
 
-// One level's internal nodes: leaf counts gathered from the children (a leaf counts 1;
-// deepest level first), or depth-first ranks handed to the children in child order (top
-// level first).
+// One internal node of a level: its leaf count gathered from its children (a leaf counts
+// 1), or its depth-first rank handed to them in child order.
+__device__ __forceinline__ void sg_level_node(const SeamScratch& S, const SgNodes& Q, int k, bool ranks) {
+    const int i = S.order[k];
+    int ch[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) ch[c] = S.ch[8 * i + c];
+    int cnt[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) cnt[c] = ch[c] >= 0 ? Q.co[ch[c]].x : 0;
+    if (!ranks) {
+        int sum = 0;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) sum += cnt[c];
+        Q.co[i].x = sum;
+    } else {
+        int off = Q.co[i].y;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            if (ch[c] < 0) continue;
+            Q.co[ch[c]].y = off;
+            off += cnt[c];
+        }
+    }
+}
+
+// The internal nodes of one deep level: counts deepest level first, ranks top level first.
 __global__ __launch_bounds__(kSgThreads) void k_sg_level(SeamGrid g, const int4* tiles, int l, int ranks) {
     LVN_SG_TILES(tiles, g.cnt[kSgCntLevel + l]) {
         SeamRun& R = g.run[tl.x];
@@ -1334,31 +1401,41 @@ __global__ __launch_bounds__(kSgThreads) void k_sg_level(SeamGrid g, const int4*
         SeamScratch S = sg_scratch(g, tl.x);
         const SgNodes Q = sg_nodes(S, g.jobs[tl.x].node_cap);
         const int first = R.lev[l], end = R.lev[l + 1];
-        for (int r = 0; r < kSgPer; ++r) {
+        for (int r = 0; r < g.per(); ++r) {
             const int k = first + tl.y + threadIdx.x + r * kSgThreads;
-            if (k >= end) continue;
-            const int i = S.order[k];
-            int ch[8];
-#pragma unroll
-            for (int c = 0; c < 8; ++c) ch[c] = S.ch[8 * i + c];
-            int cnt[8];
-#pragma unroll
-            for (int c = 0; c < 8; ++c) cnt[c] = ch[c] >= 0 ? Q.co[ch[c]].x : 0;
-            if (!ranks) {
-                int sum = 0;
-#pragma unroll
-                for (int c = 0; c < 8; ++c) sum += cnt[c];
-                Q.co[i].x = sum;
-            } else {
-                int off = Q.co[i].y;
-#pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    if (ch[c] < 0) continue;
-                    Q.co[ch[c]].y = off;
-                    off += cnt[c];
-                }
-            }
+            if (k < end) sg_level_node(S, Q, k, ranks);
         }
+    }
+}
+
+// Levels 0 .. top - 1 of one seam per workgroup: leaf counts up to the root, the
+// contouring list started with the root's cell call, ranks handed down.  A seam's leaves
+// lie on faces, so these levels hold about 3 * 4^l nodes; each level of its own was a
+// launch up and a launch down of 3 to 5 us with next to nothing to do.
+__global__ __launch_bounds__(1024) void k_sg_top(SeamGrid g, int top) {
+    const int s = blockIdx.x;
+    const SeamJobDev& J = g.jobs[s];
+    SeamRun& R = g.run[s];
+    SeamScratch S = sg_scratch(g, s);
+    const SgNodes Q = sg_nodes(S, J.node_cap);
+    const bool ok = R.status == 0;
+    const int nleaves = sg_leaves(R, J), root = R.root;
+    const bool linked = ok && nleaves > 0 && root >= 0;
+    if (!ok) top = 0;
+    for (int l = top - 1; l >= 1; --l) {
+        for (int k = R.lev[l] + threadIdx.x; k < R.lev[l + 1]; k += blockDim.x) sg_level_node(S, Q, k, false);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        R.linked = linked;
+        const bool cell = linked && root >= nleaves && ((S.shape[root] >> 56) & 1) == 0;  // an internal root
+        if (cell) S.list0[0] = make_call(root, -1, -1, -1, kCallCell);
+        R.n = R.more = cell;
+    }
+    if (!linked) return;
+    for (int l = 0; l < top; ++l) {
+        for (int k = R.lev[l] + threadIdx.x; k < R.lev[l + 1]; k += blockDim.x) sg_level_node(S, Q, k, true);
+        __syncthreads();
     }
 }
 
@@ -1370,8 +1447,8 @@ __global__ __launch_bounds__(kSgThreads) void k_sg_vertices(SeamGrid g, const in
         if (!R.linked) continue;
         SeamScratch S = sg_scratch(g, tl.x);
         const SgNodes Q = sg_nodes(S, J.node_cap);
-        const int nleaves = R.nleaves;
-        for (int r = 0; r < kSgPer; ++r) {
+        const int nleaves = sg_leaves(R, J);
+        for (int r = 0; r < g.per(); ++r) {
             const int i = tl.y + threadIdx.x + r * kSgThreads;
             if (i >= nleaves) continue;
             const uint64_t p = Q.offer[i];
@@ -1394,64 +1471,214 @@ __global__ __launch_bounds__(kSgThreads) void k_sg_vertices(SeamGrid g, const in
     }
 }
 
-// 4. One contouring round: every pending call replaced by the calls it makes.  Thread t
-// of a tile expands calls t * 4 .. t * 4 + 3 of it: it counts their calls, the workgroup
-// scans the counts, reserves the tile's block of the staging list (list1) with one
-// atomic and writes the calls at once, their nodes still in cache.  The blocks are put
-// in call order by k_sg_round_copy after k_sg_round_next has scanned each seam's tile
-// counts in tile order.
-__global__ __launch_bounds__(kSgThreads) void k_sg_round(SeamGrid g, const int4* tiles, int round, int* tsum,
-                                                          int* tbase) {
+// The calls a call may make ("candidates"), as one table over every kind and direction:
+// four (node of the call, child of it) pairs of 5 bits, then the made call's kind and
+// direction.  A cell call has 26 candidates (8 cells, 12 faces, 6 edges), a face call 8
+// (4 faces, 4 edges), an edge call 2, a finished quad itself.
+constexpr int kCandCell = 0, kCandFace = 26, kCandEdge = 50, kCandQuad = 56, kCands = 57;
+struct CandTable {
+    uint32_t v[kCands];
+};
+constexpr uint32_t cand_node(int j, int node, int child) { return (uint32_t)(node << 3 | child) << (5 * j); }
+constexpr uint32_t cand_kind(int kind, int dir) { return (uint32_t)(kind | dir << 2) << 20; }
+constexpr CandTable make_cands() {
+    CandTable t{};
+    int k = 0;
+    for (int i = 0; i < 8; ++i) t.v[k++] = cand_node(0, 0, i) | cand_kind(kCallCell, 0);
+    for (int i = 0; i < 12; ++i)
+        t.v[k++] = cand_node(0, 0, kCellFaces[i][0]) | cand_node(1, 0, kCellFaces[i][1]) |
+                   cand_kind(kCallFace, kCellFaces[i][2]);
+    for (int i = 0; i < 6; ++i) {
+        t.v[k] = cand_kind(kCallEdge, kCellEdges[i][4]);
+        for (int j = 0; j < 4; ++j) t.v[k] |= cand_node(j, 0, kCellEdges[i][j]);
+        ++k;
+    }
+    for (int d = 0; d < 3; ++d) {
+        for (int i = 0; i < 4; ++i)
+            t.v[k++] = cand_node(0, 0, kFaceFaces[d][i][0]) | cand_node(1, 1, kFaceFaces[d][i][1]) |
+                       cand_kind(kCallFace, kFaceFaces[d][i][2]);
+        for (int i = 0; i < 4; ++i) {
+            t.v[k] = cand_kind(kCallEdge, kFaceEdges[d][i][5]);
+            for (int j = 0; j < 4; ++j)
+                t.v[k] |= cand_node(j, kFaceEdgeOrder[kFaceEdges[d][i][0]][j], kFaceEdges[d][i][1 + j]);
+            ++k;
+        }
+    }
+    for (int d = 0; d < 3; ++d)
+        for (int i = 0; i < 2; ++i) {
+            t.v[k] = cand_kind(kCallEdge, kEdgeEdges[d][i][4]);
+            for (int j = 0; j < 4; ++j) t.v[k] |= cand_node(j, j, kEdgeEdges[d][i][j]);
+            ++k;
+        }
+    t.v[k] = cand_kind(kCallQuad, 0);
+    return t;
+}
+__constant__ constexpr CandTable kCandTable = make_cands();
+// Corner pairs of an edge call's four nodes, 6 bits a node (ContourProcessEdge).
+constexpr uint32_t process_corners(int dir) {
+    uint32_t v = 0;
+    for (int i = 0; i < 4; ++i)
+        v |= (uint32_t)(kEdgeCorners[kProcessEdge[dir][i]][0] | kEdgeCorners[kProcessEdge[dir][i]][1] << 3) << (6 * i);
+    return v;
+}
+
+// One candidate of a call: true if the call is made, *out = it.  The tests are Expander's.
+__device__ __forceinline__ bool sg_candidate(const SeamScratch& S, const Call& c, uint32_t cand, Call* out) {
+    const int kind = (cand >> 20) & 3, dir = (cand >> 22) & 3;
+    if (kind == kCallQuad) {
+        *out = c;
+        return true;
+    }
+    const int used = kind == kCallEdge ? 4 : kind == kCallFace ? 2 : 1;
+    int n[4];
+    uint64_t h[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int sel = (cand >> (5 * j + 3)) & 3, child = (cand >> (5 * j)) & 7;
+        const int node = sel == 0 ? c.node(0) : sel == 1 ? c.w[1] : sel == 2 ? c.w[2] : c.w[3];
+        n[j] = -1;
+        if (j < used) {  // the node itself where it is a leaf, else its child
+            const int below = S.ch[8 * node + child];
+            n[j] = (S.shape[node] >> 42) & 1 ? below : node;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) h[j] = n[j] >= 0 ? S.shape[n[j]] : 0;
+    bool made;
+    int meta = kind | dir << 2;
+    if (kind == kCallCell) {
+        made = n[0] >= 0 && ((h[0] >> 42) & 1) && !((h[0] >> 56) & 1);
+    } else if (kind == kCallFace) {
+        made = n[0] >= 0 && n[1] >= 0 && !same_chunk(h[0], h[1]) && (((h[0] | h[1]) >> 42) & 1);
+    } else {
+        made = n[0] >= 0 && n[1] >= 0 && n[2] >= 0 && n[3] >= 0 &&
+               !(same_chunk(h[0], h[1]) && same_chunk(h[0], h[2]) && same_chunk(h[0], h[3]));
+        if (made && !(((h[0] | h[1] | h[2] | h[3]) >> 42) & 1)) {
+            // ContourProcessEdge, src/octree.cpp:235-282
+            constexpr uint32_t pc0 = process_corners(0), pc1 = process_corners(1), pc2 = process_corners(2);
+            const uint32_t pc = dir == 0 ? pc0 : dir == 1 ? pc1 : pc2;
+            int min_size = 0x7fffffff;
+            bool flip = false, change = false;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int corners = (int)(h[i] >> 48) & 0xff;
+                const int size = (int)(h[i] >> 43) & 31;  // log2: the order of sizes is kept
+                const int m0 = (corners >> ((pc >> (6 * i)) & 7)) & 1;
+                const int m1 = (corners >> ((pc >> (6 * i + 3)) & 7)) & 1;
+                if (size < min_size) {
+                    min_size = size;
+                    flip = m1 != 1;
+                    change = m0 != m1;
+                }
+            }
+            made = change;
+            meta = kCallQuad | (flip ? 16 : 0);
+        }
+    }
+    if (made) *out = make_call(n[0], n[1], n[2], n[3], meta);
+    return made;
+}
+
+// 4. One contouring round: every pending call replaced by the calls it makes.  A wave
+// takes 1/16 of the tile's calls and gives every candidate of theirs a lane, in call
+// order: two dependent reads (child, then shape) decide all of them at once, whatever
+// their kinds, and a ballot puts the made ones in order in LDS.  The tile then reserves
+// its block of the staging list (list1) with one atomic and writes it in whole lines.  The
+// blocks are put in call order by k_sg_round_copy after k_sg_round_next has scanned each
+// seam's tile counts in tile order.  A thread per call ran the seven kinds and directions
+// of a wave's calls one after another, and everything twice (to count, then to write): a
+// middle round of one seam of 6,000 leaves took 62 us in 20 workgroups and takes 9 us in
+// 80, of 16 coarse seams of 25,000 leaves each 93 us and now 35 us.
+__global__ __launch_bounds__(kSgRoundThreads) void k_sg_round(SeamGrid g, const int4* tiles, int round, int* tsum,
+                                                              int* tbase) {
+    __shared__ Call stage[kSgRoundWaves][kSgStage];
+    __shared__ Call calls[kSgRoundWaves][64];
+    __shared__ int starts[kSgRoundWaves][64];  // a call's first candidate
+    __shared__ uint32_t cands[kCands];
+    __shared__ int made_by[kSgRoundWaves];
     __shared__ int base;
-    __shared__ Call stage[kSgStage];
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    if (threadIdx.x < kCands) cands[threadIdx.x] = kCandTable.v[threadIdx.x];
+    __syncthreads();
+    const int per_wave = g.tile / kSgRoundWaves;  // 16 or 64 calls
     LVN_SG_TILES(tiles, g.cnt[kSgCntRound + round]) {
         const SeamJobDev& J = g.jobs[tl.x];
         SeamRun& R = g.run[tl.x];
         SeamScratch S = sg_scratch(g, tl.x);
-        const Call* A = S.list0;
-        const int n = R.n;
-        const int i0 = tl.y + threadIdx.x * kSgPer;
+        const int n = min(R.n - (tl.y + w * per_wave), per_wave);  // calls of this wave (may be negative)
         int cnt = 0;
-        for (int q = 0; q < kSgPer && i0 + q < n; ++q) {
-            Expander e{S.ch, S.shape, S.list1, 0, 0, 0, false};
-            e.expand(A[i0 + q]);
-            cnt += e.k;
+        if (lane < n) {
+            const Call c = S.list0[tl.y + w * per_wave + lane];
+            const int kind = c.meta() & 3;
+            cnt = kind == kCallEdge ? 2 : kind == kCallFace ? 8 : kind == kCallQuad ? 1 : 26;
+            calls[w][lane] = c;
         }
-        int total;
-        const int at = sg_scan(cnt, &total);
+        const int incl = wave_inclusive(cnt);
+        starts[w][lane] = incl - cnt;
+        __builtin_amdgcn_wave_barrier();  // read by the wave's other lanes below
+        const int total = __shfl(incl, 63, 64);
+        // candidate j of the wave: the made call, if any (lanes past the end make none)
+        auto candidate = [&](int j, Call* out) {
+            if (j >= total) return false;
+            int a = 0;  // the last call that starts at or before j
+            for (int step = per_wave >> 1; step; step >>= 1)
+                if (a + step < n && starts[w][a + step] <= j) a += step;
+            const Call c = calls[w][a];
+            const int kind = c.meta() & 3, dir = (c.meta() >> 2) & 3;
+            const int row = kind == kCallEdge   ? kCandEdge + 2 * dir
+                            : kind == kCallFace ? kCandFace + 8 * dir
+                            : kind == kCallQuad ? kCandQuad
+                                                : kCandCell;
+            return sg_candidate(S, c, cands[row + j - starts[w][a]], out);
+        };
+        int made = 0;
+        bool more = false;
+        for (int j0 = 0; j0 < total; j0 += 64) {
+            Call out;
+            const bool m = candidate(j0 + lane, &out);
+            const uint64_t mask = __ballot(m);
+            const int at = made + lane_rank(mask);
+            if (m && at < kSgStage) stage[w][at] = out;
+            more |= m && (out.meta() & 3) != kCallQuad;
+            made += __popcll(mask);
+        }
+        if (lane == 0) made_by[w] = made;
+        __syncthreads();
+        int first = 0, sum = 0;
+#pragma unroll
+        for (int i = 0; i < kSgRoundWaves; ++i) {
+            first += i < w ? made_by[i] : 0;
+            sum += made_by[i];
+        }
         if (threadIdx.x == 0) {
-            base = total ? atomicAdd(&R.stage, total) : 0;
-            tsum[tk] = total;
+            base = sum ? atomicAdd(&R.stage, sum) : 0;
+            tsum[tk] = sum;
             tbase[tk] = base;
         }
         __syncthreads();
         const int b0 = base;
-        __syncthreads();  // base is rewritten by the next tile
-        if (total == 0 || b0 + total > J.list_cap) continue;  // (the seam's total then exceeds its cap)
-        // the tile's block is written from LDS in whole lines when it fits there
-        const bool in_lds = total <= kSgStage;
-        Call* dst = in_lds ? stage : S.list1 + b0;
-        int w_at = at;
-        bool m = false;
-        for (int q = 0; q < kSgPer && i0 + q < n; ++q) {
-            Expander w{S.ch, S.shape, dst, w_at, 0, 0, true};
-            w.expand(A[i0 + q]);
-            w_at += w.k;
-            m |= w.more != 0;
-        }
-        if (m) R.more = 2;
-        if (in_lds) {
-            __syncthreads();
-            Call* out = S.list1 + b0;
-            for (int i = threadIdx.x; i < total; i += kSgThreads) out[i] = stage[i];
-            __syncthreads();
+        __syncthreads();  // base and made_by are rewritten by the next tile
+        if (sum == 0 || b0 + sum > J.list_cap) continue;  // (the seam's total then exceeds its cap)
+        if (more) R.more = 2;
+        Call* dst = S.list1 + b0 + first;
+        if (made <= kSgStage) {
+            for (int i = lane; i < made; i += 64) dst[i] = stage[w][i];
+        } else {  // more than the stage holds: the candidates once more, written at once
+            int at = 0;
+            for (int j0 = 0; j0 < total; j0 += 64) {
+                Call out;
+                const bool m = candidate(j0 + lane, &out);
+                const uint64_t mask = __ballot(m);
+                if (m) dst[at + lane_rank(mask)] = out;
+                at += __popcll(mask);
+            }
         }
     }
 }
 
-// After a round, per seam (one workgroup of 1024 threads, a thread per seam): the tile
-// counts of the round scanned in tile order into the blocks' places in the next list, the
-// seam's round closed (the next list's length; the seam stays in the rounds while a
+// After a round, per seam (one workgroup of 1024 threads, g.lanes lanes per seam): the
+// tile counts of the round scanned in tile order into the blocks' places in the next list,
+// the seam's round closed (the next list's length; the seam stays in the rounds while a
 // written call still expands, counted in the round's active counter; an overflow of the
 // list or of the round limit ends it), and the next round's tile list made.
 __global__ __launch_bounds__(1024) void k_sg_round_next(SeamGrid g, int round, const int* tsum, int* toff,
@@ -1459,34 +1686,48 @@ __global__ __launch_bounds__(1024) void k_sg_round_next(SeamGrid g, int round, c
     __shared__ int fill[kXcds];
     if (threadIdx.x < kXcds) fill[threadIdx.x] = 0;
     __syncthreads();
+    const int lane = threadIdx.x & (g.lanes - 1);
     int active = 0;
-    for (int s = threadIdx.x; s < g.m; s += blockDim.x) {
+    for (int s = threadIdx.x / g.lanes; s < g.m; s += blockDim.x / g.lanes) {
         SeamRun& R = g.run[s];
         const SeamJobDev& J = g.jobs[s];
-        if (R.status == 0 && R.linked && R.more && R.ntiles > 0) {
+        int status = R.status, more = R.more, n = R.n;
+        const int ntiles = R.ntiles, linked = R.linked;
+        int base[kXcds];
+        if (status == 0 && linked && more && ntiles > 0) {
+            for (int x = 0; x < kXcds; ++x) base[x] = R.tbase[x];
             int sum = 0;
-            for (int t = 0; t < R.ntiles; ++t) {
-                const int k = sg_tile_index(g.spread, s, t, R.tbase);
-                const int v = tsum[k];
-                toff[k] = sum;
-                sum += v;
+            for (int t0 = 0; t0 < ntiles; t0 += g.lanes) {
+                const int k = t0 + lane < ntiles ? sg_tile_index(g.spread, s, t0 + lane, base) : -1;
+                const int v = k >= 0 ? tsum[k] : 0;
+                const int incl = sg_group_scan(g, v);
+                if (k >= 0) toff[k] = sum + incl - v;
+                sum += __shfl(incl, g.lanes - 1, g.lanes);
             }
-            R.rounds += 1;
-            R.stage = 0;
-            if (sum > J.list_cap || R.rounds >= kMaxRounds) {
-                set_status(&R.status, LVN_ERR_OVERFLOW);
+            const int rounds = R.rounds + 1;
+            if (sum > J.list_cap || rounds >= kMaxRounds) {
+                status = LVN_ERR_OVERFLOW;
             } else {
-                R.n = sum;
-                R.more = R.more == 2;
-                active += R.more;
+                n = sum;
+                more = more == 2;
+            }
+            if (lane == 0) {
+                R.rounds = rounds;
+                R.stage = 0;
+                if (status) set_status(&R.status, status);
+                R.n = n;
+                R.more = more;
+                active += status == 0 && more;
             }
         }
-        const int cnt = R.status == 0 && R.linked && R.more ? (R.n + kSgTile - 1) / kSgTile : 0;
-        int base[kXcds];
-        sg_place(g.spread, s, cnt, fill, base);
-        for (int t = 0; t < cnt; ++t) next[sg_tile_index(g.spread, s, t, base)] = make_int4(s, t * kSgTile, 0, 0);
-        for (int x = 0; x < kXcds; ++x) R.tbase[x] = base[x];
-        R.ntiles = cnt;
+        const int cnt = status == 0 && linked && more ? g.tiles_of(n) : 0;
+        sg_place_group(g, s, cnt, fill, base);
+        for (int t = lane; t < cnt; t += g.lanes)
+            next[sg_tile_index(g.spread, s, t, base)] = make_int4(s, t * g.tile, 0, 0);
+        if (lane == 0) {
+            for (int x = 0; x < kXcds; ++x) R.tbase[x] = base[x];
+            R.ntiles = cnt;
+        }
     }
     __syncthreads();
     const int n = sg_pad(next, fill);
@@ -1517,7 +1758,7 @@ __global__ __launch_bounds__(kSgThreads) void k_sg_triangles(SeamGrid g, const i
         const SgNodes Q = sg_nodes(S, J.node_cap);
         const Call* quads = S.list0;
         const int n = R.n;
-        for (int r = 0; r < kSgPer; ++r) {
+        for (int r = 0; r < g.per(); ++r) {
             const int i = tl.y + threadIdx.x + r * kSgThreads;
             if (i >= n) continue;
             const Call c = quads[i];
@@ -1538,7 +1779,7 @@ __global__ __launch_bounds__(kSgThreads) void k_sg_triangles(SeamGrid g, const i
         const bool ok = R.status == 0 && R.linked;
         SeamResDev r;
         r.status = R.status;
-        r.nv = ok ? R.nleaves : 0;
+        r.nv = ok ? sg_leaves(R, g.jobs[s]) : 0;
         r.nt = ok ? 2 * R.n : 0;
         r.rounds = R.rounds;
         res[s] = r;
@@ -1714,14 +1955,18 @@ int resolve_batch(void* owner, const lvn_seam_source& q, SeamSrcDev& d) {
 // the sizes the host knows, clear, select, leaves, ancestors, links, level buckets, leaf
 // counts (deepest level first), ranks (top level first), vertices, contouring rounds,
 // triangles.  The rounds run in batches without a read-back; after a batch the host reads
-// how many seams still expand.  A call descends at least one level per round, so the
-// first batch (deepest possible level + 3 rounds) normally finishes every seam.
+// how many seams still expand.  A call made in round r (from 1) has its internal nodes at
+// level r or deeper, and no internal node lies at the deepest level, so the first batch (a
+// round per level) finishes every seam.
 int run_seam_grid(Ctx* c, SeamState& st, int m, const SeamJobDev* h_jobs, const std::vector<SeamSrcDev>& srcs,
                   const SeamJobDev* d_jobs, lvn_vertex* ov, int* ot, SeamResDev* d_res) {
     // list lengths: eight interleaved sub-lists, seam k in sub-list k mod 8, each padded to
     // the longest (bounds from the seams' caps)
     const bool spread = m < kSpreadBelow;
-    auto nt = [](int64_t n) { return (n + kSgTile - 1) / kSgTile; };
+    int64_t leaves = 0;
+    for (int k = 0; k < m; ++k) leaves += h_jobs[k].leaf_cap;
+    const int tile = leaves < kSgSmallBelow ? kSgSmallTile : kSgTile;
+    auto nt = [tile](int64_t n) { return (n + tile - 1) / tile; };
     int64_t xh[kXcds] = {}, xo[kXcds] = {}, xl[kXcds] = {}, xn[kXcds] = {}, xr[kXcds] = {};
     auto add = [spread](int64_t* xs, int s, int64_t cnt) {  // sub-list lengths as sg_place makes them
         if (!spread) {
@@ -1762,44 +2007,44 @@ int run_seam_grid(Ctx* c, SeamState& st, int m, const SeamJobDev* h_jobs, const 
     int* toff = tsum + tr;
     int* tbase = toff + tr;
     int4* T = static_cast<int4*>(st.g_tiles.p);
+    int lanes = 64;
+    while (lanes > 1 && lanes * m > 1024) lanes >>= 1;
     SeamGrid g{d_jobs, static_cast<const SeamSrcDev*>(st.srcs.p), static_cast<char*>(st.scratch.p),
-               static_cast<SeamRun*>(st.g_run.p), cnt, ov, ot, m, spread ? 1 : 0};
+               static_cast<SeamRun*>(st.g_run.p), cnt, ov, ot, m, spread ? 1 : 0, tile, lanes};
+    const int top = std::min(lmax, kSgTop);
     const hipStream_t sm = c->stream;
     // tile launches: a multiple of 8 workgroups (see k_sg_tiles), looping over their lists
     static_assert(kSgGrid % kXcds == 0, "tile launches keep to one XCD per workgroup");
     auto grid = [](int64_t tiles) { return dim3((unsigned)std::min<int64_t>(tiles, kSgGrid)); };
-    const dim3 per_seam((m + kSgThreads - 1) / kSgThreads), block(kSgThreads), dev_grid(kSgGrid);
+    const dim3 per_seam((m + kSgThreads - 1) / kSgThreads), block(kSgThreads), dev_grid(kSgGrid),
+        round_grid(kSgRoundGrid);
 #define LVN_SG(...)                              \
     do {                                          \
         hipLaunchKernelGGL(__VA_ARGS__);          \
         LVN_HIP(hipGetLastError());               \
     } while (0)
-    LVN_SG(k_sg_tiles, dim3(1), dim3(1024), 0, sm, g, 3, T, 0, cnt + kSgCntHash);
-    LVN_SG(k_sg_tiles, dim3(1), dim3(1024), 0, sm, g, 6, T + o_off, 0, cnt + kSgCntOffered);
-    LVN_SG(k_sg_tiles, dim3(1), dim3(1024), 0, sm, g, 4, T + o_leaf, 0, cnt + kSgCntLeaf);
-    LVN_SG(k_sg_tiles, dim3(1), dim3(1024), 0, sm, g, 5, T + o_node, 0, cnt + kSgCntNode);
+    LVN_SG(k_sg_tiles, dim3(4), dim3(1024), 0, sm, g, kSgListHash, T, make_int4((int)o_off, (int)o_leaf, (int)o_node, 0));
     LVN_SG(k_sg_init, dev_grid, block, 0, sm, g, T);
     LVN_SG(k_sg_select, grid(to), block, 0, sm, g, T + o_off);
     LVN_SG(k_sg_leaves, grid(th), block, 0, sm, g, T);
-    LVN_SG(k_sg_seam, per_seam, block, 0, sm, g, 0);
     LVN_SG(k_sg_ancestors, grid(tl), block, 0, sm, g, T + o_leaf);
-    LVN_SG(k_sg_seam, per_seam, block, 0, sm, g, 1);
     LVN_SG(k_sg_links, grid(tn), block, 0, sm, g, T + o_node);
-    LVN_SG(k_sg_seam, per_seam, block, 0, sm, g, 2);
+    LVN_SG(k_sg_seam, per_seam, block, 0, sm, g);
     LVN_SG(k_sg_order, grid(tn), block, 0, sm, g, T + o_node);
-    LVN_SG(k_sg_tiles, dim3(lmax + 1), dim3(1024), 0, sm, g, 0, T + o_lev, (int)tn, cnt + kSgCntLevel);
-    for (int l = lmax - 1; l >= 1; --l) LVN_SG(k_sg_level, dev_grid, block, 0, sm, g, T + o_lev + l * tn, l, 0);
-    LVN_SG(k_sg_seam, per_seam, block, 0, sm, g, 3);
-    for (int l = 0; l < lmax; ++l) LVN_SG(k_sg_level, dev_grid, block, 0, sm, g, T + o_lev + l * tn, l, 1);
+    if (lmax > top)
+        LVN_SG(k_sg_tiles, dim3(lmax), dim3(1024), 0, sm, g, kSgListLevel, T + o_lev, make_int4(0, 0, 0, (int)tn));
+    for (int l = lmax - 1; l >= top; --l) LVN_SG(k_sg_level, dev_grid, block, 0, sm, g, T + o_lev + l * tn, l, 0);
+    LVN_SG(k_sg_top, dim3(m), dim3(1024), 0, sm, g, top);
+    for (int l = top; l < lmax; ++l) LVN_SG(k_sg_level, dev_grid, block, 0, sm, g, T + o_lev + l * tn, l, 1);
     LVN_SG(k_sg_vertices, grid(tl), block, 0, sm, g, T + o_leaf);
     // round r reads tile list r & 1 and makes list (r + 1) & 1
-    LVN_SG(k_sg_tiles, dim3(1), dim3(1024), 0, sm, g, 1, T + o_round, 0, cnt + kSgCntRound);
+    LVN_SG(k_sg_tiles, dim3(1), dim3(1024), 0, sm, g, kSgListRound, T + o_round, int4{});
     int round = 0;
-    for (int batch = lmax + 3; round < kMaxRounds; batch = 2) {
+    for (int batch = std::max(lmax, 1); round < kMaxRounds; batch = 2) {
         for (int k = 0; k < batch && round < kMaxRounds; ++k, ++round) {
             int4* cur = T + o_round + (round & 1) * tr;
             int4* nxt = T + o_round + ((round + 1) & 1) * tr;
-            LVN_SG(k_sg_round, dev_grid, block, 0, sm, g, cur, round, tsum, tbase);
+            LVN_SG(k_sg_round, round_grid, dim3(kSgRoundThreads), 0, sm, g, cur, round, tsum, tbase);
             LVN_SG(k_sg_round_next, dim3(1), dim3(1024), 0, sm, g, round, tsum, toff, nxt);
             LVN_SG(k_sg_round_copy, dev_grid, block, 0, sm, g, cur, round, tsum, tbase, toff);
         }
@@ -1807,18 +2052,19 @@ int run_seam_grid(Ctx* c, SeamState& st, int m, const SeamJobDev* h_jobs, const 
         LVN_HIP(hipStreamSynchronize(sm));
         if (*static_cast<const int*>(st.h_active.p) == 0) break;
     }
-    LVN_SG(k_sg_tiles, dim3(1), dim3(1024), 0, sm, g, 2, T + o_fin, 0, cnt + kSgCntFinal);
+    LVN_SG(k_sg_tiles, dim3(1), dim3(1024), 0, sm, g, kSgListFinal, T + o_fin, int4{});
     LVN_SG(k_sg_triangles, dev_grid, block, 0, sm, g, T + o_fin, d_res);
 #undef LVN_SG
     return LVN_OK;
 }
 
-// Which seam pass runs a call: the grid-wide steps (measured on the clipmap's seams: its
-// largest seam alone 3.1 against 7.8 ms, 512 seams 10.2 against 11.6 ms, all 1,798 seams
-// 32.6 against 33.4 ms) unless every seam is small, where one workgroup per seam has the
-// shorter fixed cost (a seam of 6,440 offered nodes: 0.20 against 0.38 ms; 36,606: 1.17
-// against 0.80 ms).  LVN_SEAM_PATH=grid or =workgroup in the environment overrides the
-// choice.
+// Which seam pass runs a call: the grid-wide steps unless every seam is small, where one
+// workgroup per seam is one launch in place of about forty.  A request of one seam, whole
+// call: 1,219 offered nodes 410 us by the grid against 353 by one workgroup, 2,442 nodes
+// 418 against 418, 4,888 nodes 430 against 541, 12,231 nodes 310 against 532.  Many seams
+// fill the chip with a workgroup each: 256 seams of 4,888 nodes 3.85 against 3.70 ms, of
+// 8,557 nodes 3.53 against 3.62 ms.  LVN_SEAM_PATH=grid or =workgroup in the environment
+// overrides the choice.
 bool seam_pass_grid(const std::vector<SeamJobDev>& jobs, const std::vector<SeamSrcDev>& srcs) {
     if (const char* e = getenv("LVN_SEAM_PATH")) {
         if (!strcmp(e, "grid")) return true;
@@ -1830,7 +2076,7 @@ bool seam_pass_grid(const std::vector<SeamJobDev>& jobs, const std::vector<SeamS
         for (int si = 0; si < J.src_count; ++si) offered += srcs[J.src_begin + si].count;
         largest = std::max(largest, offered);
     }
-    return largest >= 16384;
+    return largest >= ((int)jobs.size() < kSpreadBelow ? 3072 : 8192);
 }
 
 int run_seams(Ctx* c, int n, const lvn_seam_req* reqs, const lvn_seam_source* sources, lvn_seam_out* outs,
