@@ -1599,19 +1599,26 @@ __device__ __forceinline__ int corner_materials(const KArgs& a, const uint8_t* m
     return corners;
 }
 
-// The same from the solid rows, for a chunk that stores no materials: a sample's material
-// is then the default material where it is not air (density < 0) and air elsewhere.
-__device__ __forceinline__ int corner_materials_rows(const KArgs& a, const uint64_t* S, int x, int y, int z, int* cm) {
-    const int F = a.G.F;
+// The corners' solid bits from the solid rows, for a chunk that stores no materials: a
+// sample's material is then the default material where it is not air (density < 0) and air
+// elsewhere.  Two neighbouring bits of each of the voxel's four rows.
+__device__ __forceinline__ int corners_from_rows(const KArgs& a, const uint64_t* S, int x, int y, int z) {
     int corners = 0;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int cx = x + ((i >> 2) & 1), s = (y + ((i >> 1) & 1)) + F * (z + (i & 1));
-        const int bit = (int)((S[2 * s + (cx >> 6)] >> (cx & 63)) & 1ull);
-        cm[i] = bit ? a.defmat : kAir;
-        corners |= bit << i;
+    for (int j = 0; j < 4; ++j) {
+        const int jy = j & 1, jz = j >> 1;
+        const ulonglong2 w = *reinterpret_cast<const ulonglong2*>(S + 2 * ((y + jy) + a.G.F * (z + jz)));
+        const int t = (int)(uint32_t)(w.x >> x) | (x == 63 ? (int)((uint32_t)w.y << 1) : 0);
+        corners |= (t & 1) << (2 * jy + jz) | ((t >> 1) & 1) << (4 + 2 * jy + jz);
     }
     return corners;
+}
+
+// The edges with a sign change, bit e for the corners kEdgeMap[e].
+__device__ __forceinline__ int edges_of_corners(int corners) {
+    const int x = corners ^ (corners >> 4), y = corners ^ (corners >> 2), z = corners ^ (corners >> 1);
+    return (x & 15) | ((y & 3) | ((y >> 2) & 12)) << 4 |
+           ((z & 1) | ((z >> 1) & 2) | ((z >> 2) & 4) | ((z >> 3) & 8)) << 8;
 }
 
 // FindDominantMaterial, cl/octree.cl:78-138.  The reference sorts the eight corner
@@ -1779,51 +1786,74 @@ __device__ __forceinline__ void qef_fast(const KArgs& a, int chunk, const ChunkD
     const float fscale = (float)cd.scale;
 
     // The voxel's edges start at its corners, so they lie in four edge rows, (y or y + 1,
-    // z or z + 1): those rows and bases are loaded together and every edge's index is
-    // found from them, so only the hermite-data loads remain in the accumulation loop
-    // (loading those ahead as well was slower: 99 VGPRs, 4 waves per SIMD).
-    uint64_t rw[4][4];
-    int rb[4];
+    // z or z + 1), at x and x + 1: row j's six possible edges are bits 8 j .. 8 j + 5 of
+    // `have` in list order, and first[j] is the list index of the first of them.
+    uint32_t have = 0;
+    int first[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int r = (p.y + (j & 1)) + G.H * (p.z + (j >> 1));
-#pragma unroll
-        for (int q = 0; q < 4; ++q) rw[j][q] = erows[4 * r + q];
-        rb[j] = eb[r].x;
+        const uint64_t ex = erows[4 * r], ey = erows[4 * r + 1], ez = erows[4 * r + 2], hi = erows[4 * r + 3];
+        const uint64_t lt = lanemask_lt(p.x);
+        first[j] = eb[r].x + __popcll(ex & lt) + __popcll(ey & lt) + __popcll(ez & lt);
+        const uint32_t bx = (uint32_t)(ex >> p.x), by = (uint32_t)(ey >> p.x), bz = (uint32_t)(ez >> p.x);
+        uint32_t b = (bx & 1) | (by & 1) << 1 | (bz & 1) << 2 | (bx & 2) << 2 | (by & 2) << 3 | (bz & 2) << 4;
+        if (p.x == 63) b |= ((uint32_t)hi & 7) << 3;
+        have |= b << (8 * j);
     }
-    int ke[12];
-#pragma unroll
-    for (int e = 0; e < 12; ++e) {
-        const int e0 = kEdgeMap[e][0];
-        const int j = ((e0 >> 1) & 1) + 2 * (e0 & 1);  // row of the edge's lower end
-        const int k = ((emask >> e) & 1) ? edge_index_in_row(rw[j], rb[j], p.x + ((e0 >> 2) & 1), e >> 2) : -1;
-        ke[e] = k >= 0 && k < a.caps.edges ? k : -1;
-    }
+    // Edge e's bit in `have`, 5 bits each: row j = y + 2 z and slot s = 3 x + axis of its lower
+    // end's corner.
+    constexpr uint64_t kSlotOfEdge = 0ull | 16ull << 5 | 8ull << 10 | 24ull << 15 |     // x edges
+                                     1ull << 20 | 17ull << 25 | 4ull << 30 | 20ull << 35 |  // y edges
+                                     2ull << 40 | 10ull << 45 | 5ull << 50 | 13ull << 55;   // z edges
 
     // The edge's point is a0 + (a1 - a0) t per component (cl/octree.cl:266-272), scaled.  Its
     // end corners differ by exactly 1 along the edge's axis and by exactly 0 across it, and t
     // is a finite crossing in [0, 1], so (a1 - a0) t is t along the axis and +0 across it:
     // the across components are fscale * a0 (six per voxel, formed once) and the w lane is
     // +0, which leaves the dot product's fourth term +0 and makes the w sums count edges.
-    const float sx0 = fscale * (float)p.x, sx1 = fscale * (float)(p.x + 1);
-    const float sy0 = fscale * (float)p.y, sy1 = fscale * (float)(p.y + 1);
-    const float sz0 = fscale * (float)p.z, sz1 = fscale * (float)(p.z + 1);
+    const float fx = (float)p.x, fy = (float)p.y, fz = (float)p.z;
+    const float sx0 = fscale * fx, sx1 = fscale * (float)(p.x + 1);
+    const float sy0 = fscale * fy, sy1 = fscale * (float)(p.y + 1);
+    const float sz0 = fscale * fz, sz1 = fscale * (float)(p.z + 1);
     float ata0 = 0.f, ata1 = 0.f, ata2 = 0.f, ata3 = 0.f, ata4 = 0.f, ata5 = 0.f;
     Q4 atb = {0.f, 0.f, 0.f, 0.f}, mass = {0.f, 0.f, 0.f, 0.f}, nsum = {0.f, 0.f, 0.f, 0.f};
     int count = 0;
-#pragma unroll
-    for (int e = 0; e < 12; ++e) {
-        if (ke[e] < 0) continue;
-        const int e0 = kEdgeMap[e][0], axis = e >> 2;
-        const int hx = p.x + ((e0 >> 2) & 1), hy = p.y + ((e0 >> 1) & 1), hz = p.z + (e0 & 1);
-        const float4 d = ed[ke[e]];
+    // Each lane walks its own edges in the order of e, the next one's data in flight: a wave
+    // takes as many steps as its busiest voxel has edges (7 or 8 of the 12), where a step per
+    // possible edge computed all twelve indices and waited for twelve loads in turn.
+    uint32_t left = (uint32_t)emask;
+    int slot = 0;
+    bool used = false;
+    float4 d = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto next = [&]() {  // the lowest edge left
+        const int e = __builtin_ctz(left);
+        left &= left - 1;
+        slot = (int)(kSlotOfEdge >> (5 * e)) & 31;
+        const int j = slot >> 3;
+        const int row = j == 0 ? first[0] : j == 1 ? first[1] : j == 2 ? first[2] : first[3];
+        const int k = row + __popc((have >> (8 * j)) & ((1u << (slot & 7)) - 1));
+        used = ((have >> slot) & 1) && k >= 0 && k < a.caps.edges;
+        if (used) d = ed[k];
+    };
+    bool more = left != 0;
+    if (more) next();
+    while (more) {
+        const float4 c = d;
+        const int at = slot;
+        const bool take = used;
+        more = left != 0;
+        if (more) next();
+        if (!take) continue;
+        const int s = at & 7, axis = s >= 3 ? s - 3 : s;
+        const float along = fscale * ((axis == 0 ? fx : axis == 1 ? fy : fz) + c.w);
         Q4 pos, n;
-        pos.x = axis == 0 ? fscale * ((float)hx + d.w) : ((e0 >> 2) & 1) ? sx1 : sx0;
-        pos.y = axis == 1 ? fscale * ((float)hy + d.w) : ((e0 >> 1) & 1) ? sy1 : sy0;
-        pos.z = axis == 2 ? fscale * ((float)hz + d.w) : (e0 & 1) ? sz1 : sz0;
-        n.x = d.x;
-        n.y = d.y;
-        n.z = d.z;
+        pos.x = axis == 0 ? along : s >= 3 ? sx1 : sx0;
+        pos.y = axis == 1 ? along : (at & 8) ? sy1 : sy0;
+        pos.z = axis == 2 ? along : (at & 16) ? sz1 : sz0;
+        n.x = c.x;
+        n.y = c.y;
+        n.z = c.z;
         // qef_add_point, cl/qef.cl:170-191
         ata0 = ata0 + n.x * n.x;
         ata1 = ata1 + n.x * n.y;
@@ -2119,13 +2149,11 @@ __device__ __forceinline__ void qef_precise(const KArgs& a, int chunk, const Chu
 // quad count and the seam mask go to the quad and seam scans.
 // ---------------------------------------------------------------------------
 
-__device__ __forceinline__ int quad_flag(const Geometry& G, int3 p, int corners, int axis) {
+__device__ __forceinline__ int quad_flag(const Geometry& G, int3 p, int emask, int axis) {
     const int pa = axis == 0 ? p.y : axis == 1 ? p.z : p.x;
     const int pb = axis == 0 ? p.z : axis == 1 ? p.x : p.y;
     if (pa == G.N - 1 || pb == G.N - 1) return 0;  // isEdgeVoxel, cl/octree.cl:411-417
-    const int edge = axis * 4 + 3;
-    const int m1 = (corners >> kEdgeMap[edge][0]) & 1, m2 = (corners >> kEdgeMap[edge][1]) & 1;
-    return m1 != m2;
+    return (emask >> (axis * 4 + 3)) & 1;
 }
 
 template <bool kPrecise>
@@ -2150,21 +2178,30 @@ __global__ __launch_bounds__(256) void k_qef(KArgs a) {
         int qbits = 0, seam = 0;
         if (vi < V) {
             const int3 p = position_for_code((uint32_t)vcode[vi], G.depth);
-            int cm[8];
-            const int corners = rows ? corner_materials_rows(a, S, p.x, p.y, p.z, cm)
-                                     : corner_materials(a, mat, p.x, p.y, p.z, cm);
-            int emask = 0;
+            int corners, dominant;
+            if (rows && a.defmat < kNone) {  // the default material sorts before air and is the only one
+                corners = corners_from_rows(a, S, p.x, p.y, p.z);
+                dominant = corners ? a.defmat : kAir;
+            } else {
+                int cm[8];
+                if (rows) {
+                    corners = corners_from_rows(a, S, p.x, p.y, p.z);
 #pragma unroll
-            for (int e = 0; e < 12; ++e)
-                emask |= (((corners >> kEdgeMap[e][0]) & 1) != ((corners >> kEdgeMap[e][1]) & 1)) << e;
-            const int m = (dominant_material(cm) << 8) | corners;
+                    for (int i = 0; i < 8; ++i) cm[i] = (corners >> i) & 1 ? a.defmat : kAir;
+                } else {
+                    corners = corner_materials(a, mat, p.x, p.y, p.z, cm);
+                }
+                dominant = dominant_material(cm);
+            }
+            const int emask = edges_of_corners(corners);
+            const int m = (dominant << 8) | corners;
             float4 pos, nrm;
             if constexpr (kPrecise)
                 qef_precise(a, chunk, cd, p, emask, pos, nrm);
             else
                 qef_fast(a, chunk, cd, p, emask, pos, nrm);
 #pragma unroll
-            for (int axis = 0; axis < 3; ++axis) qbits |= quad_flag(G, p, corners, axis) << axis;
+            for (int axis = 0; axis < 3; ++axis) qbits |= quad_flag(G, p, emask, axis) << axis;
             seam = p.x == 0 || p.x == N - 1 || p.y == 0 || p.y == N - 1 || p.z == 0 || p.z == N - 1;
             vemask[vi] = emask | (qbits << 12);
             vmat[vi] = m;
