@@ -619,13 +619,15 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_rows(KArgs a) {
 // rows r = y + H z and loads their words together (lane j: row j).  Where its live rows
 // are dense (kDenseRow edges or more on average) it walks them in order with lane x
 // holding position x of the row: an edge's rank in the row is the popcount of the three
-// edge words below its lane (lower x) plus the lower axes at its own x, so each store
-// instruction writes one contiguous stretch of the lists.  Where they are sparse, each
-// lane walks its own row's few edges (fewer, cheaper iterations; their stores scatter
-// over the rows' stretches).  With the per-lane walk alone, lines of the clipmap batch's
-// dense rows left L2 half-written: 47 bytes reached HBM per 8 bytes of list, and the
-// stage took 3.3 ms.  Both walks write the same lists.
-constexpr int kDenseRow = 16;
+// edge words below its lane (lower x) plus the lower axes at its own x.  Where they are
+// sparse, each lane takes one edge of the wave's run of the list: it finds the edge's row
+// among the 64 bases and the edge within the row by halving the words, so 64 edges cost
+// about 140 instructions however they are spread (a lane walking each row's edges cost
+// 550 on the clipmap, whose rows hold a few edges each, and scattered their stores).
+// Either way a store instruction writes one contiguous stretch of the ids.  `split` waves
+// share 64 rows where a batch is too small to fill the chip.  Measured for the whole kernel:
+// 1,800 clipmap chunks 150 -> 80 us, 512 cave chunks 160 -> 118, one 64^3 chunk 11.3 -> 5.4.
+constexpr int kDenseRow = 32;
 
 __device__ __forceinline__ int wave_sum(int v) {
 #pragma unroll
@@ -638,7 +640,49 @@ __device__ __forceinline__ uint64_t readlane64(uint64_t v, int j) {
     return ((uint64_t)hi << 32) | lo;
 }
 
-__device__ __forceinline__ void edge_compact(const KArgs& a, int chunk, int wave, int waves) {
+// The n-th edge (from 0) of a row in slot order: its x and axis, from the row's words w
+// (x, y, z edge bits of x < 64) and hi (the edges at x = 64).
+__device__ __forceinline__ void nth_edge(const uint64_t w[3], uint32_t hi, int n, int& x, int& axis) {
+    uint32_t b[3] = {(uint32_t)w[0], (uint32_t)w[1], (uint32_t)w[2]};
+    x = 0;
+    int c = __popc(b[0]) + __popc(b[1]) + __popc(b[2]);
+    if (n >= c) {
+        n -= c;
+        x = 32;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) b[i] = (uint32_t)(w[i] >> 32);
+        c = __popc(b[0]) + __popc(b[1]) + __popc(b[2]);
+        if (n >= c) {  // the three bits at x = 64
+            n -= c;
+            x = 64;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) b[i] = (hi >> i) & 1;
+        }
+    }
+#pragma unroll
+    for (int s = 16; s > 0; s >>= 1) {
+        const uint32_t m = (1u << s) - 1;
+        c = __popc(b[0] & m) + __popc(b[1] & m) + __popc(b[2] & m);
+        const int up = n >= c ? s : 0;  // (never taken at x = 64: its bits lie lowest)
+        n -= up ? c : 0;
+        x += up;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) b[i] >>= up;
+    }
+    const int b0 = b[0] & 1, b1 = b[1] & 1;
+    axis = b0 && n == 0 ? 0 : b1 && n == b0 ? 1 : 2;
+}
+
+// Last lane whose value (ascending over the lanes) is not above v.
+__device__ __forceinline__ int last_lane_at(int value, int v) {
+    int r = 0;
+#pragma unroll
+    for (int step = 32; step > 0; step >>= 1)
+        if (__shfl(value, r + step) <= v) r += step;
+    return r;
+}
+
+__device__ __forceinline__ void edge_compact(const KArgs& a, int chunk, int wave, int waves, int split, uint4 (*stage)[2]) {
     const Geometry& G = a.G;
     const uint64_t* E = slot_ptr<const uint64_t>(a, chunk, a.L.e_rows);
     const uint32_t* count = slot_ptr<const uint32_t>(a, chunk, a.L.e_count);
@@ -656,48 +700,52 @@ __device__ __forceinline__ void edge_compact(const KArgs& a, int chunk, int wave
             if (pos < cap) order[pos] = make_int2(k, id);
         }
     };
-    const int groups = (G.edge_rows + 63) >> 6;
-    for (int g = wave; g < groups; g += waves) {
+    const int units = ((G.edge_rows + 63) >> 6) * split;
+    for (int u = wave; u < units; u += waves) {
+        const int g = u / split, part = u - g * split;
         const int rl = (g << 6) + lane;
         const int cnt = rl < G.edge_rows ? (int)(count[rl] & 0xffffu) : 0;
         uint64_t live = __ballot(cnt != 0);
         if (!live) continue;
-        int kb = 0, kyb = 0;
+        int kb = 0x7fffffff, kyb = 0;
         uint64_t w0 = 0, w1 = 0, w2 = 0, w3 = 0;
-        if (cnt) {  // a row without edges has no words
+        if (rl < G.edge_rows) {
             const int2 b = base[rl];
             kb = b.x;
             kyb = b.y;
+        }
+        if (cnt) {  // a row without edges has no words
             w0 = E[4 * rl];
             w1 = E[4 * rl + 1];
             w2 = E[4 * rl + 2];
             w3 = E[4 * rl + 3];
         }
-        if (wave_sum(cnt) < kDenseRow * __popcll(live)) {  // sparse rows: one lane per row
-            if (cnt == 0) continue;
-            const int z = div_magic(rl, G.magic_h), y = rl - z * G.H;
-            const int row_id = (y << S) | (z << (2 * S));
-            int k = kb, ky = kyb;
-            uint64_t any = w0 | w1 | w2;
-            while (any) {
-                const int x = (int)__builtin_ctzll(any);
-                any &= any - 1ull;
-                const int id = (x | row_id) << 2;
-                if ((w0 >> x) & 1ull) put(k++, ky, id, false);
-                if ((w1 >> x) & 1ull) put(k++, ky++, id | 1, true);
-                if ((w2 >> x) & 1ull) put(k++, ky, id | 2, false);
+        const int total = wave_sum(cnt);
+        if (total < kDenseRow * __popcll(live)) {  // sparse rows: one lane per edge
+            stage[lane][0] = make_uint4((uint32_t)w0, (uint32_t)(w0 >> 32), (uint32_t)w1, (uint32_t)(w1 >> 32));
+            stage[lane][1] = make_uint4((uint32_t)w2, (uint32_t)(w2 >> 32), (uint32_t)w3, (uint32_t)kyb);
+            __builtin_amdgcn_wave_barrier();  // read by the wave's other lanes
+            const int k_first = __builtin_amdgcn_readlane(kb, 0);
+            for (int i0 = part << 6; i0 < total; i0 += split << 6) {
+                const int k = k_first + min(i0 + lane, total - 1);
+                const int j = last_lane_at(kb, k);  // of equal bases the last: the row with edges
+                const int n = k - __shfl(kb, j);
+                const uint4 p = stage[j][0], q = stage[j][1];
+                const uint64_t w[3] = {(uint64_t)p.y << 32 | p.x, (uint64_t)p.w << 32 | p.z, (uint64_t)q.y << 32 | q.x};
+                int x, axis;
+                nth_edge(w, q.z, n, x, axis);
+                const int at_x = x < 64 ? (int)(w[1] >> x) & 1 : (int)(q.z >> 1) & 1;  // the y-edge at the same x
+                const int ky = (int)q.w + __popcll(w[1] & (x < 64 ? lanemask_lt(x) : ~0ull)) + (axis == 2 ? at_x : 0);
+                const int r = (g << 6) + j, z = div_magic(r, G.magic_h), y = r - z * G.H;
+                if (i0 + lane < total) put(k, ky, (x | y << S | z << (2 * S)) << 2 | axis, axis == 1);
             }
-            const int id64 = (64 | row_id) << 2;  // x = 64 (N = 64 only)
-            for (int axis = 0; axis < 3; ++axis) {
-                if (!((w3 >> axis) & 1ull)) continue;
-                put(k++, ky, id64 | axis, axis == 1);
-                ky += axis == 1 ? 1 : 0;
-            }
+            __builtin_amdgcn_wave_barrier();
             continue;
         }
-        while (live) {
+        for (int skip = 0; live; ++skip) {
             const int j = (int)__builtin_ctzll(live);
             live &= live - 1ull;
+            if (skip % split != part) continue;
             const int r = (g << 6) + j;
             const int z = div_magic(r, G.magic_h), y = r - z * G.H;
             const int row_id = (y << S) | (z << (2 * S));
@@ -1666,11 +1714,9 @@ __device__ __forceinline__ int dominant_material(const int* m) {
 // the corners anyway.  A wave takes 64 consecutive segments and loads their masks and
 // bases together (lane j: segment j).  Where its live segments are dense (kDenseRow
 // voxels or more on average) it walks them in order with lane b holding the segment's
-// voxel b: its rank is the popcount of the mask below b, so each segment's codes are one
-// contiguous store.  Where they are sparse, each lane walks its own segment (one lane
-// per segment alone scattered the dense segments' stores: 4.4 bytes reached HBM per
-// byte of codes on the clipmap batch).  Both walks write the same codes.
-__device__ __forceinline__ void voxel_compact(const KArgs& a, int chunk, int wave, int waves) {
+// voxel b: its rank is the popcount of the mask below b.  Where they are sparse, each lane
+// takes one voxel of the wave's run of the list, found as the edges are.
+__device__ __forceinline__ void voxel_compact(const KArgs& a, int chunk, int wave, int waves, int split) {
     const Geometry& G = a.G;
     const uint64_t* vmask = slot_ptr<const uint64_t>(a, chunk, a.L.v_mask);
     const int* vbase = slot_ptr<const int>(a, chunk, a.L.v_base);
@@ -1678,27 +1724,43 @@ __device__ __forceinline__ void voxel_compact(const KArgs& a, int chunk, int wav
     const int cap = a.caps.voxels;
     const int lane = threadIdx.x & 63;
     const uint64_t lt = lanemask_lt(lane);
-    const int groups = (G.voxel_segs + 63) >> 6;
-    for (int g = wave; g < groups; g += waves) {
+    const int units = ((G.voxel_segs + 63) >> 6) * split;
+    for (int u = wave; u < units; u += waves) {
+        const int g = u / split, part = u - g * split;
         const int sl = (g << 6) + lane;
-        const uint64_t own = sl < G.voxel_segs ? vmask[sl] : 0;
-        uint64_t ml = own, live = __ballot(ml != 0);
+        const uint64_t ml = sl < G.voxel_segs ? vmask[sl] : 0;
+        uint64_t live = __ballot(ml != 0);
         if (!live) continue;
-        const int bl = ml ? vbase[sl] : 0;
-        if (wave_sum(__popcll(ml)) < kDenseRow * __popcll(live)) {  // sparse: one lane per segment
-            int i = bl;
-            while (ml && i < cap) {
-                const int v = (sl << 6) + (int)__builtin_ctzll(ml);
-                ml &= ml - 1ull;
+        const int bl = sl < G.voxel_segs ? vbase[sl] : 0x7fffffff;
+        const int total = wave_sum(__popcll(ml));
+        if (total < kDenseRow * __popcll(live)) {  // sparse: one lane per voxel
+            const int i_first = __builtin_amdgcn_readlane(bl, 0);
+            for (int i0 = part << 6; i0 < total; i0 += split << 6) {
+                const int i = i_first + min(i0 + lane, total - 1);
+                const int j = last_lane_at(bl, i);
+                int n = i - __shfl(bl, j);
+                const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)ml, j), hi = (uint32_t)__shfl((int)(uint32_t)(ml >> 32), j);
+                const int c = __popc(lo);
+                int b = n >= c ? 32 : 0;
+                uint32_t m = n >= c ? hi : lo;
+                n -= n >= c ? c : 0;
+#pragma unroll
+                for (int s = 16; s > 0; s >>= 1) {
+                    const int below = __popc(m & ((1u << s) - 1)), up = n >= below ? s : 0;
+                    n -= up ? below : 0;
+                    b += up;
+                    m >>= up;
+                }
                 int x, y, z;
-                decode_voxel(G, v, x, y, z);
-                vcode[i++] = (int)code_for_position(x, y, z, G.depth);
+                decode_voxel(G, (((g << 6) + j) << 6) + b, x, y, z);
+                if (i0 + lane < total && i < cap) vcode[i] = (int)code_for_position(x, y, z, G.depth);
             }
             continue;
         }
-        while (live) {
+        for (int skip = 0; live; ++skip) {
             const int j = (int)__builtin_ctzll(live);
             live &= live - 1ull;
+            if (skip % split != part) continue;
             const int seg = (g << 6) + j;
             const uint64_t m = readlane64(ml, j);
             const int i = __builtin_amdgcn_readlane(bl, j) + __popcll(m & lt);
@@ -1712,13 +1774,14 @@ __device__ __forceinline__ void voxel_compact(const KArgs& a, int chunk, int wav
 }
 
 // Edge lists by the first `edge_blocks` workgroups of a chunk, voxel codes by the others.
-__global__ __launch_bounds__(256) void k_compact(KArgs a, int edge_blocks) {
+__global__ __launch_bounds__(256) void k_compact(KArgs a, int edge_blocks, int split) {
+    __shared__ uint4 stage[4][64][2];  // a wave's 64 edge rows
     const int chunk = blockIdx.y;
     const Counters& c = a.counters[chunk];
     if ((int)blockIdx.x < edge_blocks) {
-        if (c.edges) edge_compact(a, chunk, wave_in_chunk(), edge_blocks * 4);
+        if (c.edges) edge_compact(a, chunk, wave_in_chunk(), edge_blocks * 4, split, stage[threadIdx.x >> 6]);
     } else {
-        if (c.voxels) voxel_compact(a, chunk, wave_in_chunk() - edge_blocks * 4, ((int)gridDim.x - edge_blocks) * 4);
+        if (c.voxels) voxel_compact(a, chunk, wave_in_chunk() - edge_blocks * 4, ((int)gridDim.x - edge_blocks) * 4, split);
     }
 }
 
@@ -2574,9 +2637,14 @@ void launch_scan_quads_seams(const KArgs& a, int chunks, hipStream_t s) {
     hipLaunchKernelGGL(k_scan_quads_seams, dim3(1, chunks), dim3(kScanThreads), 0, s, a);
 }
 void launch_compact(const KArgs& a, int chunks, hipStream_t s) {
-    const unsigned eb = chunk_blocks(chunks, 64L * ((a.G.edge_rows + 63) / 64), a.row_blocks);
-    const unsigned vb = chunk_blocks(chunks, 64L * ((a.G.voxel_segs + 63) / 64), a.row_blocks);
-    hipLaunchKernelGGL(k_compact, dim3(eb + vb, chunks), dim3(256), 0, s, a, (int)eb);
+    // A wave per 64 rows, or four while one each does not fill the chip (32 waves per CU):
+    // one chunk 9.5 -> 5.4 us, 24 chunks 11 -> 7; but 1,800 chunks 80 -> 139 us, whose rows
+    // are mostly empty and looked at four times.
+    const long edge_groups = (a.G.edge_rows + 63) / 64, voxel_groups = (a.G.voxel_segs + 63) / 64;
+    const int split = (edge_groups + voxel_groups) * chunks < 32L * a.cus ? 4 : 1;
+    const unsigned eb = chunk_blocks(chunks, 64L * edge_groups * split, a.row_blocks);
+    const unsigned vb = chunk_blocks(chunks, 64L * voxel_groups * split, a.row_blocks);
+    hipLaunchKernelGGL(k_compact, dim3(eb + vb, chunks), dim3(256), 0, s, a, (int)eb, split);
 }
 // Lanes per edge of the crossing stage: the tuned value, else by field and batch size (a
 // typical 64^3 chunk has a few hundred 64-edge items, a chunk of N^3 about (N / 64)^2 of
