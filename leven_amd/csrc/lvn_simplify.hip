@@ -27,6 +27,7 @@
 #include <random>
 #include <vector>
 
+#include "lvn_device.hpp"
 #include "lvn_kernels.h"
 #include "lvn_runtime.h"
 
@@ -205,9 +206,11 @@ __device__ float qef_two(float4 p0, float4 n0, float4 p1, float4 n1, float4* out
 #pragma unroll
             for (int l = 0; l < 4; ++l) {
                 const float tau = (qq.v[l] - pp.v[l]) / (pq.v[l] * 2.f);
-                const float stt = sqrtf(tau * tau + 1.f);
+                // both square roots have arguments >= 1 and the cosine's divisor lies in
+                // [1, sqrt 2] (|tn| <= 1); a lane without a rotation is replaced below
+                const float stt = sqrt_ge1(tau * tau + 1.f);
                 const float tn = 1.f / (tau >= 0.f ? tau + stt : tau - stt);
-                const float cl = 1.f / sqrtf(1.f + tn * tn);
+                const float cl = recip_1_2(sqrt_ge1(1.f + tn * tn));
                 const float sl = tn * cl;
                 const bool zero = pq.v[l] == 0.f;
                 c.v[l] = zero ? 1.f : cl;
@@ -381,6 +384,33 @@ struct BucketOp {
     }
 };
 
+// A vertex's bucket holds the smaller ends of the triangle sides whose larger end it is, six
+// on average: up to kBucketRegs of them are read together into registers (INT_MAX past the
+// end).  Sorting and walking each bucket in memory, one dependent read after another, took
+// 211 us for 64 cave meshes, and takes 108; eight registers, too few for one bucket in most
+// waves, left it at 205.
+constexpr int kBucketRegs = 16;
+__device__ __forceinline__ void load_bucket(const int* b, int n, int* v) {
+#pragma unroll
+    for (int k = 0; k < kBucketRegs; ++k) v[k] = k < n ? b[k] : INT_MAX;
+}
+// Batcher's odd-even merge sort, its exchanges unrolled.
+__device__ __forceinline__ void sort_bucket(int* v) {
+#pragma unroll
+    for (int p = 1; p < kBucketRegs; p *= 2)
+#pragma unroll
+        for (int k = p; k >= 1; k /= 2)
+#pragma unroll
+            for (int j = k % p; j + k < kBucketRegs; j += 2 * k)
+#pragma unroll
+                for (int i = 0; i < k; ++i)
+                    if (i + j + k < kBucketRegs && (i + j) / (2 * p) == (i + j + k) / (2 * p)) {
+                        const int lo = min(v[i + j], v[i + j + k]), hi = max(v[i + j], v[i + j + k]);
+                        v[i + j] = lo;
+                        v[i + j + k] = hi;
+                    }
+}
+
 // BuildCandidateEdges (src/ng_mesh_simplify.cpp:118-172): in (max, min) key order, each
 // run of equal sides seen more than once whose ends are not boundary, except the last run
 // of all, which the reference's loop never examines.
@@ -392,6 +422,24 @@ struct EdgeOp {
         const int* b = g.bucket + 3 * (int64_t)M.tbase + g.boff[M.vbase + i];
         const bool bi = g.bnd[M.vbase + i] != 0;
         int kept = 0, k = 0;
+        if (n <= kBucketRegs) {
+            if (bi) return 0;
+            int v[kBucketRegs], open[kBucketRegs];
+            load_bucket(b, n, v);
+            const int end = i == M.last ? b[n - 1] : -1;  // the run that reaches the end is left out
+#pragma unroll
+            for (int q = 0; q < kBucketRegs - 1; ++q)  // runs of two and more, at their first side
+                open[q] = q + 1 < n && v[q + 1] == v[q] && (q == 0 || v[q - 1] != v[q]) && v[q] != end
+                              ? g.bnd[M.vbase + v[q]]
+                              : 1;
+#pragma unroll
+            for (int q = 0; q < kBucketRegs - 1; ++q)
+                if (!open[q]) {
+                    f(kept, v[q]);
+                    ++kept;
+                }
+            return kept;
+        }
         while (k < n) {
             int e = k + 1;
             while (e < n && b[e] == b[k]) ++e;
@@ -520,6 +568,15 @@ struct TriFinalOp {
 #define LVN_TILES(tiles, ntiles)                                             \
     for (int k_ = blockIdx.x; k_ < (ntiles); k_ += gridDim.x)                \
         for (int tl_m = (tiles)[k_].x, tl_s = (tiles)[k_].y, once_ = 1; once_; once_ = 0)
+
+// The same over equal parts of each tile: twice as many workgroups, for kernels whose
+// elements are long chains.
+constexpr int kSimpParts = 2;
+constexpr int kSimpPart = kSimpTile / kSimpParts;
+#define LVN_TILE_PARTS(tiles, ntiles)                                        \
+    for (int k_ = blockIdx.x; k_ < (ntiles) * kSimpParts; k_ += gridDim.x)   \
+        for (int tl_m = (tiles)[k_ / kSimpParts].x,                          \
+                 tl_s = (tiles)[k_ / kSimpParts].y + k_ % kSimpParts * kSimpPart, once_ = 1; once_; once_ = 0)
 
 // Working copy of the vertices, positions relative to the offset (:459-462).
 __global__ __launch_bounds__(kSimpThreads) void k_init_vertices(SG g) {
@@ -697,6 +754,22 @@ __global__ __launch_bounds__(kSimpThreads) void k_bucket_sort(SG g) {
             const int n = g.bcnt[M.vbase + i];
             if (n == 0) continue;
             int* b = g.bucket + 3 * (int64_t)M.tbase + g.boff[M.vbase + i];
+            if (n <= kBucketRegs) {
+                int v[kBucketRegs];
+                load_bucket(b, n, v);
+                sort_bucket(v);
+#pragma unroll
+                for (int k = 0; k < kBucketRegs; ++k) {
+                    if (k >= n) continue;
+                    b[k] = v[k];
+                    const bool once = (k == 0 || v[k - 1] != v[k]) && (k + 1 == n || v[k + 1] != v[k]);
+                    if (once && !(i == M.last && k + 1 == n)) {
+                        g.bnd[M.vbase + v[k]] = 1;
+                        g.bnd[M.vbase + i] = 1;
+                    }
+                }
+                continue;
+            }
             for (int k = 1; k < n; ++k) {
                 const int x = b[k];
                 int j = k - 1;
@@ -774,51 +847,75 @@ __global__ __launch_bounds__(kSimpThreads) void k_iter_reset(SG g) {
 }
 
 // The candidate's checks and cost (:213-275); each end keeps its cheapest valid candidate,
-// the first in edge order on ties.
+// the first in edge order on ties.  The cheap checks come first and the draws that pass
+// them are packed, so the solve (about 1,500 instructions, what bounds the kernel) runs on
+// full waves: with every draw solved in its own lane, four one after another, 64 cave
+// meshes took 49 us an iteration, and take 30.
 __global__ __launch_bounds__(kSimpThreads) void k_valid(SG g) {
-    LVN_TILES(g.dt, g.ndt) {
+    __shared__ int passed[kSimpPart];
+    __shared__ int npassed;
+    LVN_TILE_PARTS(g.dt, g.ndt) {
         SMesh& M = g.mesh[tl_m];
         const int n = min(M.draws, M.accepted);
         if (tl_s >= M.draws) continue;
         if (M.accepted < M.draws && tl_s == 0 && threadIdx.x == 0) M.fail = 1;  // too few draw positions
         const int2* edges = edges_of(g, M);
-        int valid = 0;
-        for (int r = 0; r < kSimpPer; ++r) {
+        if (threadIdx.x == 0) npassed = 0;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kSimpPart / kSimpThreads; ++r) {
             const int j = tl_s + threadIdx.x + r * kSimpThreads;
-            if (j >= n) continue;
+            bool pass = false;
+            if (j < n) {
+                const int2 e = edges[g.pick[M.dbase + j]];
+                const int va = M.vbase + e.x, vb = M.vbase + e.y;
+                const float4 pa = g.wpos[va], pb = g.wpos[vb], na = g.wnrm[va], nb = g.wnrm[vb];
+                const float cos_angle = dot_glm(na, nb);
+                const float4 d = make_float4(pb.x - pa.x, pb.y - pa.y, pb.z - pa.z, pb.w - pa.w);
+                pass = !(cos_angle < g.opt.min_angle_cosine) && !(dot_glm(d, d) > M.max_edge * M.max_edge) &&
+                       !((double)fabsf(g.wcol[va].w - g.wcol[vb].w) > 1e-3) &&
+                       !(g.vtc[va] + g.vtc[vb] > kCollapseMaxDegree);
+                if (!pass) g.pick[M.dbase + j] = -1;
+            }
+            const uint64_t mask = __ballot(pass);
+            const int lane = threadIdx.x & 63;
+            int at = 0;
+            if (lane == 0 && mask) at = atomicAdd(&npassed, __popcll(mask));
+            at = __shfl(at, 0);
+            if (pass) passed[at + __popcll(mask & ((1ull << lane) - 1))] = j;
+        }
+        __syncthreads();
+        const int np = npassed;
+        int valid = 0;
+        for (int q = threadIdx.x; q < np; q += kSimpThreads) {
+            const int j = passed[q];
             const int i = g.pick[M.dbase + j];
             const int2 e = edges[i];
             const int va = M.vbase + e.x, vb = M.vbase + e.y;
-            int ok = 0;
             const float4 pa = g.wpos[va], pb = g.wpos[vb], na = g.wnrm[va], nb = g.wnrm[vb];
-            const float cos_angle = dot_glm(na, nb);
-            const float4 d = make_float4(pb.x - pa.x, pb.y - pa.y, pb.z - pa.z, pb.w - pa.w);
             const int degree = g.vtc[va] + g.vtc[vb];
-            if (!(cos_angle < g.opt.min_angle_cosine) && !(dot_glm(d, d) > M.max_edge * M.max_edge) &&
-                !((double)fabsf(g.wcol[va].w - g.wcol[vb].w) > 1e-3) && !(degree > kCollapseMaxDegree)) {
-                float4 q;
-                float error = qef_two(pa, na, pb, nb, &q);
-                if (error > 0.f) error = 1.f / error;
-                const int penalty = max(0, degree - 10);
-                error = error + (float)penalty * (M.max_error * 0.1f);
-                if (!(error > M.max_error)) {
-                    ok = 1;
-                    g.dnrm[M.dbase + j] = make_float4((na.x - nb.x) * 0.5f, (na.y - nb.y) * 0.5f,
-                                                      (na.z - nb.z) * 0.5f, (na.w - nb.w) * 0.5f);
-                    g.dpos[M.dbase + j] = make_float4(q.x, q.y, q.z, 1.f);
-                    if (error < FLT_MAX) {
-                        const unsigned long long k2 =
-                            ((unsigned long long)__float_as_uint(error) << 32) | (unsigned long long)(uint32_t)i;
-                        atomicMin(&g.key[va], k2);
-                        atomicMin(&g.key[vb], k2);
-                    }
-                }
+            float4 x;
+            float error = qef_two(pa, na, pb, nb, &x);
+            if (error > 0.f) error = 1.f / error;
+            const int penalty = max(0, degree - 10);
+            error = error + (float)penalty * (M.max_error * 0.1f);
+            if (error > M.max_error) {
+                g.pick[M.dbase + j] = -1;
+                continue;
             }
-            g.pick[M.dbase + j] = ok ? i : -1;
-            valid += ok;
+            ++valid;
+            g.dnrm[M.dbase + j] = make_float4((na.x - nb.x) * 0.5f, (na.y - nb.y) * 0.5f, (na.z - nb.z) * 0.5f,
+                                              (na.w - nb.w) * 0.5f);
+            g.dpos[M.dbase + j] = make_float4(x.x, x.y, x.z, 1.f);
+            if (error < FLT_MAX) {
+                const unsigned long long k2 =
+                    ((unsigned long long)__float_as_uint(error) << 32) | (unsigned long long)(uint32_t)i;
+                atomicMin(&g.key[va], k2);
+                atomicMin(&g.key[vb], k2);
+            }
         }
         int tot;
-        block_scan(valid, &tot);
+        block_scan(valid, &tot);  // (its barriers also keep npassed until every thread has read it)
         if (threadIdx.x == 0 && tot) atomicAdd(&M.valid, tot);
     }
 }
@@ -826,13 +923,13 @@ __global__ __launch_bounds__(kSimpThreads) void k_valid(SG g) {
 // CollapseEdges (:281-304): an edge both of whose ends chose it collapses onto its
 // smaller end.
 __global__ __launch_bounds__(kSimpThreads) void k_collapse(SG g) {
-    LVN_TILES(g.dt, g.ndt) {
+    LVN_TILE_PARTS(g.dt, g.ndt) {
         SMesh& M = g.mesh[tl_m];
         const int n = min(M.draws, M.accepted);
         if (tl_s >= n) continue;
         const int2* edges = edges_of(g, M);
         int coll = 0;
-        for (int r = 0; r < kSimpPer; ++r) {
+        for (int r = 0; r < kSimpPart / kSimpThreads; ++r) {
             const int j = tl_s + threadIdx.x + r * kSimpThreads;
             if (j >= n) continue;
             const int i = g.pick[M.dbase + j];
@@ -870,38 +967,114 @@ __global__ void k_iter_mid(SG g) {
 // moves its counts from the old vertices to the new ones, or is dropped (marked dead) when
 // the remap makes it degenerate; degenerate input triangles are dropped in the first pass.
 // The survivors keep their order, so the final compaction gives the reference's list.
+// A tile's 1024 triangles use a few thousand consecutive vertices: their targets are read
+// once, in order, into LDS and looked up there (three scattered reads a triangle, one cache
+// line at a time, bounded the later iterations), and where many triangles change, their
+// count changes gather there too, one device atomic per vertex and tile instead of up to
+// six a triangle, which bounded the first ones.  64 cave meshes: the first iteration 84 -> 27
+// us, the mean of eleven 30 -> 22.5.
+constexpr int kRemapWindow = 4096;  // 16 KB: eight waves per SIMD
+constexpr int kRemapFew = 128;      // fewer touched triangles change the counts directly
 __global__ __launch_bounds__(kSimpThreads) void k_tri_remap(SG g) {
+    __shared__ int win[kRemapWindow];  // the window's targets, then its count changes
+    __shared__ int s_lo, s_hi, s_touched;
     LVN_TILES(g.tt, g.ntt) {
         SMesh& M = g.mesh[tl_m];
         if (!M.tpass) continue;
         const bool first = M.iter == 1;
-        int drop = 0;
+        if (threadIdx.x == 0) {
+            s_lo = INT_MAX;
+            s_hi = -1;
+            s_touched = 0;
+        }
+        int tri[kSimpPer][3], to[kSimpPer][3];
+        int lo = INT_MAX, hi = -1;
+#pragma unroll
         for (int r = 0; r < kSimpPer; ++r) {
             const int t = tl_s + threadIdx.x + r * kSimpThreads;
-            if (t >= M.nt0) continue;
-            int* p = g.tri + 3 * (int64_t)(M.tbase + t);
-            const int a = p[0];
-            if (a < 0) continue;
-            const int b = p[1], c = p[2];
-            const int a2 = remap(g, M, a), b2 = remap(g, M, b), c2 = remap(g, M, c);
-            const bool touched = a2 != a || b2 != b || c2 != c;
-            const bool degen = a2 == b2 || a2 == c2 || b2 == c2;
-            if (!touched && !(first && degen)) continue;
-            atomicSub(&g.vtc[M.vbase + a], 1);
-            atomicSub(&g.vtc[M.vbase + b], 1);
-            atomicSub(&g.vtc[M.vbase + c], 1);
-            if (degen) {
-                p[0] = -1;
-                ++drop;
+            const int* p = g.tri + 3 * (int64_t)(M.tbase + min(t, M.nt0 - 1));
+            tri[r][0] = t < M.nt0 ? p[0] : -1;
+            tri[r][1] = p[1];
+            tri[r][2] = p[2];
+        }
+#pragma unroll
+        for (int r = 0; r < kSimpPer; ++r) {
+            if (tri[r][0] < 0) continue;
+            lo = min(lo, min(tri[r][0], min(tri[r][1], tri[r][2])));
+            hi = max(hi, max(tri[r][0], max(tri[r][1], tri[r][2])));
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            lo = min(lo, __shfl_xor(lo, o));
+            hi = max(hi, __shfl_xor(hi, o));
+        }
+        __syncthreads();
+        if ((threadIdx.x & 63) == 0 && hi >= 0) {
+            atomicMin(&s_lo, lo);
+            atomicMax(&s_hi, hi);
+        }
+        __syncthreads();
+        lo = s_lo;
+        hi = s_hi;
+        const bool local = hi >= 0 && hi - lo < kRemapWindow;
+        if (local)
+            for (int e = threadIdx.x; e <= hi - lo; e += kSimpThreads) win[e] = g.tgt[M.vbase + lo + e];
+        __syncthreads();
+        int drop = 0, mine = 0;
+#pragma unroll
+        for (int r = 0; r < kSimpPer; ++r) {
+            if (tri[r][0] < 0) continue;
+            const int* a = tri[r];
+            int* b = to[r];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                const int t = local ? win[a[q] - lo] : g.tgt[M.vbase + a[q]];
+                b[q] = t != -1 ? t : a[q];
+            }
+            const bool touched = a[0] != b[0] || a[1] != b[1] || a[2] != b[2];
+            const bool degen = b[0] == b[1] || b[0] == b[2] || b[1] == b[2];
+            if (!touched && !(first && degen)) {
+                tri[r][0] = -1;  // nothing to do
                 continue;
             }
-            p[0] = a2;
-            p[1] = b2;
-            p[2] = c2;
-            atomicAdd(&g.vtc[M.vbase + a2], 1);
-            atomicAdd(&g.vtc[M.vbase + b2], 1);
-            atomicAdd(&g.vtc[M.vbase + c2], 1);
+            ++mine;
+            int* p = g.tri + 3 * (int64_t)(M.tbase + tl_s + (int)threadIdx.x + r * kSimpThreads);
+            if (degen) {
+                p[0] = b[0] = -1;
+                ++drop;
+            } else {
+                p[0] = b[0];
+                p[1] = b[1];
+                p[2] = b[2];
+            }
         }
+        if (mine) atomicAdd(&s_touched, mine);
+        __syncthreads();  // the targets are read, the touched triangles counted
+        const bool gather = local && s_touched >= kRemapFew;
+        if (gather)
+            for (int e = threadIdx.x; e <= hi - lo; e += kSimpThreads) win[e] = 0;
+        __syncthreads();
+        auto change = [&](int v, int by) {
+            if (gather && v >= lo && v <= hi)
+                atomicAdd(&win[v - lo], by);
+            else
+                atomicAdd(&g.vtc[M.vbase + v], by);
+        };
+#pragma unroll
+        for (int r = 0; r < kSimpPer; ++r) {
+            if (tri[r][0] < 0) continue;
+            const bool dropped = to[r][0] < 0;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                if (!dropped && to[r][q] == tri[r][q]) continue;  // its count stays
+                change(tri[r][q], -1);
+                if (!dropped) change(to[r][q], 1);
+            }
+        }
+        __syncthreads();
+        if (gather)
+            for (int e = threadIdx.x; e <= hi - lo; e += kSimpThreads)
+                if (win[e]) atomicAdd(&g.vtc[M.vbase + lo + e], win[e]);
         int tot;
         block_scan(drop, &tot);
         if (threadIdx.x == 0 && tot) {
@@ -1135,7 +1308,7 @@ static int run_group(SimpState& st, const SimpJob* jobs, int n, const lvn_simpli
     g.n_u = st.u_len;
     g.opt = opt;
     const dim3 B(kSimpThreads), GV = tile_grid(g.nvt, cus), GT = tile_grid(g.ntt, cus), GE = tile_grid(g.net, cus),
-               GD = tile_grid(g.ndt, cus), GM = mesh_grid(n), GW((unsigned)((n + 3) / 4));
+               GD = tile_grid(g.ndt, cus), GP = tile_grid(kSimpParts * g.ndt, cus), GM = mesh_grid(n), GW((unsigned)((n + 3) / 4));
     // candidate edges
     hipLaunchKernelGGL(k_init_vertices, GV, B, 0, stream, g);
     hipLaunchKernelGGL(k_init_triangles, GT, B, 0, stream, g);
@@ -1159,8 +1332,8 @@ static int run_group(SimpState& st, const SimpJob* jobs, int n, const lvn_simpli
         hipLaunchKernelGGL((k_mesh_scan<&SMesh::dt0, &SMesh::dtn, &SMesh::accepted, &SMesh::active>), GW, B, 0,
                            stream, g);
         hipLaunchKernelGGL(k_tile_emit<DrawOp>, GD, B, 0, stream, g, g.dt, g.ndt);
-        hipLaunchKernelGGL(k_valid, GD, B, 0, stream, g);
-        hipLaunchKernelGGL(k_collapse, GD, B, 0, stream, g);
+        hipLaunchKernelGGL(k_valid, GP, B, 0, stream, g);
+        hipLaunchKernelGGL(k_collapse, GP, B, 0, stream, g);
         hipLaunchKernelGGL(k_iter_mid, GM, dim3(256), 0, stream, g);
         hipLaunchKernelGGL(k_tri_remap, GT, B, 0, stream, g);
         hipLaunchKernelGGL(k_tile_count<EdgeKeepOp>, GE, B, 0, stream, g, g.et, g.net);
