@@ -1048,6 +1048,91 @@ __device__ __forceinline__ float4 brush_crossing(WaveOps& list, const ChunkDesc&
     return make_float4(nrm.x, nrm.y, nrm.z, crossing);
 }
 
+// The least of the wave's values, in every lane (compared as the bits of non-negative
+// floats, so a NaN loses to any number).
+__device__ __forceinline__ float wave_least(float v) {
+    uint32_t x = __float_as_uint(v);
+#define LVN_LEAST(ctrl) x = min(x, (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, ctrl, 0xf, 0xf, false));
+    LVN_LEAST(0x111)  // row_shr 1, 2, 4, 8: lane 15 of a row holds the row's
+    LVN_LEAST(0x112)
+    LVN_LEAST(0x114)
+    LVN_LEAST(0x118)
+    LVN_LEAST(0x142)  // row_bcast 15 and 31: lane 63 holds the wave's
+    LVN_LEAST(0x143)
+#undef LVN_LEAST
+    return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)x, 63));
+}
+
+// The same for one edge, the same in every lane: the ops lie one per lane, so the distances
+// of 64 of them at a point are one evaluation, and an op that can win is sampled with a
+// sample per lane.  About 310 instructions an edge up to 64 ops; 64 edges by the form above
+// take about 180 per op, and 500 for each op that can win for any of them.
+__device__ __forceinline__ float4 brush_crossing_one(WaveOps& list, const ChunkDesc& cd, int x, int y, int z, int axis) {
+    const int lane = threadIdx.x & 63;
+    const int w0x = x * cd.scale + cd.off[0], w0y = y * cd.scale + cd.off[1], w0z = z * cd.scale + cd.off[2];
+    const float p0x = (float)w0x, p0y = (float)w0y, p0z = (float)w0z;
+    const float ex = (float)(w0x + (axis == 0 ? cd.scale : 0)) - p0x;
+    const float ey = (float)(w0y + (axis == 1 ? cd.scale : 0)) - p0y;
+    const float ez = (float)(w0z + (axis == 2 ? cd.scale : 0)) - p0z;
+    const int n = cd.op_count, groups = (n + 63) >> 6;
+    constexpr float kFar = 3.402823466e+38f;
+    const float half = (float)cd.scale * 0.5f;
+    const float mx = p0x + ex * 0.5f, my = p0y + ey * 0.5f, mz = p0z + ez * 0.5f;
+    float mid = kFar;  // the lane's op's |d| at the middle (of the last group held)
+    float least = kFar;
+    for (int g = 0; g < groups; ++g) {
+        list.hold(g);
+        mid = 64 * g + lane < n ? fabsf(brush_density(list.mine(), mx, my, mz)) : kFar;
+        least = fminf(least, mid);
+    }
+    least = wave_least(least);
+    const float t = (float)min(lane, 16) * 0.0625f;  // the lane's sample (= the scan's running sum, exact)
+    const float sx = p0x + ex * t, sy = p0y + ey * t, sz = p0z + ez * t;
+    float best = kFar;
+    for (int g = 0; g < groups; ++g) {
+        if (groups > 1) {
+            list.hold(g);
+            mid = fabsf(brush_density(list.mine(), mx, my, mz));
+        }
+        const DevOp own = list.mine();
+        const float slack = 1e-5f * (((fabsf(mx - own.ox) + fabsf(my - own.oy)) + (fabsf(mz - own.oz) + half)) +
+                                     ((fabsf(own.dx) + fabsf(own.dy)) + fabsf(own.dz)));
+        const float reach = half + slack;
+        uint64_t left = __ballot(64 * g + lane < n && !(mid - reach > least));  // also taken for NaN distances
+        while (left) {
+            const DevOp op = list.at(64 * g + (int)__builtin_ctzll(left));
+            left &= left - 1;
+            const float d = fabsf(brush_density(op, sx, sy, sz));
+            if (d < best) best = d;
+        }
+    }
+    if (lane > 16) best = kFar;
+    const float found = wave_least(best);
+    const int kbest = (int)__builtin_ctzll(__ballot(best == found));
+    const float crossing = (float)kbest * 0.0625f;
+    const float px = p0x + ex * crossing;
+    const float py = p0y + ey * crossing;
+    const float pz = p0z + ez * crossing;
+    const float h = 0.001f;
+    for (int g = groups - 1; g >= 0; --g) {  // the last op holding the point decides
+        list.hold(g);
+        const uint64_t in = __ballot(64 * g + lane < n && !(brush_density(list.mine(), px, py, pz) > 0.f));
+        if (!in) continue;
+        const DevOp op = list.at(64 * g + 63 - (int)__builtin_clzll(in));
+        // lanes 0 .. 5: the points h before and behind along each axis
+        const float step = lane & 1 ? -h : h;
+        const float d = brush_density(op, lane >> 1 == 0 ? px + step : px, lane >> 1 == 1 ? py + step : py,
+                                      lane >> 1 == 2 ? pz + step : pz);
+        float q[6];
+#pragma unroll
+        for (int i = 0; i < 6; ++i) q[i] = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(d), i));
+        const float flip = op.type == 0 ? 1.f : -1.f;
+        const float3 u = normalize_or_zero(q[0] - q[1], q[2] - q[3], q[4] - q[5]);
+        return make_float4(flip * u.x, flip * u.y, flip * u.z, crossing);
+    }
+    return make_float4(0.f, 0.f, 0.f, crossing);
+}
+
 // The end samples of edge (x, y, z, axis), field indices i0 and i1: the stored field, or,
 // for a field without the cave term whose density a batch does not store (dens_cols),
 // y - H with H from the column heights: density_column's expression, bit for bit (its
@@ -1194,7 +1279,16 @@ __device__ __forceinline__ void edge_items(const KArgs& a, int chunks, int per_i
 // brushed 64^3 chunk of the reference's terrain meshed in 598 -> 325 us, a two-step edit of
 // a cached chunk (no field evaluation at all) in 1,104 -> 761 us, 24 chunks under 256
 // brushes staged, meshed and fetched in 1,554 -> 1,285 us.
-template <bool kCount>
+// Of a few chunks, those under many brushes take short items and their touched edges one by
+// one, an op per lane: 64 edges of one wave scanning 60 ops one after another were the time
+// of a one-chunk call while most of the chip was idle.  One 64^3 chunk under 60 brushes 54 us
+// by 64 edges a wave, 33 by items of 16 edges, 16 by 4 and by 2.  Under fewer than 20 brushes
+// the scan is the shorter chain, and with more chunks it costs fewer instructions: 24 chunks
+// 85 against 92 us, 64 chunks 137 against 206.  (Its own kernel: beside it the scan alone
+// took 5 to 10% longer.)
+constexpr int kOneEdgeItem = 4;
+constexpr int kFewChunks = 8, kOneEdgeOps = 20;
+template <bool kCount, bool kFew>
 __global__ __launch_bounds__(kEdgeDataThreads) void k_edge_data(KArgs a, int chunks, int per_item) {
     __shared__ int wsum[kEdgeDataThreads / 64];
     if (blockIdx.x == gridDim.x - 1) {
@@ -1212,20 +1306,35 @@ __global__ __launch_bounds__(kEdgeDataThreads) void k_edge_data(KArgs a, int chu
         const int chunk = special_chunk(a, q);
         const ChunkDesc cd = a.chunks[chunk];
         const bool cached = cd.mode == kModeCached;
-        const int edges = a.counters[chunk].edges, items = (edges + 63) >> 6;
+        const bool one = kFew && cd.op_count >= kOneEdgeOps;
+        const int per = one ? kOneEdgeItem : 64;  // edges of an item
+        const int edges = a.counters[chunk].edges, items = (edges + per - 1) / per;
         const int* ids = slot_ptr<const int>(a, chunk, a.L.e_ids);
         float4* data = slot_ptr<float4>(a, chunk, a.L.e_data);
         const int* oid = reinterpret_cast<const int*>(cd.old_ids);
         const float4* odata = reinterpret_cast<const float4*>(cd.old_data);
         WaveOps list(a, cd);
         for (int j = first_dealt(wave, dealt, waves); j < items; j += waves) {
-            const int i = 64 * j + lane;
-            const int id = i < edges ? ids[i] : 0;
+            const int i = per * j + lane;
+            const bool in = lane < per && i < edges;
+            const int id = in ? ids[i] : 0;
             EdgeAt e;
-            bool live = decode_edge(G, id, e) && i < edges;
-            if (i < edges && !live) atomicOr(&a.counters[chunk].status, kStatusLookupMiss);
+            const bool live = decode_edge(G, id, e) && in;
+            if (in && !live) atomicOr(&a.counters[chunk].status, kStatusLookupMiss);
             const bool touched = live && edge_touched(a, chunk, cd, e.i0, e.i1);
-            if (__ballot(touched)) {
+            uint64_t left = __ballot(touched);
+            if (kFew && left && one) {
+                float4 out = make_float4(0.f, 0.f, 0.f, 0.f);
+                while (left) {
+                    const int b = (int)__builtin_ctzll(left);
+                    left &= left - 1;
+                    EdgeAt at;
+                    decode_edge(G, __builtin_amdgcn_readlane(id, b), at);
+                    const float4 v = brush_crossing_one(list, cd, at.x, at.y, at.z, at.axis);
+                    if (lane == b) out = v;
+                }
+                if (touched) data[i] = out;
+            } else if (left) {
                 const float4 out = brush_crossing(list, cd, touched, e.x, e.y, e.z, e.axis);
                 if (touched) data[i] = out;
             }
@@ -2696,10 +2805,9 @@ void launch_edge_cross(const KArgs& a, int chunks, hipStream_t s) {
     // one workgroup that counts the items
     const dim3 data_grid(kEdgeDataBlocks + 1), data_block(kEdgeDataThreads);
     const int per_item = g == kCrossSampleParallel ? 64 : 64 / g;
-    if (a.work)
-        hipLaunchKernelGGL(k_edge_data<true>, data_grid, data_block, 0, s, a, chunks, per_item);
-    else
-        hipLaunchKernelGGL(k_edge_data<false>, data_grid, data_block, 0, s, a, chunks, per_item);
+    auto* const data_kernel = a.work ? (chunks <= kFewChunks ? k_edge_data<true, true> : k_edge_data<true, false>)
+                                     : (chunks <= kFewChunks ? k_edge_data<false, true> : k_edge_data<false, false>);
+    hipLaunchKernelGGL(data_kernel, data_grid, data_block, 0, s, a, chunks, per_item);
     // the item count is on the device; size the grid for 512 edge items per chunk
     switch (g) {
     case 2: launch_cross_group<2>(a, chunks, s); return;
