@@ -1,7 +1,8 @@
 """Edge and voxel lists in both of their walks (a lane per list entry where rows are sparse,
 a lane per position where they are dense) and both launch forms (four waves per 64 rows for
-a few chunks, one for many): one chunk's lists against the oracle's, and every mesh of a
-batch of 64 against that chunk's (needs a GPU)."""
+a few chunks, one for many): one chunk's lists against the oracle's, and meshes of a batch
+of 64, whose density pass stores solid planes in y-segments, against that chunk's (needs a
+GPU)."""
 import numpy as np
 import pytest
 
@@ -17,6 +18,7 @@ FIELDS = {
     "caves": (workloads.terrain_desc(), 2, -2048),
     # a few edges a row
     "hills": (workloads.heightfield_desc(), 1, -128),
+    "leven": (workloads.leven_desc(), workloads.LEVEN_SEED, 2320),
 }
 
 
@@ -26,7 +28,8 @@ def test_lists_match_oracle(field, voxels):
     desc, seed, y = FIELDS[field]
     mesher.init(desc, seed, 0)
     mesher.clear_csg_ops()
-    mn, size = (64, y // (4 * voxels) * (4 * voxels) if y < -1000 else -2 * voxels, 128), 4 * voxels
+    size = 4 * voxels
+    mn = (64, y // size * size if abs(y) > 1000 else -2 * voxels, 128)
     print(f"compact: {field} N={voxels}", flush=True)
     ctx = mesher.Context(voxels)
     g = ctx.debug_stages(mn, size)
@@ -39,10 +42,12 @@ def test_lists_match_oracle(field, voxels):
     n = 64
     b = mesher.Batch(voxels, n)
     b.set_chunks([mn] * n, [size] * n)
-    b.run()
-    assert b.counts()[:n, 4].max() == 0
-    for i in (0, 1, n // 2, n - 1):
-        for got, ref in zip(b.get_mesh(i), want):
-            assert got.shape == ref.shape and got.tobytes() == ref.tobytes()
+    for ysplit in (0, 1, 5, voxels):  # y-segments of the planes, the last ones short or empty
+        b.set_tuning(density_ysplit=ysplit)
+        b.run()
+        assert b.counts()[:n, 4].max() == 0
+        for i in (0, 1, n // 2, n - 1):
+            for got, ref in zip(b.get_mesh(i), want):
+                assert got.shape == ref.shape and got.tobytes() == ref.tobytes()
     b.close()
     ctx.close()
