@@ -440,29 +440,69 @@ __global__ __launch_bounds__(256) void k_csg(KArgs a) {
 // ---------------------------------------------------------------------------
 constexpr int kRowsPerBlock = 16;  // sample rows staged per wave
 
+// Rows [16 b, 16 b + 16) of a chunk from its materials, by one wave; `stage` is the wave's.
+__device__ __forceinline__ void solid_block(const KArgs& a, int chunk, int b, uint32_t* stage) {
+    const Geometry& G = a.G;
+    const int F = G.F, lane = threadIdx.x & 63;
+    const uint32_t* mat = slot_ptr<const uint32_t>(a, chunk, a.L.mat);
+    uint64_t* S = slot_ptr<uint64_t>(a, chunk, a.L.solid);
+    const uint8_t* bytes = reinterpret_cast<const uint8_t*>(stage);
+    const int words_total = G.field_samples >> 2;  // F is even, so F^3 is a multiple of 8
+    const int block_words = (kRowsPerBlock * F) >> 2;
+    // bytes [16 F b, 16 F (b + 1)): 4-byte aligned
+    const int w0 = b * block_words;
+    for (int j = lane; j < block_words; j += 64)
+        if (w0 + j < words_total) stage[j] = mat[w0 + j];
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    // The block's rows are 2 * rows consecutive words of S: lane 2k keeps row k's low
+    // word and lane 2k + 1 its high word, and one store writes them all.
+    const int rows = min(kRowsPerBlock, G.field_rows - b * kRowsPerBlock);
+    uint64_t word = 0;
+    for (int k = 0; k < rows; ++k) {
+        const bool s0 = lane < F && bytes[k * F + lane] != kAir;
+        const bool s1 = lane + 64 < F && bytes[k * F + lane + 64] != kAir;
+        const uint64_t lo = __ballot(s0), hi = __ballot(s1);
+        if (lane == 2 * k) word = lo;
+        if (lane == 2 * k + 1) word = hi;
+    }
+    if (lane < 2 * rows) S[2 * b * kRowsPerBlock + lane] = word;
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// A batch's chunks without brushes have solid planes, each turned by its own workgroups.  So
+// are the blocks of those with materials while a chunk has a wave for each; in larger batches
+// these, which are few, are dealt round all waves of the launch: a brushed chunk's five
+// workgroups took 14 blocks a wave one after another, and the launch waited for them (1,800
+// clipmap chunks 64 -> 30 us, 512 cave chunks 56 -> 44; 16 chunks 8 us, dealt 12).
 __global__ __launch_bounds__(256) void k_solid_rows(KArgs a) {
     __shared__ uint32_t stage[4][kRowsPerBlock * 66 / 4];
     const int chunk = blockIdx.y;
     const Geometry& G = a.G;
     const int F = G.F;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint32_t* mat = slot_ptr<const uint32_t>(a, chunk, a.L.mat);
-    uint64_t* S = slot_ptr<uint64_t>(a, chunk, a.L.solid);
-    if (chunk_mat_free(a, a.chunks[chunk])) {  // uniform over the workgroup
+    const int blocks = (G.field_rows + kRowsPerBlock - 1) / kRowsPerBlock;
+    const bool planes = chunk_mat_free(a, a.chunks[chunk]);  // uniform over the workgroup
+    const bool deal = a.mat_free && waves_per_chunk() < blocks;
+    if (!planes && !deal)
+        for (int b = wave_in_chunk(); b < blocks; b += waves_per_chunk()) solid_block(a, chunk, b, stage[wave]);
+    if (planes) {
         // the sides its items met, for the kernels from here on (an atomic per item instead
         // cost the density pass 50 us on 1,800 chunks)
+        uint64_t* S = slot_ptr<uint64_t>(a, chunk, a.L.solid);
         const uint8_t* met = slot_ptr<const uint8_t>(a, chunk, a.L.sides);
         int mine = 0;
         for (int i = lane; i < G.col_groups * a.ysplit; i += 64) mine |= met[i];
         const int sides = (__ballot(mine & kSomeSolid) ? kSomeSolid : 0) | (__ballot(mine & kSomeAir) ? kSomeAir : 0);
         if (blockIdx.x == 0 && threadIdx.x == 0) a.counters[chunk].sides = sides;
-        if (sides != (kSomeSolid | kSomeAir)) return;
         // Row (y, z) is bits [F z, F z + F) of plane y: a 64-bit window of two or three
         // consecutive group words, then F - 64 bits above it (none when F <= 64).
         const uint64_t* P = slot_ptr<const uint64_t>(a, chunk, a.L.planes);
         const uint64_t lo_mask = F >= 64 ? ~0ull : ((1ull << F) - 1ull);
         const uint64_t hi_mask = F > 64 ? ((1ull << (F - 64)) - 1ull) : 0ull;
-        for (int r = thread_in_chunk(); r < G.field_rows; r += threads_per_chunk()) {
+        const int rows = sides == (kSomeSolid | kSomeAir) ? G.field_rows : 0;
+        for (int r = thread_in_chunk(); r < rows; r += threads_per_chunk()) {
             const int z = div_magic(r, G.magic_f), y = r - z * F;
             const int t0 = F * z, g0 = t0 >> 6, sh = t0 & 63;
             const uint64_t w0 = P[g0 * F + y];
@@ -473,34 +513,14 @@ __global__ __launch_bounds__(256) void k_solid_rows(KArgs a) {
             S[2 * r] = lo & lo_mask;
             S[2 * r + 1] = hi & hi_mask;
         }
-        return;
     }
-    const uint8_t* bytes = reinterpret_cast<const uint8_t*>(stage[wave]);
-    const int blocks = (G.field_rows + kRowsPerBlock - 1) / kRowsPerBlock;
-    const int words_total = G.field_samples >> 2;  // F is even, so F^3 is a multiple of 8
-    const int block_words = (kRowsPerBlock * F) >> 2;
-    for (int b = wave_in_chunk(); b < blocks; b += waves_per_chunk()) {
-        // block b = rows [16 b, 16 b + 16) = bytes [16 F b, 16 F (b + 1)): 4-byte aligned
-        const int w0 = b * block_words;
-        for (int j = lane; j < block_words; j += 64)
-            if (w0 + j < words_total) stage[wave][j] = mat[w0 + j];
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        // The block's rows are 2 * rows consecutive words of S: lane 2k keeps row k's low
-        // word and lane 2k + 1 its high word, and one store writes them all.
-        const int rows = min(kRowsPerBlock, G.field_rows - b * kRowsPerBlock);
-        uint64_t word = 0;
-        for (int k = 0; k < rows; ++k) {
-            const bool s0 = lane < F && bytes[k * F + lane] != kAir;
-            const bool s1 = lane + 64 < F && bytes[k * F + lane + 64] != kAir;
-            const uint64_t lo = __ballot(s0), hi = __ballot(s1);
-            if (lane == 2 * k) word = lo;
-            if (lane == 2 * k + 1) word = hi;
-        }
-        if (lane < 2 * rows) S[2 * b * kRowsPerBlock + lane] = word;
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    }
+    if (!deal) return;
+    const int lists = special_chunks(a), waves = (int)(gridDim.x * gridDim.y * (blockDim.x >> 6));
+    // consecutive workgroups take distant blocks, so a few blocks spread over the CUs
+    const int first = __builtin_amdgcn_readfirstlane((int)((threadIdx.x >> 6) * gridDim.x + blockIdx.x) * (int)gridDim.y +
+                                                     (int)blockIdx.y);
+    for (int i = first; i < lists * blocks; i += waves)
+        solid_block(a, special_chunk(a, i / blocks), i % blocks, stage[wave]);
 }
 
 // Edge rows by the first `edge_blocks` workgroups of a chunk, voxel rows by the others: both
