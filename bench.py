@@ -73,16 +73,15 @@ def hbm_traffic(kernel, workload):
     with open(path) as f:
         data = json.load(f)
     for name, entries in data["kernels"].items():
-        if name.split("::")[-1].split("<")[0] == kernel and "<true>" not in name:
+        if name.split("::")[-1].split("<")[0] == kernel and "<true" not in name:
             e = max(entries, key=lambda x: x["grid"])  # the batched launch
             return e["read_bytes"] + e["write_bytes"]
     return None
 
 
 # stage -> kernels whose HBM bytes it moves (batched launch)
-STAGE_KERNELS = {"density": ["k_density"], "edge_rows": ["k_solid_rows", "k_edge_rows"],
-                 "edge_compact": ["k_edge_compact"], "edge_cross": ["k_edge_cross"], "voxel_rows": ["k_voxel_rows"],
-                 "voxel_compact": ["k_voxel_compact"], "qef": ["k_qef"], "emit": ["k_emit"]}
+STAGE_KERNELS = {"density": ["k_density"], "edge_rows": ["k_solid_rows", "k_rows"], "edge_compact": ["k_compact"],
+                 "edge_cross": ["k_edge_cross"], "qef": ["k_qef"], "emit": ["k_emit"]}
 
 
 def hbm_rates(stage_ms, workload):

@@ -1214,7 +1214,7 @@ __device__ __forceinline__ bool decode_edge(const Geometry& G, int id, EdgeAt& e
     e.z = (hidx >> (2 * G.shift)) & msk;
     e.i0 = field_index(G, e.x, e.y, e.z);
     e.i1 = e.i0 + (e.axis == 0 ? 1 : e.axis == 1 ? G.F : G.F * G.F);
-    return e.x < G.H && e.y < G.H && e.z < G.H && e.axis <= 2;  // always so for k_edge_compact's ids
+    return e.x < G.H && e.y < G.H && e.z < G.H && e.axis <= 2;  // always so for the ids of the edge lists
 }
 
 // An edge with an endpoint whose material a brush changed takes brush data
@@ -2737,18 +2737,20 @@ static unsigned persistent_blocks(const KArgs& a, int per_cu, long items) {
 // the segment is the cost (a 66-sample column is 0.18 ms of dependent octaves), so few
 // chunks are cut finely, down to two samples, until about 20,000 items fill the chip, and
 // never below three segments, which balance caves against sky; without it each segment
-// repeats the whole height term, so a cut pays only until about 3,400 items are in flight.
-// Measured (density stage, us; caves / reference terrain): one chunk 39 / 14 with 6
-// segments, 16 / 12 with these; 8 chunks 51 / 17 -> 40 / 17; 24 chunks 83 / 29 -> 74 / 24;
-// 96 chunks 347 / 54 -> 216 / 46; 500 chunks 1,087 / 202 -> 914 / 156 (with the workgroups
-// below).
+// repeats the whole height term, so a cut pays only where samples are stored (one chunk, or
+// chunks under brushes) and until about 3,400 items are in flight.
+// Measured with caves (density stage, us): one chunk 29 with 6 segments, 15 with these; 8
+// chunks 41 -> 36; 24 chunks 73 -> 69; 96 chunks 271 with one, 198 with these; 500 chunks 944
+// -> 844 (with the workgroups below).  Reference terrain, one chunk with stored samples 14
+// with 6 segments, 12 with these; batches of solid planes alone take 11 us up to 16 chunks
+// and 55 for 500 whole, 1.7 times that in two segments.
 int default_ysplit(const Geometry& G, int field_kind, int chunks) {
     const long items = (long)G.col_groups * std::max(1, chunks);
     if (field_kind == LVN_FIELD_TERRAIN_CAVES) return (int)std::clamp(20000L / items, 3L, (long)G.F / 2);
     return (int)std::clamp(3400L / items, 1L, std::min(11L, (long)G.F / 2));
 }
-// Two workgroups per CU once one per CU has every wave busy (500 chunks: 1,040 -> 914 us
-// with caves, 202 -> 156 without); below that a second one only loads tables.
+// Two workgroups per CU once one per CU has every wave busy (500 chunks: 904 -> 844 us
+// with caves, 59 -> 55 without); below that a second one only loads tables.
 int default_density_per_cu(const Geometry& G, int ysplit, int chunks, int cus) {
     return (long)G.col_groups * ysplit * chunks > 16L * cus ? 2 : 1;
 }
