@@ -881,8 +881,7 @@ enum : int {
     kSgCntFinal = 4,
     kSgCntLevel = 8,                          // + level
     kSgCntRound = kSgCntLevel + kSgLevels,        // + round: tiles of the round's list
-    kSgCntActive = kSgCntRound + kMaxRounds + 1,  // + round: seams whose calls still expand
-    kSgCounters = kSgCntActive + kMaxRounds,
+    kSgCounters = kSgCntRound + kMaxRounds + 1,
 };
 
 struct SeamGrid {
@@ -1102,7 +1101,7 @@ __global__ __launch_bounds__(1024) void k_sg_tiles(SeamGrid g, int first, int4* 
     if (threadIdx.x == 0) *total = n;
 }
 
-// Seam records and round counters cleared; every hash slot emptied.
+// Seam records cleared; every hash slot emptied.
 __global__ __launch_bounds__(kSgThreads) void k_sg_init(SeamGrid g, const int4* tiles) {
     for (int s = blockIdx.x * kSgThreads + threadIdx.x; s < g.m; s += gridDim.x * kSgThreads) {
         SeamRun& R = g.run[s];
@@ -1115,7 +1114,6 @@ __global__ __launch_bounds__(kSgThreads) void k_sg_init(SeamGrid g, const int4* 
         for (int k = 0; k <= kSgLevels; ++k) R.lev[k] = 0;
         for (int k = 0; k < kSgLevels; ++k) R.fill[k] = 0;
     }
-    if (blockIdx.x == 0 && threadIdx.x < kMaxRounds) g.cnt[kSgCntActive + threadIdx.x] = 0;
     LVN_SG_TILES(tiles, g.cnt[kSgCntHash]) {
         const SeamJobDev& J = g.jobs[tl.x];
         SeamScratch S = sg_scratch(g, tl.x);
@@ -1679,15 +1677,14 @@ __global__ __launch_bounds__(kSgRoundThreads) void k_sg_round(SeamGrid g, const 
 // After a round, per seam (one workgroup of 1024 threads, g.lanes lanes per seam): the
 // tile counts of the round scanned in tile order into the blocks' places in the next list,
 // the seam's round closed (the next list's length; the seam stays in the rounds while a
-// written call still expands, counted in the round's active counter; an overflow of the
-// list or of the round limit ends it), and the next round's tile list made.
+// written call still expands; an overflow of the list or of the round limit ends it), and
+// the next round's tile list made.
 __global__ __launch_bounds__(1024) void k_sg_round_next(SeamGrid g, int round, const int* tsum, int* toff,
                                                          int4* next) {
     __shared__ int fill[kXcds];
     if (threadIdx.x < kXcds) fill[threadIdx.x] = 0;
     __syncthreads();
     const int lane = threadIdx.x & (g.lanes - 1);
-    int active = 0;
     for (int s = threadIdx.x / g.lanes; s < g.m; s += blockDim.x / g.lanes) {
         SeamRun& R = g.run[s];
         const SeamJobDev& J = g.jobs[s];
@@ -1717,7 +1714,6 @@ __global__ __launch_bounds__(1024) void k_sg_round_next(SeamGrid g, int round, c
                 if (status) set_status(&R.status, status);
                 R.n = n;
                 R.more = more;
-                active += status == 0 && more;
             }
         }
         const int cnt = status == 0 && linked && more ? g.tiles_of(n) : 0;
@@ -1732,7 +1728,6 @@ __global__ __launch_bounds__(1024) void k_sg_round_next(SeamGrid g, int round, c
     __syncthreads();
     const int n = sg_pad(next, fill);
     if (threadIdx.x == 0) g.cnt[kSgCntRound + round + 1] = n;
-    if (active) atomicAdd(&g.cnt[kSgCntActive + round], active);
 }
 
 // The round's blocks copied from the staging list into the seam's list in call order.
@@ -1778,7 +1773,7 @@ __global__ __launch_bounds__(kSgThreads) void k_sg_triangles(SeamGrid g, const i
         const SeamRun& R = g.run[s];
         const bool ok = R.status == 0 && R.linked;
         SeamResDev r;
-        r.status = R.status;
+        r.status = R.status == 0 && R.more ? LVN_ERR_OVERFLOW : R.status;  // (every seam is done by now)
         r.nv = ok ? sg_leaves(R, g.jobs[s]) : 0;
         r.nt = ok ? 2 * R.n : 0;
         r.rounds = R.rounds;
@@ -1847,9 +1842,9 @@ struct SeamLoc {
 // Seam-stitching buffers of a context, grown on demand and kept for reuse.  Each retry
 // attempt writes its own output buffers, so every finished seam stays addressable.
 struct SeamState {
-    DevBuf in, jobs, srcs, scratch, res, offs, pv, pt, counts;
+    DevBuf in, jobs, srcs, scratch, res, pv, pt, counts;
     DevBuf g_run, g_tiles, g_tsum, g_cnt;  // grid pass: seam records, tile lists, round scans, counters
-    HostBuf h_in, h_jobs, h_srcs, h_res, h_pv, h_pt, h_counts, h_active;
+    HostBuf h_in, h_jobs, h_srcs, h_res, h_pv, h_pt, h_counts;
     std::vector<std::unique_ptr<DevBuf>> out_v, out_t;  // per attempt
     std::vector<SeamLoc> loc;                            // per seam of the last call
     std::vector<hipEvent_t> ev;                          // ends of the download chunks
@@ -1954,10 +1949,9 @@ int resolve_batch(void* owner, const lvn_seam_source& q, SeamSrcDev& d) {
 // in device memory as d_jobs and on the host as h_jobs.  Launch sequence: tile lists of
 // the sizes the host knows, clear, select, leaves, ancestors, links, level buckets, leaf
 // counts (deepest level first), ranks (top level first), vertices, contouring rounds,
-// triangles.  The rounds run in batches without a read-back; after a batch the host reads
-// how many seams still expand.  A call made in round r (from 1) has its internal nodes at
-// level r or deeper, and no internal node lies at the deepest level, so the first batch (a
-// round per level) finishes every seam.
+// triangles.  A call made in round r (from 1) has its internal nodes at
+// level r or deeper, and no internal node lies at the deepest level, so a round per level
+// ends every seam and nothing is read back.
 int run_seam_grid(Ctx* c, SeamState& st, int m, const SeamJobDev* h_jobs, const std::vector<SeamSrcDev>& srcs,
                   const SeamJobDev* d_jobs, lvn_vertex* ov, int* ot, SeamResDev* d_res) {
     // list lengths: eight interleaved sub-lists, seam k in sub-list k mod 8, each padded to
@@ -1999,8 +1993,7 @@ int run_seam_grid(Ctx* c, SeamState& st, int m, const SeamJobDev* h_jobs, const 
                   o_round = o_lev + (lmax + 1) * tn, o_fin = o_round + 2 * tr, total = o_fin + tr;
     int r;
     if ((r = st.g_run.ensure(m * sizeof(SeamRun))) || (r = st.g_tiles.ensure(total * sizeof(int4))) ||
-        (r = st.g_tsum.ensure(3 * tr * sizeof(int))) || (r = st.g_cnt.ensure(kSgCounters * sizeof(int))) ||
-        (r = st.h_active.ensure(sizeof(int))))
+        (r = st.g_tsum.ensure(3 * tr * sizeof(int))) || (r = st.g_cnt.ensure(kSgCounters * sizeof(int))))
         return r;
     int* cnt = static_cast<int*>(st.g_cnt.p);
     int* tsum = static_cast<int*>(st.g_tsum.p);
@@ -2039,18 +2032,12 @@ int run_seam_grid(Ctx* c, SeamState& st, int m, const SeamJobDev* h_jobs, const 
     LVN_SG(k_sg_vertices, grid(tl), block, 0, sm, g, T + o_leaf);
     // round r reads tile list r & 1 and makes list (r + 1) & 1
     LVN_SG(k_sg_tiles, dim3(1), dim3(1024), 0, sm, g, kSgListRound, T + o_round, int4{});
-    int round = 0;
-    for (int batch = std::max(lmax, 1); round < kMaxRounds; batch = 2) {
-        for (int k = 0; k < batch && round < kMaxRounds; ++k, ++round) {
-            int4* cur = T + o_round + (round & 1) * tr;
-            int4* nxt = T + o_round + ((round + 1) & 1) * tr;
-            LVN_SG(k_sg_round, round_grid, dim3(kSgRoundThreads), 0, sm, g, cur, round, tsum, tbase);
-            LVN_SG(k_sg_round_next, dim3(1), dim3(1024), 0, sm, g, round, tsum, toff, nxt);
-            LVN_SG(k_sg_round_copy, dev_grid, block, 0, sm, g, cur, round, tsum, tbase, toff);
-        }
-        LVN_HIP(hipMemcpyAsync(st.h_active.p, cnt + kSgCntActive + round - 1, sizeof(int), hipMemcpyDeviceToHost, sm));
-        LVN_HIP(hipStreamSynchronize(sm));
-        if (*static_cast<const int*>(st.h_active.p) == 0) break;
+    for (int round = 0; round < lmax; ++round) {
+        int4* cur = T + o_round + (round & 1) * tr;
+        int4* nxt = T + o_round + ((round + 1) & 1) * tr;
+        LVN_SG(k_sg_round, round_grid, dim3(kSgRoundThreads), 0, sm, g, cur, round, tsum, tbase);
+        LVN_SG(k_sg_round_next, dim3(1), dim3(1024), 0, sm, g, round, tsum, toff, nxt);
+        LVN_SG(k_sg_round_copy, dev_grid, block, 0, sm, g, cur, round, tsum, tbase, toff);
     }
     LVN_SG(k_sg_tiles, dim3(1), dim3(1024), 0, sm, g, kSgListFinal, T + o_fin, int4{});
     LVN_SG(k_sg_triangles, dev_grid, block, 0, sm, g, T + o_fin, d_res);
@@ -2218,17 +2205,18 @@ int run_seams(Ctx* c, int n, const lvn_seam_req* reqs, const lvn_seam_source* so
             v_off += (uint64_t)J.leaf_cap;
             t_off += 2 * (uint64_t)J.list_cap;
         }
+        // every seam's result, then the packed offsets: one read-back
+        static_assert(sizeof(SeamResDev) % 8 == 0, "the offsets follow the results");
+        const size_t res_bytes = m * sizeof(SeamResDev) + (2 * (size_t)m + 2) * 8;
         if ((r = st.jobs.ensure(m * sizeof(SeamJobDev))) || (r = st.h_jobs.ensure(m * sizeof(SeamJobDev))) ||
             (r = st.scratch.ensure(scratch)) || (r = ov.ensure(std::max<uint64_t>(v_off, 1) * sizeof(lvn_vertex))) ||
-            (r = ot.ensure(std::max<uint64_t>(t_off, 1) * 12)) || (r = st.res.ensure(m * sizeof(SeamResDev))) ||
-            (r = st.h_res.ensure(m * sizeof(SeamResDev) + (2 * (size_t)m + 2) * 8)) ||
-            (r = st.offs.ensure((2 * (size_t)m + 2) * 8)))
+            (r = ot.ensure(std::max<uint64_t>(t_off, 1) * 12)) || (r = st.res.ensure(res_bytes)) || (r = st.h_res.ensure(res_bytes)))
             return r;
         std::memcpy(st.h_jobs.p, jobs.data(), m * sizeof(SeamJobDev));
         LVN_HIP(hipMemcpyAsync(st.jobs.p, st.h_jobs.p, m * sizeof(SeamJobDev), hipMemcpyHostToDevice, c->stream));
         const auto* d_jobs = static_cast<const SeamJobDev*>(st.jobs.p);
         auto* d_res = static_cast<SeamResDev*>(st.res.p);
-        auto* d_offs = static_cast<uint64_t*>(st.offs.p);
+        auto* d_offs = reinterpret_cast<uint64_t*>(d_res + m);
         if (seam_pass_grid(jobs, srcs)) {
             if ((r = run_seam_grid(c, st, m, jobs.data(), srcs, d_jobs, static_cast<lvn_vertex*>(ov.p),
                                    static_cast<int*>(ot.p), d_res)))
@@ -2242,9 +2230,7 @@ int run_seams(Ctx* c, int n, const lvn_seam_req* reqs, const lvn_seam_source* so
         hipLaunchKernelGGL(k_seam_offsets, dim3(1), dim3(1024), 0, c->stream, d_res, m, d_offs);
         LVN_HIP(hipGetLastError());
         char* h_res = static_cast<char*>(st.h_res.p);
-        LVN_HIP(hipMemcpyAsync(h_res, d_res, m * sizeof(SeamResDev), hipMemcpyDeviceToHost, c->stream));
-        LVN_HIP(hipMemcpyAsync(h_res + m * sizeof(SeamResDev), d_offs, (2 * (size_t)m + 2) * 8, hipMemcpyDeviceToHost,
-                               c->stream));
+        LVN_HIP(hipMemcpyAsync(h_res, d_res, res_bytes, hipMemcpyDeviceToHost, c->stream));
         LVN_HIP(hipStreamSynchronize(c->stream));
         const auto* rs = reinterpret_cast<const SeamResDev*>(h_res);
         const auto* offs = reinterpret_cast<const uint64_t*>(h_res + m * sizeof(SeamResDev));
