@@ -2043,7 +2043,9 @@ __device__ __forceinline__ void qef_fast(const KArgs& a, int chunk, const ChunkD
     int count = 0;
     // Each lane walks its own edges in the order of e, the next one's data in flight: a wave
     // takes as many steps as its busiest voxel has edges (7 or 8 of the 12), where a step per
-    // possible edge computed all twelve indices and waited for twelve loads in turn.
+    // possible edge computed all twelve indices and waited for twelve loads in turn.  The
+    // kernel is bound by vector issue (1,300 of about 2,060 instructions a segment are the
+    // rotations below): 1,800 clipmap chunks 337 -> 297 us, 512 cave chunks 488 -> 461.
     uint32_t left = (uint32_t)emask;
     int slot = 0;
     bool used = false;
