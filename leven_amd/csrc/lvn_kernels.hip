@@ -1015,6 +1015,17 @@ __device__ __forceinline__ float4 density_crossing(const KArgs& a, const NoiseLd
     return crossing_normal<kKind>(Fp, T, axis, ends_known, tbest, Hbest, p0x, p0y, p0z, p1x, p1y, p1z, nh, nc);
 }
 
+// The distance from an edge's middle sample to its farther end, both as they are rounded:
+// half an edge below 2^23 voxels; beyond, where the middle of a short edge is no FP32 number,
+// up to a whole one.  (Every sample lies between the ends: the sum that places it rounds
+// monotonically.)
+__device__ __forceinline__ float farther_end(float p0x, float p0y, float p0z, float ex, float ey, float ez, float mx,
+                                             float my, float mz) {
+    // along the edge's axis; the two across add +0
+    const float back = ((mx - p0x) + (my - p0y)) + (mz - p0z);
+    return fmaxf(back, ((ex + ey) + ez) - back);
+}
+
 // FindEdgeIntersectionInfo of the CSG program, cl/apply_csg_operation.cl:443-477,
 // with BrushZeroCrossing (:86-110) and BrushNormal (:144-175): the first (t, op) in
 // the reference's t-outer, op-inner scan whose |d| is smallest, t = k/16; then the
@@ -1035,10 +1046,10 @@ __device__ __forceinline__ float4 brush_crossing(WaveOps& list, const ChunkDesc&
     const float ez = (float)(w0z + (axis == 2 ? cd.scale : 0)) - p0z;
     const int n = cd.op_count;
     constexpr int kMid = 8;
-    const float half = (float)cd.scale * 0.5f;
     float minD = 3.402823466e+38f;
     int kbest = 0;
     const float mx = p0x + ex * 0.5f, my = p0y + ey * 0.5f, mz = p0z + ez * 0.5f;
+    const float half = farther_end(p0x, p0y, p0z, ex, ey, ez, mx, my, mz);
     for (int k = 0; k < n; ++k) {
         const DevOp op = list.at(k);
         const float d = fabsf(brush_density(op, mx, my, mz));
@@ -1101,8 +1112,8 @@ __device__ __forceinline__ float4 brush_crossing_one(WaveOps& list, const ChunkD
     const float ez = (float)(w0z + (axis == 2 ? cd.scale : 0)) - p0z;
     const int n = cd.op_count, groups = (n + 63) >> 6;
     constexpr float kFar = 3.402823466e+38f;
-    const float half = (float)cd.scale * 0.5f;
     const float mx = p0x + ex * 0.5f, my = p0y + ey * 0.5f, mz = p0z + ez * 0.5f;
+    const float half = farther_end(p0x, p0y, p0z, ex, ey, ez, mx, my, mz);
     float mid = kFar;  // the lane's op's |d| at the middle (of the last group held)
     float least = kFar;
     for (int g = 0; g < groups; ++g) {

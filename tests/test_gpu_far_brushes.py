@@ -1,0 +1,55 @@
+"""Brushes far from the origin, where FP32 cannot hold every voxel position: from 2^23 voxels
+on the middle of an edge is rounded to one of its ends.  Hermite data and meshes against the
+oracle bit for bit, in both forms of the brush kernel (needs a GPU)."""
+import numpy as np
+import pytest
+
+from leven_amd import mesher, workloads
+from oracle import py_oracle
+
+pytestmark = pytest.mark.gpu
+
+N = 16
+
+
+def _ops(n, x0, scale, seed):
+    """Brushes over the chunk at x0, with centres on whole and half voxels where FP32 has them."""
+    ops, _ = workloads.make_ops(n, seed=seed, rotated=True, extent=N * scale, y_range=(-6.0 * scale, 6.0 * scale),
+                                size_range=(0.7 * scale, 5.0 * scale))
+    for op in ops:
+        op["origin"][0] = np.float32(x0) + np.float32(np.round(op["origin"][0]))
+    return ops
+
+
+@pytest.mark.parametrize("ops", [3, 40, 100])
+@pytest.mark.parametrize("x0,lod", [((1 << 23) - 8, 0), (-(1 << 23) - 8, 0), ((1 << 23) + 1000, 0), ((1 << 23) - 16, 1)])
+def test_far_brushes_match_oracle(x0, lod, ops):
+    desc = workloads.heightfield_desc()
+    mesher.init(desc, 2, 0)
+    mesher.clear_csg_ops()
+    scale = 1 << lod
+    size, mn = 4 * N * scale, (4 * x0, -2 * N * scale, 0)
+    brushes = _ops(ops, x0, scale, 7 + ops)
+    print(f"far brushes: x0={x0} lod={lod} ops={ops}", flush=True)
+    c = py_oracle.Chunk(N).generate(desc, py_oracle.perm_table(2), mn, size, ops=brushes).build()
+    ids, data = c.edges()
+    assert len(ids) > 100
+    ctx = mesher.Context(N)
+    g = ctx.debug_stages(mn, size, brushes)
+    assert (g["edge_ids"] == ids).all()
+    assert (g["edge_data"].view(np.uint32) == data.view(np.uint32)).all()
+    ctx.close()
+    # the scan of more than a few chunks: this one among eight without brushes
+    for op in brushes:
+        mesher.store_csg_op(op, mn, [v + size for v in mn])
+    b = mesher.Batch(N, 9)
+    b.set_chunks([(mn[0], mn[1] + 40 * size * k, mn[2]) for k in range(9)], [size] * 9)
+    b.run()
+    v, t, _ = b.get_mesh(0)
+    b.close()
+    mesher.clear_csg_ops()
+    pos, nrm = c.positions()
+    tri = c.triangles()
+    assert len(t) == len(tri) > 0 and (t == tri).all()
+    assert (v["pos"].view(np.uint32) == pos.view(np.uint32)).all()
+    assert (v["normal"].view(np.uint32) == nrm.view(np.uint32)).all()
