@@ -357,11 +357,13 @@ __global__ __launch_bounds__(256) void k_csg(KArgs a) {
             const int x0 = jx * kCsgX, y0 = jy * kCsgY, z0 = jz * kCsgZ;
             const int x = x0 + (lane & (kCsgX - 1)), y = y0 + lane / kCsgX;
             const bool in = x < F && y < F;
-            // the tile's samples in voxels: its box and this lane's column
+            // the tile's samples in voxels: its box (of its own samples, each rounded as they are: from
+            // 2^24 voxels on a sum of rounded numbers could leave some outside) and this lane's column
             const float lo[3] = {(float)(x0 * cd.scale + cd.off[0]), (float)(y0 * cd.scale + cd.off[1]),
                                  (float)(z0 * cd.scale + cd.off[2])};
-            const float hi[3] = {lo[0] + (float)((kCsgX - 1) * cd.scale), lo[1] + (float)((kCsgY - 1) * cd.scale),
-                                 lo[2] + (float)((kCsgZ - 1) * cd.scale)};
+            const float hi[3] = {(float)((x0 + kCsgX - 1) * cd.scale + cd.off[0]),
+                                 (float)((y0 + kCsgY - 1) * cd.scale + cd.off[1]),
+                                 (float)((z0 + kCsgZ - 1) * cd.scale + cd.off[2])};
             const float px = (float)(x * cd.scale + cd.off[0]), py = (float)(y * cd.scale + cd.off[1]);
             unsigned settled = in ? 0u : 0xffu;  // a bit per layer
             int to[kCsgZ];

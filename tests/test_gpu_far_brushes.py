@@ -1,6 +1,7 @@
 """Brushes far from the origin, where FP32 cannot hold every voxel position: from 2^23 voxels
-on the middle of an edge is rounded to one of its ends.  Hermite data and meshes against the
-oracle bit for bit, in both forms of the brush kernel (needs a GPU)."""
+on the middle of an edge is rounded to one of its ends, and from 2^24 voxels on whole samples
+are.  Materials, hermite data and meshes against the oracle bit for bit, in both forms of the
+brush kernel (needs a GPU)."""
 import numpy as np
 import pytest
 
@@ -22,7 +23,9 @@ def _ops(n, x0, scale, seed):
 
 
 @pytest.mark.parametrize("ops", [3, 40, 100])
-@pytest.mark.parametrize("x0,lod", [((1 << 23) - 8, 0), (-(1 << 23) - 8, 0), ((1 << 23) + 1000, 0), ((1 << 23) - 16, 1)])
+@pytest.mark.parametrize("x0,lod", [((1 << 23) - 8, 0), (-(1 << 23) - 8, 0), ((1 << 23) + 1000, 0), ((1 << 23) - 16, 1),
+                                    ((1 << 24) - 8, 0), ((1 << 24) + 1003, 0), (-(1 << 25) - 77, 0), ((1 << 26) + 5, 0),
+                                    ((1 << 26) + 10, 1)])
 def test_far_brushes_match_oracle(x0, lod, ops):
     desc = workloads.heightfield_desc()
     mesher.init(desc, 2, 0)
@@ -36,7 +39,8 @@ def test_far_brushes_match_oracle(x0, lod, ops):
     assert len(ids) > 100
     ctx = mesher.Context(N)
     g = ctx.debug_stages(mn, size, brushes)
-    assert (g["edge_ids"] == ids).all()
+    assert (g["materials"] == c.materials()).all()
+    assert len(g["edge_ids"]) == len(ids) and (g["edge_ids"] == ids).all()
     assert (g["edge_data"].view(np.uint32) == data.view(np.uint32)).all()
     ctx.close()
     # the scan of more than a few chunks: this one among eight without brushes
@@ -53,3 +57,29 @@ def test_far_brushes_match_oracle(x0, lod, ops):
     assert len(t) == len(tri) > 0 and (t == tri).all()
     assert (v["pos"].view(np.uint32) == pos.view(np.uint32)).all()
     assert (v["normal"].view(np.uint32) == nrm.view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("axis,at", [(0, 28), (0, 27), (1, 25), (1, 26), (1, 27), (2, 26), (2, 27)])
+def test_far_materials_match_oracle(axis, at):
+    """Tiles of samples that round to few different positions, all air but for the brushes."""
+    desc = workloads.heightfield_desc()
+    mesher.init(desc, 2, 0)
+    mesher.clear_csg_ops()
+    ctx = mesher.Context(N)
+    solid = 0
+    for k in range(8):
+        size, vox = 4 * N, [0, 64, 0]
+        vox[axis] = (1 << at) + 16 * k + k
+        brushes, _ = workloads.make_ops(30, seed=3 * at + k, extent=N, y_range=(0.0, 16.0), size_range=(0.5, 3.0))
+        for op in brushes:
+            op["type"], op["material"] = 0, 1
+            for a in range(3):
+                op["origin"][a] = np.float32(vox[a]) + np.float32(np.round(op["origin"][a]))
+        mn = tuple(4 * v for v in vox)
+        print(f"far materials: axis={axis} at=2^{at} {k}", flush=True)
+        c = py_oracle.Chunk(N).generate(desc, py_oracle.perm_table(2), mn, size, ops=brushes)
+        g = ctx.debug_stages(mn, size, brushes)
+        assert (g["materials"] == c.materials()).all()
+        solid += int((c.materials() == 1).sum())
+    ctx.close()
+    assert solid > 0
