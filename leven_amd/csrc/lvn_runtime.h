@@ -173,10 +173,8 @@ constexpr int kDefaultPersistPerCu = 2;
 constexpr int kDefaultRowBlocks = 8192;
 constexpr int kDefaultVoxelBlocks = 8192;
 
-// Device address of pinned host memory, or null for any other memory.
-char* pinned_view(void* p);
 // A mesh in device memory into the caller's host buffers (null ones are skipped), waited
-// for: one launch on `s` when they are pinned, else copies through the runtime.
+// for: one launch on `s` when they are pinned to their ends, else copies through the runtime.
 int read_mesh(const char* verts, size_t bv, const char* tris, size_t bt, const char* seams, size_t bs, lvn_vertex* v,
               int32_t* tri, lvn_seam_node* sn, hipStream_t s);
 

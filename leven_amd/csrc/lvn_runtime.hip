@@ -611,37 +611,6 @@ static int export_mesh(Ctx* c, const MeshEntry& m, bool staged, lvn_vertex* v, i
     return LVN_OK;
 }
 
-char* pinned_view(void* p) {
-    hipPointerAttribute_t at;
-    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
-        (void)hipGetLastError();  // memory the runtime does not know
-        return nullptr;
-    }
-    return at.type == hipMemoryTypeHost ? static_cast<char*>(at.devicePointer) : nullptr;
-}
-
-int read_mesh(const char* verts, size_t bv, const char* tris, size_t bt, const char* seams, size_t bs, lvn_vertex* v,
-              int32_t* tri, lvn_seam_node* sn, hipStream_t s) {
-    MeshCopy c = {{verts, tris, seams}, {nullptr, nullptr, nullptr}, {v ? bv : 0, tri ? bt : 0, sn ? bs : 0}};
-    void* out[3] = {v, tri, sn};
-    bool pinned = true;
-    for (int i = 0; i < 3; ++i) {
-        if (!c.bytes[i]) continue;
-        c.dst[i] = pinned_view(out[i]);
-        pinned = pinned && c.dst[i] && ((uintptr_t)c.dst[i] & 3) == 0;
-    }
-    if (c.bytes[0] + c.bytes[1] + c.bytes[2] == 0) return LVN_OK;
-    if (pinned) {
-        launch_copy_mesh(c, s);
-        LVN_HIP(hipGetLastError());
-        LVN_HIP(hipStreamSynchronize(s));
-        return LVN_OK;
-    }
-    for (int i = 0; i < 3; ++i)
-        if (c.bytes[i]) LVN_HIP(hipMemcpy(out[i], c.src[i], c.bytes[i], hipMemcpyDeviceToHost));
-    return LVN_OK;
-}
-
 // The last run's counters of every staged chunk in ctx.h_counters, read once per run.
 static int count_batch(Batch* b) {
     if (b->counted) return LVN_OK;
