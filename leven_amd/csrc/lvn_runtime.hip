@@ -225,12 +225,14 @@ SlotLayout make_layout(const Geometry& G, const Caps& c, bool lines) {
     L.e_base = take((uint64_t)G.edge_rows * 8);
     L.e_ids = take((uint64_t)c.edges * 4);
     L.e_data = take((uint64_t)c.edges * 16);
-    L.e_order = take((uint64_t)c.edges * 8);
     L.h_lines = take(lines ? (uint64_t)2 * G.H * G.H * kLineStride * 4 : 0);
     L.h_cols = take((uint64_t)G.F * G.F * 4);
     L.v_mask = take((uint64_t)G.voxel_segs * 8);
     L.v_base = take((uint64_t)G.voxel_segs * 4);
     L.v_code = take((uint64_t)c.voxels * 4);
+    // From here on everything is written by the QEF and what follows it, when the crossing
+    // order is no longer read: that lies in the same bytes (6.6 MB of a 64^3 slot's 66).
+    L.e_order = o;
     L.v_emask = take((uint64_t)c.voxels * 4);
     L.v_mat = take((uint64_t)c.voxels * 4);
     L.q_count = take((uint64_t)c.seam_segs * 4);
@@ -239,6 +241,7 @@ SlotLayout make_layout(const Geometry& G, const Caps& c, bool lines) {
     L.s_mask = take((uint64_t)c.seam_segs * 8);
     L.seams = take((uint64_t)c.seams * 48);
     L.verts = take((uint64_t)c.voxels * 48);
+    o = std::max(o, align256(L.e_order + (uint64_t)c.edges * 8));
     L.slot_bytes = o;
     return L;
 }

@@ -83,8 +83,10 @@ struct SlotLayout {
     uint64_t e_rows;                      // edge_rows x {x, y, z, x = 64} words (rows with edges only)
     uint64_t e_count, e_base;             // per edge row: edges | y-edges << 16; {edges, y-edges} before it
     uint64_t e_ids, e_data;
-    uint64_t e_order;                     // {rank, id} in crossing order (y-edges first)
-    uint64_t h_lines;                     // heights at k/16 (k = 1..15) along x- and z-edge lines, 2 x H x H x 15 f32
+    uint64_t e_order;                     // {rank, id} in crossing order (y-edges first); shares its bytes with
+                                          // v_emask .. verts, which are written after the crossings
+    uint64_t h_lines;                     // heights at k/16 (k = 1..15) along x- and z-edge lines, 2 x H x H lines of
+                                          // kLineStride f32
     uint64_t h_cols;                      // the height term of each field column (x, z), F x F f32 (fresh fields)
     uint64_t v_mask, v_base, v_code, v_emask, v_mat;
     uint64_t q_count, q_base, tris;       // per 64 voxels: quads | seam nodes << 16; {quads, seam nodes} before
