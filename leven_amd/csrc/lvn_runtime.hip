@@ -1228,7 +1228,11 @@ int lvn_batch_autotune(lvn_batch* bh, int32_t reps, lvn_tuning* out) {
             int32_t pick = best.*p.field;
             float pick_ms = 0.f;
             bool first = true;
-            for (int32_t v : p.values) {
+            // the present shape (automatic or set) is timed first and given up only for a faster one
+            std::vector<int32_t> values = {pick};
+            for (int32_t v : p.values)
+                if (v != pick) values.push_back(v);
+            for (int32_t v : values) {
                 lvn_tuning cand = best;
                 cand.*p.field = v;
                 if (!valid_tuning(b, cand)) continue;
