@@ -329,82 +329,105 @@ __device__ __forceinline__ int first_dealt(int wave, int dealt, int waves) {
 // ---------------------------------------------------------------------------
 // CSG material override (CSG_HermiteIndices + BrushMaterial,
 // cl/apply_csg_operation.cl:114-140,179-210): the last op whose brush contains a sample sets
-// its material.  A wave takes a tile of 16 x 4 x 8 samples, finds the ops whose bounding
-// sphere reaches it (64 tests at a time) and walks those from the last to the first, a
-// sample being settled by the first that holds it.  Tiles of all brushed chunks are dealt
-// round the grid's waves.  (The ops one after another over each chunk, a barrier after
-// each, took 82 us for one chunk under 60 brushes and 103 us for 24 or 1,800 chunks.)
+// its material.  A wave takes a run of tiles of 16 x 4 x 8 samples along z, finds the ops whose
+// bounding sphere reaches the run's column (64 tests at a time), then those that reach a tile,
+// and walks these from the last to the first, a sample being settled by the first that holds
+// it.  Runs of all brushed chunks are dealt flat over the grid's waves: a wave reads only the
+// chunks of its own runs (when every wave went through the whole list of brushed chunks, two
+// dependent reads each, the list's length was the time where ops are few: 92 us for 124
+// chunks).  A run is one tile until every wave has two of them, then longer, so most columns
+// of a chunk under a few ops cost one test.  Bound by vector issue.  Stage times in us, ops one
+// after another over each chunk with a barrier after each / every wave through the list / this:
+// one chunk of the reference's terrain under 60 brushes 100 / 18 / 18.5, 24 such chunks 104 / 35 /
+// 27.5, its clipmap 107 / 44 / 30; 512 cave chunks under 256 brushes 34.5 / 92 / 32.5, under 1,024
+// boxes 104 / 134 / 82; the cave clipmap 35 / 61 / 28.  (2,048 workgroups: 41 us for the 512 cave
+// chunks, 37 for the 24; tiles in runs along x, tested one by one: 48 and 48.)
 // ---------------------------------------------------------------------------
 constexpr int kCsgX = 16, kCsgY = 4, kCsgZ = 8;  // 64 lanes over x and y, 8 layers each
-constexpr int kCsgBlocks = 1024;
+constexpr int kCsgBlocks = 4096;
+constexpr int kCsgRunsPerWave = 2;
+
+// Squared distance from a point's coordinate to the stretch [lo, hi].
+__device__ __forceinline__ float off_stretch(float lo, float hi, float o) {
+    const float d = fmaxf(fmaxf(lo - o, o - hi), 0.f);
+    return d * d;
+}
+
+// The tiles of column (jx, jy) from layer l0 to below l1.
+__device__ __forceinline__ void csg_run(const KArgs& a, const ChunkDesc& cd, WaveOps& list, uint8_t* mat, int jx, int jy,
+                                        int l0, int l1) {
+    const int F = a.G.F, lane = threadIdx.x & 63, n = cd.op_count;
+    const int x0 = jx * kCsgX, y0 = jy * kCsgY;
+    const int x = x0 + (lane & (kCsgX - 1)), y = y0 + lane / kCsgX;
+    // the column's sides and each tile's are positions of its own samples, rounded as these
+    // are: from 2^24 voxels on a sum of rounded numbers could leave some outside
+    const float lox = (float)(x0 * cd.scale + cd.off[0]), hix = (float)((x0 + kCsgX - 1) * cd.scale + cd.off[0]);
+    const float loy = (float)(y0 * cd.scale + cd.off[1]), hiy = (float)((y0 + kCsgY - 1) * cd.scale + cd.off[1]);
+    const float px = (float)(x * cd.scale + cd.off[0]), py = (float)(y * cd.scale + cd.off[1]);
+    float r2 = 0.f, d2 = 0.f, oz = 0.f;  // of the lane's op of the group held: reach, distance from the column
+    uint64_t reach = 0;                  // the ops of the group that reach the column
+    auto hold = [&](int g) {
+        list.hold(g);
+        const DevOp op = list.mine();
+        const float r = op.radius + 1.f;
+        r2 = r * r;
+        oz = op.oz;
+        d2 = off_stretch(lox, hix, op.ox) + off_stretch(loy, hiy, op.oy);
+        reach = __ballot(64 * g + lane < n && !(d2 > r2));
+    };
+    const int last = (n - 1) >> 6;
+    if (last == 0) {
+        hold(0);
+        if (!reach) return;
+    }
+    for (int l = l0; l < l1; ++l) {
+        const int z0 = l * kCsgZ;
+        const float loz = (float)(z0 * cd.scale + cd.off[2]), hiz = (float)((z0 + kCsgZ - 1) * cd.scale + cd.off[2]);
+        unsigned outside = x < F && y < F ? 0u : 0xffu;  // a bit per layer of samples
+        if (z0 + kCsgZ > F) outside |= 0xffu << (F - z0);
+        unsigned settled = outside;
+        int to[kCsgZ] = {};
+        for (int g = last; g >= 0; --g) {
+            if (last) hold(g);
+            uint64_t near = reach & __ballot(!(d2 + off_stretch(loz, hiz, oz) > r2));
+            while (near && __ballot((settled & 0xffu) != 0xffu)) {
+                const int b = 63 - (int)__builtin_clzll(near);
+                near &= ~(1ull << b);
+                const DevOp u = list.at(64 * g + b);
+                const int newm = u.type == 0 ? (int)(uint8_t)u.material : kAir;
+#pragma unroll
+                for (int k = 0; k < kCsgZ; ++k) {
+                    const float pz = (float)((z0 + k) * cd.scale + cd.off[2]);
+                    const bool take = !((settled >> k) & 1u) && brush_density(u, px, py, pz) <= 0.f;
+                    to[k] = take ? newm : to[k];
+                    settled |= take ? 1u << k : 0u;
+                }
+            }
+        }
+        const unsigned write = settled & ~outside;
+#pragma unroll
+        for (int k = 0; k < kCsgZ; ++k)
+            if ((write >> k) & 1u) mat[field_index(a.G, x, y, z0 + k)] = (uint8_t)to[k];
+    }
+}
 
 __global__ __launch_bounds__(256) void k_csg(KArgs a) {
     const int F = a.G.F;
-    const int lane = threadIdx.x & 63;
     const int waves = grid_waves();
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) * (int)gridDim.x + (int)blockIdx.x);
     const int tx = (F + kCsgX - 1) / kCsgX, ty = (F + kCsgY - 1) / kCsgY, tz = (F + kCsgZ - 1) / kCsgZ;
-    const int items = tx * ty * tz, lists = special_chunks(a);
-    int dealt = 0;  // items of earlier chunks, modulo the number of waves
-    for (int q = 0; q < lists; ++q) {
+    const int columns = tx * ty, lists = special_chunks(a);
+    const int runs = max(1, min(tz, (int)((long)kCsgRunsPerWave * waves / max(1, columns * lists))));
+    const int per = (tz + runs - 1) / runs;  // tiles of a run
+    const int items = columns * runs, total = lists * items;
+    for (int i = wave; i < total; i += waves) {
+        const int q = i / items, j = i - q * items;
         const int chunk = special_chunk(a, q);
-        const ChunkDesc cd = a.chunks[chunk];  // a copy: the stores below could alias it
+        const ChunkDesc cd = a.chunks[chunk];  // a copy: the stores could alias it
         if (cd.op_count == 0) continue;
-        uint8_t* mat = slot_ptr<uint8_t>(a, chunk, a.L.mat);
+        const int run = j / columns, c = j - run * columns, jy = c / tx;
         WaveOps list(a, cd);
-        for (int j = first_dealt(wave, dealt, waves); j < items; j += waves) {
-            const int jz = j / (tx * ty), jy = (j - jz * tx * ty) / tx, jx = j - (jz * ty + jy) * tx;
-            const int x0 = jx * kCsgX, y0 = jy * kCsgY, z0 = jz * kCsgZ;
-            const int x = x0 + (lane & (kCsgX - 1)), y = y0 + lane / kCsgX;
-            const bool in = x < F && y < F;
-            // the tile's samples in voxels: its box (of its own samples, each rounded as they are: from
-            // 2^24 voxels on a sum of rounded numbers could leave some outside) and this lane's column
-            const float lo[3] = {(float)(x0 * cd.scale + cd.off[0]), (float)(y0 * cd.scale + cd.off[1]),
-                                 (float)(z0 * cd.scale + cd.off[2])};
-            const float hi[3] = {(float)((x0 + kCsgX - 1) * cd.scale + cd.off[0]),
-                                 (float)((y0 + kCsgY - 1) * cd.scale + cd.off[1]),
-                                 (float)((z0 + kCsgZ - 1) * cd.scale + cd.off[2])};
-            const float px = (float)(x * cd.scale + cd.off[0]), py = (float)(y * cd.scale + cd.off[1]);
-            unsigned settled = in ? 0u : 0xffu;  // a bit per layer
-            int to[kCsgZ];
-#pragma unroll
-            for (int l = 0; l < kCsgZ; ++l) {
-                to[l] = 0;
-                if (z0 + l >= F) settled |= 1u << l;
-            }
-            const unsigned outside = settled;
-            for (int g = (cd.op_count - 1) >> 6; g >= 0; --g) {
-                list.hold(g);
-                const DevOp op = list.mine();
-                const float r = op.radius + 1.f;
-                const float o[3] = {op.ox, op.oy, op.oz};
-                float d2 = 0.f;
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    const float d = fmaxf(fmaxf(lo[c] - o[c], o[c] - hi[c]), 0.f);
-                    d2 = d2 + d * d;
-                }
-                uint64_t near = __ballot(64 * g + lane < cd.op_count && !(d2 > r * r));
-                while (near && __ballot(settled != 0xffu)) {
-                    const int b = 63 - (int)__builtin_clzll(near);
-                    near &= ~(1ull << b);
-                    const DevOp u = list.at(64 * g + b);
-                    const int newm = u.type == 0 ? (int)(uint8_t)u.material : kAir;
-#pragma unroll
-                    for (int l = 0; l < kCsgZ; ++l) {
-                        const float pz = (float)((z0 + l) * cd.scale + cd.off[2]);
-                        const bool take = !((settled >> l) & 1u) && brush_density(u, px, py, pz) <= 0.f;
-                        to[l] = take ? newm : to[l];
-                        settled |= take ? 1u << l : 0u;
-                    }
-                }
-            }
-            const unsigned write = settled & ~outside;
-#pragma unroll
-            for (int l = 0; l < kCsgZ; ++l)
-                if ((write >> l) & 1u) mat[field_index(a.G, x, y, z0 + l)] = (uint8_t)to[l];
-        }
-        dealt = (dealt + items) % waves;
+        csg_run(a, cd, list, slot_ptr<uint8_t>(a, chunk, a.L.mat), c - jy * tx, jy, run * per, min(tz, run * per + per));
     }
 }
 

@@ -81,3 +81,29 @@ def test_more_lists_than_lanes():
     mins = [(40 * size * (k % 25), (-size // 2 if k % 4 else 30 * size), 40 * size * (k // 25)) for k in range(150)]
     print(f"brush lists: {sum(c > 0 for c in counts)} of {len(counts)} chunks", flush=True)
     _check(workloads.terrain_desc(), 16, mins, size, counts, 900)
+
+
+def _stage_us(chunks, stage):
+    """The stage's time for that many 4^3 chunks under a brush each."""
+    mesher.init(workloads.heightfield_desc(), 2, 0)
+    mesher.clear_csg_ops()
+    mins = [(40 * 16 * (k % 64), -8, 40 * 16 * (k // 64)) for k in range(chunks)]
+    for k, mn in enumerate(mins):
+        mesher.store_csg_op(_ops(1, k, mn, 4, 1)[0], mn, [v + 16 for v in mn])
+    b = mesher.Batch(4, chunks)
+    b.set_chunks(mins, [16] * chunks)
+    for _ in range(5):
+        b.run_timed()
+    us = 1e3 * float(np.median([b.run_timed()[stage] for _ in range(21)]))
+    mesher.clear_csg_ops()
+    b.close()
+    return us
+
+
+@pytest.mark.parametrize("stage", ["csg"])
+def test_a_wave_reads_only_its_own_chunks(stage):
+    """Twenty times the brushed chunks, all but empty: a pass whose waves each went through the
+    whole list of them would take twenty times as long."""
+    few, many = _stage_us(60, stage), _stage_us(1200, stage)
+    print(f"brush lists: {stage} {few:.1f} us for 60 chunks, {many:.1f} us for 1,200", flush=True)
+    assert many <= 6 * few
