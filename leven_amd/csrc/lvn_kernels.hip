@@ -326,6 +326,19 @@ __device__ __forceinline__ int first_dealt(int wave, int dealt, int waves) {
     return wave >= dealt ? wave - dealt : wave - dealt + waves;
 }
 
+// The sum over this lane and those below it.
+__device__ __forceinline__ int wave_upto(int v) {
+#define LVN_UPTO(ctrl, rows) v += __builtin_amdgcn_update_dpp(0, v, ctrl, rows, 0xf, false);
+    LVN_UPTO(0x111, 0xf)  // row_shr 1, 2, 4, 8: within a row of 16
+    LVN_UPTO(0x112, 0xf)
+    LVN_UPTO(0x114, 0xf)
+    LVN_UPTO(0x118, 0xf)
+    LVN_UPTO(0x142, 0xa)  // row_bcast 15: rows 0 and 2 into 1 and 3
+    LVN_UPTO(0x143, 0xc)  // row_bcast 31: the first two rows into the others
+#undef LVN_UPTO
+    return v;
+}
+
 // ---------------------------------------------------------------------------
 // CSG material override (CSG_HermiteIndices + BrushMaterial,
 // cl/apply_csg_operation.cl:114-140,179-210): the last op whose brush contains a sample sets
@@ -1310,12 +1323,7 @@ __device__ __forceinline__ void edge_items(const KArgs& a, int chunks, int per_i
         int v = 0;
         if (c < chunks && a.chunks[c].mode != kModeCached)
             v = edge_items_y(a.counters[c], per_item) + edge_items_xz(a.counters[c], per_item);
-        int sum = v;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int u = __shfl_up(sum, off);
-            if (lane >= off) sum += u;
-        }
+        const int sum = wave_upto(v);
         if (lane == 63) wsum[wave] = sum;
         __syncthreads();
         int before = carry, all = carry;
@@ -1340,6 +1348,10 @@ __device__ __forceinline__ void edge_items(const KArgs& a, int chunks, int per_i
 // brushed 64^3 chunk of the reference's terrain meshed in 598 -> 325 us, a two-step edit of
 // a cached chunk (no field evaluation at all) in 1,104 -> 761 us, 24 chunks under 256
 // brushes staged, meshed and fetched in 1,554 -> 1,285 us.
+// A wave finds its items among 64 lists at a time, a list per lane: three reads and a scan for
+// all of them.  (Going through the lists one by one, each with two dependent reads, took 70 us
+// of 124 brushed chunks' time: crossing stage 2,075 -> 2,005 us; of 24 chunks 145 -> 137, of
+// 64 680 -> 666.)
 // Of a few chunks, those under many brushes take short items and their touched edges one by
 // one, an op per lane: 64 edges of one wave scanning 60 ops one after another were the time
 // of a one-chunk call while most of the chip was idle.  One 64^3 chunk under 60 brushes 54 us
@@ -1362,20 +1374,30 @@ __global__ __launch_bounds__(kEdgeDataThreads) void k_edge_data(KArgs a, int chu
     // waves are numbered across the workgroups, so a few items spread over the CUs
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) * (int)(gridDim.x - 1) + (int)blockIdx.x);
     const int lists = special_chunks(a);
-    int dealt = 0;  // items of earlier chunks, modulo the number of waves
-    for (int q = 0; q < lists; ++q) {
-        const int chunk = special_chunk(a, q);
-        const ChunkDesc cd = a.chunks[chunk];
-        const bool cached = cd.mode == kModeCached;
-        const bool one = kFew && cd.op_count >= kOneEdgeOps;
-        const int per = one ? kOneEdgeItem : 64;  // edges of an item
-        const int edges = a.counters[chunk].edges, items = (edges + per - 1) / per;
-        const int* ids = slot_ptr<const int>(a, chunk, a.L.e_ids);
-        float4* data = slot_ptr<float4>(a, chunk, a.L.e_data);
-        const int* oid = reinterpret_cast<const int*>(cd.old_ids);
-        const float4* odata = reinterpret_cast<const float4*>(cd.old_data);
-        WaveOps list(a, cd);
-        for (int j = first_dealt(wave, dealt, waves); j < items; j += waves) {
+    int dealt = 0;  // items of earlier lists, modulo the number of waves
+    for (int first = 0; first < lists; first += 64) {
+        // 64 lists at a time, one per lane: its chunk, edges, and the items up to and with it
+        int own_chunk = 0, own_edges = 0, own_items = 0;
+        if (first + lane < lists) {
+            own_chunk = a.special[1 + first + lane];
+            own_edges = a.counters[own_chunk].edges;
+            const int per = kFew && a.chunks[own_chunk].op_count >= kOneEdgeOps ? kOneEdgeItem : 64;
+            own_items = (own_edges + per - 1) / per;
+        }
+        const int upto = wave_upto(own_items), total = __builtin_amdgcn_readlane(upto, 63);
+        for (int t = first_dealt(wave, dealt, waves); t < total; t += waves) {
+            const int q = __popcll(__ballot(upto <= t));  // the list of item t
+            const int chunk = __builtin_amdgcn_readlane(own_chunk, q), edges = __builtin_amdgcn_readlane(own_edges, q);
+            const int j = t - (__builtin_amdgcn_readlane(upto, q) - __builtin_amdgcn_readlane(own_items, q));
+            const ChunkDesc cd = a.chunks[chunk];
+            const bool cached = cd.mode == kModeCached;
+            const bool one = kFew && cd.op_count >= kOneEdgeOps;
+            const int per = one ? kOneEdgeItem : 64;  // edges of an item
+            const int* ids = slot_ptr<const int>(a, chunk, a.L.e_ids);
+            float4* data = slot_ptr<float4>(a, chunk, a.L.e_data);
+            const int* oid = reinterpret_cast<const int*>(cd.old_ids);
+            const float4* odata = reinterpret_cast<const float4*>(cd.old_data);
+            WaveOps list(a, cd);
             const int i = per * j + lane;
             const bool in = lane < per && i < edges;
             const int id = in ? ids[i] : 0;
@@ -1417,7 +1439,7 @@ __global__ __launch_bounds__(kEdgeDataThreads) void k_edge_data(KArgs a, int chu
                 if (touched || (cached && live)) atomicAdd(&a.work[6], 1ull);
             }
         }
-        dealt = (dealt + items) % waves;
+        dealt = (dealt + total) % waves;
     }
 }
 

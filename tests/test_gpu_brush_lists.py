@@ -100,7 +100,7 @@ def _stage_us(chunks, stage):
     return us
 
 
-@pytest.mark.parametrize("stage", ["csg"])
+@pytest.mark.parametrize("stage", ["csg", "edge_cross"])
 def test_a_wave_reads_only_its_own_chunks(stage):
     """Twenty times the brushed chunks, all but empty: a pass whose waves each went through the
     whole list of them would take twenty times as long."""
