@@ -233,7 +233,9 @@ int  lvn_batch_run(lvn_batch* b);
 int  lvn_batch_wait(lvn_batch* b);
 /* Same as lvn_batch_run + wait without the graph, timing each stage with HIP events
  * on the batch stream: stage_ms[0 .. LVN_NUM_STAGES - 1] in pipeline order
- * (see lvn_batch_stage_name); n_stages >= LVN_NUM_STAGES. */
+ * (see lvn_batch_stage_name); n_stages >= LVN_NUM_STAGES.  The stages edge_rows,
+ * scan_edges and edge_compact make the voxels' rows, scan and list too, in the same
+ * launches: voxel_rows, scan_voxels and voxel_compact are always 0. */
 #define LVN_NUM_STAGES 12
 
 /* Launch shapes of the batched pipeline (no counterpart in the reference, whose

@@ -54,6 +54,8 @@ constexpr int kNumStages = LVN_NUM_STAGES;
 extern const char* const kStageNames[kNumStages];
 // Launch stage `i` (0..kNumStages-1) of the pipeline.
 void launch_stage(const KArgs& a, int chunks, int i, hipStream_t s);
+// Stages 6 to 8 launch nothing: the voxels' rows, scan and list go with the edges' (2, 3 and 4).
+constexpr bool stage_launches(int i) { return i < 6 || i > 8; }
 
 // Stage launchers: `chunks` chunk slots [0, chunks) processed by one launch each.
 void launch_density(const KArgs& a, int chunks, hipStream_t s);

@@ -2953,7 +2953,7 @@ void launch_stage(const KArgs& a, int chunks, int i, hipStream_t s) {
     case 5: launch_edge_cross(a, chunks, s); break;
     case 6:
     case 7:
-    case 8: break;  // the voxel stages run with the edges' (2, 3 and 4)
+    case 8: break;  // stage_launches
     case 9: launch_qef(a, chunks, s); break;
     case 10: launch_scan_quads_seams(a, chunks, s); break;
     default: launch_emit(a, chunks, s); break;

@@ -711,13 +711,20 @@ static int time_stages(Batch* b, const KArgs& a, float* stage_ms) {
     for (auto& e : ev) LVN_HIP(hipEventCreate(&e));
     launch_clear_counters(a, std::max(b->n, 1), c->stream);
     for (int i = 0; i < kNumStages; ++i) {
+        if (!stage_launches(i)) continue;
         LVN_HIP(hipEventRecord(ev[i], c->stream));
         if (b->n) launch_stage(a, b->n, i, c->stream);
     }
     LVN_HIP(hipEventRecord(ev[kNumStages], c->stream));
     LVN_HIP(hipEventSynchronize(ev[kNumStages]));
     LVN_HIP(hipGetLastError());
-    for (int i = 0; i < kNumStages; ++i) LVN_HIP(hipEventElapsedTime(&stage_ms[i], ev[i], ev[i + 1]));
+    for (int i = 0; i < kNumStages; ++i) {
+        stage_ms[i] = 0.f;
+        if (!stage_launches(i)) continue;
+        int next = i + 1;
+        while (next < kNumStages && !stage_launches(next)) ++next;
+        LVN_HIP(hipEventElapsedTime(&stage_ms[i], ev[i], ev[next]));
+    }
     for (auto& e : ev) LVN_HIP(hipEventDestroy(e));
     return LVN_OK;
 }
@@ -1220,7 +1227,7 @@ int lvn_batch_autotune(lvn_batch* bh, int32_t reps, lvn_tuning* out) {
             {&lvn_tuning::persistent_per_cu, {1, 2}, {5}},
             {&lvn_tuning::height_lines, {1, 2}, {5}},
             {&lvn_tuning::cross_lanes, {1, 2, 4, 8, kCrossSampleParallel}, {5}},
-            {&lvn_tuning::row_blocks, {1024, 2048, 4096, 8192, 16384, 32768}, {2, 4, 6, 8}},
+            {&lvn_tuning::row_blocks, {1024, 2048, 4096, 8192, 16384, 32768}, {2, 4}},
             {&lvn_tuning::voxel_blocks, {1024, 2048, 4096, 8192, 16384, 32768}, {9, 11}},
         };
         float ms[kNumStages];
