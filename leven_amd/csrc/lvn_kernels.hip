@@ -360,10 +360,11 @@ constexpr int kCsgX = 16, kCsgY = 4, kCsgZ = 8;  // 64 lanes over x and y, 8 lay
 constexpr int kCsgBlocks = 4096;
 constexpr int kCsgRunsPerWave = 2;
 
-// Squared distance from a point's coordinate to the stretch [lo, hi].
+// Squared distance from a point's coordinate to the stretch [lo, hi]; NaN for a coordinate that
+// is no number, which a brush's distance ignores along its axes: such a brush reaches anywhere.
 __device__ __forceinline__ float off_stretch(float lo, float hi, float o) {
     const float d = fmaxf(fmaxf(lo - o, o - hi), 0.f);
-    return d * d;
+    return d * d + (o - o);
 }
 
 // The tiles of column (jx, jy) from layer l0 to below l1.
@@ -385,7 +386,7 @@ __device__ __forceinline__ void csg_run(const KArgs& a, const ChunkDesc& cd, Wav
         const float r = op.radius + 1.f;
         r2 = r * r;
         oz = op.oz;
-        d2 = off_stretch(lox, hix, op.ox) + off_stretch(loy, hiy, op.oy);
+        d2 = off_stretch(lox, hix, op.ox) + off_stretch(loy, hiy, op.oy) + (oz - oz);
         reach = __ballot(64 * g + lane < n && !(d2 > r2));
     };
     const int last = (n - 1) >> 6;

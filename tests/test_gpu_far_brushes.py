@@ -83,3 +83,27 @@ def test_far_materials_match_oracle(axis, at):
         solid += int((c.materials() == 1).sum())
     ctx.close()
     assert solid > 0
+
+
+@pytest.mark.parametrize("axis,value", [(0, np.nan), (1, np.nan), (2, np.nan), (0, np.inf), (1, -np.inf), (2, 1e30)])
+def test_brushes_without_a_place(axis, value):
+    """A brush's distance ignores the axes along which its centre is no number."""
+    desc = workloads.heightfield_desc()
+    mesher.init(desc, 2, 0)
+    mesher.clear_csg_ops()
+    mn, size = (0, -2 * N, 0), 4 * N
+    ops = _ops(40, 0, 1, 21)
+    for k in (5, 17, 18, 33):
+        ops[k]["origin"][axis] = value
+        ops[k]["type"], ops[k]["material"] = k & 1, 2
+        ops[k]["brush"], ops[k]["rotate_y"], ops[k]["dims"][:3] = 0, 0.7 * (k & 1), 1.5
+    print(f"brushes without a place: axis={axis} {value}", flush=True)
+    c = py_oracle.Chunk(N).generate(desc, py_oracle.perm_table(2), mn, size, ops=ops).build()
+    ctx = mesher.Context(N)
+    g = ctx.debug_stages(mn, size, ops)
+    ctx.close()
+    ids, data = c.edges()
+    assert (g["materials"] == c.materials()).all()
+    assert len(ids) == len(g["edge_ids"]) and (g["edge_ids"] == ids).all()
+    same = (g["edge_data"].view(np.uint32) == data.view(np.uint32)) | (np.isnan(g["edge_data"]) & np.isnan(data))
+    assert same.all()
