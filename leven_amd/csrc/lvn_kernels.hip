@@ -1611,17 +1611,14 @@ __device__ __forceinline__ void cross_edge_group(const KArgs& a, const NoiseLds&
         if (j >= 6) continue;
         const float sx = j == 0 ? h : j == 1 ? -h : 0.f;
         const float sz = j == 4 ? h : j == 5 ? -h : 0.f;
-        float H;
-        if (j == 2 || j == 3) {
-            H = hb_known ? Hbest : height_term<kKind>(Fp, T, px, pz);
-            nh += (!hb_known && j == 2) ? 1u : 0u;
-        } else {
-            H = height_term<kKind>(Fp, T, j < 2 ? px + sx : px, j < 2 ? pz : pz + sz);
-            ++nh;
-        }
         const float qx = j < 2 ? px + sx : px;
         const float qy = j == 2 ? py + h : j == 3 ? py - h : py;
         const float qz = j >= 4 ? pz + sz : pz;
+        float H = Hbest;  // the two samples above and below lie in the arg-min sample's column
+        if (!(hb_known && (j == 2 || j == 3))) {
+            H = height_term<kKind>(Fp, T, qx, qz);
+            nh += j == 3 ? 0u : 1u;
+        }
         const float aa = qy - H;
         nc += (caves && !(aa > Fp.cave_cut)) ? 1u : 0u;
         const float val = combine<kKind>(Fp, T, aa, qx, qy, qz);
