@@ -2862,15 +2862,18 @@ void launch_compact(const KArgs& a, int chunks, hipStream_t s) {
 // Crossing stage measured at 1 / 2 / 4 / 8 lanes (us): heightfield, 8 chunks 36/33/28/25,
 // 32 chunks 52/42/35/35, 200 chunks 88/84/98/108, 500 chunks 196/198/253/302; caves, 1 chunk
 // 131/67/46/32, 8 chunks 86/87/75/74, 64 chunks 415/339/382/406, 96 chunks 501/519/594/638;
-// the reference's terrain, whose 14 octaves a term make the longest chains, 1 chunk
-// 61/51/38/22, 64 chunks 87/84/79/54, 300 chunks 151/155/181/134, 500 chunks 242/261/360/268.
+// the reference's terrain, whose 14 octaves a term make the longest chains, chunks spread over
+// its clipmap, 24 chunks 91/58/48/38, 64 chunks 91/69/58/55, 90 chunks 111/80/78/79, 120 chunks
+// 152/118/125/127, 300 chunks 290/235/268/284, 1,800 chunks 956-1,017/927-933/1,198/1,311; the
+// chunks nearest its surface, 64 chunks 206/170/171/166, 200 chunks 243/202/211/211, 400 chunks
+// 348/311/362/378.
 // Sampled coarsely, caves cross more of the edges (17,000 a chunk at voxel size 1, 170,000
 // and more at 32: 50 such chunks 2,485 us with 1 lane, 2,700 with 2), hence chunk_load.
 static long full_chunks(const Geometry& G, int load) { return std::max(1L, (long)load * G.N * G.N / 4096); }
 
 int default_cross_lanes(const Geometry& G, int field_kind, int load) {
     const long n = full_chunks(G, load);
-    if (field_kind == LVN_FIELD_LEVEN_TERRAIN) return n <= 350 ? 8 : 1;
+    if (field_kind == LVN_FIELD_LEVEN_TERRAIN) return n <= 100 ? 8 : 2;
     if (field_kind == LVN_FIELD_TERRAIN_CAVES) return n <= 10 ? 8 : n <= 80 ? 2 : 1;
     return n <= 12 ? 8 : n <= 48 ? 4 : n <= 400 ? 2 : 1;
 }
