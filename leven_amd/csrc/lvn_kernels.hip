@@ -244,7 +244,7 @@ __device__ __forceinline__ int wg_next_item(int* next, int total) {
 // kCount adds the work counters of lvn_batch_work (a separate instantiation, so
 // the timed kernels carry no counting code).
 // At most 80 SGPRs and 64 VGPRs: two 1024-thread workgroups then fit a CU (8 waves per
-// SIMD; some SGPRs spill into VGPR lanes), which the tuner takes where the pass is a
+// SIMD; 50 to 54 SGPRs spill into VGPR lanes), which the tuner takes where the pass is a
 // chain of height-term lookups per column (the reference's terrain field: 0.69 -> 0.57 ms
 // on its clipmap batch); the cave field's pass takes the same time either way.
 template <bool kCount, int kKind>
@@ -540,8 +540,10 @@ __global__ __launch_bounds__(256) void k_solid_rows(KArgs a) {
 // Edge rows by the first `edge_blocks` workgroups of a chunk, voxel rows by the others: both
 // read only the solid rows, so one launch serves both (and the kernels after it: one scan,
 // one compaction), three launches of about 5 us less for one chunk.  A row without edges
-// stores its count alone: its words are never read (the QEF and the line heights look only
-// at rows with edges), which were 70% of the 243 MB of words of a clipmap batch.
+// stores its count alone, which spares 70% of the 243 MB of words of a clipmap batch: its
+// words are whatever the slot held before.  The line heights and the lists skip such a row by
+// its count; the QEF loads the words of all four rows round a voxel, and uses a row's only for
+// an edge between corners of different sign, and such an edge is in the row.
 // Row counts are packed: edges in the low half, y-edges in the high half.
 __device__ __forceinline__ void edge_rows(const KArgs& a, int chunk, int thread, int threads) {
     const Geometry& G = a.G;
@@ -702,6 +704,9 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_rows(KArgs a) {
 // Either way a store instruction writes one contiguous stretch of the ids.  `split` waves
 // share 64 rows where a batch is too small to fill the chip.  Measured for the whole kernel:
 // 1,800 clipmap chunks 150 -> 80 us, 512 cave chunks 160 -> 118, one 64^3 chunk 11.3 -> 5.4.
+// (Dense lists are bound by their stores and lose: 1,890 coarse cave chunks of 130,000 edges
+// take 1,330 us where an edge kernel and a voxel kernel took 1,283, since a crossing order entry
+// carries its id, 8 bytes instead of 4, for the crossing kernels' sake.)
 constexpr int kDenseRow = 32;
 
 __device__ __forceinline__ int wave_sum(int v) {
@@ -2046,7 +2051,9 @@ __device__ __forceinline__ void qef_fast(const KArgs& a, int chunk, const ChunkD
 
     // The voxel's edges start at its corners, so they lie in four edge rows, (y or y + 1,
     // z or z + 1), at x and x + 1: row j's six possible edges are bits 8 j .. 8 j + 5 of
-    // `have` in list order, and first[j] is the list index of the first of them.
+    // `have` in list order, and first[j] is the list index of the first of them.  Both are
+    // meaningless for a row without edges, whose words are not written (edge_rows);
+    // no edge of emask lies in one, since emask and the rows come from the same solid bits.
     uint32_t have = 0;
     int first[4];
 #pragma unroll
@@ -2184,9 +2191,9 @@ __device__ __forceinline__ void qef_fast(const KArgs& a, int chunk, const ChunkD
 // formed about the mass point, A = sum n n^T and r = sum n (n . (p - m)) (the
 // same least-squares problem as ATb - ATA m, without its cancellation), with
 // every product split exactly by an FMA (TwoProduct) and summed with Neumaier
-// compensation.  The Jacobi pseudo-inverse runs in FP32; a vertex whose
-// condition number exceeds 1e6, or with an eigenvalue within 1e-3 (relative) of
-// the truncation thresholds 0.1 / 10, is re-solved entirely in FP64.
+// compensation.  The Jacobi pseudo-inverse runs in FP32; a vertex with an eigenvalue
+// within kThresholdWindow |A|_F of the truncation thresholds 0.1 and 10 is re-solved
+// entirely in FP64.
 // ---------------------------------------------------------------------------
 
 __device__ __forceinline__ void neumaier(float& s, float& c, float x) {
@@ -2273,7 +2280,8 @@ __device__ __forceinline__ bool near_threshold(float s, float w) {
 // qef_fast's walk of a voxel's edges, for more than one pass: the precision form walks them
 // twice instead of keeping twelve points and normals, 104 registers instead of 188 and four
 // waves per SIMD instead of two: 64 chunks 168 -> 121 us.  (qef_fast keeps its own loop: by
-// this one a lone chunk's 11 us became 18.)
+// this one a lone chunk's 11 us became 18.)  As there, `have` and `first` of a row without edges
+// are meaningless, and no edge of emask lies in one.
 struct EdgeWalk {
     uint32_t have;
     int first[4];
