@@ -72,24 +72,25 @@ def hbm_traffic(kernel, workload):
         return None
     with open(path) as f:
         data = json.load(f)
+    found = []
     for name, entries in data["kernels"].items():
         if name.split("::")[-1].split("<")[0] == kernel and "<true" not in name:
             e = max(entries, key=lambda x: x["grid"])  # the batched launch
-            return e["read_bytes"] + e["write_bytes"]
-    return None
+            found.append(e["read_bytes"] + e["write_bytes"])
+    return max(found) if found else None  # of a kernel's forms, the batch's (the others run one chunk)
 
 
-# stage -> kernels whose HBM bytes it moves (batched launch)
+# stage -> kernels whose HBM bytes it moves (batched launch); the crossing stage's by its lanes per edge
 STAGE_KERNELS = {"density": ["k_density"], "edge_rows": ["k_solid_rows", "k_rows"], "edge_compact": ["k_compact"],
-                 "edge_cross": ["k_edge_cross"], "qef": ["k_qef"], "emit": ["k_emit"]}
+                 "edge_cross": [], "qef": ["k_qef"], "emit": ["k_emit"]}
 
 
-def hbm_rates(stage_ms, workload):
+def hbm_rates(stage_ms, workload, cross_kernel="k_edge_cross"):
     """HBM GB/s of each stage against the 8 TB/s peak: the committed rocprofv3 byte counts
     per batched launch over the stage times measured in this run."""
     out = {}
     for stage, kernels in STAGE_KERNELS.items():
-        total = [hbm_traffic(k, workload) for k in kernels]
+        total = [hbm_traffic(k, workload) for k in (kernels if stage != "edge_cross" else [cross_kernel])]
         if any(t is None for t in total) or stage_ms.get(stage, 0) <= 0:
             continue
         gbs = sum(total) / (stage_ms[stage] * 1e-3) / 1e9
@@ -454,8 +455,8 @@ def batched_leg(wl, args, steps, edge_cap, voxel_cap, plain=True, keep=False):
     dom = max(("density", "edge_cross"), key=lambda k: stage_ms[k])
     # the crossing stage's kernel for the tuned lanes per edge (1, 2/4/8, 16 = sample-parallel)
     lanes = tuning.get("cross_lanes", 1) if isinstance(tuning, dict) else 1
-    dom_kernel = ("k_density" if dom == "density" else
-                  "k_edge_cross_sp" if lanes == 16 else "k_edge_cross_group" if lanes in (2, 4, 8) else "k_edge_cross")
+    cross_kernel = ("k_edge_cross_sp" if lanes == 16 else "k_edge_cross_group" if lanes in (2, 4, 8) else "k_edge_cross")
+    dom_kernel = "k_density" if dom == "density" else cross_kernel
     a_d, a_c = algorithmic_flops(n, work["edges"], desc)
     dom_flops = a_d if dom == "density" else a_c
     exec_flops = d_flops if dom == "density" else c_flops
@@ -480,7 +481,7 @@ def batched_leg(wl, args, steps, edge_cap, voxel_cap, plain=True, keep=False):
                         "launch_ms": round(stage_ms[dom], 4), "executed_flops_per_launch": int(exec_flops),
                         "executed_tflops": round(exec_flops / (stage_ms[dom] * 1e-3) / 1e12, 3)},
            "tuning": tuning}
-    hbm = hbm_rates(stage_ms, wl["name"])
+    hbm = hbm_rates(stage_ms, wl["name"], cross_kernel)
     if hbm:
         out["hbm_gbs"] = hbm
     if plain:

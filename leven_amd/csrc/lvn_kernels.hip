@@ -704,9 +704,8 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_rows(KArgs a) {
 // Either way a store instruction writes one contiguous stretch of the ids.  `split` waves
 // share 64 rows where a batch is too small to fill the chip.  Measured for the whole kernel:
 // 1,800 clipmap chunks 150 -> 80 us, 512 cave chunks 160 -> 118, one 64^3 chunk 11.3 -> 5.4.
-// (Dense lists are bound by their stores and lose: 1,890 coarse cave chunks of 130,000 edges
-// take 1,330 us where an edge kernel and a voxel kernel took 1,283, since a crossing order entry
-// carries its id, 8 bytes instead of 4, for the crossing kernels' sake.)
+// (Dense lists, bound by their stores, gain nothing: 1,890 coarse cave chunks of 136,000 edges
+// take 1,535 us, an edge kernel and a voxel kernel with 4-byte order entries took 1,525.)
 constexpr int kDenseRow = 32;
 
 __device__ __forceinline__ int wave_sum(int v) {
