@@ -256,8 +256,8 @@ typedef struct lvn_tuning {
 int lvn_batch_get_tuning(lvn_batch* b, lvn_tuning* out);
 /* Set the launch shapes (validated; the captured graph is rebuilt on the next run). */
 int lvn_batch_set_tuning(lvn_batch* b, const lvn_tuning* t);
-/* Autotuner: times candidate shapes on the staged chunks (one untimed and `reps`
- * timed passes per candidate, per-stage HIP events), one parameter at a time, keeps
+/* Autotuner: times the present shape and candidates on the staged chunks (one untimed and
+ * `reps` timed passes each, per-stage HIP events), one parameter at a time, keeps
  * the fastest for the stages each parameter drives, and writes the result to *out. */
 int lvn_batch_autotune(lvn_batch* b, int32_t reps, lvn_tuning* out);
 int  lvn_batch_run_timed(lvn_batch* b, float* stage_ms, int32_t n_stages);
