@@ -768,7 +768,7 @@ __device__ __forceinline__ void edge_compact(const KArgs& a, int chunk, int wave
     const int2* base = slot_ptr<const int2>(a, chunk, a.L.e_base);
     int* ids = slot_ptr<int>(a, chunk, a.L.e_ids);
     int2* order = slot_ptr<int2>(a, chunk, a.L.e_order);
-    const int S = G.shift, cap = a.caps.edges, ey_total = a.counters[chunk].edges_y;
+    const int S = G.shift, cap = a.caps.edges, order_cap = a.caps.order, ey_total = a.counters[chunk].edges_y;
     const int lane = threadIdx.x & 63;
     const uint64_t lt = lanemask_lt(lane);
     // rank k in id order; crossing position: y-edges first, then x and z edges
@@ -776,7 +776,7 @@ __device__ __forceinline__ void edge_compact(const KArgs& a, int chunk, int wave
         if (k < cap) {
             ids[k] = id;
             const int pos = is_y ? ky : ey_total + (k - ky);
-            if (pos < cap) order[pos] = make_int2(k, id);
+            if (pos < order_cap) order[pos] = make_int2(k, id);
         }
     };
     const int units = ((G.edge_rows + 63) >> 6) * split;
@@ -1297,6 +1297,7 @@ __device__ __forceinline__ int2 edge_of_item(const KArgs& a, int chunk, int j, i
     const int ey = min(c.edges_y, c.edges), ny = (ey + per_item - 1) / per_item;
     const int pos = j < ny ? j * per_item + e : ey + (j - ny) * per_item + e;
     if (j < ny ? pos >= ey : pos >= c.edges) return make_int2(-1, 0);
+    if (pos >= a.caps.order) return make_int2(-1, 0);  // more edges than the chunk's voxels can have: refused
     const int2 o = slot_ptr<const int2>(a, chunk, a.L.e_order)[pos];
     return (unsigned)o.x < (unsigned)c.edges ? o : make_int2(-1, 0);  // entries past a capped list are not written
 }

@@ -199,6 +199,9 @@ Caps make_caps(const Geometry& G, int edge_cap, int voxel_cap) {
     Caps c;
     c.edges = edge_cap > 0 ? std::min(edge_cap, G.edge_slots) : G.edge_slots;
     c.voxels = voxel_cap > 0 ? std::min(voxel_cap, G.voxels) : G.voxels;
+    // An active voxel has twelve edges, and 3 H^2 lie beyond the last voxels: a chunk with more
+    // edges than that has more voxels than fit and is refused for these.
+    c.order = (int)std::min<int64_t>(c.edges, 12 * (int64_t)c.voxels + 3 * G.H * G.H);
     c.quads = 3 * c.voxels;
     c.seams = c.voxels;
     c.seam_segs = (c.voxels + 63) / 64;
@@ -241,7 +244,7 @@ SlotLayout make_layout(const Geometry& G, const Caps& c, bool lines) {
     L.s_mask = take((uint64_t)c.seam_segs * 8);
     L.seams = take((uint64_t)c.seams * 48);
     L.verts = take((uint64_t)c.voxels * 48);
-    o = std::max(o, align256(L.e_order + (uint64_t)c.edges * 8));
+    o = std::max(o, align256(L.e_order + (uint64_t)c.order * 8));
     L.slot_bytes = o;
     return L;
 }

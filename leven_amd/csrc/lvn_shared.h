@@ -66,6 +66,7 @@ struct Geometry {
 // Per-slot capacities of the compacted arrays.
 struct Caps {
     int edges;     // E
+    int order;     // crossing order entries: the edges that V active voxels can have, at most E
     int voxels;    // V
     int quads;     // Q (<= 3 V)
     int seams;     // <= V

@@ -9,7 +9,10 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("voxels,edges,active,slot_bytes", [
     (64, 0, 0, 69684480), (64, 262144, 131072, 32560128), (64, 131072, 12000, 7937280), (32, 0, 0, 8956160),
-    (16, 0, 0, 1186816), (8, 0, 0, 170496), (4, 0, 0, 30720)])
+    (16, 0, 0, 1186816), (8, 0, 0, 170496), (4, 0, 0, 30720),
+    # full edge capacities with room for few voxels
+    (64, 0, 8192, 23877888), (64, 0, 1024, 22585856), (64, 262144, 4096, 9656832), (64, 65536, 512, 4292864),
+    (16, 0, 64, 460800)])
 def test_slots_of_a_budget(voxels, edges, active, slot_bytes):
     w = workloads.terrain_512()
     mesher.init(w["desc"], w["seed"], 0)
@@ -17,3 +20,39 @@ def test_slots_of_a_budget(voxels, edges, active, slot_bytes):
     s = mesher.Server(voxels, 20 * slot_bytes, 4, 1, edges, active)
     assert s.stats()["slots"] >= 20
     s.close()
+
+
+def test_chunks_of_more_edges_than_their_voxels_allow():
+    """With room for 64 voxels and for every edge, a full chunk is refused, and the chunks in
+    the slots round it are meshed as ever."""
+    w = workloads.terrain_512()
+    mesher.init(w["desc"], w["seed"], 0)
+    mesher.clear_csg_ops()
+    mins, size = [(64 * k, -64 + 40 * (k & 1) * 64, 0) for k in range(6)], 64  # every other one is sky
+    # and one under a brush of a few voxels, high in the air
+    op = workloads.make_ops(1, seed=1, spheres=1)[0][0]
+    op["type"], op["material"], op["dims"][:3] = 0, 1, 1.5
+    op["origin"][:3] = [mins[1][0] / 4 + 8, mins[1][1] / 4 + 8, 8]
+    mesher.store_csg_op(op, mins[1], [v + size for v in mins[1]])
+    full, small = mesher.Batch(16, 6), mesher.Batch(16, 6, 0, 64)
+    try:
+        for b in (full, small):
+            b.set_chunks(mins, [size] * 6)
+        for run in range(2):
+            full.run()
+            small.run()
+            want, got = full.counts(), small.counts()
+            big = want[:, 1] > 64
+            assert big.any() and (want[~big, 1] > 0).any()
+            print(f"slot size: voxels {want[:, 1].tolist()}, status {got[:, 4].tolist()}", flush=True)
+            assert (got[big, 4] != 0).all() and (got[~big, 4] == 0).all()
+            for i in range(6):
+                if big[i]:
+                    with pytest.raises(mesher.LvnError):
+                        small.get_mesh(i)
+                else:
+                    assert [a.tobytes() for a in small.get_mesh(i)] == [a.tobytes() for a in full.get_mesh(i)]
+    finally:
+        mesher.clear_csg_ops()
+        full.close()
+        small.close()
